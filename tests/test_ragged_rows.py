@@ -1,0 +1,150 @@
+"""Row kernels on rows whose length or start no 16-byte chunk divides: lengths around every edge at which the
+dispatch takes another instantiation, and rows that start at odd elements (column slices of a wider buffer),
+with guard elements behind every row that must not change."""
+import pytest
+import torch
+
+from oracle import ref_torch as R
+from tritonformer_amd import _lib
+from tritonformer_amd import kernels as K
+
+from tests.util import assert_close, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+
+
+def odd_rows(t, dev, fill=7.0):
+    """`t` (rows, n) as a view that starts at element 3 of each row of a wider buffer of odd pitch."""
+    rows, n = t.shape
+    pitch = (n + 5) | 1
+    buf = torch.full((rows, pitch), fill, dtype=t.dtype, device=dev)
+    view = buf[:, 3:3 + n]
+    view.copy_(t)
+    return buf, view
+
+
+def untouched(buf, n, fill=7.0):
+    return bool((buf[:, :3] == fill).all() and (buf[:, 3 + n:] == fill).all())
+
+
+# 64 / 128 / 256 chunks of one wave, 512 / 1024 of a workgroup: one element either side of each edge
+@pytest.mark.parametrize("d", [1, 9, 511, 513, 1023, 1025, 2047, 2048, 2049, 4095, 4096, 4097, 8191, 8192, 8193])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("add", [False, True])
+def test_layernorm_rows(d, dtype, add, dev):
+    rows = 37
+    g = torch.Generator().manual_seed(d)
+    x, res, dy, ds = (torch.randn(rows, d, generator=g).to(dtype) for _ in range(4))
+    gamma, beta = torch.randn(d, generator=g).to(dtype), torch.randn(d, generator=g).to(dtype)
+    lib, st, dt = _lib.load(), _lib.stream_ptr(), _lib.dtype_code(dtype)
+    xb, xv = odd_rows(x, dev)
+    rb, rv = odd_rows(res, dev)
+    gb, gv = odd_rows(dy, dev)
+    sb, sv = odd_rows(ds, dev)
+    yb, yv = odd_rows(torch.zeros_like(x), dev)
+    tb, tv = odd_rows(torch.zeros_like(x), dev)
+    ob, ov = odd_rows(torch.zeros_like(x), dev)
+    pb, pv = odd_rows(torch.stack([gamma, beta]), dev)
+    mean, rstd = torch.empty(rows, device=dev), torch.empty(rows, device=dev)
+    dg, db = torch.empty(d, dtype=dtype, device=dev), torch.empty(d, dtype=dtype, device=dev)
+    nb = lib.tf_layernorm_bwd_partial_bytes(rows, d)
+    part = torch.empty(nb, dtype=torch.uint8, device=dev)
+    ptr = lambda t: t.data_ptr()  # noqa: E731
+    if add:
+        _lib.check(lib.tf_add_layernorm_fwd(st, dt, dt, rows, d, ptr(xv), xv.stride(0), ptr(rv), rv.stride(0), ptr(tv),
+                                            tv.stride(0), ptr(pv[0]), ptr(pv[1]), 1e-5, ptr(yv), yv.stride(0), ptr(mean), ptr(rstd)))
+        total = (x.float() + res.float()).to(dtype)
+        assert torch.equal(tv.cpu(), total) and untouched(tb, d)
+        _lib.check(lib.tf_add_layernorm_bwd(st, dt, dt, rows, d, ptr(gv), gv.stride(0), ptr(sv), sv.stride(0), ptr(tv),
+                                            tv.stride(0), ptr(pv[0]), ptr(mean), ptr(rstd), ptr(ov), ov.stride(0), ptr(dg),
+                                            ptr(db), ptr(part), nb))
+    else:
+        total = x
+        _lib.check(lib.tf_layernorm_fwd(st, dt, dt, rows, d, ptr(xv), xv.stride(0), ptr(pv[0]), ptr(pv[1]), 1e-5, ptr(yv),
+                                        yv.stride(0), ptr(mean), ptr(rstd)))
+        _lib.check(lib.tf_layernorm_bwd(st, dt, dt, rows, d, ptr(gv), gv.stride(0), ptr(xv), xv.stride(0), ptr(pv[0]), ptr(mean),
+                                        ptr(rstd), ptr(ov), ov.stride(0), ptr(dg), ptr(db), ptr(part), nb))
+    assert untouched(yb, d) and untouched(ob, d)
+    assert_close(yv, R.layer_norm(total, gamma, beta, 1e-5), dtype, "y")
+    dx, dgr, dbr = R.layer_norm_bwd(total, gamma, dy, 1e-5)
+    # one rounding of a result of order 1 (2^-11, 2^-8); d = 1 and 9 divide by a small variance
+    scale = max(1.0, dx.abs().max().item())
+    assert_close(ov, dx + ds.float() if add else dx, dtype, "dx", atol=(2e-2 if dtype == torch.float16 else 1.5e-1) * scale)
+    lim = 1e-3 if dtype == torch.float16 else 8e-3
+    assert rel_l2(db, dbr) < lim and (d == 1 or rel_l2(dg, dgr) < lim)
+
+
+# edges of the wave-per-row kernels (4096 16-bit, 2048 fp32 elements) and of the workgroup-per-row ones
+@pytest.mark.parametrize("n", [1, 7, 513, 2047, 2049, 4097, 32767, 32769, 65535, 65537])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_softmax_rows(n, dtype, dev):
+    rows = 9
+    g = torch.Generator().manual_seed(n)
+    x = (2 * torch.randn(rows, n, generator=g)).to(dtype)
+    dy = torch.randn(rows, n, generator=g).to(dtype)
+    lib, st, dt = _lib.load(), _lib.stream_ptr(), _lib.dtype_code(dtype)
+    xb, xv = odd_rows(x, dev)
+    gb, gv = odd_rows(dy, dev)
+    yb, yv = odd_rows(torch.zeros_like(x), dev)
+    ob, ov = odd_rows(torch.zeros_like(x), dev)
+    _lib.check(lib.tf_softmax_fwd(st, dt, rows, n, xv.data_ptr(), xv.stride(0), yv.data_ptr(), yv.stride(0)))
+    _lib.check(lib.tf_softmax_bwd(st, dt, rows, n, gv.data_ptr(), gv.stride(0), yv.data_ptr(), yv.stride(0), ov.data_ptr(),
+                                  ov.stride(0)))
+    assert untouched(yb, n) and untouched(ob, n)
+    tol = {torch.float32: dict(atol=1e-6, rtol=1e-4), torch.float16: dict(atol=1e-5, rtol=4e-3),
+           torch.bfloat16: dict(atol=1e-5, rtol=2e-2)}[dtype]
+    assert_close(yv, R.softmax(x.float()), dtype, "y", **tol)
+    assert_close(ov, R.softmax_bwd(yv.detach().float().cpu(), dy.float()), dtype, "dx", atol=tol["atol"] * 10, rtol=tol["rtol"])
+
+
+# 8 / 16 / 25 chunks of 256 threads in registers (16384, 32768, 51200 entries), then the streaming forward
+@pytest.mark.parametrize("v", [1, 9, 16383, 16385, 32769, 50257, 51199, 51201, 70001])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_cross_entropy_rows(v, dtype, dev):
+    rows = 11
+    g = torch.Generator().manual_seed(v)
+    x = torch.randn(rows, v, generator=g).to(dtype)
+    lab = torch.randint(0, v, (rows,), generator=g)
+    lab[0], lab[1] = 0, v - 1
+    lib, st, dt = _lib.load(), _lib.stream_ptr(), _lib.dtype_code(dtype)
+    xb, xv = odd_rows(x, dev)
+    ob, ov = odd_rows(torch.zeros_like(x), dev)
+    fb, fv = odd_rows(torch.zeros_like(x), dev)
+    labels = lab.to(dev)
+    loss, lse = torch.empty(rows, dtype=dtype, device=dev), torch.empty(rows, device=dev)
+    gout = torch.full((rows,), 4.0, dtype=dtype, device=dev)
+    _lib.check(lib.tf_cross_entropy_fwd(st, dt, rows, v, xv.data_ptr(), xv.stride(0), 0, 0, labels.data_ptr(), loss.data_ptr(),
+                                        lse.data_ptr()))
+    _lib.check(lib.tf_cross_entropy_bwd(st, dt, rows, v, xv.data_ptr(), xv.stride(0), 0, 0, labels.data_ptr(), lse.data_ptr(),
+                                        gout.data_ptr(), 1, ov.data_ptr(), ov.stride(0), 0))
+    assert untouched(ob, v)
+    assert_close(loss, R.cross_entropy(x, lab), dtype, "loss", atol=1e-2 if dtype == torch.float16 else 6e-2)
+    assert_close(ov, R.cross_entropy_bwd(x, lab, gout.cpu()), dtype, "grad", atol=1e-3, rtol=1e-2)
+    # the forward that also writes the gradient: the same bits
+    loss2, lse2 = torch.empty_like(loss), torch.empty_like(lse)
+    _lib.check(lib.tf_cross_entropy_fwd_grad(st, dt, rows, v, xv.data_ptr(), xv.stride(0), 0, 0, labels.data_ptr(),
+                                             loss2.data_ptr(), lse2.data_ptr(), fv.data_ptr(), fv.stride(0), 0, 4.0,
+                                             gout.data_ptr()))
+    assert torch.equal(fv, ov) and torch.equal(loss, loss2) and torch.equal(lse, lse2) and untouched(fb, v)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (33, 7), (100, 255), (70, 257), (513, 1733)])
+def test_column_sums_and_relu_mask_rows(rows, cols, dev):
+    g = torch.Generator().manual_seed(cols)
+    x, act = torch.randn(rows, cols, generator=g).half(), torch.randn(rows, cols, generator=g).half()
+    lib, st, dt = _lib.load(), _lib.stream_ptr(), _lib.dtype_code(torch.float16)
+    xb, xv = odd_rows(x, dev)
+    ab, av = odd_rows(act, dev)
+    ob, ov = odd_rows(torch.zeros_like(x), dev)
+    out = torch.empty(cols, device=dev)
+    nb = lib.tf_colsum_partial_bytes(rows, cols)
+    part = torch.empty(nb, dtype=torch.uint8, device=dev)
+    _lib.check(lib.tf_colsum(st, dt, _lib.TF_F32, rows, cols, xv.data_ptr(), xv.stride(0), out.data_ptr(), part.data_ptr(), nb))
+    # sums of `rows` values of order 1 in fp32, in another order
+    assert (out.cpu() - x.double().sum(0)).abs().max() < 1e-6 * rows + 1e-6
+    _lib.check(lib.tf_relu_mask(st, dt, rows, cols, xv.data_ptr(), xv.stride(0), av.data_ptr(), av.stride(0), ov.data_ptr(),
+                                ov.stride(0)))
+    assert torch.equal(ov.cpu(), torch.where(act > 0, x, torch.zeros_like(x))) and untouched(ob, cols)
+    assert torch.equal(K.mask_grad(xv, av), ov)

@@ -1,7 +1,9 @@
 // Cross-entropy forward/backward for gfx950.  HBM-bound: the forward streams
 // each logits row once (online max / sum-of-exp in the log2 domain), the
 // backward streams it once more and writes the gradient, already multiplied by
-// the upstream per-row gradient.
+// the upstream per-row gradient.  ANY: rows of any length and alignment (a vocabulary that
+// nobody padded), in the same 16-byte chunks (struct Row in rowops.h): 4095 bf16 rows of 50257 entries
+// forward 248 -> 94 us (4.4 TB/s), backward 203 -> 181 us (4.6 TB/s) against element-wise loads.
 #include "rowops.h"
 
 namespace tfa {
@@ -53,7 +55,7 @@ struct RowMap {
   __device__ __forceinline__ int64_t at(int64_t r) const { return (r / inner) * outer + (r % inner) * ld; }
 };
 
-template <typename T, bool VEC>
+template <typename T, bool ANY>
 __global__ __launch_bounds__(kCeThreads) void ce_fwd(int V, const T* __restrict__ logits, RowMap map,
                                                       const int64_t* __restrict__ labels, T* __restrict__ loss,
                                                       float* __restrict__ lse) {
@@ -61,35 +63,27 @@ __global__ __launch_bounds__(kCeThreads) void ce_fwd(int V, const T* __restrict_
   const int64_t row = blockIdx.x;
   const T* xr = logits + map.at(row);
   MaxSum acc = {-INFINITY, 0.f};
-  if (VEC) {
-    const int nchunk = V >> 3;
-    constexpr int U = 4;  // 16-byte loads in flight per thread
-    for (int c0 = threadIdx.x; c0 < nchunk; c0 += U * kCeThreads) {
-      u32x4 raw[U];
+  const int nchunk = Row<T, ANY>::chunks(V);
+  constexpr int U = 4;  // 16-byte loads in flight per thread
+  for (int c0 = threadIdx.x; c0 < nchunk; c0 += U * kCeThreads) {
+    u32x4 raw[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (c0 + u * kCeThreads < nchunk) raw[u] = ld16_stream(xr + (c0 + u * kCeThreads) * 8);
+    for (int u = 0; u < U; ++u)
+      if (c0 + u * kCeThreads < nchunk) raw[u] = Row<T, ANY>::template load<true>(xr, c0 + u * kCeThreads, V, (T)-INFINITY);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (c0 + u * kCeThreads >= nchunk) break;
-        float v[8];
-        unpack8<T>(raw[u], v);
-        float cm = v[0];
+    for (int u = 0; u < U; ++u) {
+      if (c0 + u * kCeThreads >= nchunk) break;
+      float v[8];
+      unpack8<T>(raw[u], v);
+      float cm = v[0];
 #pragma unroll
-        for (int e = 1; e < 8; ++e) cm = fmaxf(cm, v[e]);
-        cm *= kLog2e;
-        if (cm > acc.m) { acc.s *= exp2f(acc.m - cm); acc.m = cm; }
-        float part = 0.f;
+      for (int e = 1; e < 8; ++e) cm = fmaxf(cm, v[e]);
+      cm *= kLog2e;
+      if (cm > acc.m) { acc.s *= exp2f(acc.m - cm); acc.m = cm; }
+      float part = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) part += fast_exp2(v[e] * kLog2e - acc.m);
-        acc.s += part;
-      }
-    }
-  } else {
-    for (int c = threadIdx.x; c < V; c += kCeThreads) {
-      const float t = (float)xr[c] * kLog2e;
-      if (t > acc.m) { acc.s *= exp2f(acc.m - t); acc.m = t; }
-      acc.s += exp2f(t - acc.m);
+      for (int e = 0; e < 8; ++e) part += fast_exp2(v[e] * kLog2e - acc.m);
+      acc.s += part;
     }
   }
   const MaxSum tot = block_combine(acc, smem);
@@ -108,7 +102,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_fwd(int V, const T* __restrict_
 // GRAD: the same pass also writes (softmax(row) - onehot(label)) * grad_scale to the row of
 // `dlogits` -- the row is still in registers once its log-sum-exp is known, so the gradient of
 // the loss with respect to the logits costs one write instead of a second read-and-write pass.
-template <typename T, int NCH, bool GRAD>
+template <typename T, int NCH, bool GRAD, bool ANY>
 __global__ __launch_bounds__(kCeThreads) void ce_fwd_regs(int V, const T* __restrict__ logits, RowMap map,
                                                            const int64_t* __restrict__ labels, T* __restrict__ loss,
                                                            float* __restrict__ lse, T* __restrict__ dlogits,
@@ -116,12 +110,12 @@ __global__ __launch_bounds__(kCeThreads) void ce_fwd_regs(int V, const T* __rest
   __shared__ float red[2][kCeThreads / 64];
   const int64_t row = blockIdx.x;
   const T* xr = logits + map.at(row);
-  const int nchunk = V >> 3;
+  const int nchunk = Row<T, ANY>::chunks(V);
   u32x4 raw[NCH];
 #pragma unroll
   for (int u = 0; u < NCH; ++u) {
     const int c = threadIdx.x + u * kCeThreads;
-    if (c < nchunk) raw[u] = ld16_stream(xr + c * 8);
+    if (c < nchunk) raw[u] = Row<T, ANY>::template load<true>(xr, c, V, (T)-INFINITY);
   }
   float m = -INFINITY;
 #pragma unroll
@@ -188,13 +182,13 @@ __global__ __launch_bounds__(kCeThreads) void ce_fwd_regs(int V, const T* __rest
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] *= grad_scale;
-        Chunk<T>::store(dr + c * 8, v);
+        Row<T, ANY>::store(dr, c, V, pack8<T>(v));
       }
     }
   }
 }
 
-template <typename T, bool VEC>
+template <typename T, bool ANY>
 __global__ __launch_bounds__(kCeThreads) void ce_bwd(int V, const T* __restrict__ logits, RowMap map,
                                                       const int64_t* __restrict__ labels,
                                                       const float* __restrict__ lse, const T* __restrict__ gout,
@@ -205,27 +199,19 @@ __global__ __launch_bounds__(kCeThreads) void ce_bwd(int V, const T* __restrict_
   const float l2 = lse[row] * kLog2e;
   const float g = (float)gout[row * gstride];
   const int lab = (int)labels[row];
-  if (VEC) {
-    const int nchunk = V >> 3;
-    for (int c = threadIdx.x; c < nchunk; c += kCeThreads) {
-      float v[8];
-      Chunk<T>::load_stream(xr + c * 8, v);
+  const int nchunk = Row<T, ANY>::chunks(V);
+  for (int c = threadIdx.x; c < nchunk; c += kCeThreads) {
+    float v[8];
+    unpack8<T>(Row<T, ANY>::template load<true>(xr, c, V), v);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = fast_exp2(v[e] * kLog2e - l2);
-      if ((lab >> 3) == c) {
+    for (int e = 0; e < 8; ++e) v[e] = fast_exp2(v[e] * kLog2e - l2);
+    if ((lab >> 3) == c) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] -= (e == (lab & 7)) ? 1.0f : 0.0f;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= g;
-      Chunk<T>::store(dr + c * 8, v);
+      for (int e = 0; e < 8; ++e) v[e] -= (e == (lab & 7)) ? 1.0f : 0.0f;
     }
-  } else {
-    for (int c = threadIdx.x; c < V; c += kCeThreads) {
-      float p = exp2f((float)xr[c] * kLog2e - l2);
-      if (c == lab) p -= 1.0f;
-      dr[c] = (T)(p * g);
-    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] *= g;
+    Row<T, ANY>::store(dr, c, V, pack8<T>(v));
   }
 }
 
@@ -234,17 +220,21 @@ static int ce_fwd_launch(hipStream_t st, int64_t rows, int64_t V, const void* lo
                          const int64_t* labels, void* loss, float* lse) {
   const dim3 grid((unsigned)rows), block(kCeThreads);
   const RowMap none = {0, 0, 1};
-  if (row_vectorizable<T>(logits, V, map.ld) && map.outer % 8 == 0) {
-    const int64_t per_thread = (V / 8 + kCeThreads - 1) / kCeThreads;  // 16-byte chunks per thread
-#define CE_REGS(NCH) \
-  ce_fwd_regs<T, NCH, false><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, (T*)loss, lse, nullptr, none, 0.f)
-    if (per_thread <= 8) CE_REGS(8);
-    else if (per_thread <= 16) CE_REGS(16);
-    else if (per_thread <= 25) CE_REGS(25);
-    else ce_fwd<T, true><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, (T*)loss, lse);
+  const bool vec = row_vectorizable<T>(logits, V, map.ld) && map.outer % 8 == 0;
+  const int64_t per_thread = ((V + 7) / 8 + kCeThreads - 1) / kCeThreads;  // 16-byte chunks per thread
+#define CE_ARGS ((int)V, (const T*)logits, map, labels, (T*)loss, lse, nullptr, none, 0.f)
+#define CE_REGS(NCH)                                                              \
+  do {                                                                            \
+    if (vec) ce_fwd_regs<T, NCH, false, false><<<grid, block, 0, st>>>CE_ARGS;      \
+    else ce_fwd_regs<T, NCH, false, true><<<grid, block, 0, st>>>CE_ARGS;           \
+  } while (0)
+  if (per_thread <= 8) CE_REGS(8);
+  else if (per_thread <= 16) CE_REGS(16);
+  else if (per_thread <= 25) CE_REGS(25);
+  else if (vec) ce_fwd<T, false><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, (T*)loss, lse);
+  else ce_fwd<T, true><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, (T*)loss, lse);
 #undef CE_REGS
-  } else
-    ce_fwd<T, false><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, (T*)loss, lse);
+#undef CE_ARGS
   TF_CHECK_LAUNCH();
   return TF_OK;
 }
@@ -256,34 +246,38 @@ static int ce_bwd_launch(hipStream_t st, int64_t rows, int64_t V, const void* lo
   const dim3 grid((unsigned)rows), block(kCeThreads);
   if (row_vectorizable<T>(logits, V, map.ld) && row_vectorizable<T>(dlogits, V, dmap.ld) && map.outer % 8 == 0 &&
       dmap.outer % 8 == 0)
-    ce_bwd<T, true><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, lse, (const T*)gout, gstride,
-                                            (T*)dlogits, dmap);
-  else
     ce_bwd<T, false><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, lse, (const T*)gout, gstride,
                                              (T*)dlogits, dmap);
+  else
+    ce_bwd<T, true><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, lse, (const T*)gout, gstride,
+                                            (T*)dlogits, dmap);
   TF_CHECK_LAUNCH();
   return TF_OK;
 }
 
 // Forward that also leaves (softmax - onehot) * grad_scale in dlogits: one kernel when the row fits
-// the registers of a workgroup and both matrices can be accessed in 16-byte chunks, else the forward
-// followed by the backward kernel with `scale_dev` (one value of T in device memory holding
+// the registers of a workgroup, else the forward followed by the backward kernel with `scale_dev` (one value of T in device memory holding
 // grad_scale) as the upstream gradient of every row -- the same values either way.
 template <typename T>
 static int ce_fwd_grad_launch(hipStream_t st, int64_t rows, int64_t V, const void* logits, RowMap map,
                               const int64_t* labels, void* loss, float* lse, void* dlogits, RowMap dmap,
                               float grad_scale, const void* scale_dev) {
   const dim3 grid((unsigned)rows), block(kCeThreads);
-  const int64_t per_thread = (V / 8 + kCeThreads - 1) / kCeThreads;
-  if (row_vectorizable<T>(logits, V, map.ld) && map.outer % 8 == 0 && row_vectorizable<T>(dlogits, V, dmap.ld) &&
-      dmap.outer % 8 == 0 && per_thread <= 25) {
-#define CE_REGS(NCH)                                                                                               \
-  ce_fwd_regs<T, NCH, true><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, (T*)loss, lse, (T*)dlogits, \
-                                                    dmap, grad_scale)
+  const int64_t per_thread = ((V + 7) / 8 + kCeThreads - 1) / kCeThreads;
+  if (per_thread <= 25) {
+    const bool vec = row_vectorizable<T>(logits, V, map.ld) && map.outer % 8 == 0 &&
+                     row_vectorizable<T>(dlogits, V, dmap.ld) && dmap.outer % 8 == 0;
+#define CE_ARGS ((int)V, (const T*)logits, map, labels, (T*)loss, lse, (T*)dlogits, dmap, grad_scale)
+#define CE_REGS(NCH)                                                             \
+  do {                                                                           \
+    if (vec) ce_fwd_regs<T, NCH, true, false><<<grid, block, 0, st>>>CE_ARGS;      \
+    else ce_fwd_regs<T, NCH, true, true><<<grid, block, 0, st>>>CE_ARGS;           \
+  } while (0)
     if (per_thread <= 8) CE_REGS(8);
     else if (per_thread <= 16) CE_REGS(16);
     else CE_REGS(25);
 #undef CE_REGS
+#undef CE_ARGS
     TF_CHECK_LAUNCH();
     return TF_OK;
   }

@@ -1,7 +1,10 @@
 // LayerNorm forward/backward and row softmax forward/backward for gfx950.
-// All four are HBM-bound: one wave64 owns one row, holds it in registers as
-// 16-byte chunks (chunk c of the row belongs to lane c % 64), and reduces with
-// cross-lane shuffles, so every element is read from HBM exactly once.
+// All four are HBM-bound: one wave64 (long rows: one workgroup) owns one row, holds
+// it in registers as 16-byte chunks (chunk c of the row belongs to lane c % 64), and
+// reduces with cross-lane shuffles, so every element is read from HBM exactly once.
+// ANY: rows of any length and alignment, in the same chunks (struct Row in rowops.h).  31713 rows of 1021 fp16
+// elements: LayerNorm forward 58 -> 31 us (4.2 TB/s), backward 218 -> 55 us (3.5 TB/s) against element-wise
+// loads; 4000 fp32 softmax rows of 777: 13.6 -> 7.6 and 11.8 -> 8.3 us.
 #include "rowops.h"
 
 namespace tfa {
@@ -13,12 +16,23 @@ constexpr int kRowsPerBlock = 4;  // 4 waves per workgroup, one row each
 constexpr int kLnFwdRowsPerWave = TF_LN_FWD_ROWS;  // rows a wave of the forward kernel walks (with the next one in flight)
 
 // ---------------------------------------------------------------------------
-// LayerNorm forward.  NV = 16-byte chunks per lane (row length <= NV*64*8).
+// LayerNorm forward.  WPR = waves per row: 1 (a workgroup takes four rows) or 4 (one row); NV = 16-byte
+// chunks per lane (row length <= NV * WPR * 64 * 8).
 // ---------------------------------------------------------------------------
+// sum of one value per lane over the waves of a row; `slot` alternates between consecutive uses, so that one
+// barrier per sum is enough (a slot is rewritten two sums later, behind the barrier of the sum in between)
+template <int WPR> __device__ __forceinline__ float row_sum(float v, float (*red)[4], int slot) {
+  v = wave_sum(v);
+  if constexpr (WPR == 1) return v;
+  if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (red[slot][0] + red[slot][1]) + (red[slot][2] + red[slot][3]);
+}
+
 // With ADD the normalised row is s = x + res, rounded to T and also written to `sum`
 // (the residual stream after the addition); the statistics are those of the rounded s,
 // so the result equals an addition kernel followed by the plain forward.
-template <typename T, typename TP, int NV, bool ADD>
+template <typename T, typename TP, int NV, int WPR, bool ADD, bool ANY>
 __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* __restrict__ x, int64_t ldx,
                                                    const T* __restrict__ res, int64_t ldres,
                                                    T* __restrict__ sum, int64_t ldsum,
@@ -34,28 +48,31 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
   // no contraction left to the compiler (it may fuse differently per instantiation), the fused
   // operations are spelled out.
 #pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63;
-  const int nchunk = d >> 3;
-  const int64_t stride = (int64_t)gridDim.x * kRowsPerBlock;
+  typedef Row<T, ANY> R;
+  __shared__ float red[2][4];
+  const int lane = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;  // lane within the row
+  constexpr int LANES = 64 * WPR, RPB = kRowsPerBlock / WPR;
+  const int nchunk = R::chunks(d);
+  const int64_t stride = (int64_t)gridDim.x * RPB;
   u32x4 raw_x[NV], raw_r[ADD ? NV : 1];
   auto fetch = [&](int64_t row) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = lane + i * 64;
+      const int c = lane + i * LANES;
       if (c < nchunk) {
-        raw_x[i] = ld16(x + row * ldx + c * 8);
-        if (ADD) raw_r[i] = ld16(res + row * ldres + c * 8);
+        raw_x[i] = R::load(x + row * ldx, c, d);
+        if (ADD) raw_r[i] = R::load(res + row * ldres, c, d);
       }
     }
   };
-  int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
+  int64_t row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? threadIdx.x >> 6 : 0);
   if (row < rows) fetch(row);
   for (; row < rows; row += stride) {
     float v[NV][8];
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = lane + i * 64;
+      const int c = lane + i * LANES;
       if (c < nchunk) {
         unpack8<T>(raw_x[i], v[i]);
         if (ADD) {
@@ -64,7 +81,7 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[i][e] += r[e];
           const u32x4 packed = pack8<T>(v[i]);
-          st16(sum + row * ldsum + c * 8, packed);
+          R::store(sum + row * ldsum, c, d, packed);
           unpack8<T>(packed, v[i]);
         }
 #pragma unroll
@@ -75,28 +92,37 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
       }
     }
     if (row + stride < rows) fetch(row + stride);
-    const float mean = wave_sum(s) / (float)d;
+    const float mean = row_sum<WPR>(s, red, 0) / (float)d;
     float q = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      if (lane + i * 64 < nchunk) {
+      const int c = lane + i * LANES;
+      if (c < nchunk) {
+        if (ANY && (c + 1) * 8 > d) {  // the chunk that crosses the end of the row
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float t = c * 8 + e < d ? v[i][e] - mean : 0.f;
+            q = __builtin_fmaf(t, t, q);
+          }
+          continue;
+        }
 #pragma unroll
         for (int e = 0; e < 8; ++e) { const float t = v[i][e] - mean; q = __builtin_fmaf(t, t, q); }
       }
     }
-    const float var = wave_sum(q) / (float)d;
+    const float var = row_sum<WPR>(q, red, 1) / (float)d;
     const float rstd = 1.0f / sqrtf(var + eps);
     if (lane == 0) { mean_out[row] = mean; rstd_out[row] = rstd; }
     T* yr = y + row * ldy;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = lane + i * 64;
+      const int c = lane + i * LANES;
       if (c < nchunk) {
         // (gamma and beta are fetched per row: held in registers across the rows a wave walks they
         // cost a wave of occupancy, 98 against 86 VGPRs, and the kernel 0.5 us at d = 1024)
         float g[8], b[8], o[8];
-        load8<TP>(gamma + c * 8, g);
-        load8<TP>(beta + c * 8, b);
+        load8_row<TP, ANY>(gamma, c, d, g);
+        load8_row<TP, ANY>(beta, c, d, b);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           o[e] = __builtin_fmaf((v[i][e] - mean) * rstd, g[e], b[e]);
@@ -105,13 +131,13 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
           // differently per instantiation, and the two forms differ in one element in 50 000
           asm("" : "+v"(o[e]));
         }
-        Chunk<T>::store(yr + c * 8, o);
+        R::store(yr, c, d, pack8<T>(o));
       }
     }
   }
 }
 
-// Any row length / alignment: scalar loads, three passes over the row (the
+// Rows beyond the registers of a workgroup: scalar loads, three passes over the row (the
 // second and third come from cache).
 template <typename T, typename TP, bool ADD>
 __global__ __launch_bounds__(256) void ln_fwd_any(int64_t rows, int d, const T* __restrict__ x, int64_t ldx,
@@ -151,61 +177,64 @@ __global__ __launch_bounds__(256) void ln_fwd_any(int64_t rows, int d, const T* 
 // With ADD, dsum (the gradient that reaches the normalised tensor by another
 // path, e.g. along a residual stream) is added to dx before the rounding.
 // ---------------------------------------------------------------------------
-template <typename T, typename TP, int NV, bool ADD>
+template <typename T, typename TP, int NV, int WPR, bool ADD, bool ANY>
 __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* __restrict__ dy, int64_t lddy,
                                                    const T* __restrict__ dsum, int64_t lddsum,
                                                    const T* __restrict__ x, int64_t ldx,
                                                    const TP* __restrict__ gamma, const float* __restrict__ mean,
                                                    const float* __restrict__ rstd, T* __restrict__ dx,
                                                    int64_t lddx, float* __restrict__ partial) {
-  extern __shared__ float red[];  // [4][d], and behind it [d] for gamma when G_LDS
+  typedef Row<T, ANY> R;
+  extern __shared__ float dyn[];  // WPR == 1: [4][d] for the sums of the four waves; then [d] for gamma when G_LDS
+  __shared__ float red[2][4];
   // Wide rows (NV >= 4) keep gamma in LDS as fp32 and read a chunk where it is used: held in registers its
   // 8 * NV values pushed the kernel past 256 registers, one wave per SIMD and one workgroup per CU, so that
   // the 512 workgroups of a launch ran in two turns (d = 2048: 23.4 us per launch with it, 67 MB).
   constexpr bool G_LDS = NV >= 4;
-  const int lane = threadIdx.x & 63;
+  constexpr int LANES = 64 * WPR, RPB = kRowsPerBlock / WPR;
+  const int lane = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;  // lane within the row
   const int wave = threadIdx.x >> 6;
-  const int nchunk = d >> 3;
-  float* const gam = red + 4 * d;
+  const int nchunk = R::chunks(d);
+  float* const gam = dyn + (WPR == 1 ? 4 * d : 0);
   float g[G_LDS ? 1 : NV][8], dg[NV][8], db[NV][8];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = lane + i * 64;
+    const int c = lane + i * LANES;
 #pragma unroll
     for (int e = 0; e < 8; ++e) { dg[i][e] = 0.f; db[i][e] = 0.f; }
     if constexpr (!G_LDS) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) g[i][e] = 0.f;
-      if (c < nchunk) load8<TP>(gamma + c * 8, g[i]);
+      if (c < nchunk) load8_row<TP, ANY>(gamma, c, d, g[i]);
     }
   }
   if constexpr (G_LDS) {
     for (int c = threadIdx.x; c < nchunk; c += 256) {
       float gv[8];
-      load8<TP>(gamma + c * 8, gv);
+      load8_row<TP, ANY>(gamma, c, d, gv);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) gam[c * 8 + e] = gv[e];
+      for (int e = 0; e < 8; ++e) gam[c * 8 + e] = gv[e];  // (whole chunks: the buffer is padded to them)
     }
     __syncthreads();
   }
   const float inv_d = 1.0f / (float)d;
-  const int64_t stride = (int64_t)gridDim.x * kRowsPerBlock;
+  const int64_t stride = (int64_t)gridDim.x * RPB;
   u32x4 raw_x[NV], raw_dy[NV], raw_ds[ADD ? NV : 1];
   float mu_next = 0.f, rs_next = 0.f;
   auto fetch = [&](int64_t row) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = lane + i * 64;
+      const int c = lane + i * LANES;
       if (c < nchunk) {
-        raw_x[i] = ld16(x + row * ldx + c * 8);
-        raw_dy[i] = ld16(dy + row * lddy + c * 8);
-        if (ADD) raw_ds[i] = ld16(dsum + row * lddsum + c * 8);
+        raw_x[i] = R::load(x + row * ldx, c, d);
+        raw_dy[i] = R::load(dy + row * lddy, c, d);
+        if (ADD) raw_ds[i] = R::load(dsum + row * lddsum, c, d);
       }
     }
     mu_next = mean[row];
     rs_next = rstd[row];
   };
-  int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + wave;
+  int64_t row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? wave : 0);
   if (row < rows) fetch(row);
   for (; row < rows; row += stride) {
     const float mu = mu_next, rs = rs_next;
@@ -213,7 +242,7 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = lane + i * 64;
+      const int c = lane + i * LANES;
       if (c < nchunk) {
         float xv[8], dv[8], gl[8];
         unpack8<T>(raw_x[i], xv);
@@ -222,7 +251,7 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
 #pragma unroll
         for (int e = 0; e < 8; ++e) gl[e] = G_LDS ? gam[c * 8 + e] : g[G_LDS ? 0 : i][e];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < 8; ++e) {  // (beyond the end of the row dy reads as zero: nothing reaches a sum)
           xh[i][e] = (xv[e] - mu) * rs;
           gd[i][e] = dv[e] * gl[e];
           s1 += gd[i][e] * xh[i][e];
@@ -236,12 +265,12 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
       }
     }
     if (row + stride < rows) fetch(row + stride);
-    const float c1 = wave_sum(s1) * inv_d;
-    const float c2 = wave_sum(s2) * inv_d;
+    const float c1 = row_sum<WPR>(s1, red, 0) * inv_d;
+    const float c2 = row_sum<WPR>(s2, red, 1) * inv_d;
     T* dxr = dx + row * lddx;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = lane + i * 64;
+      const int c = lane + i * LANES;
       if (c < nchunk) {
         float o[8];
 #pragma unroll
@@ -249,26 +278,37 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
           o[e] = (gd[i][e] - xh[i][e] * c1 - c2) * rs;
           if (ADD) o[e] += ds[i][e];
         }
-        Chunk<T>::store(dxr + c * 8, o);
+        R::store(dxr, c, d, pack8<T>(o));
       }
     }
   }
-  // cross-wave reduction, dgamma then dbeta, through one [4][d] LDS buffer
   float* pout = partial + (int64_t)blockIdx.x * 2 * d;
+  if constexpr (WPR > 1) {  // every column belongs to one thread of the workgroup
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = lane + i * LANES;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (c * 8 + e < d) { pout[c * 8 + e] = dg[i][e]; pout[d + c * 8 + e] = db[i][e]; }
+    }
+    return;
+  }
+  // cross-wave reduction, dgamma then dbeta, through one [4][d] LDS buffer
 #pragma unroll
   for (int which = 0; which < 2; ++which) {
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = lane + i * 64;
+      const int c = lane + i * LANES;
       if (c < nchunk) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) red[wave * d + c * 8 + e] = which ? db[i][e] : dg[i][e];
+        for (int e = 0; e < 8; ++e)
+          if (!ANY || c * 8 + e < d) dyn[wave * d + c * 8 + e] = which ? db[i][e] : dg[i][e];
       }
     }
     __syncthreads();
     for (int c = threadIdx.x; c < d; c += 256)
-      pout[which * d + c] = red[c] + red[d + c] + red[2 * d + c] + red[3 * d + c];
+      pout[which * d + c] = dyn[c] + dyn[d + c] + dyn[2 * d + c] + dyn[3 * d + c];
   }
 }
 
@@ -393,14 +433,30 @@ __global__ __launch_bounds__(256) void ln_bwd_reduce_batch(LnReduceBatch batch, 
 // ---------------------------------------------------------------------------
 // Softmax (T = f16 / bf16 / float).  NV chunks of Chunk<T>::N elements per lane.
 // ---------------------------------------------------------------------------
-template <typename T, int NV>
+template <typename T> __device__ __forceinline__ void row_floats(u32x4 raw, float (&v)[Chunk<T>::N]) {
+  if constexpr (sizeof(T) == 2) unpack8<T>(raw, v);
+  else {
+    const f32x4 f = __builtin_bit_cast(f32x4, raw);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = f[i];
+  }
+}
+template <typename T, int N> __device__ __forceinline__ u32x4 row_pack(const float (&v)[N]) {
+  if constexpr (sizeof(T) == 2) return pack8<T>(v);
+  else {
+    const f32x4 f = {v[0], v[1], v[2], v[3]};
+    return __builtin_bit_cast(u32x4, f);
+  }
+}
+
+template <typename T, int NV, bool ANY>
 __global__ __launch_bounds__(256) void softmax_fwd_vec(int64_t rows, int cols, const T* __restrict__ x,
                                                         int64_t ldx, T* __restrict__ y, int64_t ldy) {
   constexpr int N = Chunk<T>::N;
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const int nchunk = cols / N;
+  const int nchunk = Row<T, ANY>::chunks(cols);
   const T* xr = x + row * ldx;
   float v[NV][N];
   float m = -INFINITY;
@@ -408,7 +464,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_vec(int64_t rows, int cols, c
   for (int i = 0; i < NV; ++i) {
     const int c = lane + i * 64;
     if (c < nchunk) {
-      Chunk<T>::load(xr + c * N, v[i]);
+      row_floats<T>(Row<T, ANY>::load(xr, c, cols, (T)-INFINITY), v[i]);
 #pragma unroll
       for (int e = 0; e < N; ++e) m = fmaxf(m, v[i][e]);
     }
@@ -430,7 +486,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_vec(int64_t rows, int cols, c
     if (c < nchunk) {
 #pragma unroll
       for (int e = 0; e < N; ++e) v[i][e] *= inv;
-      Chunk<T>::store(yr + c * N, v[i]);
+      Row<T, ANY>::store(yr, c, cols, row_pack<T>(v[i]));
     }
   }
 }
@@ -452,7 +508,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_any(int64_t rows, int cols, c
   for (int c = lane; c < cols; c += 64) yr[c] = (T)(exp2f(((float)xr[c] - m) * kLog2e) * inv);
 }
 
-template <typename T, int NV>
+template <typename T, int NV, bool ANY>
 __global__ __launch_bounds__(256) void softmax_bwd_vec(int64_t rows, int cols, const T* __restrict__ dy,
                                                         int64_t lddy, const T* __restrict__ y, int64_t ldy,
                                                         T* __restrict__ dx, int64_t lddx) {
@@ -460,15 +516,15 @@ __global__ __launch_bounds__(256) void softmax_bwd_vec(int64_t rows, int cols, c
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const int nchunk = cols / N;
+  const int nchunk = Row<T, ANY>::chunks(cols);
   float yv[NV][N], gv[NV][N];
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = lane + i * 64;
     if (c < nchunk) {
-      Chunk<T>::load(y + row * ldy + c * N, yv[i]);
-      Chunk<T>::load(dy + row * lddy + c * N, gv[i]);
+      row_floats<T>(Row<T, ANY>::load(y + row * ldy, c, cols), yv[i]);
+      row_floats<T>(Row<T, ANY>::load(dy + row * lddy, c, cols), gv[i]);
 #pragma unroll
       for (int e = 0; e < N; ++e) s += yv[i][e] * gv[i][e];
     }
@@ -481,7 +537,7 @@ __global__ __launch_bounds__(256) void softmax_bwd_vec(int64_t rows, int cols, c
       float o[N];
 #pragma unroll
       for (int e = 0; e < N; ++e) o[e] = yv[i][e] * (gv[i][e] - s);
-      Chunk<T>::store(dx + row * lddx + c * N, o);
+      Row<T, ANY>::store(dx + row * lddx, c, cols, row_pack<T>(o));
     }
   }
 }
@@ -519,23 +575,15 @@ template <bool MAX> __device__ __forceinline__ float block_reduce16(float v, flo
   return r;
 }
 
-template <typename T> __device__ __forceinline__ void chunk_floats(u32x4 raw, float (&v)[Chunk<T>::N]) {
-  if constexpr (sizeof(T) == 2) unpack8<T>(raw, v);
-  else {
-    const f32x4 f = __builtin_bit_cast(f32x4, raw);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = f[i];
-  }
-}
 // (exponentials of non-positive arguments: v_exp_f32 as it is, without the library wrapper's range
 // handling -- results below 2^-126 become zero, which is what they round to in the sum anyway)
-template <typename T, int NV>
+template <typename T, int NV, bool ANY>
 __global__ __launch_bounds__(kLongRowThreads) void softmax_fwd_long(int cols, const T* __restrict__ x, int64_t ldx,
                                                                     T* __restrict__ y, int64_t ldy) {
   constexpr int N = Chunk<T>::N;
   __shared__ float red[32];
   const int64_t row = blockIdx.x;
-  const int nchunk = cols / N;
+  const int nchunk = Row<T, ANY>::chunks(cols);
   const T* xr = x + row * ldx;
   float v[NV][N];
   float m = -INFINITY;
@@ -543,7 +591,7 @@ __global__ __launch_bounds__(kLongRowThreads) void softmax_fwd_long(int cols, co
   for (int i = 0; i < NV; ++i) {
     const int c = threadIdx.x + i * kLongRowThreads;
     if (c < nchunk) {
-      chunk_floats<T>(ld16_stream(xr + c * N), v[i]);
+      row_floats<T>(Row<T, ANY>::template load<true>(xr, c, cols, (T)-INFINITY), v[i]);
 #pragma unroll
       for (int e = 0; e < N; ++e) m = fmaxf(m, v[i][e]);
     }
@@ -566,7 +614,7 @@ __global__ __launch_bounds__(kLongRowThreads) void softmax_fwd_long(int cols, co
     if (c < nchunk) {
 #pragma unroll
       for (int e = 0; e < N; ++e) v[i][e] *= inv;
-      Chunk<T>::store(yr + c * N, v[i]);
+      Row<T, ANY>::store(yr, c, cols, row_pack<T>(v[i]));
     }
   }
 }
@@ -574,26 +622,26 @@ __global__ __launch_bounds__(kLongRowThreads) void softmax_fwd_long(int cols, co
 // y and dy stay in registers as the raw 16-byte chunks (converted where they are used: as floats, 16-bit
 // rows would need twice the registers); with HOLD_DY false dy is read a second time instead (from the
 // cache: a row is a few hundred KB), for rows whose two operands do not fit the 128 registers of a thread.
-template <typename T, int NV, bool HOLD_DY>
+template <typename T, int NV, bool HOLD_DY, bool ANY>
 __global__ __launch_bounds__(kLongRowThreads) void softmax_bwd_long(int cols, const T* __restrict__ dy, int64_t lddy,
                                                                     const T* __restrict__ y, int64_t ldy,
                                                                     T* __restrict__ dx, int64_t lddx) {
   constexpr int N = Chunk<T>::N;
   __shared__ float red[16];
   const int64_t row = blockIdx.x;
-  const int nchunk = cols / N;
+  const int nchunk = Row<T, ANY>::chunks(cols);
   u32x4 ry[NV], rg[HOLD_DY ? NV : 1];
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = threadIdx.x + i * kLongRowThreads;
     if (c < nchunk) {
-      ry[i] = ld16_stream(y + row * ldy + c * N);
-      const u32x4 g = HOLD_DY ? ld16_stream(dy + row * lddy + c * N) : ld16(dy + row * lddy + c * N);
+      ry[i] = Row<T, ANY>::template load<true>(y + row * ldy, c, cols);
+      const u32x4 g = Row<T, ANY>::template load<HOLD_DY>(dy + row * lddy, c, cols);
       if (HOLD_DY) rg[i] = g;
       float yv[N], gv[N];
-      chunk_floats<T>(ry[i], yv);
-      chunk_floats<T>(g, gv);
+      row_floats<T>(ry[i], yv);
+      row_floats<T>(g, gv);
 #pragma unroll
       for (int e = 0; e < N; ++e) s += yv[e] * gv[e];
     }
@@ -604,11 +652,11 @@ __global__ __launch_bounds__(kLongRowThreads) void softmax_bwd_long(int cols, co
     const int c = threadIdx.x + i * kLongRowThreads;
     if (c < nchunk) {
       float yv[N], gv[N], o[N];
-      chunk_floats<T>(ry[i], yv);
-      chunk_floats<T>(HOLD_DY ? rg[i] : ld16(dy + row * lddy + c * N), gv);
+      row_floats<T>(ry[i], yv);
+      row_floats<T>(HOLD_DY ? rg[i] : Row<T, ANY>::load(dy + row * lddy, c, cols), gv);
 #pragma unroll
       for (int e = 0; e < N; ++e) o[e] = yv[e] * (gv[e] - s);
-      Chunk<T>::store(dx + row * lddx + c * N, o);
+      Row<T, ANY>::store(dx + row * lddx, c, cols, row_pack<T>(o));
     }
   }
 }
@@ -631,6 +679,19 @@ static int pick_nv(int64_t nchunk) {
   return 0;
 }
 
+// LayerNorm: 16-byte chunks per lane.  Rows of up to kLnWaveRow elements belong to one wave, longer ones (up to
+// 8192) to the four waves of a workgroup: held by one wave, a row of 4096 takes 8 chunks per lane, and the backward
+// kernel's five arrays of 64 values do not fit the registers.
+constexpr int64_t kLnWaveRow = 2048;
+static int ln_pick(int64_t nchunk) {
+  if (nchunk <= 64) return 1;
+  if (nchunk <= 128) return 2;
+  if (nchunk <= 256) return 4;
+  if (nchunk <= 512) return 2;
+  if (nchunk <= 1024) return 4;
+  return 0;
+}
+
 template <typename T, typename TP, bool ADD>
 static int ln_fwd_launch(hipStream_t st, int64_t rows, int64_t d, const void* x, int64_t ldx, const void* res,
                          int64_t ldres, void* sum, int64_t ldsum, const void* gamma, const void* beta, float eps,
@@ -638,27 +699,29 @@ static int ln_fwd_launch(hipStream_t st, int64_t rows, int64_t d, const void* x,
   const dim3 grid((unsigned)ceil_div(rows, kRowsPerBlock)), block(256);
   bool vec = row_vectorizable<T>(x, d, ldx) && row_vectorizable<T>(y, d, ldy) && aligned16(gamma) && aligned16(beta);
   if (ADD) vec = vec && row_vectorizable<T>(res, d, ldres) && row_vectorizable<T>(sum, d, ldsum);
-  const int nv = vec ? pick_nv(d / 8) : 0;
+  const int nv = ln_pick((d + 7) / 8), wpr = nv > 0 && d > kLnWaveRow ? 4 : 1;
   // the row-walking kernel: kLnFwdRowsPerWave rows per wave once there are enough rows to fill the chip
-  int64_t walkers = ceil_div(rows, kRowsPerBlock * kLnFwdRowsPerWave);
+  const int64_t rpb = kRowsPerBlock / wpr;
+  int64_t walkers = ceil_div(rows, rpb * kLnFwdRowsPerWave);
   const int64_t fill = (int64_t)device_shape().cus * 4;
-  if (walkers < fill) walkers = ceil_div(rows, kRowsPerBlock) < fill ? ceil_div(rows, kRowsPerBlock) : fill;
+  if (walkers < fill) walkers = ceil_div(rows, rpb) < fill ? ceil_div(rows, rpb) : fill;
   const dim3 wgrid((unsigned)walkers);
-#define LN_FWD(NV)                                                                                             \
-  ln_fwd_vec<T, TP, NV, ADD><<<wgrid, block, 0, st>>>(rows, (int)d, (const T*)x, ldx, (const T*)res, ldres, (T*)sum, \
-                                                     ldsum, (const TP*)gamma, (const TP*)beta, eps, (T*)y, ldy, mean, \
-                                                     rstd)
-  switch (nv) {
-    case 1: LN_FWD(1); break;
-    case 2: LN_FWD(2); break;
-    case 4: LN_FWD(4); break;
-    case 8: LN_FWD(8); break;
-    default:
-      ln_fwd_any<T, TP, ADD><<<grid, block, 0, st>>>(rows, (int)d, (const T*)x, ldx, (const T*)res, ldres, (T*)sum,
-                                                     ldsum, (const TP*)gamma, (const TP*)beta, eps, (T*)y, ldy, mean,
-                                                     rstd);
+#define LN_ARGS                                                                                                    \
+  (rows, (int)d, (const T*)x, ldx, (const T*)res, ldres, (T*)sum, ldsum, (const TP*)gamma, (const TP*)beta, eps, (T*)y, \
+   ldy, mean, rstd)
+#define LN_FWD(NV, WPR)                                                        \
+  if (vec) ln_fwd_vec<T, TP, NV, WPR, ADD, false><<<wgrid, block, 0, st>>>LN_ARGS; \
+  else ln_fwd_vec<T, TP, NV, WPR, ADD, true><<<wgrid, block, 0, st>>>LN_ARGS
+  switch (nv * 10 + wpr) {
+    case 11: LN_FWD(1, 1); break;
+    case 21: LN_FWD(2, 1); break;
+    case 41: LN_FWD(4, 1); break;
+    case 24: LN_FWD(2, 4); break;
+    case 44: LN_FWD(4, 4); break;
+    default: ln_fwd_any<T, TP, ADD><<<grid, block, 0, st>>>LN_ARGS;
   }
 #undef LN_FWD
+#undef LN_ARGS
   TF_CHECK_LAUNCH();
   return TF_OK;
 }
@@ -676,23 +739,25 @@ static int ln_bwd_launch(hipStream_t st, int64_t rows, int64_t d, const void* dy
   bool vec = row_vectorizable<T>(x, d, ldx) && row_vectorizable<T>(dy, d, lddy) && row_vectorizable<T>(dx, d, lddx) &&
              aligned16(gamma);
   if (ADD) vec = vec && row_vectorizable<T>(dsum, d, lddsum);
-  const int nv = vec ? pick_nv(d / 8) : 0;
-  const size_t lds = (size_t)(nv >= 4 ? 5 : 4) * d * sizeof(float);  // wide rows keep gamma there too
-#define LN_BWD(NV)                                                                                                \
-  ln_bwd_vec<T, TP, NV, ADD><<<dim3(parts), dim3(256), lds, st>>>(rows, (int)d, (const T*)dy, lddy, (const T*)dsum,   \
-                                                                  lddsum, (const T*)x, ldx, (const TP*)gamma, mean, \
-                                                                  rstd, (T*)dx, lddx, partial)
-  switch (nv) {
-    case 1: LN_BWD(1); break;
-    case 2: LN_BWD(2); break;
-    case 4: LN_BWD(4); break;
-    case 8: LN_BWD(8); break;
-    default:
-      ln_bwd_any<T, TP, ADD><<<dim3(parts), dim3(256), 0, st>>>(rows, (int)d, (const T*)dy, lddy, (const T*)dsum,
-                                                                lddsum, (const T*)x, ldx, (const TP*)gamma, mean,
-                                                                rstd, (T*)dx, lddx, partial);
+  const int nv = ln_pick((d + 7) / 8), wpr = nv > 0 && d > kLnWaveRow ? 4 : 1;
+  // sums of the four waves of a workgroup (not needed where they share their rows); wide rows keep gamma there too
+  const size_t lds = (size_t)((wpr == 1 ? 4 * d : 0) + (nv >= 4 ? (d + 7) / 8 * 8 : 0)) * sizeof(float);
+#define LN_ARGS                                                                                                   \
+  (rows, (int)d, (const T*)dy, lddy, (const T*)dsum, lddsum, (const T*)x, ldx, (const TP*)gamma, mean, rstd, (T*)dx, lddx, \
+   partial)
+#define LN_BWD(NV, WPR)                                                                   \
+  if (vec) ln_bwd_vec<T, TP, NV, WPR, ADD, false><<<dim3(parts), dim3(256), lds, st>>>LN_ARGS; \
+  else ln_bwd_vec<T, TP, NV, WPR, ADD, true><<<dim3(parts), dim3(256), lds, st>>>LN_ARGS
+  switch (nv * 10 + wpr) {
+    case 11: LN_BWD(1, 1); break;
+    case 21: LN_BWD(2, 1); break;
+    case 41: LN_BWD(4, 1); break;
+    case 24: LN_BWD(2, 4); break;
+    case 44: LN_BWD(4, 4); break;
+    default: ln_bwd_any<T, TP, ADD><<<dim3(parts), dim3(256), 0, st>>>LN_ARGS;
   }
 #undef LN_BWD
+#undef LN_ARGS
   TF_CHECK_LAUNCH();
   if (!dgamma) return TF_OK;  // the partial sums stay where they are, for tf_layernorm_param_grads
   ln_bwd_reduce<TP><<<dim3(ceil_div(2 * d, 16)), dim3(256), 0, st>>>(parts, (int)d, partial, (TP*)dgamma, (TP*)dbeta);
@@ -705,23 +770,32 @@ static int softmax_fwd_launch(hipStream_t st, int64_t rows, int64_t cols, const 
                               int64_t ldy) {
   const dim3 grid((unsigned)ceil_div(rows, kRowsPerBlock)), block(256);
   const bool vec = row_vectorizable<T>(x, cols, ldx) && row_vectorizable<T>(y, cols, ldy);
-  const int nv = vec ? pick_nv(cols / Chunk<T>::N) : 0;
-#define SM_FWD(NV) softmax_fwd_vec<T, NV><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)x, ldx, (T*)y, ldy)
+  const int64_t nchunk = ceil_div(cols, Chunk<T>::N);
+  const int nv = pick_nv(nchunk);
+#define SM_FWD(NV)                                                                                        \
+  if (vec) softmax_fwd_vec<T, NV, false><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)x, ldx, (T*)y, ldy); \
+  else softmax_fwd_vec<T, NV, true><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)x, ldx, (T*)y, ldy)
   switch (nv) {
     case 1: SM_FWD(1); break;
     case 2: SM_FWD(2); break;
     case 4: SM_FWD(4); break;
     case 8: SM_FWD(8); break;
     default: {
-      const int lnv = vec && rows <= 0x7fffffff ? pick_long_nv<T>(cols / Chunk<T>::N) : 0;
+      const int lnv = rows <= 0x7fffffff ? pick_long_nv<T>(nchunk) : 0;
       const dim3 lgrid((unsigned)rows), lblock(kLongRowThreads);
-      if (lnv == 4) softmax_fwd_long<T, 4><<<lgrid, lblock, 0, st>>>((int)cols, (const T*)x, ldx, (T*)y, ldy);
-      else if (lnv == 8) softmax_fwd_long<T, 8><<<lgrid, lblock, 0, st>>>((int)cols, (const T*)x, ldx, (T*)y, ldy);
-      else if (lnv == 16 && sizeof(T) == 4) softmax_fwd_long<float, 16><<<lgrid, lblock, 0, st>>>((int)cols, (const float*)x, ldx, (float*)y, ldy);
+#define SM_FWD_LONG(TT, NV)                                                                                         \
+  do {                                                                                                              \
+    if (vec) softmax_fwd_long<TT, NV, false><<<lgrid, lblock, 0, st>>>((int)cols, (const TT*)x, ldx, (TT*)y, ldy);    \
+    else softmax_fwd_long<TT, NV, true><<<lgrid, lblock, 0, st>>>((int)cols, (const TT*)x, ldx, (TT*)y, ldy);         \
+  } while (0)
+      if (lnv == 4) SM_FWD_LONG(T, 4);
+      else if (lnv == 8) SM_FWD_LONG(T, 8);
+      else if (lnv == 16 && sizeof(T) == 4) SM_FWD_LONG(float, 16);
       else softmax_fwd_any<T><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)x, ldx, (T*)y, ldy);
     }
   }
 #undef SM_FWD
+#undef SM_FWD_LONG
   TF_CHECK_LAUNCH();
   return TF_OK;
 }
@@ -732,27 +806,36 @@ static int softmax_bwd_launch(hipStream_t st, int64_t rows, int64_t cols, const 
   const dim3 grid((unsigned)ceil_div(rows, kRowsPerBlock)), block(256);
   const bool vec =
       row_vectorizable<T>(dy, cols, lddy) && row_vectorizable<T>(y, cols, ldy) && row_vectorizable<T>(dx, cols, lddx);
-  const int nv = vec ? pick_nv(cols / Chunk<T>::N) : 0;
-#define SM_BWD(NV) \
-  softmax_bwd_vec<T, NV><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)dy, lddy, (const T*)y, ldy, (T*)dx, lddx)
+  const int64_t nchunk = ceil_div(cols, Chunk<T>::N);
+  const int nv = pick_nv(nchunk);
+#define SM_ARGS (rows, (int)cols, (const T*)dy, lddy, (const T*)y, ldy, (T*)dx, lddx)
+#define SM_BWD(NV)                                                      \
+  if (vec) softmax_bwd_vec<T, NV, false><<<grid, block, 0, st>>>SM_ARGS; \
+  else softmax_bwd_vec<T, NV, true><<<grid, block, 0, st>>>SM_ARGS
   switch (nv) {
     case 1: SM_BWD(1); break;
     case 2: SM_BWD(2); break;
     case 4: SM_BWD(4); break;
     case 8: SM_BWD(8); break;
     default: {
-      const int lnv = vec && rows <= 0x7fffffff ? pick_long_nv<T>(cols / Chunk<T>::N) : 0;
+      const int lnv = rows <= 0x7fffffff ? pick_long_nv<T>(nchunk) : 0;
       const dim3 lgrid((unsigned)rows), lblock(kLongRowThreads);
-#define SM_BWD_LONG(TT, NV, HOLD) \
-  softmax_bwd_long<TT, NV, HOLD><<<lgrid, lblock, 0, st>>>((int)cols, (const TT*)dy, lddy, (const TT*)y, ldy, (TT*)dx, lddx)
+#define SM_LARGS(TT) ((int)cols, (const TT*)dy, lddy, (const TT*)y, ldy, (TT*)dx, lddx)
+#define SM_BWD_LONG(TT, NV, HOLD)                                                           \
+  do {                                                                                      \
+    if (vec) softmax_bwd_long<TT, NV, HOLD, false><<<lgrid, lblock, 0, st>>>SM_LARGS(TT);     \
+    else softmax_bwd_long<TT, NV, HOLD, true><<<lgrid, lblock, 0, st>>>SM_LARGS(TT);          \
+  } while (0)
       if (lnv == 4) SM_BWD_LONG(T, 4, true);
       else if (lnv == 8) SM_BWD_LONG(T, 8, true);
       else if (lnv == 16 && sizeof(T) == 4) SM_BWD_LONG(float, 16, false);
       else softmax_bwd_any<T><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)dy, lddy, (const T*)y, ldy, (T*)dx, lddx);
 #undef SM_BWD_LONG
+#undef SM_LARGS
     }
   }
 #undef SM_BWD
+#undef SM_ARGS
   TF_CHECK_LAUNCH();
   return TF_OK;
 }

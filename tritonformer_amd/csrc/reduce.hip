@@ -26,7 +26,7 @@ static int colsum_groups(int64_t rows, int64_t cols) {
 
 // grid (col_blocks, groups).  Thread (slice, lane32) sums 8 adjacent columns
 // over rows  group_begin + slice, + 8, ...; slices are combined through LDS.
-template <typename T, bool VEC>
+template <typename T, bool ANY>
 __global__ __launch_bounds__(256) void colsum_partial(int64_t rows, int cols, const T* __restrict__ x, int64_t ldx,
                                                        float* __restrict__ partial, int rows_per_group) {
   __shared__ float red[kCsSlices][kCsColsPerBlock];
@@ -39,20 +39,12 @@ __global__ __launch_bounds__(256) void colsum_partial(int64_t rows, int cols, co
   float acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-  if (VEC) {
-    if (col0 < cols) {
-      for (int64_t r = rbeg + slice; r < rend; r += kCsSlices) {
-        float v[8];
-        Chunk<T>::load(x + r * ldx + col0, v);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += v[e];
-      }
-    }
-  } else {
+  if (col0 < cols) {
     for (int64_t r = rbeg + slice; r < rend; r += kCsSlices) {
+      float v[8];
+      unpack8<T>(Row<T, ANY>::load(x + r * ldx, col0 / 8, cols), v);
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (col0 + e < cols) acc[e] += (float)x[r * ldx + col0 + e];
+      for (int e = 0; e < 8; ++e) acc[e] += v[e];
     }
   }
 #pragma unroll
@@ -95,30 +87,21 @@ __global__ __launch_bounds__(256) void colsum_final(int groups, int cols, const 
   }
 }
 
-template <typename T, bool VEC>
+template <typename T, bool ANY>
 __global__ __launch_bounds__(256) void relu_mask_kernel(int64_t rows, int cols, const T* __restrict__ grad,
                                                          int64_t ldg, const T* __restrict__ act, int64_t lda,
                                                          T* __restrict__ out, int64_t ldo) {
-  if (VEC) {
-    const int cpr = cols >> 3;
-    const int64_t total = rows * cpr;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-      const int64_t r = i / cpr;
-      const int c = (int)(i - r * cpr) * 8;
-      float g[8], a[8];
-      Chunk<T>::load(grad + r * ldg + c, g);
-      Chunk<T>::load(act + r * lda + c, a);
+  const int cpr = Row<T, ANY>::chunks(cols);
+  const int64_t total = rows * cpr;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+    const int64_t r = i / cpr;
+    const int c = (int)(i - r * cpr);
+    float g[8], a[8];
+    unpack8<T>(Row<T, ANY>::load(grad + r * ldg, c, cols), g);
+    unpack8<T>(Row<T, ANY>::load(act + r * lda, c, cols), a);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) g[e] = a[e] > 0.f ? g[e] : 0.f;
-      Chunk<T>::store(out + r * ldo + c, g);
-    }
-  } else {
-    const int64_t total = rows * cols;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-      const int64_t r = i / cols;
-      const int c = (int)(i - r * cols);
-      out[r * ldo + c] = (float)act[r * lda + c] > 0.f ? grad[r * ldg + c] : (T)0.f;
-    }
+    for (int e = 0; e < 8; ++e) g[e] = a[e] > 0.f ? g[e] : 0.f;
+    Row<T, ANY>::store(out + r * ldo, c, cols, pack8<T>(g));
   }
 }
 
@@ -129,9 +112,9 @@ static int colsum_launch(hipStream_t st, int64_t rows, int64_t cols, const void*
   const int rpg = (int)((rows + groups - 1) / groups);
   const dim3 grid((unsigned)ceil_div(cols, kCsColsPerBlock), (unsigned)groups), block(256);
   if (row_vectorizable<T>(x, cols, ldx))
-    colsum_partial<T, true><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)x, ldx, partial, rpg);
-  else
     colsum_partial<T, false><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)x, ldx, partial, rpg);
+  else
+    colsum_partial<T, true><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)x, ldx, partial, rpg);
   TF_CHECK_LAUNCH();
   if (out_f32) colsum_final<float><<<dim3(ceil_div(cols, 32)), block, 0, st>>>(groups, (int)cols, partial, (float*)out);
   else colsum_final<T><<<dim3(ceil_div(cols, 32)), block, 0, st>>>(groups, (int)cols, partial, (T*)out);
@@ -144,15 +127,15 @@ static int relu_mask_launch(hipStream_t st, int64_t rows, int64_t cols, const vo
                             const void* act, int64_t lda, void* out, int64_t ldo) {
   const bool vec =
       row_vectorizable<T>(grad, cols, ldg) && row_vectorizable<T>(act, cols, lda) && row_vectorizable<T>(out, cols, ldo);
-  const int64_t work = vec ? rows * (cols / 8) : rows * cols;
+  const int64_t work = rows * ((cols + 7) / 8);
   int64_t blocks = (work + 255) / 256;
   if (blocks > 256 * 32) blocks = 256 * 32;
   if (blocks < 1) blocks = 1;
   if (vec)
-    relu_mask_kernel<T, true><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(rows, (int)cols, (const T*)grad, ldg,
+    relu_mask_kernel<T, false><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(rows, (int)cols, (const T*)grad, ldg,
                                                                             (const T*)act, lda, (T*)out, ldo);
   else
-    relu_mask_kernel<T, false><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(rows, (int)cols, (const T*)grad, ldg,
+    relu_mask_kernel<T, true><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(rows, (int)cols, (const T*)grad, ldg,
                                                                              (const T*)act, lda, (T*)out, ldo);
   TF_CHECK_LAUNCH();
   return TF_OK;
