@@ -77,7 +77,7 @@ int tf_device_info(int* cus, int* xcds);
  * a fixed order by a second kernel: results are bitwise reproducible).
  * Fast path needs 16-byte aligned pointers and contiguous-dimension extents
  * and leading dimensions that are multiples of 8; anything else takes a
- * slower element-wise-load path with identical arithmetic. */
+ * slower path that stages its operands through registers, with identical arithmetic. */
 int tf_gemm(void* stream, int dtype, int layout_a, int layout_b,
             int64_t M, int64_t N, int64_t K,
             const void* A, int64_t lda, const void* B, int64_t ldb,

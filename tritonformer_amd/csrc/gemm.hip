@@ -9,8 +9,9 @@
 //    s_waitcnt); the result leaves through a wave-private LDS slab so that every
 //    global store covers whole 128-byte lines;
 //  * gemm_kernel, for anything those cannot take (ragged extents, unaligned pointers,
-//    a contraction that is not a multiple of BK): operands staged through registers
-//    with per-element predication, one barrier per step.
+//    a contraction that is not a multiple of BK): operands staged through registers in
+//    16-byte chunks at any element address, one barrier per step (4113 x 1733 x 2051 fp16:
+//    231 -> 112 us forward, 219 -> 103 and 283 -> 121 us backward against element loads).
 // Both use v_mfma_f32_32x32x16_{f16,bf16} with fp32 accumulators.
 //
 // Either operand may be stored with the contraction dimension contiguous
@@ -106,13 +107,9 @@ struct Panel {
         if (gr < rmax && gk < kend) v = ld16(ptr);
         regs[j] = v;
       } else {
-        typename Vec<T>::v8 h;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const bool ok = KMAJOR ? (gr < rmax && gk + e < kend) : (gr + e < rmax && gk < kend);
-          h[e] = ok ? ptr[e] : (T)0.f;
-        }
-        regs[j] = __builtin_bit_cast(u32x4, h);
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (gr < rmax && gk < kend) v = Row<T, true>::load(ptr, 0, KMAJOR ? kend - gk : rmax - gr);
+        regs[j] = v;
       }
     }
   }
