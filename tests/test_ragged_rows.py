@@ -148,3 +148,38 @@ def test_column_sums_and_relu_mask_rows(rows, cols, dev):
                                 ov.stride(0)))
     assert torch.equal(ov.cpu(), torch.where(act > 0, x, torch.zeros_like(x))) and untouched(ob, cols)
     assert torch.equal(K.mask_grad(xv, av), ov)
+
+
+# either side of the tile edges (128, 256) and of one, two and three 64-wide stages, alone and in slices; rows shorter
+# than a chunk; operands and result start at odd elements, what lies behind the operands' rows is NaN
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (5, 3, 63), (3, 9, 130), (129, 257, 64), (255, 130, 65), (257, 127, 129),
+                                   (130, 260, 200), (33, 300, 385)])
+@pytest.mark.parametrize("cfg,splits", [(0, 1), (1, 1), (0, 2), (1, 3)])
+@pytest.mark.parametrize("la,lb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_register_staged_gemm(m, n, k, cfg, splits, la, lb, dev):
+    dtype = torch.float16 if (m + n + k) % 2 else torch.bfloat16
+    g = torch.Generator().manual_seed(m * 1000 + n * 10 + k)
+    a, b = torch.randn(m, k, generator=g).to(dtype), torch.randn(k, n, generator=g).to(dtype)
+    bias = torch.randn(1, n, generator=g).to(dtype)
+    _, av = odd_rows(a if la == _lib.KMAJOR else a.t(), dev, float("nan"))
+    _, bv = odd_rows(b.t() if lb == _lib.KMAJOR else b, dev, float("nan"))
+    _, biasv = odd_rows(bias, dev, float("nan"))
+    diag, st, dt = _lib.load_diag(), _lib.stream_ptr(), _lib.dtype_code(dtype)
+    nb = diag.tf_diag_gemm_workspace_bytes(cfg, splits, m, n, k)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=dev)
+    exact = a.double() @ b.double()
+    sums = (a.double().abs() @ b.double().abs()) * (k * 2.0 ** -24)  # fp32 sums in any order
+    for out, with_bias, dense in ((dtype, True, False), (torch.float32, False, False), (dtype, False, True)):
+        if dense:
+            cb, cv = None, torch.zeros(m, n, dtype=out, device=dev)
+        else:
+            cb, cv = odd_rows(torch.zeros(m, n, dtype=out), dev)
+        _lib.check(diag.tf_diag_gemm(st, cfg, splits, 0, dt, _lib.dtype_code(out), la, lb, m, n, k, av.data_ptr(),
+                                     av.stride(0), bv.data_ptr(), bv.stride(0), cv.data_ptr(), cv.stride(0),
+                                     biasv.data_ptr() if with_bias else None, int(with_bias), ws.data_ptr(), nb))
+        want = (exact + bias.double()).clamp_min(0) if with_bias else exact
+        # the result's own rounding: half a unit in the last place (of the smallest normal number below it)
+        ulp = {torch.float16: (2.0 ** -11, 2.0 ** -25), torch.bfloat16: (2.0 ** -8, 1e-30), torch.float32: (2.0 ** -24, 1e-30)}[out]
+        bound = sums + (want.abs() + sums) * ulp[0] + ulp[1] + 1e-7 * with_bias
+        assert ((cv.double().cpu() - want).abs() <= bound).all()
+        assert dense or untouched(cb, n)

@@ -8,10 +8,9 @@
 //    next step and the MFMAs are interleaved by hand (bare s_barrier, explicit
 //    s_waitcnt); the result leaves through a wave-private LDS slab so that every
 //    global store covers whole 128-byte lines;
-//  * gemm_kernel, for anything those cannot take (ragged extents, unaligned pointers,
-//    a contraction that is not a multiple of BK): operands staged through registers in
-//    16-byte chunks at any element address, one barrier per step (4113 x 1733 x 2051 fp16:
-//    231 -> 112 us forward, 219 -> 103 and 283 -> 121 us backward against element loads).
+//  * gemm_reg_kernel, for anything those cannot take (ragged extents, unaligned pointers,
+//    a contraction that is not a multiple of BK): the same loop and write-out with the
+//    operands staged through registers in 16-byte chunks at any element address.
 // Both use v_mfma_f32_32x32x16_{f16,bf16} with fp32 accumulators.
 //
 // Either operand may be stored with the contraction dimension contiguous
@@ -73,239 +72,12 @@ __device__ __forceinline__ int64_t c_index(const GemmParams& p, int m, int n) {
   return (int64_t)m * p.ldc + n + (int64_t)(n / p.chunk_n) * p.chunk_skip;
 }
 
-// ---------------------------------------------------------------------------
-// One operand panel: R rows (m or n) by BK of the contraction.
-// ---------------------------------------------------------------------------
-template <typename T, int R, int BK, bool KMAJOR, int NT, bool VEC>
-struct Panel {
-  static constexpr int CPR = KMAJOR ? BK / 8 : R / 8;  // 16-byte chunks per LDS row
-  static constexpr int LROWS = KMAJOR ? R : BK;        // LDS rows
-  static constexpr int NCHUNK = LROWS * CPR;
-  static constexpr int PER_THREAD = NCHUNK / NT;
-  static constexpr int BYTES = NCHUNK * 16;
-  static_assert(NCHUNK % NT == 0, "panel must divide evenly over the workgroup");
-  static_assert(KMAJOR ? (CPR == 4 || CPR == 8) : (CPR >= 16), "unsupported panel shape");
-
-  // chunk-index swizzle; an involution on c for a fixed LDS row
-  static __device__ __forceinline__ int swz(int lrow, int c) {
-    if constexpr (KMAJOR) return c ^ ((lrow / (16 / CPR)) % CPR);
-    else return c ^ ((lrow & 3) << 2);
-  }
-
-  // Global -> registers.  (row0, rmax) bound the m/n index, (k0, kend) the contraction.
-  static __device__ __forceinline__ void fetch(u32x4 (&regs)[PER_THREAD], const T* __restrict__ base, int64_t ld,
-                                               int row0, int rmax, int k0, int kend) {
-#pragma unroll
-    for (int j = 0; j < PER_THREAD; ++j) {
-      const int id = threadIdx.x + j * NT;
-      const int lrow = id / CPR, c = id % CPR;
-      const int gr = KMAJOR ? row0 + lrow : row0 + c * 8;  // m/n index of the chunk's first element
-      const int gk = KMAJOR ? k0 + c * 8 : k0 + lrow;      // contraction index of the first element
-      const T* ptr = KMAJOR ? base + (int64_t)gr * ld + gk : base + (int64_t)gk * ld + gr;
-      if (VEC) {
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (gr < rmax && gk < kend) v = ld16(ptr);
-        regs[j] = v;
-      } else {
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (gr < rmax && gk < kend) v = Row<T, true>::load(ptr, 0, KMAJOR ? kend - gk : rmax - gr);
-        regs[j] = v;
-      }
-    }
-  }
-
-  static __device__ __forceinline__ void commit(char* lds, const u32x4 (&regs)[PER_THREAD]) {
-#pragma unroll
-    for (int j = 0; j < PER_THREAD; ++j) {
-      const int id = threadIdx.x + j * NT;
-      const int lrow = id / CPR, c = id % CPR;
-      lds_st16(lds, (lrow * CPR + swz(lrow, c)) * 16, regs[j]);
-    }
-  }
-
-  // MFMA operand for the 32 rows starting at rb, contraction step ks (16 wide):
-  // lane l gets elements (row rb + l%32, k = ks*16 + (l/32)*8 + 0..7).
-  static __device__ __forceinline__ typename Vec<T>::v8 frag(const char* lds, int rb, int ks, int lane) {
-    if (KMAJOR) {
-      const int row = rb + (lane & 31);
-      const int c = ks * 2 + (lane >> 5);
-      return __builtin_bit_cast(typename Vec<T>::v8, lds_ld16(lds, (row * CPR + swz(row, c)) * 16));
-    } else {
-      const int i = lane & 15;
-      const int col = rb + 16 * ((lane >> 4) & 1) + (i & 3) * 4;
-      const int kk0 = ks * 16 + 8 * (lane >> 5) + (i >> 2);
-      const int kk1 = kk0 + 4;
-      const u32x2 lo = lds_ld8_tr(lds, (kk0 * CPR + swz(kk0, col >> 3)) * 16 + (col & 7) * 2);
-      const u32x2 hi = lds_ld8_tr(lds, (kk1 * CPR + swz(kk1, col >> 3)) * 16 + (col & 7) * 2);
-      u32x4 v = {lo[0], lo[1], hi[0], hi[1]};
-      return __builtin_bit_cast(typename Vec<T>::v8, v);
-    }
-  }
-};
-
 // Round-robin XCD dispatch -> compact per-XCD ranges, then grouped raster.
 __device__ __forceinline__ int remap_xcd(int pid, int n, int X) {
   const int xcd = pid % X, local = pid / X;
   const int q = n / X, r = n % X;
   return xcd * q + (xcd < r ? xcd : r) + local;
 }
-
-// Epilogue shared by both kernels: lane holds C[m][n .. n+3] for m = .. + lane%32.
-template <typename T, int TM, int TN, int WTM, int WTN, bool VEC>
-__device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x16 (&acc)[TM][TN], int m0, int n0, int wm,
-                                              int wn, int lane, int split) {
-  const T* bias = (const T*)p.bias;
-  T* C = (T*)p.C;
-  const float alpha = (p.alpha && p.splits <= 1) ? *p.alpha : 1.f;  // a split contraction is scaled by its reduce pass
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + wm * WTM + i * 32 + (lane & 31);
-    if (m >= p.M) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn * WTN + j * 32 + g * 8 + (lane >> 5) * 4;
-        if (n >= p.N) continue;
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][g * 4 + e] * alpha;
-        if (p.splits > 1) {
-          float* dst = p.partial + ((int64_t)split * p.M + m) * p.N + n;
-          if (VEC) {
-            f32x4 o = {v[0], v[1], v[2], v[3]};
-            *reinterpret_cast<f32x4*>(dst) = o;
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n + e < p.N) dst[e] = v[e];
-          }
-        } else {
-          if (p.mask) {
-            const T* mk = (const T*)p.mask + (int64_t)m * p.ldmask + n;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n + e < p.N && !((float)mk[e] > 0.f)) v[e] = 0.f;  // no bias / ReLU with a mask (host check)
-          }
-          if (p.out_f32) {
-            float* Cf = reinterpret_cast<float*>(p.C) + c_index(p, m, n);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              if (n + e < p.N) {
-                const float x = v[e] + (bias ? (float)bias[n + e] : 0.f);
-                Cf[e] = p.relu ? fmaxf(x, 0.f) : x;
-              }
-            }
-          } else if (VEC) {
-            typename Vec<T>::v4 o;
-            if (bias) {
-              const typename Vec<T>::v4 bv = *reinterpret_cast<const typename Vec<T>::v4*>(bias + n);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) v[e] += (float)bv[e];
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = (T)(p.relu ? fmaxf(v[e], 0.f) : v[e]);
-            *reinterpret_cast<typename Vec<T>::v4*>(C + c_index(p, m, n)) = o;
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              if (n + e < p.N) {
-                float x = v[e] + (bias ? (float)bias[n + e] : 0.f);
-                C[c_index(p, m, n) + e] = (T)(p.relu ? fmaxf(x, 0.f) : x);
-              }
-            }
-          }
-        }
-      }
-    }
-  }
-}
-
-template <typename T, int BM, int BN, int BK, int WM, int WN, bool A_KMAJOR, bool B_KMAJOR, bool VEC>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(GemmParams p) {
-  constexpr int NT = WM * WN * 64;
-  constexpr int WTM = BM / WM, WTN = BN / WN;  // wave tile
-  constexpr int TM = WTM / 32, TN = WTN / 32;  // MFMA tiles per wave
-  constexpr int GROUP_M = 8;
-  typedef Panel<T, BM, BK, A_KMAJOR, NT, VEC> PA;
-  typedef Panel<T, BN, BK, B_KMAJOR, NT, VEC> PB;
-  typedef typename Vec<T>::v8 v8;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-
-  // ---- which tile / which slice of the contraction -------------------------
-  const int tiles = p.tiles_m * p.tiles_n;
-  const int pid = (p.flags & 1) ? (int)blockIdx.x : remap_xcd(blockIdx.x, tiles * p.splits, p.xcds);
-  const int split = pid / tiles;
-  const int t = pid - split * tiles;
-  const int per_group = GROUP_M * p.tiles_n;
-  const int group = t / per_group;
-  const int first_m = group * GROUP_M;
-  const int gsz = min(p.tiles_m - first_m, GROUP_M);
-  const int tm = first_m + (t % per_group) % gsz;
-  const int tn = (t % per_group) / gsz;
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int kbeg = split * p.k_per_split;
-  const int kend = min(p.K, kbeg + p.k_per_split);
-  const int nk = (kend - kbeg + BK - 1) / BK;
-
-  const T* A = (const T*)p.A;
-  const T* B = (const T*)p.B;
-
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  u32x4 ra[PA::PER_THREAD], rb[PB::PER_THREAD];
-  constexpr int STAGE = PA::BYTES + PB::BYTES;
-
-  if (nk > 0) {
-    PA::fetch(ra, A, p.lda, m0, p.M, kbeg, kend);
-    PB::fetch(rb, B, p.ldb, n0, p.N, kbeg, kend);
-    PA::commit(smem, ra);
-    PB::commit(smem + PA::BYTES, rb);
-  }
-  __syncthreads();
-
-  for (int kt = 0; kt < nk; ++kt) {
-    const char* sa = smem + (kt & 1) * STAGE;
-    const char* sb = sa + PA::BYTES;
-    const bool more = kt + 1 < nk;
-    if (more) {
-      const int k0 = kbeg + (kt + 1) * BK;
-      PA::fetch(ra, A, p.lda, m0, p.M, k0, kend);
-      PB::fetch(rb, B, p.ldb, n0, p.N, k0, kend);
-    }
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      v8 fa[TM], fb[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) fa[i] = PA::frag(sa, wm * WTM + i * 32, ks, lane);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) fb[j] = PB::frag(sb, wn * WTN + j * 32, ks, lane);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma32(fb[j], fa[i], acc[i][j]);
-    }
-    if (more) {
-      char* da = smem + ((kt + 1) & 1) * STAGE;
-      PA::commit(da, ra);
-      PB::commit(da + PA::BYTES, rb);
-    }
-    __syncthreads();
-  }
-
-  gemm_epilogue<T, TM, TN, WTM, WTN, VEC>(p, acc, m0, n0, wm, wn, lane, split);
-}
-
 
 // ---------------------------------------------------------------------------
 // Fast path: HBM -> LDS directly (global_load_lds_dwordx4, no VGPR round trip),
@@ -387,9 +159,6 @@ struct DmaPanel {
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) ptrs[j] += KMAJOR ? (int64_t)BK : (int64_t)BK * ld;
   }
-  static __device__ __forceinline__ typename Vec<T>::v8 frag(const char* lds, int rb, int ks, int lane) {
-    return Panel<T, R, BK, KMAJOR, 64, true>::frag(lds, rb, ks, lane);
-  }
   static constexpr int READS_PER_FRAG = KMAJOR ? 1 : 2;
   // Same operand as frag(), read with volatile asm from the panel at LDS byte address `base`.
   static __device__ __forceinline__ void frag_issue(FragRegs<KMAJOR>& f, uint32_t base, int rb, int ks, int lane) {
@@ -418,7 +187,9 @@ struct DmaPanel {
 // tile) instead of 32 scattered 16-byte pieces.
 // PLAIN: the caller knows that there is no bias, ReLU, mask or sign-bit work (most launches of a
 // training step): the write-out is then straight-line code without the tests for them.
-template <typename T, typename TO, int TM, int TN, int WTM, int WTN, bool PLAIN = false, bool FULL = false>
+// ANY: rows of C, the bias and the mask start at any element and N is any number (register-staged kernel):
+// the same 16-byte accesses at element alignment, the chunk that crosses the end of a row by elements.
+template <typename T, typename TO, int TM, int TN, int WTM, int WTN, bool PLAIN = false, bool FULL = false, bool ANY = false>
 __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&acc)[TM][TN], char* smem, int m0,
                                                   int n0, int wm, int wn, int wave, int lane,
                                                   const uint8_t (*sign_bytes)[4] = nullptr) {
@@ -451,7 +222,13 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int nl = j * 32 + g * 8 + (lane >> 5) * 4;
-        if (nbase + nl < p.N) bvals[j][g] = *reinterpret_cast<const typename Vec<T>::v4*>(bias + nbase + nl);
+        if constexpr (ANY) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (nbase + nl + e < p.N) bvals[j][g][e] = bias[nbase + nl + e];
+        } else {
+          if (nbase + nl < p.N) bvals[j][g] = *reinterpret_cast<const typename Vec<T>::v4*>(bias + nbase + nl);
+        }
       }
   }
 #pragma unroll
@@ -501,7 +278,20 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
       if (FULL || (m < p.M && n < p.N)) {
         if (mask) {  // ReLU gradient mask fused into the write-out: zero where the activation is not positive
           const T* mk = (const T*)mask + (int64_t)m * p.ldmask + n;
-          if constexpr (ES == 2) {
+          if constexpr (ES == 2 && ANY) {
+            const typename Vec<T>::v8 mv = __builtin_bit_cast(typename Vec<T>::v8, Row<T, true>::load(mk, 0, p.N - n));
+            typename Vec<T>::v8 cv = __builtin_bit_cast(typename Vec<T>::v8, val);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (!((float)mv[e] > 0.f)) cv[e] = (T)0.f;
+            val = __builtin_bit_cast(u32x4, cv);
+          } else if constexpr (ANY) {
+            f32x4 cv = __builtin_bit_cast(f32x4, val);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < p.N && !((float)mk[e] > 0.f)) cv[e] = 0.f;
+            val = __builtin_bit_cast(u32x4, cv);
+          } else if constexpr (ES == 2) {
             const typename Vec<T>::v8 mv = __builtin_bit_cast(typename Vec<T>::v8, ld16(mk));
             typename Vec<T>::v8 cv = __builtin_bit_cast(typename Vec<T>::v8, val);
 #pragma unroll
@@ -517,7 +307,7 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
             val = __builtin_bit_cast(u32x4, cv);
           }
         }
-        if (sign_in) {  // the same mask from one bit per element
+        if (!ANY && sign_in) {  // the same mask from one bit per element
           unsigned bits;
           if constexpr (ES == 2) bits = sign_bytes[i][rr];  // requested before the main loop
           else bits = ((const uint8_t*)sign_in)[(int64_t)m * p.ldsign + (n >> 3)] >> (n & 7);
@@ -536,7 +326,7 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
           }
         }
         if constexpr (ES == 2) {
-          if (sign_out) {  // a chunk is 8 elements: one byte
+          if (!ANY && sign_out) {  // a chunk is 8 elements: one byte
             const typename Vec<T>::v8 cv = __builtin_bit_cast(typename Vec<T>::v8, val);
             unsigned bits = 0;
 #pragma unroll
@@ -544,7 +334,10 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
             ((uint8_t*)sign_out)[(int64_t)m * p.ldsign + (n >> 3)] = (uint8_t)bits;
           }
         }
-        st16(row0 + (int64_t)(i * 32 + rr * RPI) * p.ldc, val);
+        TO* const dst = row0 + (int64_t)(i * 32 + rr * RPI) * p.ldc;
+        if constexpr (ANY && FULL) st16_elem(dst, val, std::integral_constant<int, ES>());
+        else if constexpr (ANY) Row<TO, true>::store(dst, 0, p.N - n, val);
+        else st16(dst, val);
       }
     }
   }
@@ -919,6 +712,244 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_dma_kernel(GemmParams p
   gemm_dma_body<T, BM, BN, BK, WM, WN, A_KMAJOR, B_KMAJOR, NS>(p, pid);
 }
 
+// ---------------------------------------------------------------------------
+// Anything the direct-to-LDS kernel cannot take: extents, leading dimensions and pointers of any
+// element alignment, contractions that are not a multiple of BK.  The same tiles, LDS layout, MFMA
+// order and write-out; a panel travels HBM -> registers -> LDS in 16-byte loads at element alignment
+// (direct-to-LDS loads are kept to aligned addresses).  The loads of a stage are requested two
+// stages ahead of its MFMAs: they stay in registers for one stage and are parked in the LDS buffer
+// the other stage has just left, behind the MFMAs of the next.
+// Only a slice's last stage tests extents: every stage before it reads whole chunks without a test --
+// rows beyond M / N are clamped, a chunk that crosses the end of a contraction-strided row reads on
+// into the row after it, which exists (its products reach only entries of C that are not stored).
+// Rows shorter than a chunk could run past the last row that way: all their stages are tested.
+// Bound by the matrix pipe and the LDS traffic around it like the direct-to-LDS kernel, 25-35 % behind it by the
+// stores through the registers.  Against the kernel before it (chunks fetched one stage ahead with a test each, result
+// stored from the accumulators, 4 and 2 bytes per lane and row): 4113 x 1733 x 2051 fp16 forward 112 -> 55 us, input
+// gradient 103 -> 54, weight gradient 121 -> 61; 8192 x 50257 x 1024 forward 4232 -> 1057 (of the element-wise one),
+// 798 TFLOP/s; 8192 x 1024 x 2056 (all aligned, K % 64 != 0) 58 -> 46.
+// ---------------------------------------------------------------------------
+template <typename T, int R, int BK, bool KMAJOR, int NW>
+struct RegPanel {
+  typedef DmaPanel<T, R, BK, KMAJOR, NW> D;
+  static constexpr int PER = D::PER_WAVE;  // chunks per thread
+  static constexpr int NT = NW * 64;
+  static constexpr int ROWS = NT / D::CPR;  // LDS rows between a thread's chunks
+  static_assert(NT % D::CPR == 0 && D::NCHUNK == PER * NT, "panel must divide evenly over the threads");
+  static_assert(KMAJOR ? (ROWS / (16 / D::CPR)) % D::CPR == 0 : ROWS % 4 == 0, "a thread's chunks share one swizzle");
+
+  // Thread t owns the LDS slots t, t + NT, ... and fetches the chunk that the swizzle puts there.
+  static __device__ __forceinline__ void init(const T* (&ptrs)[PER], const T* base, int64_t ld, int row0, int rmax, int kbeg) {
+    const int t = threadIdx.x, lrow = t / D::CPR, c = D::swz(lrow, t % D::CPR);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      if (KMAJOR) {
+        ptrs[j] = base + (int64_t)min(row0 + lrow + j * ROWS, rmax - 1) * ld + kbeg + c * 8;
+      } else {
+        const int gr = row0 + c * 8 < rmax ? row0 + c * 8 : row0;
+        ptrs[j] = base + (int64_t)(kbeg + lrow + j * ROWS) * ld + gr;
+      }
+    }
+  }
+  static __device__ __forceinline__ u32x4 fetch(const T* ptr) {
+    return ld16_elem<false>(ptr, std::integral_constant<int, 2>());
+  }
+  // chunk j of the stage that starts at contraction index k0, zero from kend on
+  static __device__ __forceinline__ u32x4 fetch_tested(const T* ptr, int j, int k0, int kend, int row0, int rmax) {
+    const int t = threadIdx.x, lrow = t / D::CPR, c = D::swz(lrow, t % D::CPR);
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (KMAJOR) {
+      const int left = kend - (k0 + c * 8);
+      if (left > 0) v = Row<T, true>::load(ptr, 0, left);
+    } else if (k0 + lrow + j * ROWS < kend) {
+      const int gr = row0 + c * 8 < rmax ? row0 + c * 8 : row0;
+      v = Row<T, true>::load(ptr, 0, rmax - gr);
+    }
+    return v;
+  }
+};
+
+template <typename T, int BM, int BN, int BK, int WM, int WN, int WPE, bool A_KMAJOR, bool B_KMAJOR>
+__global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_reg_kernel(GemmParams p) {
+  constexpr int NW = WM * WN, NT = NW * 64;
+  constexpr int WTM = BM / WM, WTN = BN / WN;
+  constexpr int TM = WTM / 32, TN = WTN / 32;
+  constexpr int GROUP_M = 8;
+  constexpr int KSTEPS = BK / 16;
+  typedef RegPanel<T, BM, BK, A_KMAJOR, NW> PA;
+  typedef RegPanel<T, BN, BK, B_KMAJOR, NW> PB;
+  typedef typename Vec<T>::v8 v8;
+  constexpr int STAGE = PA::D::BYTES + PB::D::BYTES;
+  constexpr int LPS = PA::PER + PB::PER;  // chunks per thread per stage
+  static_assert(KSTEPS == 4, "stores, loads and hand-over are dealt over four contraction steps");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int pid = (p.flags & 1) ? (int)blockIdx.x : remap_xcd(blockIdx.x, tiles * p.splits, p.xcds);
+  const int split = pid / tiles;
+  const int t = pid - split * tiles;
+  const int per_group = GROUP_M * p.tiles_n;
+  const int group = t / per_group;
+  const int first_m = group * GROUP_M;
+  const int gsz = min(p.tiles_m - first_m, GROUP_M);
+  const int tm = first_m + (t % per_group) % gsz;
+  const int tn = (t % per_group) / gsz;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int kbeg = split * p.k_per_split;
+  const int kend = min(p.K, kbeg + p.k_per_split);
+  const int nk = (kend - kbeg + BK - 1) / BK;
+  // stages that need no test: all but the last one, none where a row may be shorter than a chunk
+  const int nfree = (A_KMAJOR || p.lda >= 8) && (B_KMAJOR || p.ldb >= 8) ? nk - 1 : 0;
+
+  const T* pa[PA::PER];
+  const T* pb[PB::PER];
+  PA::init(pa, (const T*)p.A, p.lda, m0, p.M, kbeg);
+  PB::init(pb, (const T*)p.B, p.ldb, n0, p.N, kbeg);
+
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  u32x4 regs[LPS];
+  // chunk q of the next stage to be fetched (which starts at contraction index k0) into its register
+  auto load_item = [&](int q, int k0, auto tested_c) {
+    constexpr bool TESTED = decltype(tested_c)::value;
+    if (q < PA::PER) {
+      regs[q] = TESTED ? PA::fetch_tested(pa[q], q, k0, kend, m0, p.M) : PA::fetch(pa[q]);
+      pa[q] += A_KMAJOR ? (int64_t)BK : (int64_t)BK * p.lda;
+    } else {
+      regs[q] = TESTED ? PB::fetch_tested(pb[q - PA::PER], q - PA::PER, k0, kend, n0, p.N) : PB::fetch(pb[q - PA::PER]);
+      pb[q - PA::PER] += B_KMAJOR ? (int64_t)BK : (int64_t)BK * p.ldb;
+    }
+  };
+  auto store_item = [&](char* dst, int q) {
+    if (q < PA::PER) lds_st16(dst, (int)threadIdx.x * 16 + q * NT * 16, regs[q]);
+    else lds_st16(dst, PA::D::BYTES + (int)threadIdx.x * 16 + (q - PA::PER) * NT * 16, regs[q]);
+  };
+  auto barrier = [&]() {  // bare: __syncthreads() would wait for the loads in flight as well
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  FragRegs<A_KMAJOR> fa[2][TM];
+  FragRegs<B_KMAJOR> fb[2][TN];
+  constexpr int NMFMA = TM * TN;
+  constexpr int NR = TM + TN;
+  constexpr int RPS = (NR + NMFMA - 1) / NMFMA;
+  constexpr int RSLOTS = (NR + RPS - 1) / RPS;
+  auto read_item = [&](const char* stage, int ks, int buf, int item) {
+    const uint32_t sa_addr = lds_address(stage), sb_addr = sa_addr + PA::D::BYTES;
+    if (item < TM) PA::D::frag_issue(fa[buf][item], sa_addr, wm * WTM + item * 32, ks, lane);
+    else PB::D::frag_issue(fb[buf][item - TM], sb_addr, wn * WTN + (item - TM) * 32, ks, lane);
+  };
+  typedef std::integral_constant<bool, true> yes_t;
+  typedef std::integral_constant<bool, false> no_t;
+
+  // ---- prologue: stage 0 into LDS, stage 1 into the registers, the first operands
+#pragma unroll
+  for (int q = 0; q < LPS; ++q) {
+    if (nfree > 0) load_item(q, kbeg, no_t());
+    else load_item(q, kbeg, yes_t());
+  }
+#pragma unroll
+  for (int q = 0; q < LPS; ++q) store_item(smem, q);
+  if (nk > 1) {
+#pragma unroll
+    for (int q = 0; q < LPS; ++q) {
+      if (nfree > 1) load_item(q, kbeg + BK, no_t());
+      else load_item(q, kbeg + BK, yes_t());
+    }
+  }
+  wait_lgkmcnt<0>();
+  barrier();
+#pragma unroll
+  for (int r = 0; r < NR; ++r) read_item(smem, 0, 0, r);
+
+  // ---- one stage: everything that is not an MFMA sits behind one, pinned by scheduling barriers.
+  // MORE: another stage follows (its chunks are in the registers: stored behind steps 0 and 1);
+  // LOAD: and one after that, whose chunks are requested behind steps 1 and 2 (TESTED: by extents).
+  auto stage = [&](char* cur, char* nxt, int k2, auto more_c, auto load_c, auto tested_c) {
+    constexpr bool MORE = decltype(more_c)::value, LOAD = decltype(load_c)::value;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      const bool last = ks + 1 == KSTEPS;
+      wait_lgkmcnt<0>();  // this step's operands, requested a step ago; at the last step also the stores
+      __builtin_amdgcn_sched_barrier(0);
+      if (last && MORE) {
+        barrier();  // everyone's stores of the next stage are in, everyone has read the last operands of `cur`
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int m = 0; m < NMFMA; ++m) {
+        const int i = m / TN, j = m % TN;
+        acc[i][j] = mfma32(fb[ks & 1][j].template get<v8>(), fa[ks & 1][i].template get<v8>(), acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!last || MORE) {
+#pragma unroll
+          for (int r = m * RPS; r < (m + 1) * RPS && r < NR; ++r) {
+            if (last) read_item(nxt, 0, 0, r);
+            else read_item(cur, ks + 1, (ks + 1) & 1, r);
+          }
+        }
+        // the extras of steps 0 to 2, dealt over their MFMAs: half of the stores, the other half and half of the
+        // loads, the other half of the loads
+        constexpr int H = LPS / 2;
+        const int q0 = m * H / NMFMA, q1 = (m + 1) * H / NMFMA;
+#pragma unroll
+        for (int q = q0; q < q1; ++q) {
+          if (MORE && ks == 0) store_item(nxt, q);
+          if (MORE && ks == 1) store_item(nxt, H + q);
+          if (LOAD && ks == 1) load_item(q, k2, tested_c);
+          if (LOAD && ks == 2) load_item(H + q, k2, tested_c);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  static_assert(LPS % 2 == 0 && RSLOTS <= NMFMA, "halves of a stage's chunks; a step's reads fit behind its MFMAs");
+  int kt = 0;
+  auto cur = [&]() { return smem + (kt & 1) * STAGE; };
+  auto nxt = [&]() { return smem + ((kt + 1) & 1) * STAGE; };
+  for (; kt + 2 < nfree; ++kt) stage(cur(), nxt(), 0, yes_t(), yes_t(), no_t());
+  for (; kt + 2 < nk; ++kt) stage(cur(), nxt(), kbeg + (kt + 2) * BK, yes_t(), yes_t(), yes_t());
+  if (kt + 1 < nk) {
+    stage(cur(), nxt(), 0, yes_t(), no_t(), no_t());
+    ++kt;
+  }
+  stage(cur(), nxt(), 0, no_t(), no_t(), no_t());
+
+  __syncthreads();  // all waves are done reading the last pipeline stage
+  const bool full = m0 + BM <= p.M && n0 + BN <= p.N;
+  if (p.splits > 1) {
+    // fp32 partial of this contraction slice: a plain (M, N) matrix, written like an fp32 result
+    GemmParams q = p;
+    q.C = p.partial + (int64_t)split * p.M * p.N;
+    q.ldc = p.N;
+    q.bias = nullptr;
+    q.relu = 0;
+    q.mask = nullptr;
+    q.alpha = nullptr;
+    q.chunk_n = p.N;
+    q.chunk_skip = 0;
+    if (full) gemm_epilogue_lds<T, float, TM, TN, WTM, WTN, true, true, true>(q, acc, smem, m0, n0, wm, wn, wave, lane);
+    else gemm_epilogue_lds<T, float, TM, TN, WTM, WTN, true, false, true>(q, acc, smem, m0, n0, wm, wn, wave, lane);
+  } else if (p.out_f32) {
+    gemm_epilogue_lds<T, float, TM, TN, WTM, WTN, false, false, true>(p, acc, smem, m0, n0, wm, wn, wave, lane);
+  } else {
+    const bool plain = !p.bias && !p.relu && !p.mask && !p.alpha;
+    if (plain && full) gemm_epilogue_lds<T, T, TM, TN, WTM, WTN, true, true, true>(p, acc, smem, m0, n0, wm, wn, wave, lane);
+    else gemm_epilogue_lds<T, T, TM, TN, WTM, WTN, false, false, true>(p, acc, smem, m0, n0, wm, wn, wave, lane);
+  }
+}
+
 // Up to sixteen independent products of one operand layout in ONE launch: workgroup ids
 // [first[i], first[i+1]) belong to problem i.  Used for weight gradients, whose output has
 // few tiles: side by side they fill the chip with fewer, longer contraction slices.
@@ -942,32 +973,46 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_dma_group_kernel(GemmGr
 }
 
 // Sum the split-contraction partials in a fixed order and apply the epilogue.
-// VEC4: N and ldc multiples of 4, 16-byte aligned partials, 8-byte aligned C.
-template <typename T, typename TO, bool VEC4>
+//  kReduceRows: N and ldc multiples of 4, 16-byte aligned partials, 8-byte aligned C: four columns of a row at a time
+//  kReduceFlat: C is one dense (M, N) matrix and there is no bias, so partials and result are the same flat sequence,
+//               taken four elements at a time whatever N is (2051 x 1733 x 4113 in four slices, both passes: 65 -> 61 us)
+//  kReduceAny:  element by element
+enum ReduceMode { kReduceAny, kReduceRows, kReduceFlat };
+template <typename T, typename TO, ReduceMode MODE>
 __global__ __launch_bounds__(256) void gemm_reduce(int M, int N, int splits, const float* __restrict__ partial,
                                                     const T* __restrict__ bias, int relu, TO* __restrict__ C,
                                                     int64_t ldc, int chunk_n, int64_t chunk_skip,
                                                     const float* __restrict__ alpha_ptr) {
   const int64_t total = (int64_t)M * N;
   const float alpha = alpha_ptr ? *alpha_ptr : 1.f;
-  if (VEC4) {
+  if (MODE != kReduceAny) {
+    struct alignas(sizeof(TO) * 4) Quad { TO v[4]; };
     const int64_t quads = total >> 2;
     for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < quads; q += (int64_t)gridDim.x * 256) {
-      f32x4 s = *reinterpret_cast<const f32x4*>(partial + q * 4);
-      for (int k = 1; k < splits; ++k) s += *reinterpret_cast<const f32x4*>(partial + (int64_t)k * total + q * 4);
       const int64_t i = q * 4;
-      const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
-      TO o[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float x = s[e] * alpha + (bias ? (float)bias[n + e] : 0.f);
-        o[e] = (TO)(relu ? fmaxf(x, 0.f) : x);
-      }
-      struct alignas(sizeof(TO) * 4) Quad { TO v[4]; };
+      auto part = [&](int k) {  // a slice of an odd number of elements starts at any of them
+        const float* src = partial + (int64_t)k * total + i;
+        if (MODE == kReduceRows) return *reinterpret_cast<const f32x4*>(src);
+        return __builtin_bit_cast(f32x4, ld16_elem<false>(src, std::integral_constant<int, 4>()));
+      };
+      f32x4 s = part(0);
+      for (int k = 1; k < splits; ++k) s += part(k);
+      const int m = MODE == kReduceRows ? (int)(i / N) : 0, n = MODE == kReduceRows ? (int)(i - (int64_t)m * N) : 0;
       Quad qd;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) qd.v[e] = o[e];
-      store_out(C + (int64_t)m * ldc + n + (int64_t)(n / chunk_n) * chunk_skip, qd);
+      for (int e = 0; e < 4; ++e) {
+        const float x = s[e] * alpha + (MODE == kReduceRows && bias ? (float)bias[n + e] : 0.f);
+        qd.v[e] = (TO)(relu ? fmaxf(x, 0.f) : x);
+      }
+      if (MODE == kReduceRows) store_out(C + (int64_t)m * ldc + n + (int64_t)(n / chunk_n) * chunk_skip, qd);
+      else store_out(C + i, qd);
+    }
+    if (MODE == kReduceFlat && blockIdx.x == 0 && threadIdx.x < (total & 3)) {
+      const int64_t i = (quads << 2) + threadIdx.x;
+      float s = 0.f;
+      for (int k = 0; k < splits; ++k) s += partial[(int64_t)k * total + i];
+      s *= alpha;
+      C[i] = (TO)(relu ? fmaxf(s, 0.f) : s);
     }
   } else {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
@@ -1073,7 +1118,10 @@ static GemmPlan plan_for(int cfg, int64_t M, int64_t N, int64_t K, double* cost_
 #define TF_STEP_256x128 1.0
 #endif
   const double fixed = pl.bm * pl.bn >= 256 * 256 ? 10.0 : 7.0;
-  const double per_step = pl.bm * pl.bn >= 256 * 256 ? 1.65 : (pl.bm * pl.bn >= 256 * 128 ? TF_STEP_256x128 : 1.1);
+  // register-staged: 8192 x 1024 x 50257 takes 393 steps of 256x256 tiles in 911 us, 786 of 128x128 in 1340
+  // (with the figures of the direct-to-LDS tiles 960 x 768 x 50257 ran on 128x128 tiles: 160 us instead of 129)
+  const double per_step = !kCfgs[cfg].dma ? (pl.bm * pl.bn >= 256 * 256 ? 2.25 : 1.6)
+                          : pl.bm * pl.bn >= 256 * 256 ? 1.65 : (pl.bm * pl.bn >= 256 * 128 ? TF_STEP_256x128 : 1.1);
   auto cost_of = [&](int64_t nsplit, int64_t steps) {
     const int64_t rounds = (tiles * nsplit + slots - 1) / slots;
     double c = (double)rounds * (fixed + per_step * (double)steps);
@@ -1147,12 +1195,10 @@ static void allow_big_lds(K kernel, int bytes) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
-template <typename T, int BM, int BN, int BK, int WM, int WN, bool AK, bool BKM, bool VEC>
-static int launch_one(hipStream_t st, const GemmParams& p) {
-  typedef Panel<T, BM, BK, AK, WM * WN * 64, VEC> PA;
-  typedef Panel<T, BN, BK, BKM, WM * WN * 64, VEC> PB;
-  constexpr int lds = 2 * (PA::BYTES + PB::BYTES);
-  auto kernel = gemm_kernel<T, BM, BN, BK, WM, WN, AK, BKM, VEC>;
+template <typename T, int BM, int BN, int BK, int WM, int WN, int WPE, bool AK, bool BKM>
+static int launch_reg(hipStream_t st, const GemmParams& p) {
+  constexpr int lds = 2 * (BM + BN) * BK * 2;
+  auto kernel = gemm_reg_kernel<T, BM, BN, BK, WM, WN, WPE, AK, BKM>;
   static bool once = (allow_big_lds(kernel, lds), true);
   (void)once;
   const unsigned grid = (unsigned)(p.tiles_m * p.tiles_n * p.splits);
@@ -1185,9 +1231,9 @@ static int launch_dma(hipStream_t st, const GemmParams& p) {
 #endif
 constexpr int kStagesNarrow = TF_STAGES_NARROW;
 
-template <typename T, bool AK, bool BKM, bool VEC>
-static int launch_cfg(hipStream_t st, const GemmPlan& pl, const GemmParams& p) {
-  if (kCfgs[pl.cfg].dma && VEC && p.K % pl.bk == 0) {
+template <typename T, bool AK, bool BKM>
+static int launch_cfg(hipStream_t st, bool vec, const GemmPlan& pl, const GemmParams& p) {
+  if (kCfgs[pl.cfg].dma && vec && p.K % pl.bk == 0) {
     switch (pl.cfg) {
       case 2: return launch_dma<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
       case 3: return launch_dma<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, p);
@@ -1195,8 +1241,8 @@ static int launch_cfg(hipStream_t st, const GemmPlan& pl, const GemmParams& p) {
       case 5: return launch_dma<T, 128, 256, 64, 2, 4, 2, AK, BKM, kStagesNarrow>(st, p);
     }
   }
-  if (pl.bm == 256 && pl.bn == 256) return launch_one<T, 256, 256, 64, 2, 4, AK, BKM, VEC>(st, p);
-  if (pl.bm == 128 && pl.bn == 128) return launch_one<T, 128, 128, 64, 2, 2, AK, BKM, VEC>(st, p);
+  if (pl.bm == 256 && pl.bn == 256) return launch_reg<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
+  if (pl.bm == 128 && pl.bn == 128) return launch_reg<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, p);
   return TF_EINVAL;
 }
 
@@ -1205,18 +1251,22 @@ template <typename T>
 static int launch_reduce(hipStream_t st, const GemmParams& p) {
   if (p.splits <= 1) return TF_OK;
   const int64_t total = (int64_t)p.M * p.N;
-  const bool v4 = p.N % 4 == 0 && p.ldc % 4 == 0 && p.chunk_n % 4 == 0 && p.chunk_skip % 4 == 0 &&
-                  (reinterpret_cast<uintptr_t>(p.C) & 15) == 0;
-  int64_t blocks = ((v4 ? total / 4 : total) + 255) / 256;
+  const bool c16 = (reinterpret_cast<uintptr_t>(p.C) & 15) == 0;
+  const bool rows = c16 && p.N % 4 == 0 && p.ldc % 4 == 0 && p.chunk_n % 4 == 0 && p.chunk_skip % 4 == 0;
+  const bool flat = c16 && !p.bias && p.ldc == p.N && p.chunk_n == p.N;
+  int64_t blocks = ((rows || flat ? total / 4 : total) + 255) / 256;
   if (blocks > 4096) blocks = 4096;
   if (blocks < 1) blocks = 1;
   const dim3 g((unsigned)blocks), b(256);
   const T* bias = (const T*)p.bias;
-#define REDUCE(TO, V4) \
-  gemm_reduce<T, TO, V4><<<g, b, 0, st>>>(p.M, p.N, p.splits, p.partial, bias, p.relu, (TO*)p.C, p.ldc, p.chunk_n, \
-                                          p.chunk_skip, p.alpha)
-  if (p.out_f32) { if (v4) REDUCE(float, true); else REDUCE(float, false); }
-  else { if (v4) REDUCE(T, true); else REDUCE(T, false); }
+#define REDUCE(TO, MODE) \
+  gemm_reduce<T, TO, MODE><<<g, b, 0, st>>>(p.M, p.N, p.splits, p.partial, bias, p.relu, (TO*)p.C, p.ldc, p.chunk_n, \
+                                            p.chunk_skip, p.alpha)
+#define REDUCE_MODE(TO) \
+  do { if (rows) REDUCE(TO, kReduceRows); else if (flat) REDUCE(TO, kReduceFlat); else REDUCE(TO, kReduceAny); } while (0)
+  if (p.out_f32) REDUCE_MODE(float);
+  else REDUCE_MODE(T);
+#undef REDUCE_MODE
 #undef REDUCE
   TF_CHECK_LAUNCH();
   return TF_OK;
@@ -1226,7 +1276,7 @@ template <typename T>
 static int gemm_dispatch(hipStream_t st, int la, int lb, bool vec, const GemmPlan& pl, const GemmParams& p) {
   const bool ak = la == TF_OP_KMAJOR, bk = lb == TF_OP_KMAJOR;
   int rc;
-#define GO(AK, BKM) rc = vec ? launch_cfg<T, AK, BKM, true>(st, pl, p) : launch_cfg<T, AK, BKM, false>(st, pl, p)
+#define GO(AK, BKM) rc = launch_cfg<T, AK, BKM>(st, vec, pl, p)
   if (ak && bk) GO(true, true);
   else if (ak && !bk) GO(true, false);
   else if (!ak && bk) GO(false, true);
