@@ -1,0 +1,136 @@
+"""The native launch path against the Python launchers it stands in for: the same call with the native functions
+answering None (the general path) gives the same bits, for operands of every form -- contiguous ones, which the
+native path takes, and strided, misaligned or empty ones, which it hands back."""
+import pytest
+import torch
+
+from tritonformer_amd import kernels as K
+
+
+class HandsBack:
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def both(monkeypatch, call):
+    outcomes = []
+    for general in (False, True):
+        with monkeypatch.context() as m:
+            if general:
+                m.setattr(K, "launch", HandsBack)
+            try:
+                out = call()
+                outcomes.append([t for t in (out if isinstance(out, tuple) else (out,)) if isinstance(t, torch.Tensor)])
+            except (ValueError, TypeError) as e:
+                outcomes.append(type(e))
+    native, general = outcomes
+    if isinstance(general, type):
+        assert native is general
+        return
+    assert len(native) == len(general)
+    for a, b in zip(native, general):
+        assert a.shape == b.shape and a.dtype == b.dtype and a.stride() == b.stride() and torch.equal(a, b)
+
+
+def forms(t):
+    """`t`, and tensors equal to it: other strides, an odd start, every second column of a wider one."""
+    wide = torch.zeros(t.shape[:-1] + (2 * t.shape[-1],), dtype=t.dtype, device=t.device)
+    wide[..., ::2] = t
+    odd = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
+    out = {"plain": t, "strided": wide[..., ::2], "odd": odd}
+    if t.ndim >= 2:
+        out["transposed"] = t.transpose(-1, -2).contiguous().transpose(-1, -2)
+    return out
+
+
+def randn(*shape, dtype=torch.float16):
+    return torch.randn(*shape, device="cuda").to(dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["plain", "strided", "odd", "transposed"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,k,n", [(1, 64, 64), (77, 128, 264), (130, 67, 33)])
+def test_products(m, k, n, dtype, form, dev, monkeypatch):
+    torch.manual_seed(m + k)
+    a, b, bias, g = randn(2, m, k, dtype=dtype), randn(k, n, dtype=dtype), randn(n, dtype=dtype), randn(2, m, n, dtype=dtype)
+    af, bf, gf, biasf = forms(a)[form], forms(b)[form], forms(g)[form], forms(bias).get(form, bias)
+    both(monkeypatch, lambda: K.gemm(af, b, biasf, True))
+    both(monkeypatch, lambda: K.gemm(a, bf, None))
+    both(monkeypatch, lambda: K.gemm_relu_bits(af, bf, biasf))
+    both(monkeypatch, lambda: K.mm_dw(af, gf, torch.float32))
+    both(monkeypatch, lambda: K.mm_dw(a, gf))
+    both(monkeypatch, lambda: K.unbroadcast_leading(gf))
+    both(monkeypatch, lambda: K.mask_grad(gf, g))
+    both(monkeypatch, lambda: K.cast_pack([bf.float(), b.float()], dtype))
+    act, bits = K.gemm_relu_bits(a, b, bias)
+    if bits is not None:
+        both(monkeypatch, lambda: K.mm_masked_bits(af, bf, bits, act))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["plain", "strided", "odd", "transposed"])
+@pytest.mark.parametrize("d", [64, 129])
+def test_rows(d, form, dev, monkeypatch):
+    torch.manual_seed(d)
+    x, r, g = (randn(2, 19, d) for _ in range(3))
+    al, be = randn(d).float(), randn(d).float()
+    xf, gf, alf = forms(x)[form], forms(g)[form], forms(al).get(form, al)
+    both(monkeypatch, lambda: K.layernorm_fwd(xf, alf, be, 1e-5))
+    both(monkeypatch, lambda: K.add_layernorm_fwd(xf, r, alf, be, 1e-5))
+    y, mean, rstd = K.layernorm_fwd(x, al, be, 1e-5)
+    for leave in (False, True):  # partial sums: the buffer's unused tail is whatever memory held
+        both(monkeypatch, lambda: K.layernorm_bwd(gf, xf, alf, mean, rstd, leave)[: 1 if leave else 3])
+        both(monkeypatch, lambda: K.add_layernorm_bwd(gf, r, xf, alf, mean, rstd, leave)[: 1 if leave else 3])
+    for dtype in (torch.float32, torch.bfloat16):
+        both(monkeypatch, lambda: K.softmax_fwd(xf.to(dtype)))
+        both(monkeypatch, lambda: K.softmax_bwd(gf.to(dtype), x.to(dtype)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias", ["none", "dense", "dense-odd-pitch", "alibi"])
+@pytest.mark.parametrize("s,hd", [(64, 32), (192, 64), (96, 128)])
+def test_attention(s, hd, bias, dev, monkeypatch):
+    torch.manual_seed(s)
+    b, nh = 2, 3
+    extra = {"none": None, "dense": randn(nh, s + 8, s + 8), "dense-odd-pitch": randn(nh, s + 3, s + 3),
+             "alibi": torch.tensor([0.5, 0.25, 0.125], device="cuda", dtype=torch.float16)}[bias]
+    qkv, g = randn(b, s, 3, nh, hd), randn(b, s, nh * hd)
+    out, lse = K.flash_packed_fwd(qkv, extra)
+    both(monkeypatch, lambda: K.flash_packed_fwd(qkv, extra))
+    for gf in forms(g).values():
+        both(monkeypatch, lambda: K.flash_packed_bwd(gf, out, qkv, lse, extra))
+    for q, k, v, go in [tuple(randn(b, s, nh, hd).transpose(1, 2) for _ in range(4)),
+                        tuple(randn(b, nh, s, hd) for _ in range(4)),
+                        (randn(b, nh, s, hd),) + tuple(randn(b, s, nh, hd).transpose(1, 2) for _ in range(3))]:
+        both(monkeypatch, lambda: K.flash_wrapper_fwd(q, k, v, extra))
+        o, l = K.flash_wrapper_fwd(q, k, v, extra)
+        both(monkeypatch, lambda: K.flash_wrapper_bwd(go, o, q, k, v, l, extra))
+
+
+@pytest.mark.gpu
+def test_refused_calls_are_refused_alike(dev, monkeypatch):
+    x, w = randn(2, 8, 64), randn(64, 64)
+    for call in [lambda: K.gemm(x[0], w), lambda: K.gemm(x, w[:32]), lambda: K.gemm(x.float(), w.float()),
+                 lambda: K.gemm(x, w.bfloat16()), lambda: K.gemm(x, w.cpu()), lambda: K.gemm(x, w, w[0, :32]),
+                 lambda: K.layernorm_fwd(x[0], w[0], w[0], 1e-5), lambda: K.layernorm_fwd(x, w[0, :8], w[0, :8], 1e-5),
+                 lambda: K.add_layernorm_fwd(x, x[:1], w[0], w[0], 1e-5), lambda: K.softmax_fwd(w),
+                 lambda: K.mask_grad(x, x.bfloat16()), lambda: K.mm_dw(x, x[:1]), lambda: K.cast_pack([w, w[:32]], torch.float16),
+                 lambda: K.flash_wrapper_fwd(*(randn(1, 1, 64, 48) for _ in range(3))),
+                 lambda: K.flash_wrapper_fwd(*(randn(1, 1, 80, 64) for _ in range(3)))]:
+        with pytest.raises((ValueError, TypeError)):
+            call()
+        both(monkeypatch, call)
+
+
+def test_tensors_off_the_gpu_are_handed_back():
+    native = K.launch()
+    x, w = torch.zeros(1, 8, 64, dtype=torch.float16), torch.zeros(64, 64, dtype=torch.float16)
+    assert native.linear(x, w, None, False) is None
+    assert native.layernorm(x, None, w[0], w[0], 1e-5) is None
+    assert native.softmax_fwd(x) is None and native.cast_pack([w], torch.bfloat16) is None
+    assert native.linear("x", w, None, False) is None
+    with pytest.raises(ValueError):
+        K.gemm(x, w)
+    with pytest.raises(TypeError):
+        native.linear(x, w)

@@ -4,7 +4,9 @@ Run as ``python -m tritonformer_amd._build`` (recompiles what changed; ``--force
 recompiles everything).  Every ``csrc/*.hip`` file is compiled to an object (in
 parallel) and linked into ``libtritonformer_amd.so`` next to this file, where
 ``_lib.py`` loads it with ctypes; ``csrc/diag/*.hip`` become
-``libtritonformer_amd_diag.so`` (diagnostics, never loaded by an operator).
+``libtritonformer_amd_diag.so`` (diagnostics, never loaded by an operator), and
+``csrc/launch.cpp`` becomes ``_launch.so``, the extension module through which the
+launchers of ``kernels.py`` reach the product library without ctypes.
 
 The product library carries a hash of the sources it was built from
 (``tf_source_hash``); ``_lib.load`` compares it with the sources next to it and
@@ -14,6 +16,7 @@ import hashlib
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -24,6 +27,8 @@ INCLUDE = os.path.join(ROOT, "include")
 OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(HERE, "libtritonformer_amd.so")
 DIAG_LIB_PATH = os.path.join(HERE, "libtritonformer_amd_diag.so")
+LAUNCH_SRC = os.path.join(CSRC, "launch.cpp")
+LAUNCH_PATH = os.path.join(HERE, "_launch.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -48,9 +53,9 @@ def _headers():
 
 
 def source_hash():
-    """sha256 over every file the product library is built from (names and contents)."""
+    """sha256 over every file the product library and its extension module are built from (names and contents)."""
     h = hashlib.sha256()
-    for path in [os.path.join(CSRC, f) for f in sources()] + _headers():
+    for path in [os.path.join(CSRC, f) for f in sources()] + _headers() + [LAUNCH_SRC]:
         h.update(os.path.basename(path).encode())
         with open(path, "rb") as fh:
             h.update(fh.read())
@@ -82,6 +87,25 @@ def _link(objs, path):
     os.replace(tmp, path)
 
 
+def _build_launch():
+    # host code only, against the torch that is installed: the product library is found next to the module
+    import torch
+
+    base = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    tmp = LAUNCH_PATH + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DTF_SOURCE_HASH="{source_hash()}"',
+           "-isystem", os.path.join(base, "include"), "-isystem", os.path.join(base, "include/torch/csrc/api/include"),
+           "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"], LAUNCH_SRC, "-o", tmp,
+           "-L" + HERE, "-ltritonformer_amd", "-L" + os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10",
+           "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compiling launch.cpp failed:\n{r.stderr}")
+    os.replace(tmp, LAUNCH_PATH)
+
+
 def build_library(verbose=True, jobs=None, force=True):
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
@@ -98,8 +122,9 @@ def build_library(verbose=True, jobs=None, force=True):
                 print(f"[{job[1]}] {err}", file=sys.stderr)
     _link([o for o, _ in results[: len(srcs)]], LIB_PATH)
     _link([o for o, _ in results[len(srcs):]], DIAG_LIB_PATH)
+    _build_launch()
     if verbose:
-        print(f"built {LIB_PATH} from {len(srcs)} sources, {DIAG_LIB_PATH} from {len(diag)}")
+        print(f"built {LIB_PATH} from {len(srcs)} sources, {DIAG_LIB_PATH} from {len(diag)}, {LAUNCH_PATH}")
     return LIB_PATH
 
 

@@ -99,8 +99,10 @@ class LnParamGrads(ctypes.Structure):
 
 
 DIAG_LIB_PATH = os.path.join(_HERE, "libtritonformer_amd_diag.so")
+LAUNCH_PATH = os.path.join(_HERE, "_launch.so")
 
 _lib = None
+_launch = None
 _diag = None
 
 
@@ -130,6 +132,24 @@ def load():
                 )
         _lib = lib
     return _lib
+
+
+def launch():
+    """The extension module of csrc/launch.cpp (same sources as the library, or it is refused): each of its
+    functions runs one operator on plain contiguous tensors and returns None for any other form of call."""
+    global _launch
+    if _launch is None:
+        lib = load()
+        if not os.path.exists(LAUNCH_PATH):
+            raise ImportError(f"{LAUNCH_PATH} is missing: build it with `python -m tritonformer_amd._build`")
+        from . import _launch as module
+
+        if module.source_hash != lib.tf_source_hash().decode():
+            raise ImportError(f"{LAUNCH_PATH} and {LIB_PATH} were built from different sources: rebuild them with "
+                              "`python -m tritonformer_amd._build`")
+        module.set_check(check)
+        _launch = module
+    return _launch
 
 
 class _Diag:

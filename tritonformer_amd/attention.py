@@ -9,6 +9,8 @@ from . import _deferred
 from ._amp import amp_bwd, amp_fwd, cached_conversion
 from .kernels import (
     cast_pack,
+    flash_packed_bwd,
+    flash_packed_fwd,
     flash_wrapper_bwd,
     flash_wrapper_bwd_attn_bias,
     flash_wrapper_fwd,
@@ -83,9 +85,7 @@ class PackedCausalAttention(Function):
         if not qkv.is_contiguous():
             qkv = qkv.contiguous()
         b, s, _, nh, hd = qkv.shape
-        q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        out = torch.empty((b, s, nh, hd), dtype=qkv.dtype, device=qkv.device)
-        _, lse = flash_wrapper_fwd(q, k, v, attn_bias, out=out.permute(0, 2, 1, 3))
+        out, lse = flash_packed_fwd(qkv, attn_bias)
         ctx.save_for_backward(lse, qkv, out, attn_bias)
         return out.view(b, s, nh * hd)
 
@@ -93,13 +93,7 @@ class PackedCausalAttention(Function):
     @amp_bwd
     def backward(ctx: Any, grad_output: torch.Tensor):
         lse, qkv, out, attn_bias = ctx.saved_tensors
-        b, s, _, nh, hd = qkv.shape
-        q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        dqkv = torch.empty_like(qkv)
-        grads = tuple(dqkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        grad_output = grad_output.reshape(b, s, nh, hd).permute(0, 2, 1, 3)
-        flash_wrapper_bwd(grad_output, out.permute(0, 2, 1, 3), q, k, v, lse, attn_bias, grads=grads)
-        return dqkv, None
+        return flash_packed_bwd(grad_output, out, qkv, lse, attn_bias), None
 
 
 class AttentionBlock(Function):
@@ -128,9 +122,7 @@ class AttentionBlock(Function):
         packed = cached_conversion([wq, wk, wv, wo], x.dtype, cast_pack)
         w_qkv, w_o = packed[:, : 3 * d], packed[:, 3 * d:]
         qkv = mm(x, w_qkv).view(b, s, 3, num_heads, hd)
-        q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        attn = torch.empty((b, s, num_heads, hd), dtype=x.dtype, device=x.device)
-        _, lse = flash_wrapper_fwd(q, k, v, attn_bias, out=attn.permute(0, 2, 1, 3))
+        attn, lse = flash_packed_fwd(qkv, attn_bias)
         attn = attn.view(b, s, d)
         ctx.save_for_backward(x, packed, qkv, attn, lse, attn_bias)
         ctx.weight_dtype = wq.dtype
@@ -142,12 +134,8 @@ class AttentionBlock(Function):
         x, packed, qkv, attn, lse, attn_bias = ctx.saved_tensors
         b, s, _, nh, hd = qkv.shape
         w_qkv, w_o = packed[:, : 3 * nh * hd], packed[:, 3 * nh * hd:]
-        d_attn = mm(grad_output, w_o.T).view(b, s, nh, hd).permute(0, 2, 1, 3)
-        q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        dqkv = torch.empty_like(qkv)
-        grads = tuple(dqkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
-        flash_wrapper_bwd(d_attn, attn.view(b, s, nh, hd).permute(0, 2, 1, 3), q, k, v, lse, attn_bias, grads=grads)
-        dqkv = dqkv.view(b, s, 3 * nh * hd)
+        d_attn = mm(grad_output, w_o.T)
+        dqkv = flash_packed_bwd(d_attn, attn, qkv, lse, attn_bias).view(b, s, 3 * nh * hd)
         if ctx.defer_to is not None:
             # launched later, together with those of other layers, in whole rounds of workgroups
             _deferred.submit([(x, dqkv, 3, ctx.defer_to[:3], ctx.weight_dtype),
