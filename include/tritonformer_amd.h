@@ -402,6 +402,12 @@ int tf_relu_mask(void* stream, int dtype, int64_t rows, int64_t cols,
                  const void* grad, int64_t ldg, const void* act, int64_t lda,
                  void* out, int64_t ldo);
 
+/* masked = where(act > 0, grad, 0) and sums[c] = sum_r masked[r, c] in one pass: the bits of
+ * tf_relu_mask followed by tf_colsum (out_dtype and partial as there). */
+int tf_relu_mask_colsum(void* stream, int dtype, int out_dtype, int64_t rows, int64_t cols,
+                        const void* grad, int64_t ldg, const void* act, int64_t lda,
+                        void* masked, int64_t ldm, void* sums, float* partial, int64_t partial_bytes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -264,6 +264,8 @@ def test_row_kernels_reject_bad_arguments():
     assert lib.tf_cross_entropy_fwd(None, 0, 6, 64, FAKE, 64, 3, 100, FAKE, FAKE, FAKE) == -1   # groups overlap
     assert lib.tf_colsum(None, 0, 0, 16, 64, FAKE, 64, FAKE, None, 0) == -5
     assert lib.tf_colsum(None, 0, 1, 16, 64, FAKE, 64, FAKE, FAKE, 1 << 20) == -2   # bf16 sums of fp16 input
+    assert lib.tf_relu_mask_colsum(None, 0, 0, 16, 64, FAKE, 64, FAKE, 64, FAKE, 64, FAKE, None, 0) == -5
+    assert lib.tf_relu_mask_colsum(None, 0, 0, 16, 64, FAKE, 64, FAKE, 64, FAKE, 63, FAKE, FAKE, 1 << 20) == -1
     assert lib.tf_relu_mask(None, 0, 4, 64, None, 64, FAKE, 64, FAKE, 64) == -1
     # empty inputs are accepted and launch nothing
     assert lib.tf_softmax_fwd(None, 0, 0, 64, FAKE, 64, FAKE, 64) == 0

@@ -62,6 +62,7 @@ def test_products(m, k, n, dtype, form, dev, monkeypatch):
     both(monkeypatch, lambda: K.mm_dw(a, gf))
     both(monkeypatch, lambda: K.unbroadcast_leading(gf))
     both(monkeypatch, lambda: K.mask_grad(gf, g))
+    both(monkeypatch, lambda: K.mask_grad_sums(gf, g, torch.float32))
     both(monkeypatch, lambda: K.cast_pack([bf.float(), b.float()], dtype))
     act, bits = K.gemm_relu_bits(a, b, bias)
     if bits is not None:

@@ -130,7 +130,7 @@ def test_cross_entropy_rows(v, dtype, dev):
     assert torch.equal(fv, ov) and torch.equal(loss, loss2) and torch.equal(lse, lse2) and untouched(fb, v)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 1), (33, 7), (100, 255), (70, 257), (513, 1733)])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (33, 7), (100, 255), (70, 257), (513, 1733), (97, 512)])
 def test_column_sums_and_relu_mask_rows(rows, cols, dev):
     g = torch.Generator().manual_seed(cols)
     x, act = torch.randn(rows, cols, generator=g).half(), torch.randn(rows, cols, generator=g).half()
@@ -148,6 +148,16 @@ def test_column_sums_and_relu_mask_rows(rows, cols, dev):
                                 ov.stride(0)))
     assert torch.equal(ov.cpu(), torch.where(act > 0, x, torch.zeros_like(x))) and untouched(ob, cols)
     assert torch.equal(K.mask_grad(xv, av), ov)
+    # mask and sums in one pass: the bits of the two passes, from odd and from whole rows
+    _lib.check(lib.tf_colsum(st, dt, _lib.TF_F32, rows, cols, ov.data_ptr(), ov.stride(0), out.data_ptr(), part.data_ptr(), nb))
+    fb, fv = odd_rows(torch.zeros_like(x), dev)
+    sums = torch.empty(cols, device=dev)
+    _lib.check(lib.tf_relu_mask_colsum(st, dt, _lib.TF_F32, rows, cols, xv.data_ptr(), xv.stride(0), av.data_ptr(),
+                                       av.stride(0), fv.data_ptr(), fv.stride(0), sums.data_ptr(), part.data_ptr(), nb))
+    assert torch.equal(fv, ov) and torch.equal(sums, out) and untouched(fb, cols)
+    for a, b in [(xv, av), (xv.contiguous(), av.contiguous())]:
+        masked, s = K.mask_grad_sums(a, b, torch.float32)
+        assert torch.equal(masked, ov) and torch.equal(s, out)
 
 
 # either side of the tile edges (128, 256) and of one, two and three 64-wide stages, alone and in slices; rows shorter

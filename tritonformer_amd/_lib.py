@@ -67,6 +67,7 @@ SIGNATURES = {
     "tf_colsum_partial_bytes": (_i64, [_i64, _i64]),
     "tf_colsum_noalloc": (_i, [_vp, _i, _i, _i64, _i64, _vp, _i64, _vp]),
     "tf_colsum_noalloc_max_partial_bytes": (_i64, []),
+    "tf_relu_mask_colsum": (_i, [_vp, _i, _i, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64]),
     "tf_relu_mask": (_i, [_vp, _i, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64]),
 }
 

@@ -496,6 +496,22 @@ TF_FN(relu_mask, 2) {
   return THPVariable_Wrap(out);
 }
 
+// relu_mask_colsum(grad, act, fp32) -> (where(act > 0, grad, 0), its sums over every dimension but the last)
+TF_FN(relu_mask_colsum, 3) {
+  const Tensor *g = dense(args.a[0]), *act = dense(args.a[1]);
+  if (!alike(g, act) || !is16(*g)) Py_RETURN_NONE;
+  const int64_t rows = rows_of(*g), cols = last(*g), bytes = tf_colsum_partial_bytes(rows, cols);
+  const at::ScalarType type = args.a[2] == Py_True ? at::kFloat : g->scalar_type();
+  Tensor out = make(g->sizes(), *g), sums = make({cols}, *g, type), part = make({bytes}, *g, at::kByte);
+  if (!call([&] {
+        return tf_relu_mask_colsum(stream(), code(g->scalar_type()), code(type), rows, cols, g->data_ptr(), cols,
+                                   act->data_ptr(), cols, out.data_ptr(), cols, sums.data_ptr(),
+                                   static_cast<float*>(part.data_ptr()), bytes);
+      }))
+    return nullptr;
+  return tuple_of({&out, &sums});
+}
+
 // colsum(x, fp32) -> sums over every dimension but the last
 TF_FN(colsum, 2) {
   const Tensor* x = dense(args.a[0]);
@@ -521,7 +537,8 @@ PyObject* set_check(PyObject*, PyObject* f) {
 PyMethodDef methods[] = {
     TF_ENTRY(linear), TF_ENTRY(linear_bits), TF_ENTRY(linear_masked), TF_ENTRY(weight_grad), TF_ENTRY(cast_pack),
     TF_ENTRY(attn_fwd), TF_ENTRY(attn_bwd), TF_ENTRY(attn_packed_fwd), TF_ENTRY(attn_packed_bwd), TF_ENTRY(layernorm),
-    TF_ENTRY(layernorm_bwd), TF_ENTRY(softmax_fwd), TF_ENTRY(softmax_bwd), TF_ENTRY(relu_mask), TF_ENTRY(colsum),
+    TF_ENTRY(layernorm_bwd), TF_ENTRY(softmax_fwd), TF_ENTRY(softmax_bwd), TF_ENTRY(relu_mask), TF_ENTRY(relu_mask_colsum),
+    TF_ENTRY(colsum),
     {"set_check", set_check, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

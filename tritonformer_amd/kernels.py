@@ -358,6 +358,17 @@ def mask_grad(grad, out_act):
     return out
 
 
+def mask_grad_sums(grad, out_act, out_dtype=None):
+    """``(mask_grad(grad, out_act), unbroadcast_leading(of it, out_dtype))``, the same bits in one pass over
+    contiguous operands."""
+    if out_dtype is None or out_dtype == torch.float32 or out_dtype == grad.dtype:
+        out = launch().relu_mask_colsum(grad, out_act, out_dtype == torch.float32)
+        if out is not None:
+            return out
+    masked = mask_grad(grad, out_act)
+    return masked, unbroadcast_leading(masked, out_dtype)
+
+
 # --------------------------------------------------------------------------- attention
 def _attn_layout(q, *others):
     """All tensors must share q's strides, unit stride along hd and 16-byte

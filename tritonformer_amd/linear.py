@@ -5,7 +5,7 @@ from torch.autograd import Function
 
 from . import _deferred
 from ._amp import amp_bwd, amp_fwd, cached_conversion
-from .kernels import (cast_pack, gemm, gemm_relu_bits, mask_grad, mm, mm_dw, mm_dw_group, mm_masked_bits,
+from .kernels import (cast_pack, gemm, gemm_relu_bits, mask_grad, mask_grad_sums, mm, mm_dw, mm_dw_group, mm_masked_bits,
                       unbroadcast_leading)
 
 
@@ -17,10 +17,14 @@ RELU_BITS = True
 PACK_CASTS = True
 
 
+def _bias_grad_dtype(ctx, index):
+    """fp32 sums are stored unrounded for an fp32 master bias (as the weight gradients are), else in 16 bits."""
+    return torch.float32 if ctx.arg_dtypes[index] == torch.float32 else None
+
+
 def _bias_grad(ctx, grad, index):
-    """Column sums of ``grad`` as the gradient of the bias passed at argument ``index``: fp32 sums
-    stored unrounded for an fp32 master bias (as the weight gradients are), else in 16 bits."""
-    return unbroadcast_leading(grad, torch.float32 if ctx.arg_dtypes[index] == torch.float32 else None)
+    """Column sums of ``grad`` as the gradient of the bias passed at argument ``index``."""
+    return unbroadcast_leading(grad, _bias_grad_dtype(ctx, index))
 
 
 def _deferral_target(ctx, index=1):
@@ -119,9 +123,11 @@ class LinearBiasReLU(Function):
     @amp_bwd
     def backward(ctx, grad_output):
         inputs, weights, out_w_act = ctx.saved_tensors
-        grad_output = mask_grad(grad_output, out_w_act)
+        if ctx.needs_input_grad[2]:
+            grad_output, grad_bias = mask_grad_sums(grad_output, out_w_act, _bias_grad_dtype(ctx, 2))
+        else:
+            grad_output, grad_bias = mask_grad(grad_output, out_w_act), None
         grad_input, grad_weights = _grads(ctx, grad_output, inputs, weights)
-        grad_bias = _bias_grad(ctx, grad_output, 2) if ctx.needs_input_grad[2] else None
         return grad_input, grad_weights, grad_bias
 
 
