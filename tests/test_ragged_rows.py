@@ -99,6 +99,40 @@ def test_softmax_rows(n, dtype, dev):
     assert_close(ov, R.softmax_bwd(yv.detach().float().cpu(), dy.float()), dtype, "dx", atol=tol["atol"] * 10, rtol=tol["rtol"])
 
 
+def masked_rows(n, dtype, seed):
+    """Rows as masking leaves them, and rows whose maximum is of large magnitude."""
+    g = torch.Generator().manual_seed(seed)
+    lowest = torch.finfo(dtype).min
+    rows = [torch.full((n,), lowest)]                                   # masked throughout: uniform
+    for fill in (lowest, float("-inf")):
+        head, few, most = (2 * torch.randn(n, generator=g) for _ in range(3))
+        head[: n // 2] = fill
+        few[n // 3 : n // 3 + 24] = fill
+        most[torch.arange(n) != n // 3] = fill
+        rows += [head, few, most]
+    for big in (6e4, -6e4) if dtype == torch.float16 else (1e10, -1e10, 3e38, -3e38):
+        one = 2 * torch.randn(n, generator=g)
+        one[n // 2] = big
+        rows += [torch.full((n,), big), one]
+    return torch.stack(rows).to(dtype)
+
+
+# either side of the wave-per-row kernels' end (4096 16-bit, 2048 fp32 elements), the longest rows of the
+# workgroup-per-row ones and those beyond; ragged and whole
+@pytest.mark.parametrize("n", [513, 2048, 2049, 4096, 4097, 4104, 32769, 65535, 65536, 65537])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_softmax_of_masked_rows(n, dtype, dev):
+    x = masked_rows(n, dtype, n)
+    y = K.softmax_fwd(x.to(dev)[None])[0]
+    want = torch.softmax(x.double(), -1)
+    # fp32 exponentials (relative error below 1e-5 down to exp(-100)) and sums, one rounding of the result
+    ulp, least = {torch.float32: (2.0 ** -24, 2.0 ** -126), torch.float16: (2.0 ** -11, 2.0 ** -25),
+                  torch.bfloat16: (2.0 ** -8, 2.0 ** -126)}[dtype]
+    assert ((y.double().cpu() - want).abs() <= want * (ulp + 1e-5) + least).all()
+    dx = K.softmax_bwd(torch.ones_like(y)[None], y[None])
+    assert torch.isfinite(dx).all()
+
+
 # 8 / 16 / 25 chunks of 256 threads in registers (16384, 32768, 51200 entries), then the streaming forward
 @pytest.mark.parametrize("v", [1, 9, 16383, 16385, 32769, 50257, 51199, 51201, 70001])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
