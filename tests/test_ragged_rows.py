@@ -164,6 +164,29 @@ def test_cross_entropy_rows(v, dtype, dev):
     assert torch.equal(fv, ov) and torch.equal(loss, loss2) and torch.equal(lse, lse2) and untouched(fb, v)
 
 
+# vocabularies held in registers and streamed (beyond 51200), ragged and whole; the masked tokens fill whole chunks of
+# the first ones of a thread, with -inf and with the type's lowest value
+@pytest.mark.parametrize("v", [257, 16385, 51199, 51201, 51208, 70001, 128257])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_cross_entropy_of_masked_rows(v, dtype, dev):
+    g = torch.Generator().manual_seed(v)
+    x = torch.randn(6, v, generator=g)
+    for r, fill in enumerate((float("-inf"), torch.finfo(dtype).min)):
+        x[3 * r, 64:80] = fill
+        x[3 * r + 1, : v - 40] = fill
+        x[3 * r + 2, torch.arange(v) % 16 >= 8] = fill
+    x = x.to(dtype)
+    lab = torch.full((6,), v - 1 - (v - 1) % 16, dtype=torch.int64)
+    gout = torch.full((6,), 4.0, dtype=dtype)
+    loss, lse, _, _ = K.cross_entropy_fwd(x.to(dev), lab.to(dev))
+    grad = K.cross_entropy_bwd(gout.to(dev), x.to(dev), lab.to(dev), lse)
+    assert torch.isfinite(loss).all() and torch.isfinite(grad).all()
+    assert_close(loss, R.cross_entropy(x, lab), dtype, "loss", atol=1e-2 if dtype == torch.float16 else 6e-2)
+    assert_close(grad, R.cross_entropy_bwd(x, lab, gout), dtype, "grad", atol=1e-3, rtol=1e-2)
+    _, _, both = K.shifted_cross_entropy_fwd_grad(x.to(dev).repeat_interleave(2, 0).view(6, 2, v), lab.to(dev)[:, None].expand(6, 2), 4.0)
+    assert torch.equal(both[:, 0], grad)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (33, 7), (100, 255), (70, 257), (513, 1733), (97, 512)])
 def test_column_sums_and_relu_mask_rows(rows, cols, dev):
     g = torch.Generator().manual_seed(cols)

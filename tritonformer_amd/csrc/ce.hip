@@ -80,9 +80,12 @@ __global__ __launch_bounds__(kCeThreads) void ce_fwd(int V, const T* __restrict_
       for (int e = 1; e < 8; ++e) cm = fmaxf(cm, v[e]);
       cm *= kLog2e;
       if (cm > acc.m) { acc.s *= exp2f(acc.m - cm); acc.m = cm; }
+      // nothing but masked entries so far (-inf, or a lowest value whose multiple is): they count as exp2(-inf - 0),
+      // where -inf - (-inf) is NaN
+      const float shift = acc.m == -INFINITY ? 0.f : acc.m;
       float part = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) part += fast_exp2(v[e] * kLog2e - acc.m);
+      for (int e = 0; e < 8; ++e) part += fast_exp2(v[e] * kLog2e - shift);
       acc.s += part;
     }
   }
