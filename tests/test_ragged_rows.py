@@ -133,6 +133,34 @@ def test_softmax_of_masked_rows(n, dtype, dev):
     assert torch.isfinite(dx).all()
 
 
+# ragged rows whose small probabilities are subnormal numbers
+@pytest.mark.parametrize("n", [777, 2049, 4097, 32769, 65537])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_softmax_of_ragged_rows_keeps_subnormal_numbers(n, dtype, dev):
+    x = torch.linspace(-100, 0, n).to(dtype).repeat(2, 1)
+    y = K.softmax_fwd(x.to(dev)[None])[0].double().cpu()
+    want = torch.softmax(x.double(), -1)
+    # as in the test above, with two units of the smallest number: those of the exponential and of the quotient
+    ulp, least = (2.0 ** -24, 2.0 ** -149) if dtype == torch.float32 else (2.0 ** -8, 2.0 ** -133)
+    assert ((want < 2.0 ** -126) & (want > 4 * least)).sum() > n // 50
+    assert ((y - want).abs() <= want * (ulp + 1e-5) + 2 * least).all()
+
+
+# ... and where the upstream gradient, a loss scale, lifts them into the normal numbers of the type
+@pytest.mark.parametrize("v", [1001, 50257, 70001])
+def test_cross_entropy_gradient_of_ragged_rows_keeps_subnormal_numbers(v, dev):
+    x = torch.linspace(-100, 0, v).bfloat16().repeat(2, 1)
+    lab, gout = torch.full((2,), v - 1), torch.full((2,), 1024.0, dtype=torch.bfloat16)
+    loss, lse, _, _ = K.cross_entropy_fwd(x.to(dev), lab.to(dev))
+    grad = K.cross_entropy_bwd(gout.to(dev), x.to(dev), lab.to(dev), lse).double().cpu()
+    want = torch.softmax(x.double(), -1)
+    assert ((want < 2.0 ** -126) & (want > 2.0 ** -140)).any()
+    want[:, v - 1] -= 1.0
+    # one rounding of the result, of half the smallest bf16 number (2^-133, over 1024) at least; logarithm and argument of
+    # the exponential in fp32; a unit of the subnormal exponential
+    assert ((grad / 1024 - want).abs() <= want.abs() * (2.0 ** -8 + 1e-4) + 2.0 ** -144 + 2.0 ** -149).all()
+
+
 # 8 / 16 / 25 chunks of 256 threads in registers (16384, 32768, 51200 entries), then the streaming forward
 @pytest.mark.parametrize("v", [1, 9, 16383, 16385, 32769, 50257, 51199, 51201, 70001])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

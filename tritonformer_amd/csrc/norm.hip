@@ -575,8 +575,9 @@ template <bool MAX> __device__ __forceinline__ float block_reduce16(float v, flo
   return r;
 }
 
-// (exponentials of non-positive arguments: v_exp_f32 as it is, without the library wrapper's range
-// handling -- results below 2^-126 become zero, which is what they round to in the sum anyway)
+// Exponentials of non-positive arguments.  Whole rows: v_exp_f32 as it is, results below 2^-126 become zero (as they
+// always have there).  ANY: the library function, which keeps the subnormal numbers.
+template <bool ANY> __device__ __forceinline__ float long_exp2(float x) { return ANY ? exp2f(x) : __builtin_amdgcn_exp2f(x); }
 template <typename T, int NV, bool ANY>
 __global__ __launch_bounds__(kLongRowThreads) void softmax_fwd_long(int cols, const T* __restrict__ x, int64_t ldx,
                                                                     T* __restrict__ y, int64_t ldy) {
@@ -605,7 +606,7 @@ __global__ __launch_bounds__(kLongRowThreads) void softmax_fwd_long(int cols, co
       // and from |m| of 1e10 on the rounding of m * log2e alone exceeds the range of the exponential.  The operation
       // more shows where few rows leave the memory idle: 100 x 65536 fp32 9.5 -> 9.9 us, 1000 x 8192 fp16 7.3 -> 7.4)
 #pragma unroll
-      for (int e = 0; e < N; ++e) { v[i][e] = __builtin_amdgcn_exp2f((v[i][e] - m) * kLog2e); s += v[i][e]; }
+      for (int e = 0; e < N; ++e) { v[i][e] = long_exp2<ANY>((v[i][e] - m) * kLog2e); s += v[i][e]; }
     }
   }
   const float inv = 1.0f / block_reduce16<false>(s, red, 1);
