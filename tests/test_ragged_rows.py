@@ -278,3 +278,20 @@ def test_register_staged_gemm(m, n, k, cfg, splits, la, lb, dev):
         bound = sums + (want.abs() + sums) * ulp[0] + ulp[1] + 1e-7 * with_bias
         assert ((cv.double().cpu() - want).abs() <= bound).all()
         assert dense or untouched(cb, n)
+
+
+# the chunk that crosses the end of a row holds r elements of it; alone, behind one whole chunk, behind many
+@pytest.mark.parametrize("r", range(1, 8))
+def test_row_kernels_at_every_remainder_of_a_chunk(r, dev):
+    for n in (r, 8 + r, 640 + r):
+        for dtype in (torch.float16, torch.bfloat16):
+            if n > 3:  # (the variance of up to three elements may be of any smallness)
+                test_layernorm_rows(n, dtype, False, dev)
+                test_layernorm_rows(n, dtype, True, dev)
+            test_cross_entropy_rows(n, dtype, dev)
+        for dtype in (torch.float16, torch.bfloat16, torch.float32):
+            test_softmax_rows(n, dtype, dev)
+        test_column_sums_and_relu_mask_rows(33, n, dev)
+    test_layernorm_rows(2048 + r, torch.float16, True, dev)
+    test_softmax_rows(4096 + r, torch.float16, dev)
+    test_cross_entropy_rows(51200 + r, torch.float16, dev)

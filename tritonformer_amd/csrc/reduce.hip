@@ -34,6 +34,7 @@ __global__ __launch_bounds__(256) void colsum_partial(int64_t rows, int cols, co
                                                        float* __restrict__ partial, int rows_per_group,
                                                        const T* __restrict__ act, int64_t lda, T* __restrict__ out,
                                                        int64_t ldo) {
+  typedef Row<T, ANY> R;
   __shared__ float red[kCsSlices][kCsColsPerBlock];
   const int lane32 = threadIdx.x & 31;
   const int slice = threadIdx.x >> 5;
@@ -47,13 +48,15 @@ __global__ __launch_bounds__(256) void colsum_partial(int64_t rows, int cols, co
   if (col0 < cols) {
     for (int64_t r = rbeg + slice; r < rend; r += kCsSlices) {
       float v[8];
-      unpack8<T>(Row<T, ANY>::load(x + r * ldx, col0 / 8, cols), v);
+      const u32x4 rx = R::template fetch<true>(x + r * ldx, col0 / 8, cols);
+      const u32x4 ra = MASK ? R::template fetch<true>(act + r * lda, col0 / 8, cols) : rx;
+      unpack8<T>(R::template settle<true>(rx, col0 / 8, cols), v);
       if constexpr (MASK) {
         float a[8];
-        unpack8<T>(Row<T, ANY>::load(act + r * lda, col0 / 8, cols), a);
+        unpack8<T>(R::template settle<true>(ra, col0 / 8, cols), a);
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = a[e] > 0.f ? v[e] : 0.f;
-        Row<T, ANY>::store(out + r * ldo, col0 / 8, cols, pack8<T>(v));
+        R::template store<true>(out + r * ldo, col0 / 8, cols, pack8<T>(v));
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[e] += v[e];
@@ -103,17 +106,19 @@ template <typename T, bool ANY>
 __global__ __launch_bounds__(256) void relu_mask_kernel(int64_t rows, int cols, const T* __restrict__ grad,
                                                          int64_t ldg, const T* __restrict__ act, int64_t lda,
                                                          T* __restrict__ out, int64_t ldo) {
-  const int cpr = Row<T, ANY>::chunks(cols);
+  typedef Row<T, ANY> R;
+  const int cpr = R::chunks(cols);
   const int64_t total = rows * cpr;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
     const int64_t r = i / cpr;
     const int c = (int)(i - r * cpr);
     float g[8], a[8];
-    unpack8<T>(Row<T, ANY>::load(grad + r * ldg, c, cols), g);
-    unpack8<T>(Row<T, ANY>::load(act + r * lda, c, cols), a);
+    const u32x4 rg = R::template fetch<true>(grad + r * ldg, c, cols), ra = R::template fetch<true>(act + r * lda, c, cols);
+    unpack8<T>(R::template settle<true>(rg, c, cols), g);
+    unpack8<T>(R::template settle<true>(ra, c, cols), a);
 #pragma unroll
     for (int e = 0; e < 8; ++e) g[e] = a[e] > 0.f ? g[e] : 0.f;
-    Row<T, ANY>::store(out + r * ldo, c, cols, pack8<T>(g));
+    R::template store<true>(out + r * ldo, c, cols, pack8<T>(g));
   }
 }
 

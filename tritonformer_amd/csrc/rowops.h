@@ -49,6 +49,8 @@ template <> __device__ __forceinline__ void load8<float>(const float* p, float (
 // ANY = false: the caller has checked that rows are aligned and whole chunks (row_vectorizable).
 typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
 template <bool STREAM> __device__ __forceinline__ u32x4 ld16_elem(const void* p, std::integral_constant<int, 2>) {
   const u32x4_a2* q = reinterpret_cast<const u32x4_a2*>(p);
   return STREAM ? __builtin_nontemporal_load(q) : *q;
@@ -75,30 +77,76 @@ template <typename T, bool ANY> struct Row {
     for (int e = 0; e < N; ++e) t.v[e] = c * N + e < n ? p[e] : fill;
     return __builtin_bit_cast(u32x4, t);
   }
-  static __device__ __forceinline__ void store(T* row, int c, int n, u32x4 v) {
+  // The same in two halves for SHORT rows, one chunk per lane, where every wave has a chunk that crosses the end and the
+  // tested element loads above, each waited for, are most of the time: `fetch` takes the 16 bytes that end with the row
+  // in its place, `settle` moves their elements down.  (63488 x 71 fp16, LayerNorm forward: 28.5 us with
+  // element loads, 22.5 so, 22.1 in a loop over elements; with a residual 40.2, 28.9 and 31.2.  In longer rows the moves, made
+  // for every chunk, cost more than the element loads of the one: 8192 x 1537 14.4 -> 18.3.)
+  template <bool SHORT> static __device__ __forceinline__ u32x4 fetch(const T* row, int c, int n, T fill = (T)0.f) {
+    if (!ANY || !SHORT || n < N) return load(row, c, n, fill);
+    return ld16_elem<false>(row + min(c * N, n - N), size_t_());
+  }
+  template <bool SHORT> static __device__ __forceinline__ u32x4 settle(u32x4 raw, int c, int n, T fill = (T)0.f) {
+    if (!ANY || !SHORT || n < N || (c + 1) * N <= n) return raw;
+    const int up = ((c + 1) * N - n) * (int)sizeof(T) * 8;  // bits to move down by, 16 to 112
+    struct Words { uint64_t lo, hi; };
+    Words w = __builtin_bit_cast(Words, raw);
+    w.lo = up >= 64 ? w.hi >> (up & 63) : w.lo >> up | w.hi << (64 - up);
+    w.hi = up >= 64 ? 0 : w.hi >> up;
+    struct { T v[8 / sizeof(T)]; } f8;
+#pragma unroll
+    for (int e = 0; e < 8 / (int)sizeof(T); ++e) f8.v[e] = fill;
+    const uint64_t f = __builtin_bit_cast(uint64_t, f8);
+    if (f != 0) {
+      w.hi |= up >= 64 ? f : f << (64 - up);
+      if (up > 64) w.lo |= f << (128 - up);
+    }
+    return __builtin_bit_cast(u32x4, w);
+  }
+  template <bool SHORT = false> static __device__ __forceinline__ void store(T* row, int c, int n, u32x4 v) {
     T* p = row + c * N;
     if constexpr (!ANY) { st16(p, v); return; }
     if ((c + 1) * N <= n) {  // lines are filled by neighbouring lanes and stores: write-back, see st16
       st16_elem(p, v, size_t_());
       return;
     }
-    struct alignas(16) Elems { T v[N]; };
-    const Elems t = __builtin_bit_cast(Elems, v);
+    if constexpr (!SHORT) {
+      struct alignas(16) Elems { T v[N]; };
+      const Elems t = __builtin_bit_cast(Elems, v);
 #pragma unroll
-    for (int e = 0; e < N; ++e)
-      if (c * N + e < n) p[e] = t.v[e];
+      for (int e = 0; e < N; ++e)
+        if (c * N + e < n) p[e] = t.v[e];
+      return;
+    }
+    // SHORT: what is left of the row in pieces of 8, 4 and 2 bytes
+    char* q = reinterpret_cast<char*>(p);
+    const int left = (n - c * N) * (int)sizeof(T);
+    if (left & 8) {
+      *reinterpret_cast<u32x2_a2*>(q) = u32x2{v[0], v[1]};
+      q += 8;
+      v[0] = v[2], v[1] = v[3];
+    }
+    if (left & 4) {
+      *reinterpret_cast<u32_a2*>(q) = v[0];
+      q += 4;
+      v[0] = v[1];
+    }
+    if (sizeof(T) == 2 && (left & 2)) *reinterpret_cast<uint16_t*>(q) = (uint16_t)v[0];
   }
 };
 // eight elements from index 8 c on of a vector of n elements (16-bit or fp32) as fp32, zero beyond its end
-template <typename TP, bool ANY> __device__ __forceinline__ void load8_row(const TP* p, int c, int n, float (&v)[8]) {
+template <typename TP, bool ANY, bool SHORT = false>
+__device__ __forceinline__ void load8_row(const TP* p, int c, int n, float (&v)[8]) {
   if constexpr (!ANY) {
     load8<TP>(p + c * 8, v);
   } else if constexpr (sizeof(TP) == 2) {
-    unpack8<TP>(Row<TP, true>::load(p, c, n), v);
+    typedef Row<TP, true> R;
+    unpack8<TP>(R::template settle<SHORT>(R::template fetch<SHORT>(p, c, n), c, n), v);
   } else {
-    const f32x4 a = __builtin_bit_cast(f32x4, Row<float, true>::load(p, 2 * c, n));
+    typedef Row<float, true> R;
+    const f32x4 a = __builtin_bit_cast(f32x4, R::template settle<SHORT>(R::template fetch<SHORT>(p, 2 * c, n), 2 * c, n));
     f32x4 b = {};
-    if (8 * c + 4 < n) b = __builtin_bit_cast(f32x4, Row<float, true>::load(p, 2 * c + 1, n));
+    if (8 * c + 4 < n) b = __builtin_bit_cast(f32x4, R::template settle<SHORT>(R::template fetch<SHORT>(p, 2 * c + 1, n), 2 * c + 1, n));
 #pragma unroll
     for (int i = 0; i < 4; ++i) { v[i] = a[i]; v[4 + i] = b[i]; }
   }
