@@ -218,6 +218,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_bwd(int V, const T* __restrict_
                                                       const int64_t* __restrict__ labels,
                                                       const float* __restrict__ lse, const T* __restrict__ gout,
                                                       int64_t gstride, T* __restrict__ dlogits, RowMap dmap) {
+  typedef Row<T, ANY> R;
   const int64_t row = blockIdx.x;
   const T* xr = logits + map.at(row);
   T* dr = dlogits + dmap.at(row);
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_bwd(int V, const T* __restrict_
   const int nchunk = Row<T, ANY>::chunks(V);
   for (int c = threadIdx.x; c < nchunk; c += kCeThreads) {
     float v[8];
-    unpack8<T>(Row<T, ANY>::template load<true>(xr, c, V), v);
+    unpack8<T>(R::template settle<true>(R::template fetch<true, true>(xr, c, V), c, V), v);
     grad_probs<ANY>(v, l2);
     if ((lab >> 3) == c) {
 #pragma unroll
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_bwd(int V, const T* __restrict_
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] *= g;
-    Row<T, ANY>::store(dr, c, V, pack8<T>(v));
+    R::template store<true>(dr, c, V, pack8<T>(v));
   }
 }
 

@@ -82,9 +82,10 @@ template <typename T, bool ANY> struct Row {
   // in its place, `settle` moves their elements down.  (63488 x 71 fp16, LayerNorm forward: 28.5 us with
   // element loads, 22.5 so, 22.1 in a loop over elements; with a residual 40.2, 28.9 and 31.2.  In longer rows the moves, made
   // for every chunk, cost more than the element loads of the one: 8192 x 1537 14.4 -> 18.3.)
-  template <bool SHORT> static __device__ __forceinline__ u32x4 fetch(const T* row, int c, int n, T fill = (T)0.f) {
-    if (!ANY || !SHORT || n < N) return load(row, c, n, fill);
-    return ld16_elem<false>(row + min(c * N, n - N), size_t_());
+  template <bool SHORT, bool STREAM = false>
+  static __device__ __forceinline__ u32x4 fetch(const T* row, int c, int n, T fill = (T)0.f) {
+    if (!ANY || !SHORT || n < N) return load<STREAM>(row, c, n, fill);
+    return ld16_elem<STREAM>(row + min(c * N, n - N), size_t_());
   }
   template <bool SHORT> static __device__ __forceinline__ u32x4 settle(u32x4 raw, int c, int n, T fill = (T)0.f) {
     if (!ANY || !SHORT || n < N || (c + 1) * N <= n) return raw;
