@@ -110,6 +110,24 @@ def test_attention(s, hd, bias, dev, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", ["plain", "odd"])
+def test_products_without_sign_bits_are_tried_once(form, dev, monkeypatch):
+    """A contraction that no kernel writes or reads sign bits for (not a multiple of 64; operands at odd elements): the
+    plain product follows the native refusal, without a second attempt through the general launcher."""
+    torch.manual_seed(0)
+    k = 72 if form == "plain" else 128
+    a, b, bias, act = (forms(t)[form] for t in (randn(2, 77, k), randn(k, 264), randn(264), randn(2, 77, 264).relu()))
+    bits = torch.zeros(2 * 77, 33, dtype=torch.uint8, device="cuda")
+    want, masked = K.gemm(a, b, bias, True), K.gemm(a, b, None, False, act)
+    monkeypatch.setattr(K, "_gemm_bits", lambda *args: pytest.fail("tried a second time"))
+    out, none = K.gemm_relu_bits(a, b, bias)
+    assert none is None and torch.equal(out, want)
+    assert torch.equal(K.mm_masked_bits(a, b, bits, act), masked)
+    with pytest.raises(ValueError):
+        K.mm_masked_bits(a, b, bits)
+
+
+@pytest.mark.gpu
 def test_refused_calls_are_refused_alike(dev, monkeypatch):
     x, w = randn(2, 8, 64), randn(64, 64)
     for call in [lambda: K.gemm(x[0], w), lambda: K.gemm(x, w[:32]), lambda: K.gemm(x.float(), w.float()),

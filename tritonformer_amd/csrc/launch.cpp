@@ -178,7 +178,8 @@ TF_FN(linear, 4) {
   return THPVariable_Wrap(out);
 }
 
-// linear_bits(a, b, bias | None) -> (relu(a @ b + bias), sign bits); None also where no kernel writes the bits
+// linear_bits(a, b, bias | None) -> (relu(a @ b + bias), sign bits); False where no kernel writes the bits of a product
+// of this shape: the caller goes on with another product and need not try this one again
 TF_FN(linear_bits, 3) {
   Operands p;
   if (!operands(args.a[0], args.a[1], args.a[2], &p) || p.n % 8) Py_RETURN_NONE;
@@ -191,11 +192,11 @@ TF_FN(linear_bits, 3) {
                                  bits.data_ptr(), nullptr, p.n / 8);
       }, TF_ESHAPE, &rc))
     return nullptr;
-  if (rc != TF_OK) Py_RETURN_NONE;
+  if (rc != TF_OK) Py_RETURN_FALSE;
   return tuple_of({&out, &bits});
 }
 
-// linear_masked(a, b, bits) -> (a @ b) * mask
+// linear_masked(a, b, bits) -> (a @ b) * mask; False as above
 TF_FN(linear_masked, 3) {
   Operands p;
   const Tensor* bits = dense(args.a[2]);
@@ -210,7 +211,7 @@ TF_FN(linear_masked, 3) {
                                  p.n / 8);
       }, TF_ESHAPE, &rc))
     return nullptr;
-  if (rc != TF_OK) Py_RETURN_NONE;
+  if (rc != TF_OK) Py_RETURN_FALSE;
   return THPVariable_Wrap(out);
 }
 

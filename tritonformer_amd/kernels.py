@@ -125,6 +125,8 @@ def gemm_relu_bits(a, b, bias=None):
     the activation's size (reference mask_grad reads the activation, kernels/activation.py:27-44).
     The bits are None when the kernel that produces them cannot take the problem."""
     out = launch().linear_bits(a, b, bias)
+    if out is False:
+        return gemm(a, b, bias, True), None
     if out is not None:
         return out
     _check_linear(a, b, bias)
@@ -151,6 +153,10 @@ def mm_masked_bits(a, b, bits, act=None):
     operands) which this product may miss although the one that wrote the bits met them; ``act``,
     the activation the bits were taken from, then serves as the mask (``mm(..., mask_act=act)``)."""
     out = launch().linear_masked(a, b, bits)
+    if out is False and act is not None:
+        return gemm(a, b, None, False, act)
+    if out is False:
+        check(_BITS_NOT_SERVED)
     if out is not None:
         return out
     _check_linear(a, b, None)
