@@ -142,6 +142,17 @@ def test_refused_calls_are_refused_alike(dev, monkeypatch):
         both(monkeypatch, call)
 
 
+@pytest.mark.gpu
+def test_attention_bias_without_dimensions_is_refused_alike(dev, monkeypatch):
+    qkv = randn(1, 64, 3, 2, 64)
+    bias = qkv.new_zeros(())
+    q, k, v = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+    for call in (lambda: K.flash_wrapper_fwd(q, k, v, bias), lambda: K.flash_packed_fwd(qkv, bias)):
+        with pytest.raises(ValueError):
+            call()
+        both(monkeypatch, call)
+
+
 def test_tensors_off_the_gpu_are_handed_back():
     native = K.launch()
     x, w = torch.zeros(1, 8, 64, dtype=torch.float16), torch.zeros(64, 64, dtype=torch.float16)

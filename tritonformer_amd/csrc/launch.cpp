@@ -271,7 +271,7 @@ bool attn_bias(PyObject* o, const Tensor& q, int64_t nh, int64_t s, const Tensor
   *out = nullptr;
   if (o == Py_None) return true;
   const Tensor* b = plain(o);
-  if (!b || b->size(0) != nh) return false;
+  if (!b || b->dim() < 1 || b->size(0) != nh) return false;
   *out = b;
   if (b->dim() == 1) return b->scalar_type() == at::kHalf && b->is_contiguous();
   return b->dim() == 3 && b->scalar_type() == q.scalar_type() && b->size(1) == b->size(2) && b->size(1) >= s &&
@@ -376,7 +376,7 @@ TF_FN(attn_packed_bwd, 5) {
   const Tensor *g = dense(args.a[0]), *o = dense(args.a[1]), *t = dense(args.a[2]), *lse = dense(args.a[3]), *bias;
   if (!g || !o || !lse || !packed_qkv(t)) Py_RETURN_NONE;
   const int64_t b = t->size(0), s = t->size(1), nh = t->size(3), hd = t->size(4), d = nh * hd;
-  if (g->numel() != b * s * d || o->numel() != b * s * d || g->size(0) != b || g->size(1) != s || o->size(0) != b ||
+  if (g->numel() != b * s * d || o->numel() != b * s * d || g->dim() < 2 || o->dim() < 2 || g->size(0) != b || g->size(1) != s || o->size(0) != b ||
       o->size(1) != s || g->scalar_type() != t->scalar_type() || o->scalar_type() != t->scalar_type() || !aligned(*g) ||
       !aligned(*o) || lse->scalar_type() != at::kFloat || lse->numel() != b * nh * s ||
       !attn_bias(args.a[4], *t, nh, s, &bias))
