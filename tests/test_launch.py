@@ -1,9 +1,13 @@
 """The native launch path against the Python launchers it stands in for: the same call with the native functions
 answering None (the general path) gives the same bits, for operands of every form -- contiguous ones, which the
 native path takes, and strided, misaligned or empty ones, which it hands back."""
+import sys
+
 import pytest
 import torch
 
+import tritonformer_amd
+from tritonformer_amd import _lib
 from tritonformer_amd import kernels as K
 
 
@@ -164,3 +168,19 @@ def test_tensors_off_the_gpu_are_handed_back():
         K.gemm(x, w)
     with pytest.raises(TypeError):
         native.linear(x, w)
+
+
+def test_a_module_of_another_torch_is_refused(monkeypatch):
+    monkeypatch.setattr(_lib, "_launch", None)
+    assert _lib.launch().host_abi.startswith(f"torch {torch.__version__} ")
+    monkeypatch.setattr(_lib, "_launch", None)
+    with monkeypatch.context() as m:  # it loads, but was compiled against another torch
+        m.setattr(torch, "__version__", "0.0.0")
+        with pytest.raises(ImportError, match="rebuild"):
+            _lib.launch()
+    assert _lib._launch is None
+    with monkeypatch.context() as m:  # it does not load at all
+        m.delattr(tritonformer_amd, "_launch", raising=False)
+        m.setitem(sys.modules, "tritonformer_amd._launch", None)
+        with pytest.raises(ImportError, match="rebuild"):
+            _lib.launch()

@@ -87,6 +87,14 @@ def _link(objs, path):
     os.replace(tmp, path)
 
 
+def host_abi():
+    """What the extension module is compiled against beside this repository's sources: its inlined accessors read the
+    torch tensors of this very build, through the C API of this interpreter."""
+    import torch
+
+    return f"torch {torch.__version__} {torch.version.git_version}, {sysconfig.get_config_var('SOABI')}"
+
+
 def _build_launch():
     # host code only, against the torch that is installed: the product library is found next to the module
     import torch
@@ -96,6 +104,7 @@ def _build_launch():
     tmp = LAUNCH_PATH + ".tmp"
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DTF_SOURCE_HASH="{source_hash()}"',
+           f'-DTF_HOST_ABI="{host_abi()}"',
            "-isystem", os.path.join(base, "include"), "-isystem", os.path.join(base, "include/torch/csrc/api/include"),
            "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"], LAUNCH_SRC, "-o", tmp,
            "-L" + HERE, "-ltritonformer_amd", "-L" + os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10",

@@ -136,18 +136,27 @@ def load():
 
 
 def launch():
-    """The extension module of csrc/launch.cpp (same sources as the library, or it is refused): each of its
-    functions runs one operator on plain contiguous tensors and returns None for any other form of call."""
+    """The extension module of csrc/launch.cpp (same sources as the library, compiled against the torch and the
+    interpreter that run, or it is refused): each of its functions runs one operator on plain contiguous tensors and
+    returns None for any other form of call."""
     global _launch
     if _launch is None:
         lib = load()
         if not os.path.exists(LAUNCH_PATH):
             raise ImportError(f"{LAUNCH_PATH} is missing: build it with `python -m tritonformer_amd._build`")
-        from . import _launch as module
+        from . import _build
 
+        try:
+            from . import _launch as module
+        except ImportError as e:  # a symbol that this torch does not have
+            raise ImportError(f"{LAUNCH_PATH} does not load into this process ({_build.host_abi()}): rebuild it with "
+                              "`python -m tritonformer_amd._build`") from e
         if module.source_hash != lib.tf_source_hash().decode():
             raise ImportError(f"{LAUNCH_PATH} and {LIB_PATH} were built from different sources: rebuild them with "
                               "`python -m tritonformer_amd._build`")
+        if module.host_abi != _build.host_abi():
+            raise ImportError(f"{LAUNCH_PATH} was built for {module.host_abi}, this process has {_build.host_abi()}: "
+                              "rebuild it with `python -m tritonformer_amd._build`")
         module.set_check(check)
         _launch = module
     return _launch

@@ -28,6 +28,9 @@
 #ifndef TF_SOURCE_HASH
 #define TF_SOURCE_HASH ""
 #endif
+#ifndef TF_HOST_ABI
+#define TF_HOST_ABI ""
+#endif
 
 namespace {
 
@@ -549,6 +552,8 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_launch", "native launch path 
 
 PyMODINIT_FUNC PyInit__launch() {
   PyObject* m = PyModule_Create(&module_def);
-  if (m && PyModule_AddStringConstant(m, "source_hash", TF_SOURCE_HASH) < 0) Py_CLEAR(m);
+  if (m && (PyModule_AddStringConstant(m, "source_hash", TF_SOURCE_HASH) < 0 ||
+            PyModule_AddStringConstant(m, "host_abi", TF_HOST_ABI) < 0))
+    Py_CLEAR(m);
   return m;
 }
