@@ -107,21 +107,26 @@ def layout_name(la, lb):
             (1, 1): "X^T.dY (both k-strided)", (1, 0): "A k-strided, B k-contiguous"}[(la, lb)]
 
 
+def key_flop(key):
+    """Algorithmic FLOPs of one call recorded by GemmTimer."""
+    problems = key[1:] if key[0] == "group" else [key[2:]]
+    return sum(2.0 * m * n * k for m, n, k in problems)
+
+
 def gemm_table(by_shape, reps, workload, dtype_name):
     """Markdown table of the instrumented GEMM calls: one row per distinct call, HIP-event time per call."""
     rows = []
     for key, (cnt, ms) in by_shape.items():
         if key[0] == "group":
-            probs = key[1:]
-            flop = sum(2.0 * m * n * k for m, n, k in probs)
-            what = "grouped dW: " + " + ".join(f"{m}x{n}x{k}" for m, n, k in probs)
+            what = "grouped dW: " + " + ".join(f"{m}x{n}x{k}" for m, n, k in key[1:])
             layout = layout_name(1, 1)
         elif key[0] == "bits":
             _, lb, m, n, k = key
-            flop, what, layout = 2.0 * m * n * k, f"{m}x{n}x{k} (ReLU sign bits)", layout_name(0, lb)
+            what, layout = f"{m}x{n}x{k} (ReLU sign bits)", layout_name(0, lb)
         else:
             la, lb, m, n, k = key
-            flop, what, layout = 2.0 * m * n * k, f"{m}x{n}x{k}", layout_name(la, lb)
+            what, layout = f"{m}x{n}x{k}", layout_name(la, lb)
+        flop = key_flop(key)
         us = ms / cnt * 1e3
         rows.append((ms / reps, f"| {what} | {layout} | {cnt // reps} | {us:.1f} | {flop / us / 1e6:.0f} | {ms / reps:.3f} |"))
     rows.sort(key=lambda r: -r[0])
@@ -176,9 +181,39 @@ def family_rooflines(by_family, reps):
     return out
 
 
+def _linear_key(a, b):
+    m, k, n = a.numel() // a.shape[-1], b.shape[0], b.shape[1]
+    return (0, 1 if b.stride(1) == 1 and b.stride(0) >= n else 0, m, n, k)
+
+
+def _attn_native_flop(fwd):
+    def work(q):  # (B, nh, S, hd), or the packed (B, S, 3, nh, hd)
+        b, nh, s, hd = q.shape if q.ndim == 4 else (q.shape[0], q.shape[3], q.shape[1], q.shape[4])
+        return (2.0 if fwd else 5.0) * b * nh * s * s * hd
+    return work
+
+
+# function of the native launchers (kernels.launch()) -> what a call of it is: the key of a product, or
+# (kernel family, work) as below; None: neither (memory passes outside the families)
+NATIVE_CALLS = {
+    "linear": lambda a, b, bias, relu: _linear_key(a, b),
+    "linear_bits": lambda a, b, bias: ("bits",) + _linear_key(a, b)[1:],
+    "linear_masked": lambda a, b, bits: ("bits",) + _linear_key(a, b)[1:],
+    "weight_grad": lambda x, g, fp32: (1, 1, x.shape[-1], g.shape[-1], x.numel() // x.shape[-1]),
+    "attn_fwd": lambda q, *rest: ("attention", _attn_native_flop(True)(q)),
+    "attn_packed_fwd": lambda qkv, bias: ("attention", _attn_native_flop(True)(qkv)),
+    "attn_bwd": lambda g, o, q, *rest: ("attention", _attn_native_flop(False)(q)),
+    "attn_packed_bwd": lambda g, o, qkv, *rest: ("attention", _attn_native_flop(False)(qkv)),
+    "layernorm": lambda x, res, *rest: ("layernorm", (4.0 if res is None else 8.0) * x.numel()),
+    "layernorm_bwd": lambda g, s, x, *rest: ("layernorm", (6.0 if s is None else 8.0) * x.numel()),
+    "cast_pack": None, "softmax_fwd": None, "softmax_bwd": None, "relu_mask": None, "relu_mask_colsum": None, "colsum": None,
+}
+
+
 class GemmTimer:
-    """HIP events on the current (launch) stream around every tf_gemm / tf_gemm_scaled / tf_gemm_relu_bits /
-    tf_gemm_group call, and around every attention, LayerNorm and cross-entropy call (`by_family`)."""
+    """HIP events on the current (launch) stream around every product (tf_gemm / tf_gemm_scaled / tf_gemm_relu_bits /
+    tf_gemm_group), and around every attention, LayerNorm and cross-entropy call (`by_family`), whichever way the
+    launcher reaches the library: through the extension module or through ctypes."""
 
     def __init__(self, events=8192):
         self.records = []
@@ -241,6 +276,34 @@ class GemmTimer:
         kernels._gemm_group = timed_group
         kernels._gemm_bits = timed_bits
 
+        native = kernels.launch()
+        self._launch_orig = kernels.launch
+
+        class TimedLaunch:  # stands in for the extension module
+            def __getattr__(_, name):
+                return getattr(native, name)
+
+        timed_launch = TimedLaunch()
+        for name, describe in NATIVE_CALLS.items():
+            if describe is None:
+                continue
+
+            def timed_native(*args, _call=getattr(native, name), _describe=describe):
+                e0, e1 = self._event(), self._event()
+                e0.record()
+                out = _call(*args)
+                e1.record()
+                if out is not None and out is not False:  # handed back or refused: nothing was launched
+                    what = _describe(*args)
+                    if what[0] in FAMILY_BOUND:
+                        self.family_records.append((*what, e0, e1))
+                    else:
+                        self.records.append((what, e0, e1))
+                return out
+
+            setattr(timed_launch, name, timed_native)
+        kernels.launch = lambda: timed_launch
+
         # the other kernel families: events around the C-ABI call itself (the launchers look the entry
         # point up on the library object at every call, so replacing the attribute is enough)
         self._lib = kernels.load()
@@ -267,6 +330,7 @@ class GemmTimer:
         self._kernels._gemm_scaled = self._orig_scaled
         self._kernels._gemm_group = self._orig_group
         self._kernels._gemm_bits = self._orig_bits
+        self._kernels.launch = self._launch_orig
         for name, orig in self._lib_orig.items():
             setattr(self._lib, name, orig)
         torch.cuda.synchronize()
@@ -575,6 +639,9 @@ def main():
         launches = _lib.load_diag().tf_diag_gemm_launch_count() - count0  # kernels: a product cut along N is two
         total_ms = sum(t for _, t in gt.by_shape.values())
         gflops = gemm_flops(L, d, f, S, B) * reps
+        seen = sum(c * key_flop(key) for key, (c, _) in gt.by_shape.items())
+        if abs(seen - gflops) > 1e-6 * gflops:  # a launcher that the timer does not wrap: no figure rather than a wrong one
+            sys.exit(f"bench.py: the instrumented products account for {seen / reps:.6g} of the step's {gflops / reps:.6g} FLOP")
         achieved = gflops / (total_ms * 1e-3) / 1e12
         out["roofline"] = {
             "bound": "mfma",
