@@ -280,6 +280,29 @@ def test_register_staged_gemm(m, n, k, cfg, splits, la, lb, dev):
         assert dense or untouched(cb, n)
 
 
+# operands whose contraction is strided and whose rows are shorter than a chunk, dense (pitch 1 to 7): no stage goes
+# untested then, over one to seven stages, whole and in slices
+@pytest.mark.parametrize("m,n", [(1, 1), (3, 5), (7, 7), (5, 300), (257, 3)])
+@pytest.mark.parametrize("k", [65, 130, 200, 385])
+@pytest.mark.parametrize("cfg,splits", [(0, 1), (1, 1), (0, 2), (1, 3)])
+def test_register_staged_gemm_of_rows_shorter_than_a_chunk(m, n, k, cfg, splits, dev):
+    g = torch.Generator().manual_seed(m * 1000 + n * 10 + k)
+    a, b = torch.randn(m, k, generator=g).half(), torch.randn(k, n, generator=g).half()
+    diag, st, dt = _lib.load_diag(), _lib.stream_ptr(), _lib.dtype_code(torch.float16)
+    nb = diag.tf_diag_gemm_workspace_bytes(cfg, splits, m, n, k)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=dev)
+    exact = a.double() @ b.double()
+    bound = (a.double().abs() @ b.double().abs()) * (k * 2.0 ** -24) + exact.abs() * 2.0 ** -24  # fp32 sums in any order
+    for la, lb in ((1, 1), (0, 1), (1, 0)):
+        # behind the last row lies NaN, which a read past it would bring into a sum
+        av, bv = ((torch.cat([t.flatten(), torch.full((64,), float("nan"), dtype=t.dtype)]).to(dev), t.shape[1])
+                  for t in (a.t().contiguous() if la else a, b if lb else b.t().contiguous()))
+        cb, cv = odd_rows(torch.zeros(m, n), dev)
+        _lib.check(diag.tf_diag_gemm(st, cfg, splits, 0, dt, _lib.TF_F32, la, lb, m, n, k, av[0].data_ptr(), av[1],
+                                     bv[0].data_ptr(), bv[1], cv.data_ptr(), cv.stride(0), None, 0, ws.data_ptr(), nb))
+        assert ((cv.double().cpu() - exact).abs() <= bound).all() and untouched(cb, n)
+
+
 # the chunk that crosses the end of a row holds r elements of it; alone, behind one whole chunk, behind many
 @pytest.mark.parametrize("r", range(1, 8))
 def test_row_kernels_at_every_remainder_of_a_chunk(r, dev):
