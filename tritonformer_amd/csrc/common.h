@@ -16,7 +16,6 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -107,14 +106,6 @@ __device__ __forceinline__ u32x4 lds_ld16(const char* base, int byte_off) {
 __device__ __forceinline__ void lds_st16(char* base, int byte_off, u32x4 v) {
   *reinterpret_cast<u32x4*>(base + byte_off) = v;
 }
-// Transposing 8-byte LDS read: within each group of 16 lanes, lane i supplies
-// the address of 4 consecutive 16-bit elements; viewing the 16 loads as a
-// 4x16 matrix (row = i/4, 4 columns per lane), lane j receives column j.
-__device__ __forceinline__ u32x2 lds_ld8_tr(const char* base, int byte_off) {
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(base + byte_off));
-  return __builtin_bit_cast(u32x2, v);
-}
 
 // ---- LDS reads as volatile asm ---------------------------------------------
 // The compiler neither reorders these nor waits for them (and does not make them
@@ -131,6 +122,9 @@ template <int OFF> __device__ __forceinline__ void lds_read128_at(u32x4& dst, ui
   constexpr int IMM = OFF < 65536 ? OFF : OFF % 32768;  // the instruction's offset field is 16 bits
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr + (uint32_t)(OFF - IMM)), "n"(IMM));
 }
+// Transposing 8-byte LDS read: within each group of 16 lanes, lane i supplies
+// the address of 4 consecutive 16-bit elements; viewing the 16 loads as a
+// 4x16 matrix (row = i/4, 4 columns per lane), lane j receives column j.
 template <int OFF> __device__ __forceinline__ void lds_read64_tr_at(u32x2& dst, uint32_t addr) {
   static_assert(OFF >= 0, "offset");
   constexpr int IMM = OFF < 65536 ? OFF : OFF % 32768;  // the instruction's offset field is 16 bits

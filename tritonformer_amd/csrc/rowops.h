@@ -8,18 +8,12 @@ namespace tfa {
 template <typename T> struct Chunk {  // 16-bit types: 8 elements per 16 bytes
   static constexpr int N = 8;
   static __device__ __forceinline__ void load(const T* p, float (&v)[8]) { unpack8<T>(ld16(p), v); }
-  static __device__ __forceinline__ void load_stream(const T* p, float (&v)[8]) { unpack8<T>(ld16_stream(p), v); }
   static __device__ __forceinline__ void store(T* p, const float (&v)[8]) { st16(p, pack8<T>(v)); }
 };
 template <> struct Chunk<float> {
   static constexpr int N = 4;
   static __device__ __forceinline__ void load(const float* p, float (&v)[4]) {
     f32x4 r = *reinterpret_cast<const f32x4*>(p);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = r[i];
-  }
-  static __device__ __forceinline__ void load_stream(const float* p, float (&v)[4]) {
-    f32x4 r = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = r[i];
   }
