@@ -161,6 +161,19 @@ def test_cross_entropy_gradient_of_ragged_rows_keeps_subnormal_numbers(v, dev):
     assert ((grad / 1024 - want).abs() <= want.abs() * (2.0 ** -8 + 1e-4) + 2.0 ** -144 + 2.0 ** -149).all()
 
 
+# fp32 results against 64 bits, and against what fp32 operands and results alone cost: the argument of the exponential in
+# fp32, exponential and sum exactly rounded.  A fifth above that is left for an exponential of one unit in the last place
+# and a sum in pairs (measured 1.07 to 1.13; with serial sums and x * log2e - m * log2e in one step 1.24 to 1.33).
+@pytest.mark.parametrize("n", [2051, 4097, 20001, 65535])
+def test_softmax_of_long_ragged_rows_loses_nothing_to_its_sums(n, dev):
+    x = 2 * torch.randn(1000, n, generator=torch.Generator().manual_seed(n))
+    want = torch.softmax(x.double(), -1)
+    t = (x - x.amax(-1, keepdim=True)) * torch.tensor(1.4426950408889634)
+    e = torch.exp2(t.double()).float()
+    least = ((e * (1 / e.double().sum(-1, keepdim=True).float())).double() - want).norm()
+    assert (K.softmax_fwd(x.to(dev)[None])[0].cpu().double() - want).norm() < 1.2 * least
+
+
 # 8 / 16 / 25 chunks of 256 threads in registers (16384, 32768, 51200 entries), then the streaming forward
 @pytest.mark.parametrize("v", [1, 9, 16383, 16385, 32769, 50257, 51199, 51201, 70001])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
