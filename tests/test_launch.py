@@ -132,6 +132,26 @@ def test_products_without_sign_bits_are_tried_once(form, dev, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(3, 1), (1, 4), (3, 4)])
+def test_attention_of_expanded_operands(dims, dev, monkeypatch):
+    """Batches or heads that share their memory: every one has results of its own."""
+    torch.manual_seed(1)
+    b, nh, s, hd = 3, 4, 128, 64
+    small = [randn(b // dims[0], nh // dims[1], s, hd) for _ in range(3)]
+    q, k, v = (t.expand(b, nh, s, hd) for t in small)
+    g = randn(b, nh, s, hd)
+    full = [t.contiguous() for t in (q, k, v)]
+    want, lse = K.flash_wrapper_fwd(*full)
+    grads = K.flash_wrapper_bwd(g, want, *full, lse)
+    out, lse2 = K.flash_wrapper_fwd(q, k, v)
+    assert torch.equal(out, want) and torch.equal(lse2, lse) and out.stride() == want.stride()
+    for a, e in zip(K.flash_wrapper_bwd(g, out, q, k, v, lse), grads):
+        assert torch.equal(a, e)
+    both(monkeypatch, lambda: K.flash_wrapper_fwd(q, k, v))
+    both(monkeypatch, lambda: K.flash_wrapper_bwd(g, out, q, k, v, lse))
+
+
+@pytest.mark.gpu
 def test_refused_calls_are_refused_alike(dev, monkeypatch):
     x, w = randn(2, 8, 64), randn(64, 64)
     for call in [lambda: K.gemm(x[0], w), lambda: K.gemm(x, w[:32]), lambda: K.gemm(x.float(), w.float()),

@@ -307,6 +307,23 @@ bool attn_backward(int dt, int64_t b, int64_t nh, int64_t s, int64_t hd, const v
   });
 }
 
+// No two elements share memory (expanded dimensions and sliding windows do): results are laid out with these strides.
+bool disjoint(const Tensor& t) {
+  int64_t need = 1;
+  for (int64_t floor = 0;;) {  // dimensions in the order of their strides
+    int64_t st = INT64_MAX, span = 0;
+    for (int64_t i = 0; i < t.dim(); ++i) {
+      if (t.size(i) <= 1 || t.stride(i) < floor || t.stride(i) > st) continue;
+      if (t.stride(i) == st) return false;
+      st = t.stride(i), span = t.size(i);
+    }
+    if (st == INT64_MAX) return true;
+    if (st < need) return false;
+    need = st * span;
+    floor = st + 1;
+  }
+}
+
 // q, k, v (B, nh, S, hd): one dtype, one set of strides, rows of whole 16-byte chunks
 bool attn_inputs(PyObject* const* a, const Tensor** q, const Tensor** k, const Tensor** v) {
   *q = plain(a[0]), *k = plain(a[1]), *v = plain(a[2]);
@@ -315,7 +332,7 @@ bool attn_inputs(PyObject* const* a, const Tensor** q, const Tensor** k, const T
   for (const Tensor* o : {*q, *k, *v})
     if (o->sizes() != t.sizes() || o->strides() != t.strides() || o->scalar_type() != t.scalar_type() || !aligned(*o))
       return false;
-  return t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 &&
+  return t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && disjoint(t) &&
          attn_sizes(t.size(2), t.size(3));
 }
 

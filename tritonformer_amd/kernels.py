@@ -381,6 +381,10 @@ def _attn_layout(q, *others):
     aligned rows; otherwise everything is copied to contiguous (B, nh, S, hd)."""
     ok = q.stride(-1) == 1 and all(s % 8 == 0 for s in q.stride()[:-1]) and q.data_ptr() % 16 == 0
     ok = ok and all(t.stride() == q.stride() and t.data_ptr() % 16 == 0 for t in others)
+    # results are laid out with q's strides: no two of its elements may share memory (expanded dimensions)
+    need = 1
+    for st, n in sorted((st, n) for st, n in zip(q.stride(), q.shape) if n > 1):
+        ok, need = ok and st >= need, st * n
     if ok:
         return (q,) + tuple(others)
     return tuple(t.contiguous() for t in (q,) + tuple(others))
