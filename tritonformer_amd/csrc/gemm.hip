@@ -722,8 +722,8 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_dma_kernel(GemmParams p
 // Rows shorter than a chunk could run past the last row that way: all their stages are tested.
 // Bound by the matrix pipe and the LDS traffic around it like the direct-to-LDS kernel, 25-35 % behind it by the
 // stores through the registers.  Against the kernel before it (chunks fetched one stage ahead with a test each, result
-// stored from the accumulators, 4 and 2 bytes per lane and row): 4113 x 1733 x 2051 fp16 forward 112 -> 55 us, input
-// gradient 103 -> 54, weight gradient 121 -> 61; 8192 x 50257 x 1024 forward 4232 -> 1057 (of the element-wise one),
+// stored from the accumulators, 4 and 2 bytes per lane and row): 4113 x 1733 x 2051 fp16 forward 112 -> 57 us, input
+// gradient 103 -> 56, weight gradient 121 -> 59; 8192 x 50257 x 1024 forward 4232 -> 1057 (of the element-wise one),
 // 798 TFLOP/s; 8192 x 1024 x 2056 (all aligned, K % 64 != 0) 58 -> 46.
 // ---------------------------------------------------------------------------
 template <typename T, int R, int BK, bool KMAJOR, int NW>
