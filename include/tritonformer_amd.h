@@ -356,9 +356,8 @@ int tf_cross_entropy_fwd(void* stream, int dtype, int64_t rows, int64_t V,
  * :110-127 as one kernel).  The values equal, bit for bit, tf_cross_entropy_bwd with every
  * gout[r] = grad_scale (as a value of `dtype`); rows of dlogits are addressed like those of
  * logits with (ldd, inner_rows, outer_stride_d).  `grad_scale_dev`: one value of `dtype` in device
- * memory holding grad_scale, used only when the one-kernel form does not apply (longer rows,
- * unaligned matrices: forward and backward kernels then run one after the other); may be null
- * otherwise.  grad_scale = 1024 keeps fp16 probabilities of 1e-5 out of the subnormal range. */
+ * memory holding grad_scale, used only when the one-kernel form does not apply (longer rows:
+ * forward and backward kernels then run one after the other); may be null otherwise.  grad_scale = 1024 keeps fp16 probabilities of 1e-5 out of the subnormal range. */
 int tf_cross_entropy_fwd_grad(void* stream, int dtype, int64_t rows, int64_t V,
                               const void* logits, int64_t ld, int64_t inner_rows, int64_t outer_stride,
                               const int64_t* labels, void* loss, float* lse,

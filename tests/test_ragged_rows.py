@@ -331,3 +331,42 @@ def test_row_kernels_at_every_remainder_of_a_chunk(r, dev):
     test_layernorm_rows(2048 + r, torch.float16, True, dev)
     test_softmax_rows(4096 + r, torch.float16, dev)
     test_cross_entropy_rows(51200 + r, torch.float16, dev)
+
+
+# a NaN or an infinity stays in its row (and its column, where a kernel sums over rows): what is fetched beyond the end of
+# a row, or twice, belongs to no result
+@pytest.mark.parametrize("n", [33, 65, 519, 1021, 2051, 4099])
+def test_non_finite_values_stay_in_their_rows(n, dev):
+    g = torch.Generator().manual_seed(n)
+    x, dy = (torch.randn(1, 13, n, generator=g).half().to(dev) for _ in range(2))
+    gamma, beta = (torch.randn(n, generator=g).half().to(dev) for _ in range(2))
+    lab = torch.randint(0, n, (13,), generator=g).to(dev)
+    bad = x.clone()
+    bad[0, 3, n - 1], bad[0, 7, 0], bad[0, 12, n - 1] = float("nan"), float("inf"), float("inf")
+    keep = [r for r in range(13) if r not in (3, 7, 12)]
+
+    def outcomes(t):
+        y, mean, rstd = K.layernorm_fwd(t, gamma, beta, 1e-5)
+        total, z, _, _ = K.add_layernorm_fwd(t, dy, gamma, beta, 1e-5)
+        s = K.softmax_fwd(t)
+        loss, lse, _, _ = K.cross_entropy_fwd(t[0], lab)
+        ds = K.softmax_bwd(dy, s)
+        dl = K.cross_entropy_bwd(torch.ones_like(loss), t[0], lab, lse)
+        return [y[0], K.layernorm_bwd(dy, t, gamma, mean, rstd)[0][0], total[0], z[0], s[0], ds[0], loss[:, None], dl]
+
+    for a, b in zip(outcomes(bad), outcomes(x)):
+        assert torch.equal(a[keep], b[keep]) and torch.isfinite(a[keep]).all()
+    # ReLU mask and its column sums: an activation that is NaN is not positive
+    act = bad.clone()
+    act[0, 5, n - 1] = 1.0
+    grad = dy.clone()
+    grad[0, 5, n - 1] = float("nan")
+    masked, sums = K.mask_grad_sums(grad, act, torch.float32)
+    assert masked[0, 3, n - 1] == 0 and torch.isnan(sums[n - 1]) and torch.isfinite(sums[: n - 1]).all()
+    # products: the last row of A and the last column of B, which lie at the edges of their tiles
+    b = torch.randn(n, 67, generator=g).half().to(dev)
+    worse = b.clone()
+    worse[0, 66] = float("inf")
+    out, want = K.gemm(bad, worse), K.gemm(x, b)
+    assert torch.equal(out[0, keep, :66], want[0, keep, :66]) and not torch.isfinite(out[0, 3]).any()
+    assert not torch.isfinite(out[0, :, 66]).any()
