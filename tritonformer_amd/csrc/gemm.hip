@@ -609,16 +609,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
       for (int m = 0; m < NMFMA; ++m) {
         const int i = m / TN, j = m % TN;
         if (last && m == HAND && MORE) {
-          // (Measurement switches, never defined by the build: TF_ABL_NO_LOAD_WAIT_TILE / TF_ABL_NO_HANDOVER_BARRIER_TILE
-          // = BM * BN of the configuration whose wait / barrier is compiled out.  The results of such a build are
-          // wrong; its step time says what the wait costs -- how the need for a third stage was found.)
-#ifdef TF_ABL_NO_LOAD_WAIT_TILE
-          if (BM * BN != TF_ABL_NO_LOAD_WAIT_TILE)
-#endif
           wait_vmcnt<(NS == 3 && MORE2) ? LPS : 0>();  // this wave's loads of the next stage have landed
-#ifdef TF_ABL_NO_HANDOVER_BARRIER_TILE
-          if (BM * BN != TF_ABL_NO_HANDOVER_BARRIER_TILE)
-#endif
           barrier();        // ... and everyone's; everyone has read the last operands of `cur`
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1111,16 +1102,13 @@ static GemmPlan plan_for(int cfg, int64_t M, int64_t N, int64_t K, double* cost_
   // gradients: few output tiles, long contraction); never beyond one full round of
   // workgroups, and every slice keeps at least 16 steps so that the fp32 partial
   // traffic stays small.
-#ifndef TF_STEP_256x128
-#define TF_STEP_256x128 1.0
-#endif
   const double fixed = pl.bm * pl.bn >= 256 * 256 ? 10.0 : 7.0;
   // register-staged: 8192 x 1024 x 50257 takes 393 steps of 256x256 tiles in 911 us, 786 of 128x128 in 1340
   // (with the figures of the direct-to-LDS tiles 960 x 768 x 50257 ran on 128x128 tiles: 160 us instead of 129)
   // Over 46 products of odd extents (64 to 16384, 64 to 8192, 64 to 4096, all layouts) the choice was within a tenth of the
   // better tile every time.
   const double per_step = !kCfgs[cfg].dma ? (pl.bm * pl.bn >= 256 * 256 ? 2.25 : 1.6)
-                          : pl.bm * pl.bn >= 256 * 256 ? 1.65 : (pl.bm * pl.bn >= 256 * 128 ? TF_STEP_256x128 : 1.1);
+                          : pl.bm * pl.bn >= 256 * 256 ? 1.65 : (pl.bm * pl.bn >= 256 * 128 ? 1.0 : 1.1);
   auto cost_of = [&](int64_t nsplit, int64_t steps) {
     const int64_t rounds = (tiles * nsplit + slots - 1) / slots;
     double c = (double)rounds * (fixed + per_step * (double)steps);
@@ -1137,11 +1125,7 @@ static GemmPlan plan_for(int cfg, int64_t M, int64_t N, int64_t K, double* cost_
   // A long contraction whose tiles leave part of a round idle (0.75 of a round: the LM-head input gradient
   // of a narrow model) may be cheaper in more, shorter slices that fill whole rounds: by the cost model,
   // among slice counts that keep 16 steps per slice, and only when it wins by a tenth.
-#ifdef TF_NO_SPLIT_SEARCH
-  if (false) {
-#else
   if (allow_split && force_splits <= 0 && tiles % slots != 0 && ksteps >= 256) {
-#endif
     double best = cost_of(splits, (ksteps + splits - 1) / splits) * 0.9;
     for (int64_t sp = 2; sp <= 16 && ksteps / sp >= 16; ++sp) {
       const double c = cost_of(sp, (ksteps + sp - 1) / sp);
@@ -1224,11 +1208,7 @@ static int launch_dma(hipStream_t st, const GemmParams& p) {
 // The register-staged kernel handles everything (ragged extents, unaligned
 // pointers); the direct-to-LDS kernel needs the vector conditions and a
 // contraction extent that is a multiple of its BK.
-// LDS stages of the 256x128 / 128x256 configurations (a diagnostic build may impose 2)
-#ifndef TF_STAGES_NARROW
-#define TF_STAGES_NARROW 3
-#endif
-constexpr int kStagesNarrow = TF_STAGES_NARROW;
+constexpr int kStagesNarrow = 3;  // LDS stages of the 256x128 / 128x256 configurations
 
 template <typename T, bool AK, bool BKM>
 static int launch_cfg(hipStream_t st, bool vec, const GemmPlan& pl, const GemmParams& p) {
@@ -1621,9 +1601,6 @@ GroupPlan plan_group(int la, int lb, int count, const tf_gemm_problem* pr) {
     // workgroups; the split tail pays its fp32 partials and the reduce pass (about six steps' worth).
     bool same_k = true;
     for (int i = 1; i < count; ++i) same_k = same_k && pr[i].K == pr[0].K;
-#ifdef TF_NO_GROUP_CUT
-    same_k = false;
-#endif
     if (splits == 1 && tiles > cus && tiles % cus != 0 && same_k && count < kMaxGroup) {
       const int64_t ksteps = pr[0].K / 64;
       const int64_t rounds_whole = tiles / cus;
