@@ -312,6 +312,40 @@ def test_short_contractions_take_every_peeled_form_of_the_main_loop(layouts, dev
                 assert_close(out, want, name=f"{layouts} K={K} cfg {cfg} splits {splits}")
 
 
+@pytest.mark.parametrize("layouts", ["fwd", "dx", "dw"])
+@pytest.mark.parametrize("M,N", [(8, 8), (64, 64), (72, 56), (128, 192), (200, 328)])
+def test_small_tiles_give_the_bits_of_the_large_ones(layouts, M, N, dev):
+    """The configurations for few tiles (64x64, 128x64) at the edges of their tiles: one to five stages (their main
+    loop peels three), bias and ReLU, and slices of one stage.  An unsplit contraction sums the same steps in the same order
+    as the 128x128 tiles do, so the bits are the same; slices are rounded once more: half an ulp of fp16 per element."""
+    from tritonformer_amd import _lib
+
+    d = _lib.load_diag()
+    g = torch.Generator().manual_seed(37)
+    la, lb = {"fwd": (0, 1), "dx": (0, 0), "dw": (1, 1)}[layouts]
+    stream = torch.cuda.current_stream().cuda_stream
+    bias = torch.randn(N, generator=g).half().to(dev)
+    for K in (64, 128, 192, 256, 320):
+        a = torch.randn((M, K) if la == 0 else (K, M), generator=g).half().to(dev)
+        b = (torch.randn((N, K) if lb == 0 else (K, N), generator=g) / K ** 0.5).half().to(dev)
+
+        def run(cfg, splits=1, epilogue=False):
+            out = torch.full((M + 1, N), 7.0, dtype=torch.float16, device=dev)
+            nb = d.tf_diag_gemm_workspace_bytes(cfg, splits, M, N, K)
+            ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=dev)
+            _lib.check(d.tf_diag_gemm(stream, cfg, splits, 0, 0, 0, la, lb, M, N, K, a.data_ptr(), a.stride(0),
+                                      b.data_ptr(), b.stride(0), out.data_ptr(), N, bias.data_ptr() if epilogue else None,
+                                      int(epilogue), ws.data_ptr(), nb))
+            assert (out[M] == 7.0).all(), "row beyond the result written"
+            return out[:M]
+
+        for cfg in (6, 7):
+            assert torch.equal(run(cfg), run(3)), f"K={K} cfg {cfg}"
+            assert torch.equal(run(cfg, epilogue=True), run(3, epilogue=True)), f"K={K} cfg {cfg}, bias and ReLU"
+            want = (a.float() if la == 0 else a.float().T) @ (b.float().T if lb == 0 else b.float())
+            assert (run(cfg, K // 64).float() - want).abs().max() <= 2 ** -10 * want.abs().max()
+
+
 @pytest.mark.parametrize("dims,use_bias", [((2, 128, 256, 1024), False), ((3, 77, 136, 264), True),
                                            ((1, 100, 333, 129), True)])
 def test_fused_mlp_equals_two_functions(dims, use_bias, dev):

@@ -26,6 +26,7 @@
 // Workgroup ids are remapped so that each XCD (which receive ids round-robin)
 // works on a compact block of neighbouring tiles and shares the A/B panels
 // through its own L2.  The number of XCDs and of CUs is read from the device.
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -118,11 +119,15 @@ struct DmaPanel {
   static constexpr int WLOADS = NCHUNK / 64;   // wave-level loads per panel
   static constexpr int PER_WAVE = WLOADS / NW;
   static_assert(WLOADS % NW == 0 && PER_WAVE >= 1, "panel must divide evenly over the waves");
-  static_assert(KMAJOR ? (CPR == 4 || CPR == 8) : (CPR >= 16), "unsupported panel shape");
+  static_assert(KMAJOR ? (CPR == 4 || CPR == 8) : (CPR >= 4), "unsupported panel shape");
 
+  // K-minor: a transposing read takes 32 bytes of each of four neighbouring rows per 16 lanes.  Rows of 256 bytes and
+  // more begin at the same bank, rows of 128 bytes at every other half of them; four rows of 64 bytes fill them.
   static __device__ __forceinline__ int swz(int lrow, int c) {
     if constexpr (KMAJOR) return c ^ ((lrow / (16 / CPR)) % CPR);
-    else return c ^ ((lrow & 3) << 2);
+    else if constexpr (CPR >= 16) return c ^ ((lrow & 3) << 2);
+    else if constexpr (CPR == 8) return c ^ ((lrow & 3) << 1);
+    else return c;
   }
 
   // Global address of each of this lane's chunks for the step starting at kbeg.
@@ -485,14 +490,14 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
   // Mask bits of a 16-bit result: this lane's bytes (one per 8-element chunk it will store, in the
   // order of the write-out) are requested here, a whole main loop ahead of their use -- loaded in
   // the write-out they would sit between every LDS read and the store that needs both.
-  static_assert(64 / (WTN * 2 / 16) * 4 == 32, "four wave-wide stores per 32-row block of a 16-bit result");
+  static_assert(WTN == 64 || WTN == 32, "four or two wave-wide stores per 32-row block of a 16-bit result");
   uint8_t sign_bytes[TM][4] = {};
   if (p.sign_in && !p.out_f32) {
     constexpr int CH16 = WTN * 2 / 16, RPI16 = 64 / CH16;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
+      for (int rr = 0; rr < 32 / RPI16; ++rr) {
         const int m = m0 + wm * WTM + i * 32 + rr * RPI16 + lane / CH16, n = n0 + wn * WTN + (lane % CH16) * 8;
         if (m < p.M && n < p.N) sign_bytes[i][rr] = ((const uint8_t*)p.sign_in)[(int64_t)m * p.ldsign + (n >> 3)];
       }
@@ -654,8 +659,8 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
     if (kt < nk) stage(smem + (kt & 1) * STAGE, smem + ((kt + 1) & 1) * STAGE, nullptr, no_t(), no_t(), no_t());
   }
 
-  static_assert(NW * 32 * (WTN * 4 + 16) <= 2 * STAGE, "epilogue staging must fit in the pipeline LDS");
-  static_assert(NW * 32 * (WTN * 2 + 16) + BM * BN / 8 <= 2 * STAGE, "... and so must the image of a tile's sign bits behind it");
+  static_assert(NW * 32 * (WTN * 4 + 16) <= NS * STAGE, "epilogue staging must fit in the pipeline LDS");
+  static_assert(NW * 32 * (WTN * 2 + 16) + BM * BN / 8 <= NS * STAGE, "... and so must the image of a tile's sign bits behind it");
   const bool full = m0 + BM <= p.M && n0 + BN <= p.N;  // no row or column of the tile lies outside C: stores need no test
   if (p.splits > 1) {
     // fp32 partial of this contraction slice: a plain (M, N) matrix, written like an fp32 result
@@ -683,13 +688,15 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
     } else {
       // the two sign-bit launches of a fused MLP, on full tiles of a plain (unchunked) result whose bit rows take
       // 16-byte pieces: write-outs of their own, nothing tested per store
-      const bool bits_fast = full && !p.mask && !p.alpha && p.chunk_skip == 0 && p.ldsign % 16 == 0 &&
+      const bool bits_fast = BN >= 128 && full && !p.mask && !p.alpha && p.chunk_skip == 0 && p.ldsign % 16 == 0 &&
                              ((reinterpret_cast<uintptr_t>(p.sign_out) | reinterpret_cast<uintptr_t>(p.sign_in)) & 15) == 0;
-      if (plain && full) gemm_epilogue_lds<T, T, TM, TN, WTM, WTN, true, true>(p, acc, smem, m0, n0, wm, wn, wave, lane);
-      else if (plain) gemm_epilogue_lds<T, T, TM, TN, WTM, WTN, true>(p, acc, smem, m0, n0, wm, wn, wave, lane);
-      else if (bits_fast && p.sign_out && p.relu) gemm_epilogue_bits<T, BM, BN, TM, TN, WTM, WTN, true>(p, acc, smem, m0, n0, wm, wn, wave, lane, sign_bytes);
-      else if (bits_fast && p.sign_in && !p.bias && !p.relu) gemm_epilogue_bits<T, BM, BN, TM, TN, WTM, WTN, false>(p, acc, smem, m0, n0, wm, wn, wave, lane, sign_bytes);
-      else gemm_epilogue_lds<T, T, TM, TN, WTM, WTN>(p, acc, smem, m0, n0, wm, wn, wave, lane, sign_bytes);
+      if (plain && full) return gemm_epilogue_lds<T, T, TM, TN, WTM, WTN, true, true>(p, acc, smem, m0, n0, wm, wn, wave, lane);
+      if (plain) return gemm_epilogue_lds<T, T, TM, TN, WTM, WTN, true>(p, acc, smem, m0, n0, wm, wn, wave, lane);
+      if constexpr (BN >= 128) {
+        if (bits_fast && p.sign_out && p.relu) return gemm_epilogue_bits<T, BM, BN, TM, TN, WTM, WTN, true>(p, acc, smem, m0, n0, wm, wn, wave, lane, sign_bytes);
+        if (bits_fast && p.sign_in && !p.bias && !p.relu) return gemm_epilogue_bits<T, BM, BN, TM, TN, WTM, WTN, false>(p, acc, smem, m0, n0, wm, wn, wave, lane, sign_bytes);
+      }
+      gemm_epilogue_lds<T, T, TM, TN, WTM, WTN>(p, acc, smem, m0, n0, wm, wn, wave, lane, sign_bytes);
     }
   }
 }
@@ -1070,6 +1077,8 @@ static const TileCfg kCfgs[] = {
     {128, 128, 64, 4, 1},  // 3: direct-to-LDS, 64 KB LDS, two workgroups per CU, wave tile 64x64
     {256, 128, 64, 8, 1},  // 4: direct-to-LDS, three stages = 144 KB LDS, waves 4x2, wave tile 64x64
     {128, 256, 64, 8, 1},  // 5: direct-to-LDS, three stages = 144 KB LDS, waves 2x4, wave tile 64x64
+    {64, 64, 64, 4, 1},    // 6: direct-to-LDS, three stages = 48 KB LDS, waves 2x2, wave tile 32x32: few tiles
+    {128, 64, 64, 4, 1},   // 7: direct-to-LDS, three stages = 72 KB LDS, waves 4x1, wave tile 32x64: few tiles
 };
 constexpr int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
 
@@ -1085,7 +1094,7 @@ constexpr GemmForce kNoForce = {-1, 0, 0};
 // rocprofv3 kernel durations on MI355X: one "round" of workgroups (one per CU)
 // costs a fixed part (launch, cold first loads, result write-out) plus a part
 // per 64-wide contraction step.
-static GemmPlan plan_for(int cfg, int64_t M, int64_t N, int64_t K, double* cost_us, bool allow_split,
+static GemmPlan plan_for(int64_t cus, int cfg, int64_t M, int64_t N, int64_t K, double* cost_us, bool allow_split,
                          int force_splits = 0) {
   GemmPlan pl;
   pl.cfg = cfg;
@@ -1097,7 +1106,7 @@ static GemmPlan plan_for(int cfg, int64_t M, int64_t N, int64_t K, double* cost_
   const int64_t tiles = (int64_t)pl.tiles_m * pl.tiles_n;
   const int64_t ksteps = (K + pl.bk - 1) / pl.bk;
   const int wg_per_cu = pl.bm * pl.bn <= 128 * 128 ? 2 : 1;
-  const int64_t slots = (int64_t)device_shape().cus * wg_per_cu;
+  const int64_t slots = cus * wg_per_cu;
   // Split the contraction only when the tiles alone leave most CUs idle (weight
   // gradients: few output tiles, long contraction); never beyond one full round of
   // workgroups, and every slice keeps at least 16 steps so that the fp32 partial
@@ -1143,14 +1152,35 @@ static GemmPlan plan_for(int cfg, int64_t M, int64_t N, int64_t K, double* cost_
   return pl;
 }
 
-static GemmPlan make_plan(int64_t M, int64_t N, int64_t K, bool vec, bool allow_split = true,
+// Time (microseconds) of a direct-to-LDS launch that leaves CUs or their second workgroup idle, where the cost above --
+// made for whole rounds -- is 1.3 to 2 times too high: a fixed part plus a time per 64-wide step that rises with the
+// workgroups per CU (`fill`), since operands come faster and the clock is higher while few CUs work.  Fits to 348 products
+// of 16 to 4096 rows, 128 to 6144 columns and contractions of 64 to 8192, operand B from HBM.
+static double part_round_us(int64_t cus, const GemmPlan& pl, int64_t M, int64_t N) {
+  const double steps = (double)(pl.k_per_split / pl.bk);
+  const double fill = (double)((int64_t)pl.tiles_m * pl.tiles_n * pl.splits) / (double)cus;
+  auto rise = [](double x, double from, double to) { return x <= from ? 0.0 : x >= to ? 1.0 : (x - from) / (to - from); };
+  const double more = 0.7 * std::max(0.0, fill - 1);  // start and write-out of every further workgroup of a CU
+  double c = 0;
+  switch (pl.cfg) {
+    case 2: c = 5.4 + steps * (0.95 + 0.70 * rise(fill, 0.35, 1)); break;
+    case 3: c = 2.5 + steps * (0.67 + 0.43 * rise(fill, 0.6, 2)); break;
+    case 4: c = 3.8 + steps * (0.64 + 0.36 * rise(fill, 0.25, 1)); break;
+    case 6: c = 2.7 + more + steps * std::max(0.27 + 0.05 * rise(fill, 0.5, 1), 0.27 * fill); break;
+    case 7: c = 2.9 + more + steps * std::max(0.36 + 0.14 * rise(fill, 0.5, 1), 0.40 * fill); break;
+  }
+  if (pl.splits > 1) c += 3.0 + (pl.splits + 0.5) * (double)M * (double)N * 4.0 / 5.0e6;
+  return c;
+}
+
+static GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec, bool allow_split = true,
                           double* cost_us = nullptr, const GemmForce& force = kNoForce) {
   const bool dma = vec && K % 64 == 0;
   if (cost_us) *cost_us = -1.0;  // stays negative when the configuration is forced
   if (force.cfg >= 0 && force.cfg < kNumCfgs) {
     int cfg = force.cfg;
     if (kCfgs[cfg].dma && !dma) cfg = kCfgs[cfg].bm * kCfgs[cfg].bn >= 256 * 256 ? 0 : 1;  // register-staged twin
-    return plan_for(cfg, M, N, K, nullptr, allow_split, force.splits);
+    return plan_for(cus, cfg, M, N, K, nullptr, allow_split, force.splits);
   }
   // candidates: 256x256 and 256x128 / 128x128 tiles, direct-to-LDS kernels when their
   // preconditions hold, the register-staged twins otherwise
@@ -1158,12 +1188,27 @@ static GemmPlan make_plan(int64_t M, int64_t N, int64_t K, bool vec, bool allow_
   const int cand_reg[2] = {0, 1};
   const int* cand = dma ? cand_dma : cand_reg;
   const int ncand = dma ? 3 : 2;
-  GemmPlan best = plan_for(cand[0], M, N, K, nullptr, allow_split, force.splits);
+  GemmPlan best = plan_for(cus, cand[0], M, N, K, nullptr, allow_split, force.splits);
   double best_cost = 1e30;
   for (int i = 0; i < ncand; ++i) {
     double c;
-    const GemmPlan pl = plan_for(cand[i], M, N, K, &c, allow_split, force.splits);
+    const GemmPlan pl = plan_for(cus, cand[i], M, N, K, &c, allow_split, force.splits);
     if (c < best_cost) { best_cost = c; best = pl; }
+  }
+  // Tiles that do not fill one round of workgroups: smaller ones occupy more CUs.  A 256x128 tile's step takes 0.64 us on
+  // an idle chip, a 64x64 one's 0.27, and start and write-out shrink with the tile: 128 x 1024 x 1024 14.4 -> 6.9 us,
+  // 960 x 768 x 768 12.1 -> 6.3, 2048 x 1024 x 1024 15.1 -> 9.5.  Beyond one round the larger tiles are the better ones
+  // throughout (2048 x 4096 x 1024: 21 against 29 us).  The slices of the contraction stay those of the larger tile: the
+  // same sums in the same order, whatever the tile.
+  const int64_t wgs = (int64_t)best.tiles_m * best.tiles_n * best.splits;
+  if (dma && wgs <= cus * (best.cfg == 3 ? 2 : 1)) {
+    const GemmPlan best_large = best;
+    double best_us = 0.95 * part_round_us(cus, best, M, N);
+    for (int cfg : {6, 7}) {
+      const GemmPlan pl = plan_for(cus, cfg, M, N, K, nullptr, allow_split, best_large.splits);
+      const double us = part_round_us(cus, pl, M, N);
+      if (us < best_us) { best_us = us; best = pl; best_cost = std::min(best_cost, us); }
+    }
   }
   if (cost_us) *cost_us = best_cost;
   return best;
@@ -1208,7 +1253,7 @@ static int launch_dma(hipStream_t st, const GemmParams& p) {
 // The register-staged kernel handles everything (ragged extents, unaligned
 // pointers); the direct-to-LDS kernel needs the vector conditions and a
 // contraction extent that is a multiple of its BK.
-constexpr int kStagesNarrow = 3;  // LDS stages of the 256x128 / 128x256 configurations
+constexpr int kStagesNarrow = 3;  // LDS stages of the configurations below 256x256 but 128x128
 
 template <typename T, bool AK, bool BKM>
 static int launch_cfg(hipStream_t st, bool vec, const GemmPlan& pl, const GemmParams& p) {
@@ -1218,6 +1263,8 @@ static int launch_cfg(hipStream_t st, bool vec, const GemmPlan& pl, const GemmPa
       case 3: return launch_dma<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, p);
       case 4: return launch_dma<T, 256, 128, 64, 4, 2, 2, AK, BKM, kStagesNarrow>(st, p);
       case 5: return launch_dma<T, 128, 256, 64, 2, 4, 2, AK, BKM, kStagesNarrow>(st, p);
+      case 6: return launch_dma<T, 64, 64, 64, 2, 2, 2, AK, BKM, kStagesNarrow>(st, p);
+      case 7: return launch_dma<T, 128, 64, 64, 4, 1, 2, AK, BKM, kStagesNarrow>(st, p);
     }
   }
   if (pl.bm == 256 && pl.bn == 256) return launch_reg<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
@@ -1319,11 +1366,8 @@ static int64_t round_unit(int64_t tiles_m, int64_t cus) {
 // that runs as a split contraction on the otherwise idle CUs instead of a nearly empty last
 // round (LM-head weight gradient: 4 x 197 tiles = 3 rounds + 20 tiles).  Returns the number
 // of tail columns, 0 for no cut.
-static int64_t tail_columns(int64_t M, int64_t N, int64_t K, bool vec, bool allow_split, const GemmForce& force) {
-  if (!allow_split || force.cfg >= 0 || force.splits > 0 || K < 32 * 64 || (force.flags & 64)) return 0;
-  const int64_t cus = device_shape().cus;
-  double uncut;
-  const GemmPlan pl = make_plan(M, N, K, vec, allow_split, &uncut);
+static int64_t tail_columns(int64_t cus, int64_t M, int64_t N, int64_t K, const GemmPlan& pl) {
+  if (K < 32 * 64) return 0;
   const int64_t tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
   const int64_t unit = round_unit(tiles_m, cus);
   const int64_t tn1 = (tiles_n / unit) * unit;
@@ -1341,26 +1385,58 @@ static int64_t tail_columns(int64_t M, int64_t N, int64_t K, bool vec, bool allo
 // together are cheaper than the best single launch (q/k/v projection 8192 x 3072 x 1024: one
 // round of 256x256 tiles + 1024 columns of 128x128 tiles, 0.2 ms per training step less than
 // three rounds of 128x128 tiles).
-static int64_t round_cut_columns(int64_t M, int64_t N, int64_t K, bool vec, bool allow_split, const GemmForce& force,
-                                 bool allow_cut) {
-  if (!allow_cut || force.cfg >= 0 || force.splits > 0 || !(vec && K % 64 == 0) || (force.flags & 64)) return 0;
-  const int64_t cus = device_shape().cus;
-  double uncut, whole, rest;
-  (void)make_plan(M, N, K, vec, allow_split, &uncut);
-  if (uncut < 0) return 0;
+static int64_t round_cut_columns(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec, bool allow_split, double uncut) {
+  if (!(vec && K % 64 == 0) || uncut < 0) return 0;
+  double whole, rest;
   const int64_t tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
   if (tiles_m * tiles_n <= cus) return 0;
   const int64_t unit = round_unit(tiles_m, cus);
   const int64_t tn1 = (tiles_n / unit) * unit;
   if (tn1 <= 0 || tn1 * 256 >= N) return 0;
-  (void)plan_for(2, M, tn1 * 256, K, &whole, false);
-  (void)make_plan(M, N - tn1 * 256, K, vec, allow_split, &rest);
+  (void)plan_for(cus, 2, M, tn1 * 256, K, &whole, false);
+  (void)make_plan(cus, M, N - tn1 * 256, K, vec, allow_split, &rest);
   if (rest < 0) return 0;
   return whole + rest + 3.0 < uncut ? N - tn1 * 256 : 0;
 }
 
-static int64_t single_need(int64_t M, int64_t N, int64_t K, bool vec) {
-  const GemmPlan pl = make_plan(M, N, K, vec);
+// How a product is run: cut along N (`tail` columns, 0 = uncut) or as `plan`.  Cut along N only where the result is one
+// matrix and no mask rides on it; split only where neither a mask nor sign bits do.
+enum RouteKind { kRoutePlain, kRouteSigns, kRouteMask, kRouteChunked };
+struct Route {
+  GemmPlan plan;
+  int64_t tail;
+};
+static Route find_route(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec, RouteKind kind) {
+  const bool split = kind == kRoutePlain || kind == kRouteChunked;
+  double uncut;
+  Route r = {make_plan(cus, M, N, K, vec, split, &uncut), 0};
+  if (kind == kRoutePlain) r.tail = tail_columns(cus, M, N, K, r.plan);
+  if (r.tail == 0 && (kind == kRoutePlain || kind == kRouteSigns)) r.tail = round_cut_columns(cus, M, N, K, vec, split, uncut);
+  if (r.tail > 0 && kind == kRouteSigns) {
+    // the bits of both parts have to be served (a cut at a multiple of 256 columns keeps whole bytes and the 16-byte
+    // pieces of the bit rows)
+    const GemmPlan p1 = make_plan(cus, M, N - r.tail, K, vec, false), p2 = make_plan(cus, M, r.tail, K, vec, false);
+    if (!(kCfgs[p1.cfg].dma && kCfgs[p2.cfg].dma && K % p1.bk == 0 && K % p2.bk == 0)) r.tail = 0;
+  }
+  return r;
+}
+// The route follows from these figures alone and takes 1 to 4 us to find -- as long as a launch -- several times per
+// product (workspace, both alignments, parts of a cut): each thread keeps the last ones it found, 256 at most.
+static Route route(int64_t M, int64_t N, int64_t K, bool vec, RouteKind kind) {
+  struct Entry {
+    int64_t M, N, K, tag;
+    Route r;
+  };
+  static thread_local Entry cache[256];  // all zero at first: no product has M = 0
+  const int64_t cus = device_shape().cus, tag = cus * 8 + kind * 2 + (vec ? 1 : 0);
+  const uint64_t h = ((uint64_t)M * 0x9e3779b97f4a7c15u + (uint64_t)N * 0xc2b2ae3d27d4eb4fu + (uint64_t)K * 0x165667b19e3779f9u + (uint64_t)tag) *
+                     0x9e3779b97f4a7c15u;
+  Entry& e = cache[h >> 56];
+  if (e.M != M || e.N != N || e.K != K || e.tag != tag) e = {M, N, K, tag, find_route(cus, M, N, K, vec, kind)};
+  return e.r;
+}
+
+static int64_t plan_need(const GemmPlan& pl, int64_t M, int64_t N) {
   return pl.splits > 1 ? (int64_t)pl.splits * M * N * (int64_t)sizeof(float) : 0;
 }
 
@@ -1371,15 +1447,10 @@ extern "C" int64_t tf_gemm_workspace_bytes(int layout_a, int layout_b, int64_t M
   // the caller's alignment is unknown here: cover both kernel families
   int64_t need = 0;
   for (int vec = 0; vec < 2; ++vec) {
-    int64_t n = single_need(M, N, K, vec != 0);
-    int64_t tail = tail_columns(M, N, K, vec != 0, true, kNoForce);
-    if (tail == 0) tail = round_cut_columns(M, N, K, vec != 0, true, kNoForce, true);
-    if (tail > 0) {
-      const int64_t n1 = single_need(M, N - tail, K, vec != 0), n2 = single_need(M, tail, K, vec != 0);
-      if (n1 > n) n = n1;
-      if (n2 > n) n = n2;
-    }
-    if (n > need) need = n;
+    const Route r = route(M, N, K, vec != 0, kRoutePlain);
+    need = std::max(need, plan_need(r.plan, M, N));
+    if (r.tail > 0)
+      for (int64_t n : {N - r.tail, r.tail}) need = std::max(need, plan_need(route(M, n, K, vec != 0, kRouteChunked).plan, M, n));
   }
   return need;
 }
@@ -1432,39 +1503,29 @@ static int gemm_entry(void* stream, int dtype, int out_dtype, int layout_a, int 
   const bool vec = aligned16(A) && aligned16(B) && aligned16(C) && (!bias || aligned16(bias)) && a_contig % 8 == 0 &&
                    b_contig % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && N % 8 == 0 && ldc % 8 == 0 &&
                    (!mask_act || (aligned16(mask_act) && ld_mask % 8 == 0));
-  if (chunk_n == N) {
-    // (a launch with sign bits takes no split contraction: its cut is the one into unsplit products, and only
-    // where the bits of both parts are served -- a cut at a multiple of 256 columns keeps whole bytes and the
-    // 16-byte pieces of the bit rows)
-    const bool may_split = mask_act == nullptr && !signs;
-    int64_t tail = signs ? 0 : tail_columns(M, N, K, vec, may_split, force);
-    if (tail == 0) tail = round_cut_columns(M, N, K, vec, may_split, force, mask_act == nullptr);
-    if (tail > 0 && signs) {
-      const GemmPlan p1 = make_plan(M, N - tail, K, vec, false, nullptr, force), p2 = make_plan(M, tail, K, vec, false, nullptr, force);
-      if (!(kCfgs[p1.cfg].dma && kCfgs[p2.cfg].dma && K % p1.bk == 0 && K % p2.bk == 0)) tail = 0;
-    }
-    if (tail > 0) {  // whole rounds first, then the narrow remainder as a split contraction
-      const int64_t n1 = N - tail;
-      const int64_t osz = out_dtype == TF_F32 ? 4 : 2;
-      const char* b2 = (const char*)B + (layout_b == TF_OP_KMAJOR ? n1 * ldb : n1) * 2;
-      const void* bias2 = bias ? (const char*)bias + n1 * 2 : nullptr;
-      const void* mask2 = mask_act ? (const char*)mask_act + n1 * 2 : nullptr;
-      void* so2 = sign_out ? (char*)sign_out + n1 / 8 : nullptr;
-      const void* si2 = sign_in ? (const char*)sign_in + n1 / 8 : nullptr;
-      const int rc = gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, n1, K, A, lda, B, ldb, C, ldc, 0, 0, bias,
-                                relu, mask_act, ld_mask, workspace, workspace_bytes, sign_out, sign_in, ld_sign, force, alpha);
-      if (rc != TF_OK) return rc;
-      return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, tail, K, A, lda, b2, ldb, (char*)C + n1 * osz,
-                        ldc, 0, 0, bias2, relu, mask2, ld_mask, workspace, workspace_bytes, so2, si2, ld_sign, force,
-                        alpha);
-    }
+  const bool forced = force.cfg >= 0 || force.splits > 0 || (force.flags & 64);
+  Route rt;
+  if (forced) rt = {make_plan(device_shape().cus, M, N, K, vec, mask_act == nullptr && !signs, nullptr, force), 0};
+  else rt = route(M, N, K, vec, mask_act ? kRouteMask : signs ? kRouteSigns : chunk_n != N ? kRouteChunked : kRoutePlain);
+  if (rt.tail > 0) {  // whole rounds first, then the narrow remainder as a split contraction
+    const int64_t tail = rt.tail, n1 = N - tail;
+    const int64_t osz = out_dtype == TF_F32 ? 4 : 2;
+    const char* b2 = (const char*)B + (layout_b == TF_OP_KMAJOR ? n1 * ldb : n1) * 2;
+    const void* bias2 = bias ? (const char*)bias + n1 * 2 : nullptr;
+    void* so2 = sign_out ? (char*)sign_out + n1 / 8 : nullptr;
+    const void* si2 = sign_in ? (const char*)sign_in + n1 / 8 : nullptr;
+    const int rc = gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, n1, K, A, lda, B, ldb, C, ldc, 0, 0, bias,
+                              relu, nullptr, 0, workspace, workspace_bytes, sign_out, sign_in, ld_sign, force, alpha);
+    if (rc != TF_OK) return rc;
+    return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, tail, K, A, lda, b2, ldb, (char*)C + n1 * osz,
+                      ldc, 0, 0, bias2, relu, nullptr, 0, workspace, workspace_bytes, so2, si2, ld_sign, force, alpha);
   }
-  const GemmPlan pl = make_plan(M, N, K, vec, mask_act == nullptr && !signs, nullptr, force);
+  const GemmPlan pl = rt.plan;
   // the sign bits exist in the write-out of the direct-to-LDS kernels only
   // (TF_ESHAPE, so that a caller can tell "this product is not served, use the activation as mask"
   // from a malformed call)
   if (signs && !(kCfgs[pl.cfg].dma && vec && K % pl.bk == 0 && pl.splits == 1)) return TF_ESHAPE;
-  const int64_t need = pl.splits > 1 ? (int64_t)pl.splits * M * N * (int64_t)sizeof(float) : 0;
+  const int64_t need = plan_need(pl, M, N);
   if (need > 0 && (!workspace || workspace_bytes < need)) return TF_EWORKSPACE;
   if (need > 0 && !aligned16(workspace)) return TF_EALIGN;
   if ((int64_t)pl.tiles_m * pl.tiles_n * pl.splits > 0x7fffffff) return TF_EINVAL;
@@ -1535,9 +1596,7 @@ extern "C" int64_t tf_diag_gemm_workspace_bytes(int cfg, int splits, int64_t M, 
   const GemmForce force = {cfg < 0 ? -1 : cfg, splits, 0};
   int64_t need = 0;
   for (int vec = 0; vec < 2; ++vec) {
-    const GemmPlan pl = make_plan(M, N, K, vec != 0, true, nullptr, force);
-    const int64_t n = pl.splits > 1 ? (int64_t)pl.splits * M * N * (int64_t)sizeof(float) : 0;
-    if (n > need) need = n;
+    need = std::max(need, plan_need(make_plan(device_shape().cus, M, N, K, vec != 0, true, nullptr, force), M, N));
   }
   return need;
 }
