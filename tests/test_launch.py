@@ -204,3 +204,81 @@ def test_a_module_of_another_torch_is_refused(monkeypatch):
         m.setitem(sys.modules, "tritonformer_amd._launch", None)
         with pytest.raises(ImportError, match="rebuild"):
             _lib.launch()
+
+
+# ------------------------------------------------------------------------------------------ several launches in one call
+class _OneByOne:
+    """The extension module without the functions that run a whole block."""
+
+    def __init__(self, native):
+        self._native = native
+
+    def __getattr__(self, name):
+        return (lambda *a: None) if name in ("attn_block", "attn_block_dqkv", "mlp") else getattr(self._native, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("autocast", [False, True])
+@pytest.mark.parametrize("batch,seq,d,heads,ffn,bias", [(2, 64, 128, 2, 512, False), (3, 192, 96, 3, 200, True),
+                                                        (1, 96, 128, 1, 129, True)])
+def test_blocks_in_one_call_give_the_bits_of_their_launches(dtype, autocast, batch, seq, d, heads, ffn, bias, dev, monkeypatch):
+    """Attention and MLP blocks, forward and backward: weights in 16 bits and fp32 masters, contractions that no sign bits
+    are served for (96 columns), widths that no row of chunks fits (129)."""
+    import tritonformer_amd as T
+    from tritonformer_amd import kernels as K
+
+    g = torch.Generator().manual_seed(5)
+    wt = torch.float32 if autocast else dtype
+    rnd = lambda *s: (torch.randn(s, generator=g) * 0.1).to(dev)
+    x = rnd(batch, seq, d).to(dtype)
+    wa = [rnd(d, d).to(wt) for _ in range(4)]
+    wm = [rnd(d, ffn).to(wt), rnd(ffn).to(wt) if bias else None, rnd(ffn, d).to(wt), rnd(d).to(wt) if bias else None]
+    slopes = torch.tensor([2.0 ** -(i + 1) for i in range(heads)], device=dev, dtype=torch.float16) if bias else None
+
+    def run():
+        leaves = [None if t is None else t.clone().requires_grad_(True) for t in [x, *wa, *wm]]
+        with torch.autocast("cuda", dtype=dtype, enabled=autocast):
+            out = T.mlp_fused_relu.apply(T.attention_block.apply(*leaves[:5], heads, slopes), *leaves[5:])
+            assert torch.is_autocast_enabled("cuda") == autocast
+        out.backward(torch.ones_like(out))
+        return [out] + [t.grad for t in leaves if t is not None]
+
+    together = run()
+    native = K.launch()
+    monkeypatch.setattr(K, "launch", lambda: _OneByOne(native))
+    for a, b in zip(together, run()):
+        assert torch.equal(a, b)
+
+
+def test_pick_takes_what_the_exhaustive_search_takes():
+    """The packing of pending weight gradients against the search over ways to reach a sum, written out."""
+    import random
+
+    from tritonformer_amd import _deferred as D
+
+    class Item:
+        def __init__(self, tiles, key):
+            self.tiles, self.key = tiles, key
+
+    def search(items, cus, split):
+        reach = {0: ()}
+        for i, it in enumerate(items):
+            if it.key == items[0].key:
+                for s, sub in list(reach.items()):
+                    if len(sub) < D._MAX_GROUP:
+                        reach.setdefault(s + it.tiles, sub + (i,))
+        best, best_rank = None, None
+        for s, sub in reach.items():
+            if sub:
+                f = 0.9 * s * (cus // s) / cus if split and 2 * s <= cus else D._fill(s, cus)
+                rank = (min(f, D._FILL), 0 in sub, s)
+                if best_rank is None or rank > best_rank:
+                    best, best_rank = sub, rank
+        return best, best_rank[0]
+
+    rng = random.Random(3)
+    for _ in range(200):
+        items = [Item(rng.choice([1, 3, 9, 27, 36, 64, 200, 432]), rng.random() < 0.9) for _ in range(rng.randint(1, 26))]
+        for split in (False, True):
+            assert D._pick(items, 256, split) == search(items, 256, split)

@@ -61,8 +61,16 @@ def cached_conversion(weights, dtype, convert):
     return out
 
 
+def _is_parameter(value):
+    """isinstance(value, Parameter); that check runs Python code, so the two usual types are told apart ahead of it."""
+    kind = type(value)
+    return kind is torch.nn.Parameter or (kind is not torch.Tensor and isinstance(value, torch.nn.Parameter))
+
+
 def _cast(value, dtype):
     if isinstance(value, torch.Tensor):
+        if value.dtype == dtype:
+            return value
         if value.is_floating_point() and value.is_cuda and value.dtype != torch.float64:
             if _cache_on and value.dtype == torch.float32 and value.ndim == 2 and isinstance(value, torch.nn.Parameter):
                 return cached_conversion([value], dtype, lambda ws, dt: ws[0].to(dt))
@@ -84,16 +92,19 @@ def amp_fwd(fwd=None, *, keep=()):
         ctx._dtype = torch.get_autocast_dtype("cuda")
         ctx._fwd_used_autocast = False
         # dtypes the caller passed in, before any autocast cast (fp32 master weights)
-        ctx.arg_dtypes = tuple(a.dtype if isinstance(a, torch.Tensor) else None for a in args)
+        ctx.arg_dtypes = tuple([a.dtype if isinstance(a, torch.Tensor) else None for a in args])
         ctx.amp_active = torch.is_autocast_enabled("cuda")  # for bodies that cast their `keep` arguments themselves
         # the parameters as the caller holds them (autocast hands the body 16-bit copies): where a deferred
         # gradient is delivered
-        ctx.arg_params = tuple(a if isinstance(a, torch.nn.Parameter) else None for a in args)
+        ctx.arg_params = tuple([a if _is_parameter(a) else None for a in args])
         if ctx.amp_active:
             dtype = torch.bfloat16 if ctx._dtype == torch.bfloat16 else torch.float16
-            with torch.autocast(device_type="cuda", enabled=False):
-                cast = tuple(a if i in keep else _cast(a, dtype) for i, a in enumerate(args))
-                return fwd(ctx, *cast)
+            # the switch alone: entering an autocast region with enabled=False costs 8 us per graph node
+            torch.set_autocast_enabled("cuda", False)
+            try:
+                return fwd(ctx, *[a if i in keep else _cast(a, dtype) for i, a in enumerate(args)])
+            finally:
+                torch.set_autocast_enabled("cuda", True)
         return fwd(ctx, *args)
 
     return wrapper

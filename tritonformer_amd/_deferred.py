@@ -20,6 +20,7 @@ import contextlib
 
 import torch
 
+from ._lib import launch
 from .kernels import layernorm_param_grads, mm_dw_group
 
 # products per launch (the grouped GEMM entry point takes up to sixteen)
@@ -84,33 +85,13 @@ def _fill(tiles, cus):
     return tiles / (-(-tiles // cus) * cus)
 
 
-def _fill_split(tiles, cus):
-    """The share of the chip a launch keeps busy when the grouped GEMM may split contractions: at most half
-    a round of tiles runs as cus // tiles slices per tile (fp32 partial sums and a second pass: rated 0.9)."""
-    if 2 * tiles <= cus:
-        return 0.9 * tiles * (cus // tiles) / cus
-    return _fill(tiles, cus)
-
-
-def _pick(items, cus, rate=_fill):
+def _pick(items, cus, split=False):
     """Indices of up to _MAX_GROUP products (of the first one's kind) whose tiles best fill whole rounds;
-    among equals the oldest, then the most tiles.  Returns (indices, fill)."""
-    reach = {0: ()}
-    for idx, it in enumerate(items):
-        if it.key != items[0].key:
-            continue
-        for s, sub in list(reach.items()):
-            if len(sub) < _MAX_GROUP and s + it.tiles not in reach:
-                reach[s + it.tiles] = sub + (idx,)
-    best, best_rank = None, None
-    for s, sub in reach.items():
-        if not sub:
-            continue
-        f = rate(s, cus)
-        rank = (min(f, _FILL), 0 in sub, s)
-        if best_rank is None or rank > best_rank:
-            best, best_rank = sub, rank
-    return best, best_rank[0]
+    among equals the oldest, then the most tiles.  Returns (indices, fill).  ``split``: as if the grouped GEMM may split
+    contractions -- at most half a round of tiles runs as cus // tiles slices per tile (fp32 partial sums and a second
+    pass: rated 0.9)."""
+    key = items[0].key
+    return launch().pick([it.tiles if it.key == key else 0 for it in items], cus, _MAX_GROUP, _FILL, split)
 
 
 def _launch(items):
@@ -128,12 +109,15 @@ def _launch(items):
 
 def _next_launch(items, cus, final):
     """Indices of the products to launch now, or None to wait for more."""
+    waiting = not final and len(items) < _MAX_PENDING
+    if waiting and sum([it.tiles for it in items]) < _FILL * cus:
+        return None  # all of them together are no round
     sub, fill = _pick(items, cus)
     if fill < _FILL:
-        if not final and len(items) < _MAX_PENDING:
+        if waiting:
             return None
         # nothing more is coming (or too much is held): what fills the chip best, split contractions included
-        sub, fill = _pick(items, cus, _fill_split)
+        sub, fill = _pick(items, cus, True)
     return sub
 
 

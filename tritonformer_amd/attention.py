@@ -5,8 +5,8 @@ from typing import Any, Tuple
 import torch
 from torch.autograd import Function
 
-from . import _deferred
-from ._amp import amp_bwd, amp_fwd, cached_conversion
+from . import _deferred, kernels
+from ._amp import amp_bwd, amp_fwd, cached_conversion, weight_cast_cache_enabled
 from .kernels import (
     cast_pack,
     flash_packed_bwd,
@@ -119,13 +119,21 @@ class AttentionBlock(Function):
         ctx.defer_to = weights if _deferred.active() and same and _deferred.deferrable(weights) else None
         # the four (d, d) weights side by side in one 16-bit (d, 4d) matrix, one conversion kernel;
         # the GEMMs take its first three column blocks and its last one as strided operands
-        packed = cached_conversion([wq, wk, wv, wo], x.dtype, cast_pack)
+        cached = weight_cast_cache_enabled()
+        packed = cached_conversion([wq, wk, wv, wo], x.dtype, cast_pack) if cached else None
+        ctx.weight_dtype = wq.dtype
+        block = kernels.launch().attn_block(x, [wq, wk, wv, wo], packed, num_heads, attn_bias)
+        if block is not None:
+            out, packed, qkv, attn, lse = block
+            ctx.save_for_backward(x, packed, qkv, attn, lse, attn_bias)
+            return out
+        if packed is None:
+            packed = cast_pack([wq, wk, wv, wo], x.dtype)
         w_qkv, w_o = packed[:, : 3 * d], packed[:, 3 * d:]
         qkv = mm(x, w_qkv).view(b, s, 3, num_heads, hd)
         attn, lse = flash_packed_fwd(qkv, attn_bias)
         attn = attn.view(b, s, d)
         ctx.save_for_backward(x, packed, qkv, attn, lse, attn_bias)
-        ctx.weight_dtype = wq.dtype
         return mm(attn, w_o)
 
     @staticmethod
@@ -133,9 +141,12 @@ class AttentionBlock(Function):
     def backward(ctx: Any, grad_output: torch.Tensor):
         x, packed, qkv, attn, lse, attn_bias = ctx.saved_tensors
         b, s, _, nh, hd = qkv.shape
-        w_qkv, w_o = packed[:, : 3 * nh * hd], packed[:, 3 * nh * hd:]
-        d_attn = mm(grad_output, w_o.T)
-        dqkv = flash_packed_bwd(d_attn, attn, qkv, lse, attn_bias).view(b, s, 3 * nh * hd)
+        w_qkv = packed[:, : 3 * nh * hd]
+        dqkv = kernels.launch().attn_block_dqkv(grad_output, attn, qkv, packed, lse, attn_bias)
+        if dqkv is None:
+            d_attn = mm(grad_output, packed[:, 3 * nh * hd:].T)
+            dqkv = flash_packed_bwd(d_attn, attn, qkv, lse, attn_bias)
+        dqkv = dqkv.view(b, s, 3 * nh * hd)
         if ctx.defer_to is not None:
             # launched later, together with those of other layers, in whole rounds of workgroups
             _deferred.submit([(x, dqkv, 3, ctx.defer_to[:3], ctx.weight_dtype),

@@ -20,8 +20,10 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cmath>
 #include <initializer_list>
+#include <unordered_set>
 
 #include "../../include/tritonformer_amd.h"
 
@@ -548,6 +550,239 @@ TF_FN(colsum, 2) {
   return THPVariable_Wrap(out);
 }
 
+// ------------------------------------------------------------------------------------------ blocks
+// Several launches of one graph node in one call: at a few hundred tokens a node is bound by the host, and every return to
+// Python between two launches costs 2 to 3 us.
+
+// c (m, n) = relu?(a (m, k) . b + bias), b as the header's layouts have it
+bool product(const Tensor& like, int lb, int64_t m, int64_t n, int64_t k, const void* a, const void* b, int64_t ldb, void* c,
+             const void* bias = nullptr, int relu = 0) {
+  const int dt = code(like.scalar_type());
+  const int64_t bytes = tf_gemm_workspace_bytes(TF_OP_KMAJOR, lb, m, n, k);
+  Tensor ws = scratch(bytes, like);
+  return call([&] {
+    return tf_gemm_out_chunked(stream(), dt, dt, TF_OP_KMAJOR, lb, m, n, k, a, k, b, ldb, c, n, 0, 0, bias, relu, nullptr, 0,
+                               ptr(ws), bytes);
+  });
+}
+
+// `n` matrices (float32 or `to`) of one shape side by side in `to`, as rows x cols each; false: an operand of another form
+// (no error set) or a failed call (error set)
+bool pack(const Tensor* const* w, int n, int64_t rows, int64_t cols, at::ScalarType to, Tensor* out) {
+  const void* src[4];
+  for (int i = 0; i < n; ++i) {
+    if (!w[i] || w[i]->sizes() != w[0]->sizes() || w[i]->scalar_type() != w[0]->scalar_type()) return false;
+    src[i] = w[i]->data_ptr();
+  }
+  const at::ScalarType from = w[0]->scalar_type();
+  if (from != at::kFloat && from != to) return false;
+  *out = make({rows, n * cols}, *w[0], to);
+  return call([&] { return tf_cast_pack(stream(), code(from), code(to), n, rows, cols, src, cols, out->data_ptr(), n * cols); });
+}
+
+// attn_block(x (B, S, d), [wq, wk, wv, wo], packed | None, heads, bias | None)
+//   -> (attention(x wq, x wk, x wv) wo, packed (d, 4d), qkv (B, S, 3, nh, hd), attention output (B, S, d), lse)
+TF_FN(attn_block, 5) {
+  const Tensor *x = dense(args.a[0]), *bias;
+  if (!x || x->dim() != 3 || !is16(*x) || !aligned(*x) || !PyList_Check(args.a[1]) || PyList_GET_SIZE(args.a[1]) != 4)
+    Py_RETURN_NONE;
+  const int64_t b = x->size(0), s = x->size(1), d = x->size(2), nh = PyLong_AsLongLong(args.a[3]);
+  if (nh == -1 && PyErr_Occurred()) return nullptr;
+  if (nh <= 0 || d % nh || !attn_sizes(s, d / nh) || !attn_bias(args.a[4], *x, nh, s, &bias)) Py_RETURN_NONE;
+  const int64_t hd = d / nh, m = b * s;
+  Tensor packed;
+  if (args.a[2] != Py_None) {
+    const Tensor* p = dense(args.a[2]);
+    if (!p || p->dim() != 2 || p->size(0) != d || p->size(1) != 4 * d || p->scalar_type() != x->scalar_type()) Py_RETURN_NONE;
+    packed = *p;
+  } else {
+    const Tensor* w[4];
+    for (int i = 0; i < 4; ++i) {
+      w[i] = dense(PyList_GET_ITEM(args.a[1], i));
+      if (!w[i] || w[i]->dim() != 2 || w[i]->size(0) != d || w[i]->size(1) != d) Py_RETURN_NONE;
+    }
+    if (!pack(w, 4, d, d, x->scalar_type(), &packed)) {
+      if (PyErr_Occurred()) return nullptr;
+      Py_RETURN_NONE;
+    }
+  }
+  const char* w = static_cast<const char*>(packed.data_ptr());
+  Tensor qkv = make({b, s, 3, nh, hd}, *x), attn = make({b, s, d}, *x), lse = make({b, nh, s}, *x, at::kFloat),
+         out = make({b, s, d}, *x);
+  const char* q = static_cast<const char*>(qkv.data_ptr());
+  if (!product(*x, TF_OP_KMINOR, m, 3 * d, d, x->data_ptr(), w, 4 * d, qkv.data_ptr()) ||
+      !attn_forward(code(x->scalar_type()), b, nh, s, hd, q, q + 2 * d, q + 4 * d, attn.data_ptr(), {s * 3 * d, hd, 3 * d},
+                    {s * d, hd, d}, lse.data_ptr<float>(), bias) ||
+      !product(*x, TF_OP_KMINOR, m, d, d, attn.data_ptr(), w + 6 * d, 4 * d, out.data_ptr()))
+    return nullptr;
+  return tuple_of({&out, &packed, &qkv, &attn, &lse});
+}
+
+// attn_block_dqkv(grad_out (B, S, d), attention output, qkv, packed, lse, bias | None) -> gradient of qkv
+TF_FN(attn_block_dqkv, 6) {
+  const Tensor *g = dense(args.a[0]), *o = dense(args.a[1]), *t = dense(args.a[2]), *w = dense(args.a[3]),
+               *lse = dense(args.a[4]), *bias;
+  if (!g || !o || !w || !lse || !packed_qkv(t)) Py_RETURN_NONE;
+  const int64_t b = t->size(0), s = t->size(1), nh = t->size(3), hd = t->size(4), d = nh * hd;
+  if (g->dim() != 3 || g->size(0) != b || g->size(1) != s || g->size(2) != d || o->sizes() != g->sizes() || w->dim() != 2 ||
+      w->size(0) != d || w->size(1) != 4 * d || g->scalar_type() != t->scalar_type() || o->scalar_type() != t->scalar_type() ||
+      w->scalar_type() != t->scalar_type() || !aligned(*o) || lse->scalar_type() != at::kFloat ||
+      lse->numel() != b * nh * s || !attn_bias(args.a[5], *t, nh, s, &bias))
+    Py_RETURN_NONE;
+  Tensor d_attn = make(g->sizes(), *t), dqkv = make(t->sizes(), *t), delta = make({b, nh, s}, *t, at::kFloat);
+  const char* q = static_cast<const char*>(t->data_ptr());
+  char* dq = static_cast<char*>(dqkv.data_ptr());
+  if (!product(*t, TF_OP_KMAJOR, b * s, d, d, g->data_ptr(), static_cast<const char*>(w->data_ptr()) + 6 * d, 4 * d,
+               d_attn.data_ptr()) ||
+      !attn_backward(code(t->scalar_type()), b, nh, s, hd, q, q + 2 * d, q + 4 * d, o->data_ptr(), d_attn.data_ptr(), dq,
+                     dq + 2 * d, dq + 4 * d, {s * 3 * d, hd, 3 * d}, {s * d, hd, d}, lse->data_ptr<float>(),
+                     delta.data_ptr<float>(), bias))
+    return nullptr;
+  return THPVariable_Wrap(dqkv);
+}
+
+// mlp(x (B, S, k), w1 (k, f), b1 | None, w2 (f, n), b2 | None, with_bits)
+//   -> (relu(x w1 + b1) w2 + b2, hidden, sign bits | None, w1 and w2 in x's dtype)
+TF_FN(mlp, 6) {
+  const Tensor *x = dense(args.a[0]), *w1 = dense(args.a[1]), *w2 = dense(args.a[3]);
+  const Tensor *b1 = nullptr, *b2 = nullptr;
+  if (!x || !w1 || !w2 || x->dim() != 3 || !is16(*x) || w1->dim() != 2 || w2->dim() != 2 || w1->size(0) != last(*x) ||
+      w2->size(0) != w1->size(1) || w1->scalar_type() != w2->scalar_type())
+    Py_RETURN_NONE;
+  const int64_t k = w1->size(0), f = w1->size(1), n = w2->size(1), m = rows_of(*x);
+  auto bias = [&](PyObject* o, int64_t size, const Tensor** out) {
+    if (o == Py_None) return true;
+    *out = dense(o);
+    return *out && (*out)->dim() == 1 && (*out)->size(0) == size && (*out)->scalar_type() == x->scalar_type();
+  };
+  if (!bias(args.a[2], f, &b1) || !bias(args.a[4], n, &b2)) Py_RETURN_NONE;
+  Tensor c1, c2;
+  if (w1->scalar_type() == x->scalar_type()) {
+    c1 = *w1, c2 = *w2;
+  } else {
+    const int64_t each = w1->numel();
+    if (w1->scalar_type() != at::kFloat || w2->numel() != each || each % 8) Py_RETURN_NONE;
+    const Tensor a = w1->view({1, each}), b = w2->view({1, each});
+    const Tensor* w[2] = {&a, &b};
+    Tensor both;
+    if (!pack(w, 2, 1, each, x->scalar_type(), &both)) {
+      if (PyErr_Occurred()) return nullptr;
+      Py_RETURN_NONE;
+    }
+    c1 = both.narrow(1, 0, each).view({k, f}), c2 = both.narrow(1, each, each).view({f, n});
+  }
+  Tensor hidden = make({x->size(0), x->size(1), f}, *x), out = make({x->size(0), x->size(1), n}, *x), bits;
+  const void *p1 = b1 ? b1->data_ptr() : nullptr, *p2 = b2 ? b2->data_ptr() : nullptr;
+  int rc = TF_ESHAPE;
+  if (args.a[5] == Py_True && f % 8 == 0) {
+    bits = make({m, f / 8}, *x, at::kByte);
+    const int dt = code(x->scalar_type());
+    if (!call([&] {
+          return tf_gemm_relu_bits(stream(), dt, dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x->data_ptr(), k, c1.data_ptr(), f,
+                                   hidden.data_ptr(), f, p1, bits.data_ptr(), nullptr, f / 8);
+        }, TF_ESHAPE, &rc))
+      return nullptr;
+  }
+  if (rc != TF_OK && !product(*x, TF_OP_KMINOR, m, f, k, x->data_ptr(), c1.data_ptr(), f, hidden.data_ptr(), p1, 1)) return nullptr;
+  if (!product(*x, TF_OP_KMINOR, m, n, f, hidden.data_ptr(), c2.data_ptr(), n, out.data_ptr(), p2)) return nullptr;
+  if (rc == TF_OK) return tuple_of({&out, &hidden, &bits, &c1, &c2});
+  PyObject* t = tuple_of({&out, &hidden, &hidden, &c1, &c2});
+  if (t) {
+    Py_INCREF(Py_None);
+    PyObject* old = PyTuple_GET_ITEM(t, 2);
+    PyTuple_SET_ITEM(t, 2, Py_None);
+    Py_DECREF(old);
+  }
+  return t;
+}
+
+// ------------------------------------------------------------------------------------------ optimizer
+// adamw([params], [grads], [first moments], [second moments], [16-bit copies] | None, dtype of the copies, lr, beta1, beta2,
+// eps, weight decay, step): dense float32 tensors of one size each (the copies 16-bit); nothing is returned but True
+TF_FN(adamw, 12) {
+  for (int i = 0; i < 4; ++i)
+    if (!PyList_Check(args.a[i]) || PyList_GET_SIZE(args.a[i]) != PyList_GET_SIZE(args.a[0])) Py_RETURN_NONE;
+  const Py_ssize_t n = PyList_GET_SIZE(args.a[0]);
+  const bool copies = args.a[4] != Py_None;
+  if ((copies && (!PyList_Check(args.a[4]) || PyList_GET_SIZE(args.a[4]) != n)) || !THPDtype_Check(args.a[5])) Py_RETURN_NONE;
+  const at::ScalarType type = reinterpret_cast<THPDtype*>(args.a[5])->scalar_type;
+  std::vector<tf_adamw_tensor> items((size_t)n);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    void* at[5] = {};
+    int64_t count = 0;
+    for (int j = 0; j < (copies ? 5 : 4); ++j) {
+      const Tensor* t = dense(PyList_GET_ITEM(args.a[j], i));
+      if (!t || t->scalar_type() != (j < 4 ? at::kFloat : type) || (j && t->numel() != count)) Py_RETURN_NONE;
+      count = t->numel();
+      at[j] = t->data_ptr();
+    }
+    items[(size_t)i] = {at[0], at[1], at[2], at[3], at[4], count};
+  }
+  double f[5];
+  for (int j = 0; j < 5; ++j) {
+    if (!PyFloat_Check(args.a[6 + j]) && !PyLong_Check(args.a[6 + j])) Py_RETURN_NONE;
+    f[j] = PyFloat_AsDouble(args.a[6 + j]);
+  }
+  const int64_t step = PyLong_AsLongLong(args.a[11]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!call([&] {
+        return tf_adamw_step(stream(), code(type), (int)n, items.data(), (float)f[0], (float)f[1], (float)f[2], (float)f[3],
+                             (float)f[4], step);
+      }))
+    return nullptr;
+  Py_RETURN_TRUE;
+}
+
+// ------------------------------------------------------------------------------------------ gradient queue
+// pick(tiles of the pending products (0: not of the first one's kind), cus, most, full, split) -> (indices, fill): the
+// products, `most` at the most, whose tiles best fill whole rounds of workgroups; among equals with the oldest, then the
+// most tiles.  `split`: tiles up to half a round count as filled by slices (at 0.9).  Sums of tiles are reached in the order
+// of the products, the first way to a sum is kept.
+PyObject* pick(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 5 || !PyList_Check(a[0])) return PyErr_Format(PyExc_TypeError, "pick takes a list and four numbers");
+  const Py_ssize_t count = PyList_GET_SIZE(a[0]);
+  const int64_t cus = PyLong_AsLongLong(a[1]), most = PyLong_AsLongLong(a[2]);
+  const double full = PyFloat_AsDouble(a[3]);
+  const int split = PyObject_IsTrue(a[4]);
+  std::vector<int64_t> tiles((size_t)count);
+  for (Py_ssize_t i = 0; i < count; ++i) tiles[(size_t)i] = PyLong_AsLongLong(PyList_GET_ITEM(a[0], i));
+  if (PyErr_Occurred()) return nullptr;
+  if (count < 1 || count > 64 || cus < 1) return PyErr_Format(PyExc_ValueError, "1 to 64 products");
+  struct Way {
+    int64_t sum;
+    uint64_t members;
+  };
+  std::vector<Way> ways{{0, 0}};
+  std::unordered_set<int64_t> reached{0};
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    if (tiles[(size_t)i] <= 0) continue;
+    const size_t before = ways.size();
+    for (size_t w = 0; w < before; ++w) {
+      const Way from = ways[w];
+      if (__builtin_popcountll(from.members) < most && reached.insert(from.sum + tiles[(size_t)i]).second)
+        ways.push_back({from.sum + tiles[(size_t)i], from.members | uint64_t(1) << i});
+    }
+  }
+  Way best{0, 0};
+  double best_fill = -1;
+  for (const Way& w : ways) {
+    if (!w.members) continue;
+    double f = split && 2 * w.sum <= cus ? 0.9 * (double)w.sum * (double)(cus / w.sum) / (double)cus
+                                         : (double)w.sum / (double)((w.sum + cus - 1) / cus * cus);
+    f = std::min(f, full);
+    const bool old = w.members & 1, best_old = best.members & 1;
+    if (f > best_fill || (f == best_fill && (old > best_old || (old == best_old && w.sum > best.sum)))) best = w, best_fill = f;
+  }
+  PyObject* indices = PyTuple_New(__builtin_popcountll(best.members));
+  if (!indices) return nullptr;
+  Py_ssize_t at = 0;
+  for (Py_ssize_t i = 0; i < count; ++i)
+    if (best.members >> i & 1) PyTuple_SET_ITEM(indices, at++, PyLong_FromSsize_t(i));
+  return Py_BuildValue("(Nd)", indices, best_fill);
+  END_HANDLE_TH_ERRORS
+}
+
 PyObject* set_check(PyObject*, PyObject* f) {
   Py_INCREF(f);
   Py_XSETREF(g_check, f);
@@ -559,7 +794,7 @@ PyMethodDef methods[] = {
     TF_ENTRY(linear), TF_ENTRY(linear_bits), TF_ENTRY(linear_masked), TF_ENTRY(weight_grad), TF_ENTRY(cast_pack),
     TF_ENTRY(attn_fwd), TF_ENTRY(attn_bwd), TF_ENTRY(attn_packed_fwd), TF_ENTRY(attn_packed_bwd), TF_ENTRY(layernorm),
     TF_ENTRY(layernorm_bwd), TF_ENTRY(softmax_fwd), TF_ENTRY(softmax_bwd), TF_ENTRY(relu_mask), TF_ENTRY(relu_mask_colsum),
-    TF_ENTRY(colsum),
+    TF_ENTRY(colsum), TF_ENTRY(attn_block), TF_ENTRY(attn_block_dqkv), TF_ENTRY(mlp), TF_ENTRY(pick), TF_ENTRY(adamw),
     {"set_check", set_check, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

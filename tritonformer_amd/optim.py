@@ -6,7 +6,7 @@ from typing import Optional
 
 import torch
 
-from ._lib import AdamTensor, check, dtype_code, load
+from ._lib import AdamTensor, check, dtype_code, launch, load
 from .kernels import require_cuda, stream_ptr
 
 
@@ -56,17 +56,25 @@ class AdamW(torch.optim.Optimizer):
                 st["step"] += 1
                 by_step.setdefault(st["step"], []).append((p, p.grad.contiguous(), st))
             for step, items in by_step.items():
-                arr = (AdamTensor * len(items))()
-                for a, (p, g, st) in zip(arr, items):
-                    a.param, a.grad = p.data_ptr(), g.data_ptr()
-                    a.exp_avg, a.exp_avg_sq = st["exp_avg"].data_ptr(), st["exp_avg_sq"].data_ptr()
-                    a.shadow = st["shadow"].data_ptr() if "shadow" in st else None
-                    a.count = p.numel()
-                check(lib.tf_adamw_step(stream_ptr(), dtype_code(self.shadow_dtype or torch.float16), len(items),
-                                        ctypes.cast(arr, ctypes.c_void_p), group["lr"], group["betas"][0],
-                                        group["betas"][1], group["eps"], group["weight_decay"], step))
+                params, grads, states = zip(*items)
+                copies = [st["shadow"] for st in states] if all(["shadow" in st for st in states]) else None
+                done = None
+                if copies is not None or not any(["shadow" in st for st in states]):
+                    done = launch().adamw(list(params), list(grads), [st["exp_avg"] for st in states],
+                                          [st["exp_avg_sq"] for st in states], copies, self.shadow_dtype or torch.float16,
+                                          group["lr"], group["betas"][0], group["betas"][1], group["eps"],
+                                          group["weight_decay"], step)
+                if done is None:
+                    arr = (AdamTensor * len(items))()
+                    for a, (p, g, st) in zip(arr, items):
+                        a.param, a.grad = p.data_ptr(), g.data_ptr()
+                        a.exp_avg, a.exp_avg_sq = st["exp_avg"].data_ptr(), st["exp_avg_sq"].data_ptr()
+                        a.shadow = st["shadow"].data_ptr() if "shadow" in st else None
+                        a.count = p.numel()
+                    check(lib.tf_adamw_step(stream_ptr(), dtype_code(self.shadow_dtype or torch.float16), len(items),
+                                            ctypes.cast(arr, ctypes.c_void_p), group["lr"], group["betas"][0],
+                                            group["betas"][1], group["eps"], group["weight_decay"], step))
                 # the kernel wrote through raw pointers: tell autograd (and anything keyed on the
                 # version counter, like the cache of 16-bit weight copies) that the values changed
-                for p, _, _ in items:
-                    torch.autograd.graph.increment_version(p)
+                torch.autograd.graph.increment_version(params)
         return loss
