@@ -207,6 +207,37 @@ def test_cross_entropy_rows(v, dtype, dev):
 
 # vocabularies held in registers and streamed (beyond 51200), ragged and whole; the masked tokens fill whole chunks of
 # the first ones of a thread, with -inf and with the type's lowest value
+@pytest.mark.parametrize("v", [2047, 2048, 2049, 2055, 2112, 50257])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_cross_entropy_gradient_is_the_same_bits_wherever_its_rows_start(v, dtype, dev):
+    """The gradient kernel counts its chunks from the line in which a row starts, from the row's start (short rows, in place)
+    or over aligned rows: 70 rows of odd pitch start at every element of a line, labels at the ends of the row and of its
+    first and last chunks.  The same rows padded with -inf to aligned ones have the same sums and so the same bits."""
+    g = torch.Generator().manual_seed(v)
+    rows = 70
+    x = (2 * torch.randn(rows, v, generator=g)).to(dtype).to(dev)
+    at = [0, 1, 7, 8, 63, 64, v - 1, v - 2, v - 8, v - 9]
+    labels = torch.tensor([at[i % len(at)] for i in range(rows)], device=dev)
+    gout = torch.randn(rows, generator=g).to(dtype).to(dev)
+    lse = torch.logsumexp(x.float(), 1)
+    wide = (v + 7) // 8 * 8
+    aligned = torch.full((rows, wide), float("-inf"), dtype=dtype, device=dev)
+    aligned[:, :v] = x
+
+    def run(logits, out):
+        _lib.check(_lib.load().tf_cross_entropy_bwd(
+            torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype), rows, logits.shape[1], logits.data_ptr(), logits.stride(0),
+            0, 0, labels.data_ptr(), lse.data_ptr(), gout.data_ptr(), 1, out.data_ptr(), out.stride(0), 0))
+        return out
+
+    want = run(aligned, torch.empty_like(aligned))[:, :v]
+    buf, view = odd_rows(x, dev)
+    out_buf, out = odd_rows(torch.zeros_like(x), dev)
+    assert torch.equal(run(view, out), want) and untouched(out_buf, v)
+    assert torch.equal(run(x, torch.empty_like(x)), want)
+    assert torch.equal(run(view, view), want) and untouched(buf, v)
+
+
 @pytest.mark.parametrize("v", [257, 16385, 51199, 51201, 51208, 70001, 128257])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_cross_entropy_of_masked_rows(v, dtype, dev):

@@ -3,7 +3,7 @@
 // backward streams it once more and writes the gradient, already multiplied by
 // the upstream per-row gradient.  ANY: rows of any length and alignment (a vocabulary that
 // nobody padded), in the same 16-byte chunks (struct Row in rowops.h): 4095 bf16 rows of 50257 entries
-// forward 233 -> 81 us (5.1 TB/s), backward 208 -> 187 us (4.4 TB/s) against element-wise loads.
+// forward 233 -> 81 us (5.1 TB/s), backward 208 -> 170 us (4.8 TB/s) against element-wise loads.
 #include "rowops.h"
 
 namespace tfa {
@@ -213,11 +213,19 @@ __global__ __launch_bounds__(kCeThreads, NCH == 8 ? 4 : 1) void ce_fwd_regs(int 
   }
 }
 
-template <typename T, bool ANY>
+// How ce_bwd walks its rows; bound by memory.  kCeAligned: whole aligned chunks.  kCeShort: chunks counted from the start of
+// the row, wherever it lies.  kCeLines: chunks counted from the 128-byte line in which the row of the gradient starts, so that
+// a wave's access covers whole lines instead of leaving a piece of one to the next: 4095 x 50257 bf16 187 -> 170 us
+// (4.8 TB/s), 2047 x 32001 50.7 -> 44.3, 8192 x 4097 27.3 -> 24.6, but 8192 x 1001 12.1 -> 12.8 (written through, these
+// stores take 183, 53 and 54 us).  The values are the same bits in every form: an element depends on nothing but itself.
+enum CeRows { kCeAligned, kCeShort, kCeLines };
+constexpr int64_t kCeLinesFrom = 2048;
+template <typename T, CeRows FORM>
 __global__ __launch_bounds__(kCeThreads) void ce_bwd(int V, const T* __restrict__ logits, RowMap map,
                                                       const int64_t* __restrict__ labels,
                                                       const float* __restrict__ lse, const T* __restrict__ gout,
                                                       int64_t gstride, T* __restrict__ dlogits, RowMap dmap) {
+  constexpr bool ANY = FORM != kCeAligned;
   typedef Row<T, ANY> R;
   const int64_t row = blockIdx.x;
   const T* xr = logits + map.at(row);
@@ -225,18 +233,28 @@ __global__ __launch_bounds__(kCeThreads) void ce_bwd(int V, const T* __restrict_
   const float l2 = lse[row] * kLog2e;
   const float g = (float)gout[row * gstride];
   const int lab = (int)labels[row];
-  const int nchunk = Row<T, ANY>::chunks(V);
+  const int before = FORM == kCeLines ? (int)((reinterpret_cast<uintptr_t>(dr) & 127) / sizeof(T)) : 0;  // of the line, ahead of the row
+  const int nchunk = FORM == kCeLines ? (V + before + 7) / 8 : R::chunks(V);
   for (int c = threadIdx.x; c < nchunk; c += kCeThreads) {
+    int first = c * 8 - before;
+    if (FORM == kCeLines && first <= -8) continue;
+    // a chunk that crosses an end of the row is taken as the eight elements at that end: its neighbour writes some of
+    // them as well, the same bits
+    const bool inside = FORM != kCeLines || (first >= 0 && first + 8 <= V);
+    if (FORM == kCeLines) first = min(max(first, 0), V - 8);
     float v[8];
-    unpack8<T>(R::template settle<true>(R::template fetch<true, true>(xr, c, V), c, V), v);
+    if (FORM == kCeLines) unpack8<T>(ld16_elem<true>(xr + first, std::integral_constant<int, 2>()), v);
+    else unpack8<T>(R::template settle<true>(R::template fetch<true, true>(xr, c, V), c, V), v);
     grad_probs<ANY>(v, l2);
-    if ((lab >> 3) == c) {
+    if ((unsigned)(lab - first) < 8u) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] -= (e == (lab & 7)) ? 1.0f : 0.0f;
+      for (int e = 0; e < 8; ++e) v[e] -= (e == lab - first) ? 1.0f : 0.0f;
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] *= g;
-    R::template store<true>(dr, c, V, pack8<T>(v));
+    if (FORM != kCeLines) R::template store<true>(dr, c, V, pack8<T>(v));
+    else if (inside) *reinterpret_cast<u32x4*>(dr + first) = pack8<T>(v);
+    else st16_elem(dr + first, pack8<T>(v), std::integral_constant<int, 2>());
   }
 }
 
@@ -269,13 +287,15 @@ static int ce_bwd_launch(hipStream_t st, int64_t rows, int64_t V, const void* lo
                          const int64_t* labels, const float* lse, const void* gout, int64_t gstride,
                          void* dlogits, RowMap dmap) {
   const dim3 grid((unsigned)rows), block(kCeThreads);
-  if (row_vectorizable<T>(logits, V, map.ld) && row_vectorizable<T>(dlogits, V, dmap.ld) && map.outer % 8 == 0 &&
-      dmap.outer % 8 == 0)
-    ce_bwd<T, false><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, lse, (const T*)gout, gstride,
-                                             (T*)dlogits, dmap);
-  else
-    ce_bwd<T, true><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, lse, (const T*)gout, gstride,
-                                            (T*)dlogits, dmap);
+  const bool aligned = row_vectorizable<T>(logits, V, map.ld) && row_vectorizable<T>(dlogits, V, dmap.ld) &&
+                       map.outer % 8 == 0 && dmap.outer % 8 == 0;
+#define CE_BWD(FORM)                                                                                                  \
+  ce_bwd<T, FORM><<<grid, block, 0, st>>>((int)V, (const T*)logits, map, labels, lse, (const T*)gout, gstride, (T*)dlogits, \
+                                          dmap)
+  if (aligned) CE_BWD(kCeAligned);
+  else if (V >= kCeLinesFrom && logits != dlogits) CE_BWD(kCeLines);
+  else CE_BWD(kCeShort);
+#undef CE_BWD
   TF_CHECK_LAUNCH();
   return TF_OK;
 }
