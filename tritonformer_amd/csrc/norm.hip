@@ -29,6 +29,29 @@ template <int WPR> __device__ __forceinline__ float row_sum(float v, float (*red
   return (red[slot][0] + red[slot][1]) + (red[slot][2] + red[slot][3]);
 }
 
+// Access to the chunks of a LayerNorm row of NV chunks per lane.  The chunk that crosses the end of a ragged row lies among a
+// lane's upper NV / 2 (a row takes NV only if NV / 2 do not hold it): those are fetched as 16 bytes inside the row and
+// moved down (Row::settle), so that no wave stands waiting for eight element loads in the midst of its prefetch.  fp16, us:
+// backward 31713 x 1021 68.0 -> 46.0 (1024 columns: 42.2), 31713 x 777 60.7 -> 41.8, 20000 x 2051 121 -> 99, 8000 x 8191
+// 156 -> 140; forward 31713 x 1021 33.0 -> 30.0, 8000 x 8191 69.7 -> 62.6.
+template <typename T, int NV, bool ANY, int FROM = NV / 2> struct RowEnds {
+  typedef Row<T, ANY> R;
+  static __device__ __forceinline__ u32x4 fetch(const T* row, int c, int i, int n) {
+    return i >= FROM ? R::template fetch<true>(row, c, n) : R::template fetch<false>(row, c, n);
+  }
+  static __device__ __forceinline__ u32x4 settle(u32x4 raw, int c, int i, int n) {
+    return i >= FROM ? R::template settle<true>(raw, c, n) : raw;
+  }
+  static __device__ __forceinline__ void store(T* row, int c, int i, int n, u32x4 v) {
+    if (i >= FROM) R::template store<true>(row, c, n, v);
+    else R::template store<false>(row, c, n, v);
+  }
+  template <typename TP> static __device__ __forceinline__ void load8(const TP* p, int c, int i, int n, float (&v)[8]) {
+    if (i >= FROM) load8_row<TP, ANY, true>(p, c, n, v);
+    else load8_row<TP, ANY, false>(p, c, n, v);
+  }
+};
+
 // With ADD the normalised row is s = x + res, rounded to T and also written to `sum`
 // (the residual stream after the addition); the statistics are those of the rounded s,
 // so the result equals an addition kernel followed by the plain forward.
@@ -49,7 +72,8 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
   // operations are spelled out.
 #pragma clang fp contract(off)
   typedef Row<T, ANY> R;
-  constexpr bool SHORT = NV == 1;
+  // (four chunks per lane with a residual: 31713 x 1537 88 us by elements, 102 so)
+  typedef RowEnds<T, NV, ANY, ADD && NV == 4 && WPR == 1 ? NV : NV / 2> E;
   __shared__ float red[2][4];
   const int lane = WPR == 1 ? threadIdx.x & 63 : threadIdx.x;  // lane within the row
   constexpr int LANES = 64 * WPR, RPB = kRowsPerBlock / WPR;
@@ -61,8 +85,8 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
     for (int i = 0; i < NV; ++i) {
       const int c = lane + i * LANES;
       if (c < nchunk) {
-        raw_x[i] = R::template fetch<SHORT>(x + row * ldx, c, d);
-        if (ADD) raw_r[i] = R::template fetch<SHORT>(res + row * ldres, c, d);
+        raw_x[i] = E::fetch(x + row * ldx, c, i, d);
+        if (ADD) raw_r[i] = E::fetch(res + row * ldres, c, i, d);
       }
     }
   };
@@ -75,14 +99,14 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
     for (int i = 0; i < NV; ++i) {
       const int c = lane + i * LANES;
       if (c < nchunk) {
-        unpack8<T>(R::template settle<SHORT>(raw_x[i], c, d), v[i]);
+        unpack8<T>(E::settle(raw_x[i], c, i, d), v[i]);
         if (ADD) {
           float r[8];
-          unpack8<T>(R::template settle<SHORT>(raw_r[i], c, d), r);
+          unpack8<T>(E::settle(raw_r[i], c, i, d), r);
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[i][e] += r[e];
           const u32x4 packed = pack8<T>(v[i]);
-          R::template store<SHORT>(sum + row * ldsum, c, d, packed);
+          E::store(sum + row * ldsum, c, i, d, packed);
           unpack8<T>(packed, v[i]);
         }
 #pragma unroll
@@ -122,8 +146,8 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
         // (gamma and beta are fetched per row: held in registers across the rows a wave walks they
         // cost a wave of occupancy, 98 against 86 VGPRs, and the kernel 0.5 us at d = 1024)
         float g[8], b[8], o[8];
-        load8_row<TP, ANY, SHORT>(gamma, c, d, g);
-        load8_row<TP, ANY, SHORT>(beta, c, d, b);
+        E::template load8<TP>(gamma, c, i, d, g);
+        E::template load8<TP>(beta, c, i, d, b);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           o[e] = __builtin_fmaf((v[i][e] - mean) * rstd, g[e], b[e]);
@@ -132,7 +156,7 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
           // differently per instantiation, and the two forms differ in one element in 50 000
           asm("" : "+v"(o[e]));
         }
-        R::template store<SHORT>(yr, c, d, pack8<T>(o));
+        E::store(yr, c, i, d, pack8<T>(o));
       }
     }
   }
@@ -186,7 +210,7 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
                                                    const float* __restrict__ rstd, T* __restrict__ dx,
                                                    int64_t lddx, float* __restrict__ partial) {
   typedef Row<T, ANY> R;
-  constexpr bool SHORT = NV == 1;
+  typedef RowEnds<T, NV, ANY> E;
   extern __shared__ float dyn[];  // WPR == 1: [4][d] for the sums of the four waves; then [d] for gamma when G_LDS
   __shared__ float red[2][4];
   // Wide rows (NV >= 4) keep gamma in LDS as fp32 and read a chunk where it is used: held in registers its
@@ -207,13 +231,13 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
     if constexpr (!G_LDS) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) g[i][e] = 0.f;
-      if (c < nchunk) load8_row<TP, ANY, SHORT>(gamma, c, d, g[i]);
+      if (c < nchunk) E::template load8<TP>(gamma, c, i, d, g[i]);
     }
   }
   if constexpr (G_LDS) {
     for (int c = threadIdx.x; c < nchunk; c += 256) {
       float gv[8];
-      load8_row<TP, ANY, SHORT>(gamma, c, d, gv);
+      load8_row<TP, ANY>(gamma, c, d, gv);
 #pragma unroll
       for (int e = 0; e < 8; ++e) gam[c * 8 + e] = gv[e];  // (whole chunks: the buffer is padded to them)
     }
@@ -228,9 +252,9 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
     for (int i = 0; i < NV; ++i) {
       const int c = lane + i * LANES;
       if (c < nchunk) {
-        raw_x[i] = R::template fetch<SHORT>(x + row * ldx, c, d);
-        raw_dy[i] = R::template fetch<SHORT>(dy + row * lddy, c, d);
-        if (ADD) raw_ds[i] = R::template fetch<SHORT>(dsum + row * lddsum, c, d);
+        raw_x[i] = E::fetch(x + row * ldx, c, i, d);
+        raw_dy[i] = E::fetch(dy + row * lddy, c, i, d);
+        if (ADD) raw_ds[i] = E::fetch(dsum + row * lddsum, c, i, d);
       }
     }
     mu_next = mean[row];
@@ -247,9 +271,9 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
       const int c = lane + i * LANES;
       if (c < nchunk) {
         float xv[8], dv[8], gl[8];
-        unpack8<T>(R::template settle<SHORT>(raw_x[i], c, d), xv);
-        unpack8<T>(R::template settle<SHORT>(raw_dy[i], c, d), dv);
-        if (ADD) unpack8<T>(R::template settle<SHORT>(raw_ds[i], c, d), ds[i]);
+        unpack8<T>(E::settle(raw_x[i], c, i, d), xv);
+        unpack8<T>(E::settle(raw_dy[i], c, i, d), dv);
+        if (ADD) unpack8<T>(E::settle(raw_ds[i], c, i, d), ds[i]);
 #pragma unroll
         for (int e = 0; e < 8; ++e) gl[e] = G_LDS ? gam[c * 8 + e] : g[G_LDS ? 0 : i][e];
 #pragma unroll
@@ -280,7 +304,7 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
           o[e] = (gd[i][e] - xh[i][e] * c1 - c2) * rs;
           if (ADD) o[e] += ds[i][e];
         }
-        R::template store<SHORT>(dxr, c, d, pack8<T>(o));
+        E::store(dxr, c, i, d, pack8<T>(o));
       }
     }
   }
