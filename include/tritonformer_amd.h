@@ -129,6 +129,13 @@ int tf_gemm_relu_bits(void* stream, int dtype, int out_dtype, int layout_a, int 
                       const void* A, int64_t lda, const void* B, int64_t ldb,
                       void* C, int64_t ldc, const void* bias,
                       void* bits_out, const void* bits_in, int64_t ld_bits);
+/* tf_gemm (bits_out null) or tf_gemm_relu_bits with bits_out, with the bias as its fp32 master: each value is
+ * rounded to the operand dtype where it is read, so the results are those of the call with a bias converted
+ * before it.  With bits_out no workspace is needed. */
+int tf_gemm_master_bias(void* stream, int dtype, int layout_a, int layout_b, int64_t M, int64_t N, int64_t K,
+                        const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc,
+                        const float* bias, int relu, void* bits_out, int64_t ld_bits,
+                        void* workspace, int64_t workspace_bytes);
 int64_t tf_gemm_workspace_bytes(int layout_a, int layout_b, int64_t M, int64_t N, int64_t K);
 /* C = alpha * (A . B), no bias / ReLU / mask; `alpha`: ONE fp32 value in DEVICE memory, read by
  * the kernel when it writes its result (applied to the fp32 sums before the rounding to

@@ -346,6 +346,37 @@ def test_small_tiles_give_the_bits_of_the_large_ones(layouts, M, N, dev):
             assert (run(cfg, K // 64).float() - want).abs().max() <= 2 ** -10 * want.abs().max()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (33, 129, 70), (200, 328, 192), (512, 768, 4096), (4096, 2304, 1024)])
+def test_master_bias_is_the_bias_converted_ahead(dtype, M, N, K, dev):
+    """A bias read as fp32 and rounded in the product: register-staged and direct-to-LDS kernels, split contractions, a product
+    cut along N, with ReLU and with sign bits -- the bits of the product with a converted bias."""
+    from tritonformer_amd import _lib
+
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(N)
+    x, w = torch.randn(M, K, generator=g).to(dtype).to(dev), (torch.randn(K, N, generator=g) / K ** 0.5).to(dtype).to(dev)
+    bias = torch.randn(N, generator=g).to(dev)
+    low = bias.to(dtype)
+    st, code = torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
+    nb = lib.tf_gemm_workspace_bytes(0, 1, M, N, K)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=dev)
+    a, b = torch.empty(M, N, dtype=dtype, device=dev), torch.empty(M, N, dtype=dtype, device=dev)
+    for relu in (0, 1):
+        _lib.check(lib.tf_gemm(st, code, 0, 1, M, N, K, x.data_ptr(), K, w.data_ptr(), N, a.data_ptr(), N, low.data_ptr(), relu,
+                               ws.data_ptr(), nb))
+        _lib.check(lib.tf_gemm_master_bias(st, code, 0, 1, M, N, K, x.data_ptr(), K, w.data_ptr(), N, b.data_ptr(), N,
+                                           bias.data_ptr(), relu, None, 0, ws.data_ptr(), nb))
+        assert torch.equal(a, b), f"relu {relu}"
+    if N % 8 == 0:
+        ba, bb = (torch.zeros(M, N // 8, dtype=torch.uint8, device=dev) for _ in range(2))
+        rc = [lib.tf_gemm_relu_bits(st, code, code, 0, 1, M, N, K, x.data_ptr(), K, w.data_ptr(), N, a.data_ptr(), N,
+                                    low.data_ptr(), ba.data_ptr(), None, N // 8),
+              lib.tf_gemm_master_bias(st, code, 0, 1, M, N, K, x.data_ptr(), K, w.data_ptr(), N, b.data_ptr(), N,
+                                      bias.data_ptr(), 1, bb.data_ptr(), N // 8, None, 0)]
+        assert rc == [0, 0] and torch.equal(a, b) and torch.equal(ba, bb)
+
+
 @pytest.mark.parametrize("dims,use_bias", [((2, 128, 256, 1024), False), ((3, 77, 136, 264), True),
                                            ((1, 100, 333, 129), True)])
 def test_fused_mlp_equals_two_functions(dims, use_bias, dev):

@@ -67,7 +67,7 @@ def _is_parameter(value):
     return kind is torch.nn.Parameter or (kind is not torch.Tensor and isinstance(value, torch.nn.Parameter))
 
 
-def _cast(value, dtype):
+def cast_argument(value, dtype):
     if isinstance(value, torch.Tensor):
         if value.dtype == dtype:
             return value
@@ -77,7 +77,7 @@ def _cast(value, dtype):
             return value.to(dtype)
         return value
     if isinstance(value, (list, tuple)):
-        return type(value)(_cast(v, dtype) for v in value)
+        return type(value)(cast_argument(v, dtype) for v in value)
     return value
 
 
@@ -102,7 +102,7 @@ def amp_fwd(fwd=None, *, keep=()):
             # the switch alone: entering an autocast region with enabled=False costs 8 us per graph node
             torch.set_autocast_enabled("cuda", False)
             try:
-                return fwd(ctx, *[a if i in keep else _cast(a, dtype) for i, a in enumerate(args)])
+                return fwd(ctx, *[a if i in keep else cast_argument(a, dtype) for i, a in enumerate(args)])
             finally:
                 torch.set_autocast_enabled("cuda", True)
         return fwd(ctx, *args)

@@ -40,11 +40,12 @@ struct GemmParams {
   const void* A;
   const void* B;
   void* C;
-  const void* bias;
+  const void* bias;  // of type T, or fp32 (bias_f32: an fp32 master, rounded to T where it is read)
   float* partial;
   int M, N, K;
   int64_t lda, ldb, ldc;
   int relu;
+  int bias_f32;
   int splits, k_per_split;
   int tiles_m, tiles_n;
   int flags;  // bit 0: skip the XCD remap (set by the diagnostic entry point only)
@@ -182,6 +183,19 @@ struct DmaPanel {
   }
 };
 
+// bias[n .. n + 3] in T
+template <typename T> __device__ __forceinline__ typename Vec<T>::v4 bias4(const GemmParams& p, int n) {
+  if (!p.bias_f32) return *reinterpret_cast<const typename Vec<T>::v4*>((const T*)p.bias + n);
+  const f32x4 b = *reinterpret_cast<const f32x4*>((const float*)p.bias + n);
+  typename Vec<T>::v4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = (T)b[e];
+  return r;
+}
+template <typename T> __device__ __forceinline__ T bias1(const void* bias, int f32, int n) {
+  return f32 ? (T)((const float*)bias)[n] : ((const T*)bias)[n];
+}
+
 // Epilogue of the direct-to-LDS kernel.  Each wave rounds its accumulators (after
 // bias / ReLU), parks one 32-row block at a time in a private LDS region and
 // reads it back row-contiguously, so every global store instruction writes whole
@@ -201,7 +215,7 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
   constexpr int RPI = 64 / CH;            // rows covered by one wave-wide access
   constexpr int EPC = 16 / ES;            // elements per chunk
   char* mine = smem + wave * (32 * ROWB);
-  const T* bias = PLAIN ? nullptr : (const T*)p.bias;
+  const void* bias = PLAIN ? nullptr : p.bias;
   const bool relu = !PLAIN && p.relu;
   const void* mask = PLAIN ? nullptr : p.mask;
   const void* sign_in = PLAIN ? nullptr : p.sign_in;
@@ -227,9 +241,9 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
         if constexpr (ANY) {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            if (nbase + nl + e < p.N) bvals[j][g][e] = bias[nbase + nl + e];
+            if (nbase + nl + e < p.N) bvals[j][g][e] = bias1<T>(bias, p.bias_f32, nbase + nl + e);
         } else {
-          if (nbase + nl < p.N) bvals[j][g] = *reinterpret_cast<const typename Vec<T>::v4*>(bias + nbase + nl);
+          if (nbase + nl < p.N) bvals[j][g] = bias4<T>(p, nbase + nl);
         }
       }
   }
@@ -383,17 +397,16 @@ __device__ __forceinline__ void gemm_epilogue_bits(const GemmParams& p, f32x16 (
   constexpr int IMG = NW * 32 * ROWB;  // the bit image lies behind the waves' slabs
   static_assert(BN / 8 % 16 == 0, "rows of the bit image are whole 16-byte pieces");
   char* mine = smem + wave * (32 * ROWB);
-  const T* bias = (const T*)p.bias;
   T* C = (T*)p.C;
   const int nbase = n0 + wn * WTN;
   const int n_lane = nbase + (lane % CH) * 8;
   T* const row0 = C + (int64_t)(m0 + wm * WTM + lane / CH) * p.ldc + n_lane + (int64_t)(n_lane / p.chunk_n) * p.chunk_skip;
   typename Vec<T>::v4 bvals[TN][4] = {};
-  if (BITS_OUT && bias) {
+  if (BITS_OUT && p.bias) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) bvals[j][g] = *reinterpret_cast<const typename Vec<T>::v4*>(bias + nbase + j * 32 + g * 8 + (lane >> 5) * 4);
+      for (int g = 0; g < 4; ++g) bvals[j][g] = bias4<T>(p, nbase + j * 32 + g * 8 + (lane >> 5) * 4);
   }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -975,7 +988,7 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_dma_group_kernel(GemmGr
 enum ReduceMode { kReduceAny, kReduceRows, kReduceFlat };
 template <typename T, typename TO, ReduceMode MODE>
 __global__ __launch_bounds__(256) void gemm_reduce(int M, int N, int splits, const float* __restrict__ partial,
-                                                    const T* __restrict__ bias, int relu, TO* __restrict__ C,
+                                                    const void* __restrict__ bias, int bias_f32, int relu, TO* __restrict__ C,
                                                     int64_t ldc, int chunk_n, int64_t chunk_skip,
                                                     const float* __restrict__ alpha_ptr) {
   const int64_t total = (int64_t)M * N;
@@ -996,7 +1009,7 @@ __global__ __launch_bounds__(256) void gemm_reduce(int M, int N, int splits, con
       Quad qd;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float x = s[e] * alpha + (MODE == kReduceRows && bias ? (float)bias[n + e] : 0.f);
+        const float x = s[e] * alpha + (MODE == kReduceRows && bias ? (float)bias1<T>(bias, bias_f32, n + e) : 0.f);
         qd.v[e] = (TO)(relu ? fmaxf(x, 0.f) : x);
       }
       if (MODE == kReduceRows) store_out(C + (int64_t)m * ldc + n + (int64_t)(n / chunk_n) * chunk_skip, qd);
@@ -1015,7 +1028,7 @@ __global__ __launch_bounds__(256) void gemm_reduce(int M, int N, int splits, con
       for (int k = 0; k < splits; ++k) s += partial[(int64_t)k * total + i];
       const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
       s *= alpha;
-      if (bias) s += (float)bias[n];
+      if (bias) s += (float)bias1<T>(bias, bias_f32, n);
       C[(int64_t)m * ldc + n + (int64_t)(n / chunk_n) * chunk_skip] = (TO)(relu ? fmaxf(s, 0.f) : s);
     }
   }
@@ -1284,9 +1297,8 @@ static int launch_reduce(hipStream_t st, const GemmParams& p) {
   if (blocks > 4096) blocks = 4096;
   if (blocks < 1) blocks = 1;
   const dim3 g((unsigned)blocks), b(256);
-  const T* bias = (const T*)p.bias;
 #define REDUCE(TO, MODE) \
-  gemm_reduce<T, TO, MODE><<<g, b, 0, st>>>(p.M, p.N, p.splits, p.partial, bias, p.relu, (TO*)p.C, p.ldc, p.chunk_n, \
+  gemm_reduce<T, TO, MODE><<<g, b, 0, st>>>(p.M, p.N, p.splits, p.partial, p.bias, p.bias_f32, p.relu, (TO*)p.C, p.ldc, p.chunk_n, \
                                             p.chunk_skip, p.alpha)
 #define REDUCE_MODE(TO) \
   do { if (rows) REDUCE(TO, kReduceRows); else if (flat) REDUCE(TO, kReduceFlat); else REDUCE(TO, kReduceAny); } while (0)
@@ -1474,8 +1486,10 @@ static int gemm_entry(void* stream, int dtype, int out_dtype, int layout_a, int 
                       int64_t K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc,
                       int64_t chunk_n, int64_t chunk_stride, const void* bias, int relu, const void* mask_act,
                       int64_t ld_mask, void* workspace, int64_t workspace_bytes, void* sign_out, const void* sign_in,
-                      int64_t ld_sign, const GemmForce& force = kNoForce, const float* alpha = nullptr) {
+                      int64_t ld_sign, const GemmForce& force = kNoForce, const float* alpha = nullptr,
+                      bool bias_f32 = false) {
   if (!A || !B || !C) return TF_EINVAL;
+  if (bias_f32 && (reinterpret_cast<uintptr_t>(bias) & 3)) return TF_EALIGN;
   if (alpha && (reinterpret_cast<uintptr_t>(alpha) & 3)) return TF_EALIGN;
   const bool signs = sign_out || sign_in;
   if (signs) {
@@ -1511,14 +1525,15 @@ static int gemm_entry(void* stream, int dtype, int out_dtype, int layout_a, int 
     const int64_t tail = rt.tail, n1 = N - tail;
     const int64_t osz = out_dtype == TF_F32 ? 4 : 2;
     const char* b2 = (const char*)B + (layout_b == TF_OP_KMAJOR ? n1 * ldb : n1) * 2;
-    const void* bias2 = bias ? (const char*)bias + n1 * 2 : nullptr;
+    const void* bias2 = bias ? (const char*)bias + n1 * (bias_f32 ? 4 : 2) : nullptr;
     void* so2 = sign_out ? (char*)sign_out + n1 / 8 : nullptr;
     const void* si2 = sign_in ? (const char*)sign_in + n1 / 8 : nullptr;
     const int rc = gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, n1, K, A, lda, B, ldb, C, ldc, 0, 0, bias,
-                              relu, nullptr, 0, workspace, workspace_bytes, sign_out, sign_in, ld_sign, force, alpha);
+                              relu, nullptr, 0, workspace, workspace_bytes, sign_out, sign_in, ld_sign, force, alpha, bias_f32);
     if (rc != TF_OK) return rc;
     return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, tail, K, A, lda, b2, ldb, (char*)C + n1 * osz,
-                      ldc, 0, 0, bias2, relu, nullptr, 0, workspace, workspace_bytes, so2, si2, ld_sign, force, alpha);
+                      ldc, 0, 0, bias2, relu, nullptr, 0, workspace, workspace_bytes, so2, si2, ld_sign, force, alpha,
+                      bias_f32);
   }
   const GemmPlan pl = rt.plan;
   // the sign bits exist in the write-out of the direct-to-LDS kernels only
@@ -1535,6 +1550,7 @@ static int gemm_entry(void* stream, int dtype, int out_dtype, int layout_a, int 
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
   p.relu = relu ? 1 : 0;
+  p.bias_f32 = bias_f32 ? 1 : 0;
   p.splits = pl.splits; p.k_per_split = pl.k_per_split;
   p.tiles_m = pl.tiles_m; p.tiles_n = pl.tiles_n;
   p.flags = force.flags;
@@ -1569,6 +1585,15 @@ extern "C" int tf_gemm_relu_bits(void* stream, int dtype, int out_dtype, int lay
   if (!bits_out && !bits_in) return TF_EINVAL;
   return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, N, K, A, lda, B, ldb, C, ldc, 0, 0, bias,
                     bits_out ? 1 : 0, nullptr, 0, nullptr, 0, bits_out, bits_in, ld_bits);
+}
+
+extern "C" int tf_gemm_master_bias(void* stream, int dtype, int layout_a, int layout_b, int64_t M, int64_t N, int64_t K,
+                                   const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc,
+                                   const float* bias, int relu, void* bits_out, int64_t ld_bits, void* workspace,
+                                   int64_t workspace_bytes) {
+  if (!bias) return TF_EINVAL;
+  return gemm_entry(stream, dtype, dtype, layout_a, layout_b, M, N, K, A, lda, B, ldb, C, ldc, 0, 0, bias, relu, nullptr, 0,
+                    workspace, workspace_bytes, bits_out, nullptr, ld_bits, kNoForce, nullptr, true);
 }
 
 extern "C" int tf_gemm_scaled(void* stream, int dtype, int out_dtype, int layout_a, int layout_b, int64_t M, int64_t N,
@@ -1763,6 +1788,7 @@ extern "C" int tf_gemm_group(void* stream, int dtype, int out_dtype, int layout_
     p.M = (int)q.M; p.N = (int)q.N; p.K = (int)q.K;
     p.lda = q.lda; p.ldb = q.ldb; p.ldc = q.ldc;
     p.relu = 0;
+    p.bias_f32 = 0;
     p.tiles_m = (int)((q.M + 255) / 256); p.tiles_n = (int)((q.N + 255) / 256);
     const int64_t ksteps = q.K / 64;
     const int64_t steps_per = (ksteps + want - 1) / want;

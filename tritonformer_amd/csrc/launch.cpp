@@ -556,13 +556,16 @@ TF_FN(colsum, 2) {
 
 // c (m, n) = relu?(a (m, k) . b + bias), b as the header's layouts have it
 bool product(const Tensor& like, int lb, int64_t m, int64_t n, int64_t k, const void* a, const void* b, int64_t ldb, void* c,
-             const void* bias = nullptr, int relu = 0) {
+             const Tensor* bias = nullptr, int relu = 0) {
   const int dt = code(like.scalar_type());
   const int64_t bytes = tf_gemm_workspace_bytes(TF_OP_KMAJOR, lb, m, n, k);
   Tensor ws = scratch(bytes, like);
   return call([&] {
-    return tf_gemm_out_chunked(stream(), dt, dt, TF_OP_KMAJOR, lb, m, n, k, a, k, b, ldb, c, n, 0, 0, bias, relu, nullptr, 0,
-                               ptr(ws), bytes);
+    if (bias && bias->scalar_type() == at::kFloat)
+      return tf_gemm_master_bias(stream(), dt, TF_OP_KMAJOR, lb, m, n, k, a, k, b, ldb, c, n, bias->data_ptr<float>(), relu,
+                                 nullptr, 0, ptr(ws), bytes);
+    return tf_gemm_out_chunked(stream(), dt, dt, TF_OP_KMAJOR, lb, m, n, k, a, k, b, ldb, c, n, 0, 0,
+                               bias ? bias->data_ptr() : nullptr, relu, nullptr, 0, ptr(ws), bytes);
   });
 }
 
@@ -641,9 +644,9 @@ TF_FN(attn_block_dqkv, 6) {
   return THPVariable_Wrap(dqkv);
 }
 
-// mlp(x (B, S, k), w1 (k, f), b1 | None, w2 (f, n), b2 | None, with_bits)
+// mlp(x (B, S, k), w1 (k, f), b1 | None, w2 (f, n), b2 | None, with_bits, master_biases: fp32 ones are taken as well)
 //   -> (relu(x w1 + b1) w2 + b2, hidden, sign bits | None, w1 and w2 in x's dtype)
-TF_FN(mlp, 6) {
+TF_FN(mlp, 7) {
   const Tensor *x = dense(args.a[0]), *w1 = dense(args.a[1]), *w2 = dense(args.a[3]);
   const Tensor *b1 = nullptr, *b2 = nullptr;
   if (!x || !w1 || !w2 || x->dim() != 3 || !is16(*x) || w1->dim() != 2 || w2->dim() != 2 || w1->size(0) != last(*x) ||
@@ -653,7 +656,8 @@ TF_FN(mlp, 6) {
   auto bias = [&](PyObject* o, int64_t size, const Tensor** out) {
     if (o == Py_None) return true;
     *out = dense(o);
-    return *out && (*out)->dim() == 1 && (*out)->size(0) == size && (*out)->scalar_type() == x->scalar_type();
+    return *out && (*out)->dim() == 1 && (*out)->size(0) == size &&
+           ((*out)->scalar_type() == x->scalar_type() || (args.a[6] == Py_True && (*out)->scalar_type() == at::kFloat && aligned(**out)));
   };
   if (!bias(args.a[2], f, &b1) || !bias(args.a[4], n, &b2)) Py_RETURN_NONE;
   Tensor c1, c2;
@@ -672,19 +676,21 @@ TF_FN(mlp, 6) {
     c1 = both.narrow(1, 0, each).view({k, f}), c2 = both.narrow(1, each, each).view({f, n});
   }
   Tensor hidden = make({x->size(0), x->size(1), f}, *x), out = make({x->size(0), x->size(1), n}, *x), bits;
-  const void *p1 = b1 ? b1->data_ptr() : nullptr, *p2 = b2 ? b2->data_ptr() : nullptr;
   int rc = TF_ESHAPE;
   if (args.a[5] == Py_True && f % 8 == 0) {
     bits = make({m, f / 8}, *x, at::kByte);
     const int dt = code(x->scalar_type());
     if (!call([&] {
+          if (b1 && b1->scalar_type() == at::kFloat)
+            return tf_gemm_master_bias(stream(), dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x->data_ptr(), k, c1.data_ptr(), f,
+                                       hidden.data_ptr(), f, b1->data_ptr<float>(), 1, bits.data_ptr(), f / 8, nullptr, 0);
           return tf_gemm_relu_bits(stream(), dt, dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x->data_ptr(), k, c1.data_ptr(), f,
-                                   hidden.data_ptr(), f, p1, bits.data_ptr(), nullptr, f / 8);
+                                   hidden.data_ptr(), f, b1 ? b1->data_ptr() : nullptr, bits.data_ptr(), nullptr, f / 8);
         }, TF_ESHAPE, &rc))
       return nullptr;
   }
-  if (rc != TF_OK && !product(*x, TF_OP_KMINOR, m, f, k, x->data_ptr(), c1.data_ptr(), f, hidden.data_ptr(), p1, 1)) return nullptr;
-  if (!product(*x, TF_OP_KMINOR, m, n, f, hidden.data_ptr(), c2.data_ptr(), n, out.data_ptr(), p2)) return nullptr;
+  if (rc != TF_OK && !product(*x, TF_OP_KMINOR, m, f, k, x->data_ptr(), c1.data_ptr(), f, hidden.data_ptr(), b1, 1)) return nullptr;
+  if (!product(*x, TF_OP_KMINOR, m, n, f, hidden.data_ptr(), c2.data_ptr(), n, out.data_ptr(), b2)) return nullptr;
   if (rc == TF_OK) return tuple_of({&out, &hidden, &bits, &c1, &c2});
   PyObject* t = tuple_of({&out, &hidden, &hidden, &c1, &c2});
   if (t) {

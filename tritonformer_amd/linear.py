@@ -4,7 +4,7 @@ import torch
 from torch.autograd import Function
 
 from . import _deferred, kernels
-from ._amp import amp_bwd, amp_fwd, cached_conversion, weight_cast_cache_enabled
+from ._amp import amp_bwd, amp_fwd, cached_conversion, cast_argument, weight_cast_cache_enabled
 from .kernels import (cast_pack, gemm, gemm_relu_bits, mask_grad, mask_grad_sums, mm, mm_dw, mm_dw_group, mm_masked_bits,
                       unbroadcast_leading)
 
@@ -141,19 +141,21 @@ class MLPReLU(Function):
     (two Functions and an in-place mask kernel, linear.py:47-102)."""
 
     @staticmethod
-    @amp_fwd(keep=(1, 3))
+    @amp_fwd(keep=(1, 2, 3, 4))
     def forward(ctx, input, w1, b1, w2, b2):
         # the weights as the caller holds them: where their gradients go when they are deferred
         ctx.defer_to = (w1, w2) if _deferred.active() and GROUP_DW and _deferred.deferrable((w1, w2)) else None
         block = None
         # conversions of unequal weights and those that are kept between passes are made below
         if w1.dtype == input.dtype or (ctx.amp_active and PACK_CASTS and not weight_cast_cache_enabled()):
-            block = kernels.launch().mlp(input, w1, b1, w2, b2, bool(RELU_BITS))
+            block = kernels.launch().mlp(input, w1, b1, w2, b2, bool(RELU_BITS), ctx.amp_active)
         if block is not None:
             out, hidden, ctx.relu_bits, w1, w2 = block
             ctx.save_for_backward(input, w1, w2, hidden)
             ctx.has_bias = (b1 is not None, b2 is not None)
             return out
+        if ctx.amp_active:
+            b1, b2 = cast_argument(b1, input.dtype), cast_argument(b2, input.dtype)
         if ctx.amp_active and (w1.dtype != input.dtype or w2.dtype != input.dtype):
             # what autocast's cast of the two weights does -- as ONE conversion kernel over both when
             # they are stored alike (two matrices of d*f elements each seen as two rows)
