@@ -205,8 +205,6 @@ def test_cross_entropy_rows(v, dtype, dev):
     assert torch.equal(fv, ov) and torch.equal(loss, loss2) and torch.equal(lse, lse2) and untouched(fb, v)
 
 
-# vocabularies held in registers and streamed (beyond 51200), ragged and whole; the masked tokens fill whole chunks of
-# the first ones of a thread, with -inf and with the type's lowest value
 @pytest.mark.parametrize("v", [2047, 2048, 2049, 2055, 2112, 50257])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_cross_entropy_gradient_is_the_same_bits_wherever_its_rows_start(v, dtype, dev):
@@ -238,6 +236,27 @@ def test_cross_entropy_gradient_is_the_same_bits_wherever_its_rows_start(v, dtyp
     assert torch.equal(run(view, view), want) and untouched(buf, v)
 
 
+# every length of the last chunk, in the first, an inner and the last of a thread's chunks: the rows padded with -inf to
+# whole chunks add zeros to the same sums
+@pytest.mark.parametrize("v0", [0, 8, 2040, 4096, 16376, 30000, 51192])
+def test_cross_entropy_forward_takes_every_end_of_a_row(v0, dev):
+    for v in range(v0 + 1, v0 + 9):
+        g = torch.Generator().manual_seed(v)
+        x = (2 * torch.randn(3, v, generator=g)).half()
+        wide = torch.full((3, (v + 7) // 8 * 8), float("-inf"), dtype=x.dtype)
+        wide[:, :v] = x
+        labels = torch.tensor([0, v - 1, v // 2], device=dev)
+        got = []
+        for t in (odd_rows(x, dev)[1], wide.to(dev)):
+            loss, lse = torch.empty(3, dtype=x.dtype, device=dev), torch.empty(3, device=dev)
+            _lib.check(_lib.load().tf_cross_entropy_fwd(_lib.stream_ptr(), _lib.dtype_code(x.dtype), 3, t.shape[1], t.data_ptr(),
+                                                        t.stride(0), 0, 0, labels.data_ptr(), loss.data_ptr(), lse.data_ptr()))
+            got.append((loss, lse))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), v
+
+
+# vocabularies held in registers and streamed (beyond 51200), ragged and whole; the masked tokens fill whole chunks of
+# the first ones of a thread, with -inf and with the type's lowest value
 @pytest.mark.parametrize("v", [257, 16385, 51199, 51201, 51208, 70001, 128257])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_cross_entropy_of_masked_rows(v, dtype, dev):

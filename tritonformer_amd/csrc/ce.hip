@@ -16,7 +16,8 @@ constexpr int kCeThreads = 256;
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 // The probabilities of a gradient chunk, exp2(x * log2e - l2).  ANY: also where they are subnormal numbers, which an
 // upstream gradient may lift into the range of the type -- only a chunk that has one takes the library function
-// (4095 x 50257 bf16, forward with gradient: 246 us without, 276 with that function for every element, 263 this way).
+// (4095 x 50257 bf16, forward with gradient, as it then was: 246 us without, 276 with that function for every element, 263
+// this way).
 template <bool ANY> __device__ __forceinline__ void grad_probs(float (&v)[8], float l2) {
   float least = 0.f;
 #pragma unroll
@@ -135,12 +136,21 @@ __global__ __launch_bounds__(kCeThreads, NCH == 8 ? 4 : 1) void ce_fwd_regs(int 
 #pragma unroll
   for (int u = 0; u < NCH; ++u) {
     const int c = threadIdx.x + u * kCeThreads;
-    if (c < nchunk) raw[u] = Row<T, ANY>::template load<true>(xr, c, V, (T)-INFINITY);
+    if (c < nchunk) raw[u] = Row<T, ANY>::template fetch<true, true>(xr, c, V, (T)-INFINITY);
   }
   float m = -INFINITY;
 #pragma unroll
   for (int u = 0; u < NCH; ++u) {
-    if (threadIdx.x + u * kCeThreads < nchunk) {
+    const int c = threadIdx.x + u * kCeThreads;
+    if (c < nchunk) {
+      // The chunk that crosses the end of the row is the 16 bytes that end with it, moved down -- behind a branch that one
+      // wave takes (the empty statement keeps the moves from being made for every chunk).  Eight tested element loads in
+      // its place held up the loads in flight.  bf16 with gradient, us: 4095 x 50257 190 -> 173, 2047 x 33001 70.7 -> 58,
+      // 8192 x 1001 24.0 -> 20.5; forward alone 8192 x 4097 19.1 -> 16.7, 8192 x 1001 13.3 -> 11.9, 4095 x 50257 82 as before.
+      if (ANY && (c + 1) * 8 > V) {
+        asm volatile("");
+        raw[u] = Row<T, ANY>::template settle<true>(raw[u], c, V, (T)-INFINITY);
+      }
       float v[8];
       unpack8<T>(raw[u], v);
 #pragma unroll
@@ -156,7 +166,7 @@ __global__ __launch_bounds__(kCeThreads, NCH == 8 ? 4 : 1) void ce_fwd_regs(int 
 #pragma unroll
   for (int w = 1; w < kCeThreads / 64; ++w) m = fmaxf(m, red[0][w]);
   // The later passes convert the row again: bf16 rows kept as floats from one pass to the next took 25 chunks to 290
-  // registers, one wave per SIMD (4095 x 50257 bf16, forward with gradient: 263 -> 188 us, 50304 193 -> 153).
+  // registers, one wave per SIMD (4095 x 50257 bf16, forward with gradient: 263 -> 188 us, 173 since; 50304 193 -> 153).
 #pragma unroll
   for (int u = 0; u < NCH; ++u) asm("" : "+v"(raw[u]));
   const float m2 = m * kLog2e;
