@@ -174,6 +174,35 @@ def test_softmax_of_long_ragged_rows_loses_nothing_to_its_sums(n, dev):
     assert (K.softmax_fwd(x.to(dev)[None])[0].cpu().double() - want).norm() < 1.2 * least
 
 
+# every length of the last chunk of rows that a workgroup holds (4, 8 and 16 chunks per thread; backward operands of the last
+# read twice): padded to whole chunks with -inf and zeros, the rows have the same terms
+@pytest.mark.parametrize("dtype,n0", [(torch.float16, 4096), (torch.float16, 40000), (torch.bfloat16, 65528), (torch.float32, 2048),
+                                      (torch.float32, 16384), (torch.float32, 20000), (torch.float32, 65528)])
+def test_softmax_of_long_rows_takes_every_end(dtype, n0, dev):
+    lib, st, dt = _lib.load(), _lib.stream_ptr(), _lib.dtype_code(dtype)
+    for n in range(n0 + 1, n0 + 8):
+        x = torch.randn(3, n, generator=torch.Generator().manual_seed(n)).to(dtype)
+        got = []
+        for pad in (0, -n % 8):
+            wide = torch.cat([x, torch.full((3, pad), float("-inf"), dtype=dtype)], 1)
+            dy = torch.cat([x, torch.zeros(3, pad, dtype=dtype)], 1)
+            put = (lambda t: t.to(dev)) if pad else (lambda t: odd_rows(t, dev)[1])
+            wide, dy, y, dx = put(wide), put(dy), put(torch.zeros_like(wide)), put(torch.zeros_like(wide))
+            _lib.check(lib.tf_softmax_fwd(st, dt, 3, n + pad, wide.data_ptr(), wide.stride(0), y.data_ptr(), y.stride(0)))
+            if pad:  # the backward of one forward
+                got[0] = (got[0][0], y[:, :n].clone(), got[0][1])
+                y[:, :n] = got[0][0]
+            _lib.check(lib.tf_softmax_bwd(st, dt, 3, n + pad, dy.data_ptr(), dy.stride(0), y.data_ptr(), y.stride(0),
+                                          dx.data_ptr(), dx.stride(0)))
+            got.append((y[:, :n], dx[:, :n]))
+        # the compiler may contract the terms of a sum otherwise in the two kernels: 128 terms of a thread and 10 steps between
+        # threads in fp32, twice, sum |y dy| < 6 in the backward, and one rounding of a result (2^-24: a subnormal one of fp16)
+        sums, eps = 2 * 138 * 2.0 ** -24, torch.finfo(dtype).eps
+        y0, y1, dx0, dx1 = [t.double() for t in (*got[0], got[1][1])]
+        assert ((y0 - y1).abs() <= y1 * (sums + eps) + 2.0 ** -24).all(), n
+        assert ((dx0 - dx1).abs() <= y0 * 6 * sums + dx1.abs() * eps + 2.0 ** -24).all(), n
+
+
 # 8 / 16 / 25 chunks of 256 threads in registers (16384, 32768, 51200 entries), then the streaming forward
 @pytest.mark.parametrize("v", [1, 9, 16383, 16385, 32769, 50257, 51199, 51201, 70001])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

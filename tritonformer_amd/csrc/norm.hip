@@ -635,6 +635,16 @@ template <bool ANY, int N> __device__ __forceinline__ void long_exp2(float (&v)[
     for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_exp2f(v[e]);
   }
 }
+// The chunk that crosses the end of a ragged row, fetched as the 16 bytes that end with it.  Called behind a branch that one
+// wave of the row takes: the empty statement keeps the moves from being made for every chunk.  Eight tested element loads in
+// its place, each waited for, held the row up at the workgroup's reduction (us, forward / backward): fp16 4000 x 5001
+// 48.1 -> 28.6 / 37.8 -> 30.0, 2000 x 20001 47.7 -> 38.1 / 52.0 -> 49.1, 4096 x 50257 200 -> 195 / 294 -> 286; fp32 2000 x 33001
+// 110 -> 106 / 170 -> 161.  (All loads of the row ahead of the first conversion: the same forward, the backward of 50304
+// fp16 columns 212 -> 216 and 2 % slower in ragged rows, fp32 rows of 8 chunks in scratch.)
+template <typename T> __device__ __forceinline__ void long_row_end(u32x4& raw, int c, int cols, T fill = (T)0.f) {
+  asm volatile("");
+  raw = Row<T, true>::template settle<true>(raw, c, cols, fill);
+}
 template <typename T, int NV, bool ANY>
 __global__ __launch_bounds__(kLongRowThreads) void softmax_fwd_long(int cols, const T* __restrict__ x, int64_t ldx,
                                                                     T* __restrict__ y, int64_t ldy) {
@@ -649,7 +659,9 @@ __global__ __launch_bounds__(kLongRowThreads) void softmax_fwd_long(int cols, co
   for (int i = 0; i < NV; ++i) {
     const int c = threadIdx.x + i * kLongRowThreads;
     if (c < nchunk) {
-      row_floats<T>(Row<T, ANY>::template load<true>(xr, c, cols, (T)-INFINITY), v[i]);
+      u32x4 raw = Row<T, ANY>::template fetch<true, true>(xr, c, cols, (T)-INFINITY);
+      if (ANY && (c + 1) * N > cols) long_row_end<T>(raw, c, cols, (T)-INFINITY);
+      row_floats<T>(raw, v[i]);
 #pragma unroll
       for (int e = 0; e < N; ++e) m = fmaxf(m, v[i][e]);
     }
@@ -698,8 +710,12 @@ __global__ __launch_bounds__(kLongRowThreads) void softmax_bwd_long(int cols, co
   for (int i = 0; i < NV; ++i) {
     const int c = threadIdx.x + i * kLongRowThreads;
     if (c < nchunk) {
-      ry[i] = Row<T, ANY>::template load<true>(y + row * ldy, c, cols);
-      const u32x4 g = Row<T, ANY>::template load<HOLD_DY>(dy + row * lddy, c, cols);
+      ry[i] = Row<T, ANY>::template fetch<true, true>(y + row * ldy, c, cols);
+      u32x4 g = Row<T, ANY>::template fetch<true, HOLD_DY>(dy + row * lddy, c, cols);
+      if (ANY && (c + 1) * N > cols) {
+        long_row_end<T>(ry[i], c, cols);
+        long_row_end<T>(g, c, cols);
+      }
       if (HOLD_DY) rg[i] = g;
       float yv[N], gv[N];
       row_floats<T>(ry[i], yv);
@@ -713,9 +729,11 @@ __global__ __launch_bounds__(kLongRowThreads) void softmax_bwd_long(int cols, co
   for (int i = 0; i < NV; ++i) {
     const int c = threadIdx.x + i * kLongRowThreads;
     if (c < nchunk) {
+      u32x4 g = HOLD_DY ? rg[i] : Row<T, ANY>::template fetch<true>(dy + row * lddy, c, cols);
+      if (!HOLD_DY && ANY && (c + 1) * N > cols) long_row_end<T>(g, c, cols);
       float yv[N], gv[N], o[N];
       row_floats<T>(ry[i], yv);
-      row_floats<T>(HOLD_DY ? rg[i] : Row<T, ANY>::load(dy + row * lddy, c, cols), gv);
+      row_floats<T>(g, gv);
 #pragma unroll
       for (int e = 0; e < N; ++e) o[e] = yv[e] * (gv[e] - s);
       Row<T, ANY>::store(dx + row * lddx, c, cols, row_pack<T>(o));
