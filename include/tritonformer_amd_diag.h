@@ -33,7 +33,20 @@ int tf_diag_gemm(void* stream, int cfg, int splits, int flags, int dtype, int ou
                  int layout_a, int layout_b, int64_t M, int64_t N, int64_t K,
                  const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc,
                  const void* bias, int relu, void* workspace, int64_t workspace_bytes);
+/* tf_gemm_relu_bits with the tile choice imposed in the same way. */
+int tf_diag_gemm_relu_bits(void* stream, int cfg, int dtype, int out_dtype, int layout_a, int layout_b,
+                           int64_t M, int64_t N, int64_t K,
+                           const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc,
+                           const void* bias, void* bits_out, const void* bits_in, int64_t ld_bits);
 int64_t tf_diag_gemm_workspace_bytes(int cfg, int splits, int64_t M, int64_t N, int64_t K);
+
+/* The launches that a product becomes on a device of `cus` compute units; nothing is launched and no device is needed.
+ *   vec   1: the preconditions of the direct-to-LDS kernels other than K % 64 == 0 hold;
+ *   kind  0 = tf_gemm, tf_gemm_out, tf_gemm_scaled; 1 = tf_gemm_relu_bits; 2 = with mask_act;
+ *         3 = column blocks (tf_gemm_out_chunked with 0 < chunk_n < N).
+ * Each launch is a row of four in `launches` (HOST memory, `room` rows): columns, configuration (as cfg above),
+ * slices of the contraction, elements of the contraction per slice.  Returns their number. */
+int tf_diag_gemm_route(int cus, int64_t M, int64_t N, int64_t K, int vec, int kind, int64_t* launches, int room);
 
 /* GEMM kernels launched by libtritonformer_amd.so since it was loaded (the reduce passes of
  * split contractions are not counted; one tf_gemm* call may launch two kernels when the

@@ -77,6 +77,9 @@ SIGNATURES = {
 DIAG_SIGNATURES = {
     "tf_diag_gemm": ("main", _i, [_vp, _i, _i, _i, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64,
                                   _vp, _i, _vp, _i64]),
+    "tf_diag_gemm_relu_bits": ("main", _i, [_vp, _i, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64,
+                                            _vp, _vp, _vp, _i64]),
+    "tf_diag_gemm_route": ("main", _i, [_i, _i64, _i64, _i64, _i, _i, ctypes.POINTER(_i64), _i]),
     "tf_diag_gemm_workspace_bytes": ("main", _i64, [_i, _i, _i64, _i64, _i64]),
     "tf_diag_gemm_launch_count": ("main", _i64, []),
     "tf_diag_mfma_rate": ("diag", _i, [_vp, _i, _vp, _i, _i, _vp]),

@@ -1212,7 +1212,10 @@ static GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec
   // an idle chip, a 64x64 one's 0.27, and start and write-out shrink with the tile: 128 x 1024 x 1024 14.4 -> 6.9 us,
   // 960 x 768 x 768 12.1 -> 6.3, 2048 x 1024 x 1024 15.1 -> 9.5.  Beyond one round the larger tiles are the better ones
   // throughout (2048 x 4096 x 1024: 21 against 29 us).  The slices of the contraction stay those of the larger tile: the
-  // same sums in the same order, whatever the tile.
+  // same sums in the same order, whatever the tile.  The cost handed back stays the larger tile's: the cuts below compare it
+  // with that of whole rounds, and the two scales are not comparable (mixed, 247 of 400 000 products were cut otherwise: 1920 x
+  // 8512 x 2304 79 us for 86 but 3968 x 4160 x 512 25.2 for 24.0 and 384 x 35840 x 2048 83.9 for 80.5, 16 of them with other
+  // slices and so with sums in another order).
   const int64_t wgs = (int64_t)best.tiles_m * best.tiles_n * best.splits;
   if (dma && wgs <= cus * (best.cfg == 3 ? 2 : 1)) {
     const GemmPlan best_large = best;
@@ -1220,7 +1223,7 @@ static GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec
     for (int cfg : {6, 7}) {
       const GemmPlan pl = plan_for(cus, cfg, M, N, K, nullptr, allow_split, best_large.splits);
       const double us = part_round_us(cus, pl, M, N);
-      if (us < best_us) { best_us = us; best = pl; best_cost = std::min(best_cost, us); }
+      if (us < best_us) { best_us = us; best = pl; }
     }
   }
   if (cost_us) *cost_us = best_cost;
@@ -1614,6 +1617,32 @@ extern "C" int tf_diag_gemm(void* stream, int cfg, int splits, int flags, int dt
   const GemmForce force = {cfg < 0 ? -1 : cfg, splits, flags};
   return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, N, K, A, lda, B, ldb, C, ldc, 0, 0, bias, relu,
                     nullptr, 0, workspace, workspace_bytes, nullptr, nullptr, 0, force);
+}
+extern "C" int tf_diag_gemm_relu_bits(void* stream, int cfg, int dtype, int out_dtype, int layout_a, int layout_b, int64_t M,
+                                      int64_t N, int64_t K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C,
+                                      int64_t ldc, const void* bias, void* bits_out, const void* bits_in, int64_t ld_bits) {
+  if (cfg >= kNumCfgs || (!bits_out && !bits_in)) return TF_EINVAL;
+  const GemmForce force = {cfg < 0 ? -1 : cfg, 0, 0};
+  return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, N, K, A, lda, B, ldb, C, ldc, 0, 0, bias,
+                    bits_out ? 1 : 0, nullptr, 0, nullptr, 0, bits_out, bits_in, ld_bits, force);
+}
+// The launches of a product, in the order in which gemm_entry makes them: rows of {columns, configuration, slices,
+// contraction elements per slice} from `at` on.  Returns the rows there are then, -1 where `room` does not hold them.
+static int route_launches(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec, RouteKind kind, int64_t (*rows)[4], int at,
+                          int room) {
+  const Route r = find_route(cus, M, N, K, vec, kind);
+  if (r.tail > 0) {
+    at = route_launches(cus, M, N - r.tail, K, vec, kind, rows, at, room);
+    return at < 0 ? at : route_launches(cus, M, r.tail, K, vec, kind, rows, at, room);
+  }
+  if (at >= room) return -1;
+  const int64_t row[4] = {N, r.plan.cfg, r.plan.splits, r.plan.k_per_split};
+  std::copy(row, row + 4, rows[at]);
+  return at + 1;
+}
+extern "C" int tf_diag_gemm_route(int cus, int64_t M, int64_t N, int64_t K, int vec, int kind, int64_t* launches, int room) {
+  if (cus < 1 || M <= 0 || N <= 0 || K <= 0 || kind < 0 || kind > kRouteChunked || !launches || room < 1) return TF_EINVAL;
+  return route_launches(cus, M, N, K, vec != 0, (RouteKind)kind, reinterpret_cast<int64_t(*)[4]>(launches), 0, room);
 }
 extern "C" int64_t tf_diag_gemm_workspace_bytes(int cfg, int splits, int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || cfg >= kNumCfgs) return 0;
