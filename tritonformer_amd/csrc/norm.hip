@@ -211,7 +211,9 @@ __global__ __launch_bounds__(256) void ln_bwd_vec(int64_t rows, int d, const T* 
                                                    const float* __restrict__ rstd, T* __restrict__ dx,
                                                    int64_t lddx, float* __restrict__ partial) {
   typedef Row<T, ANY> R;
-  typedef RowEnds<T, NV, ANY> E;
+  // (four chunks per lane with a residual by elements: with the moves it takes 276 registers, one wave per SIMD -- 31713 x 1025
+  // 69 us by elements, 81 with them, 8192 x 1537 35 and 39)
+  typedef RowEnds<T, NV, ANY, ADD && NV == 4 && WPR == 1 ? NV : NV / 2> E;
   extern __shared__ float dyn[];  // WPR == 1: [4][d] for the sums of the four waves; then [d] for gamma when G_LDS
   __shared__ float red[2][4];
   // Wide rows (NV >= 4) keep gamma in LDS as fp32 and read a chunk where it is used: held in registers its
