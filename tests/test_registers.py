@@ -34,3 +34,9 @@ def test_layernorm_backward_keeps_two_waves_per_simd(norm_kernels):
     kernels = {k: v for k, v in norm_kernels.items() if "ln_bwd_vec" in k}
     assert len(kernels) == 80  # 4 pairs of types, 5 row widths, with and without a residual, whole and ragged rows
     assert {k: v for k, v in kernels.items() if v[0] > 256 or v[1]} == {}
+
+
+def test_layernorm_forward_of_ragged_rows_and_fp32_parameters_keeps_four_waves_per_simd(norm_kernels):
+    kernels = {k: v for k, v in norm_kernels.items() if re.search(r"ln_fwd_vecIDF16b?_?fLi\dELi\dELb\dELb1E", k)}
+    assert len(kernels) == 20
+    assert {k: v for k, v in kernels.items() if v[0] > 128 or v[1]} == {}

@@ -47,8 +47,12 @@ template <typename T, int NV, bool ANY, int FROM = NV / 2> struct RowEnds {
     if (i >= FROM) R::template store<true>(row, c, n, v);
     else R::template store<false>(row, c, n, v);
   }
+  // Elements of gamma or beta.  fp32 ones beyond one chunk per lane are read by elements at the end of the row: eight of them are
+  // two accesses with moves each, which took the forward kernels from 101 to 146 registers, four waves per SIMD to three
+  // (fp16, us, by elements / with moves / here: 8192 x 1025 12.2 / 15.9 / 12.5, 31713 x 1537 48 / 56 / 47, 2048 x 6001 with a
+  // residual 22.0 / 25.8 / 20.9).
   template <typename TP> static __device__ __forceinline__ void load8(const TP* p, int c, int i, int n, float (&v)[8]) {
-    if (i >= FROM) load8_row<TP, ANY, true>(p, c, n, v);
+    if (i >= FROM && (sizeof(TP) == 2 || NV == 1)) load8_row<TP, ANY, true>(p, c, n, v);
     else load8_row<TP, ANY, false>(p, c, n, v);
   }
 };
