@@ -11,14 +11,12 @@ from tritonformer_amd import _build
 LLVM = os.path.join(os.path.dirname(os.path.dirname(_build.HIPCC)), "llvm", "bin")
 
 
-@pytest.fixture(scope="module")
-def norm_kernels(tmp_path_factory):
-    """{mangled name: (vector registers, bytes of scratch)} of csrc/norm.hip"""
-    obj, src = os.path.join(_build.OBJ_DIR, "norm.o"), os.path.join(_build.CSRC, "norm.hip")
+def kernels_of(name, d):
+    """{mangled name: (vector registers, bytes of scratch)} of csrc/<name>.hip; `d`: a folder for what is unpacked"""
+    obj, src = os.path.join(_build.OBJ_DIR, f"{name}.o"), os.path.join(_build.CSRC, f"{name}.hip")
     if not os.path.exists(obj) or os.path.getmtime(obj) < os.path.getmtime(src):
-        pytest.skip("no object of csrc/norm.hip as it is: only the linked library is here")
-    d = tmp_path_factory.mktemp("norm")
-    fat, code = str(d / "norm.fat"), str(d / "norm.co")
+        pytest.skip(f"no object of csrc/{name}.hip as it is: only the linked library is here")
+    fat, code = str(d / "fat"), str(d / "code")
     run = lambda *cmd: subprocess.run(cmd, check=True, capture_output=True, text=True).stdout
     run(f"{LLVM}/llvm-objcopy", f"--dump-section=.hip_fatbin={fat}", obj, str(d / "copy.o"))
     run(f"{LLVM}/clang-offload-bundler", "--unbundle", "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950",
@@ -27,6 +25,11 @@ def norm_kernels(tmp_path_factory):
     found = re.findall(r"\.name:\s+(\S+)\n\s+\.private_segment_fixed_size:\s+(\d+)(?:\n\s+\..*)*?\n\s+\.vgpr_count:\s+(\d+)",
                        notes)
     return {name: (int(regs), int(scratch)) for name, scratch, regs in found}
+
+
+@pytest.fixture(scope="module")
+def norm_kernels(tmp_path_factory):
+    return kernels_of("norm", tmp_path_factory.mktemp("norm"))
 
 
 def test_layernorm_backward_keeps_two_waves_per_simd(norm_kernels):
@@ -40,3 +43,10 @@ def test_layernorm_forward_of_ragged_rows_and_fp32_parameters_keeps_four_waves_p
     kernels = {k: v for k, v in norm_kernels.items() if re.search(r"ln_fwd_vecIDF16b?_?fLi\dELi\dELb\dELb1E", k)}
     assert len(kernels) == 20
     assert {k: v for k, v in kernels.items() if v[0] > 128 or v[1]} == {}
+
+
+def test_cross_entropy_forward_of_whole_rows_holds_a_row_and_little_else(tmp_path):
+    """Five registers per chunk of the row, eight more: what the compiler needs where it follows one test per chunk."""
+    kernels = {k: v for k, v in kernels_of("ce", tmp_path).items() if re.search(r"ce_fwd_regsIDF16b?_?Li\d+ELb0ELb0E", k)}
+    assert len(kernels) == 6
+    assert {k: v for k, v in kernels.items() if v[0] > 5 * int(re.search(r"Li(\d+)E", k)[1]) + 8 or v[1]} == {}
