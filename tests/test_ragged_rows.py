@@ -265,6 +265,38 @@ def test_cross_entropy_gradient_is_the_same_bits_wherever_its_rows_start(v, dtyp
     assert torch.equal(run(view, view), want) and untouched(buf, v)
 
 
+@pytest.mark.parametrize("v", [2048, 2051, 50257])
+def test_cross_entropy_gradient_of_subnormal_probabilities_is_the_same_bits_in_both_ragged_forms(v, dev):
+    """Chunks from the line (results of their own) and from the row's start (in place) cut a row differently, and a chunk takes
+    the library exponential if one of its elements is subnormal: probabilities on both sides of 2^-126, which two lanes write
+    at the ends of a row, lifted into bf16's numbers by the upstream gradient."""
+    g = torch.Generator().manual_seed(v)
+    rows = 70
+    x = -80 - 20 * torch.rand(rows, v, generator=g)
+    x[:, v // 2] = 0
+    x = x.bfloat16().to(dev)
+    labels = torch.tensor([[0, 7, v // 2, v - 8, v - 1][i % 5] for i in range(rows)], device=dev)
+    lse = torch.logsumexp(x.float(), 1)
+    gout = torch.full((rows,), 2.0 ** 20, dtype=torch.bfloat16, device=dev)
+
+    def run(logits, out):
+        _lib.check(_lib.load().tf_cross_entropy_bwd(
+            torch.cuda.current_stream().cuda_stream, _lib.dtype_code(torch.bfloat16), rows, v, logits.data_ptr(),
+            logits.stride(0), 0, 0, labels.data_ptr(), lse.data_ptr(), gout.data_ptr(), 1, out.data_ptr(), out.stride(0), 0))
+        return out
+
+    buf, view = odd_rows(x, dev)
+    out_buf, out = odd_rows(torch.zeros_like(x), dev)
+    lines = run(view, out).clone()
+    want = torch.softmax(x.cpu().double(), 1)
+    for end in (slice(0, 8), slice(v - 8, v)):
+        assert (want[:, end] < 2.0 ** -126).any() and (want[:, end] > 2.0 ** -126).any()
+    assert untouched(out_buf, v) and torch.equal(run(view, view), lines) and untouched(buf, v)
+    want[torch.arange(rows), labels.cpu()] -= 1
+    # as in the test of subnormal numbers above
+    assert ((lines.cpu().double() / 2.0 ** 20 - want).abs() <= want.abs() * (2.0 ** -8 + 1e-4) + 2.0 ** -148).all()
+
+
 # every length of the last chunk, in the first, an inner and the last of a thread's chunks: the rows padded with -inf to
 # whole chunks add zeros to the same sums
 @pytest.mark.parametrize("v0", [0, 8, 2040, 4096, 16376, 30000, 51192])

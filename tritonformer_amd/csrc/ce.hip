@@ -229,7 +229,9 @@ __global__ __launch_bounds__(kCeThreads, NCH == 8 ? 4 : 1) void ce_fwd_regs(int 
 // the row, wherever it lies.  kCeLines: chunks counted from the 128-byte line in which the row of the gradient starts, so that
 // a wave's access covers whole lines instead of leaving a piece of one to the next: 4095 x 50257 bf16 187 -> 170 us
 // (4.8 TB/s), 2047 x 32001 50.7 -> 44.3, 8192 x 4097 27.3 -> 24.6, but 8192 x 1001 12.1 -> 12.8 (written through, these
-// stores take 183, 53 and 54 us).  The values are the same bits in every form: an element depends on nothing but itself.
+// stores take 183, 53 and 54 us).  The values of the last two are the same bits: an element depends on nothing but itself, and
+// where a chunk holds a probability below 2^-126 the library function gives its other elements what v_exp_f32 would.  Whole
+// aligned rows flush such probabilities to zero.
 enum CeRows { kCeAligned, kCeShort, kCeLines };
 constexpr int64_t kCeLinesFrom = 2048;
 template <typename T, CeRows FORM>
