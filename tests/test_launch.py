@@ -251,6 +251,136 @@ def test_blocks_in_one_call_give_the_bits_of_their_launches(dtype, autocast, bat
         assert torch.equal(a, b)
 
 
+class _Counted:
+    """The extension module; counts the answers of the functions that run a whole block, and those that are None."""
+
+    def __init__(self, native):
+        self._native, self.answers = native, {}
+
+    def __getattr__(self, name):
+        fn = getattr(self._native, name)
+        if name not in ("attn_block", "attn_block_dqkv", "mlp", "adamw"):
+            return fn
+
+        def counted(*args):
+            out = fn(*args)
+            served, declined = self.answers.get(name, (0, 0))
+            self.answers[name] = (served + (out is not None), declined + (out is None))
+            return out
+
+        return counted
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("autocast,cache", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("form", ["plain", "strided", "odd", "transposed"])
+def test_blocks_serve_plain_operands_and_hand_back_the_others(form, autocast, cache, dev, monkeypatch):
+    """Inputs, weights and biases of every form, kept 16-bit weights: the bits of the launches one by one, and the block
+    functions are the ones that ran wherever every operand is plain (the weights that the cache holds in 16 bits are, whatever
+    form they were converted from)."""
+    import tritonformer_amd as T
+    from tritonformer_amd import kernels as K
+
+    torch.manual_seed(11)
+    dtype, wt = torch.float16, torch.float32 if autocast else torch.float16
+    shape = lambda t: forms(t).get(form, t)
+    x = shape(randn(2, 64, 128))
+    ws = [torch.nn.Parameter(shape(torch.randn(s, device=dev) * 0.1).to(wt)) for s in
+          [(128, 128)] * 4 + [(128, 512), (512,), (512, 128), (128,)]]
+    grad = shape(randn(2, 64, 128))
+    T.set_weight_cast_cache(cache)
+
+    def run():
+        T.clear_weight_cast_cache()
+        for w in ws:
+            w.grad = None
+        leaf = x.detach().requires_grad_(True)
+        with torch.autocast("cuda", dtype=dtype, enabled=autocast):
+            out = T.mlp_fused_relu.apply(T.attention_block.apply(leaf, *ws[:4], 2, None), *ws[4:])
+        out.backward(grad)
+        return [out.detach(), leaf.grad] + [w.grad for w in ws]
+
+    try:
+        native = K.launch()
+        counted = _Counted(native)
+        monkeypatch.setattr(K, "launch", lambda: counted)
+        together = run()
+        monkeypatch.setattr(K, "launch", lambda: _OneByOne(native))
+        for a, b in zip(together, run()):
+            assert torch.equal(a, b)
+    finally:
+        T.set_weight_cast_cache(False)
+    assert set(counted.answers) >= {"attn_block", "attn_block_dqkv"}
+    if form == "plain":
+        assert all(declined == 0 for _, declined in counted.answers.values()) and ("mlp" in counted.answers) == (not cache)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shadow_dtype", [None, torch.float16, torch.bfloat16])
+def test_adamw_takes_its_tensors_natively_or_one_by_one(shadow_dtype, dev, monkeypatch):
+    """The native hand-over of the tensors against the ctypes one: the same parameters, moments and copies; an empty parameter
+    goes the second way, with every other of its step."""
+    from tritonformer_amd import optim
+
+    native, counted = optim.launch(), []
+
+    def steps(launch, sizes):
+        monkeypatch.setattr(optim, "launch", launch)
+        g = torch.Generator().manual_seed(2)
+        params = [torch.randn(s, generator=g).to(dev).requires_grad_(True) for s in sizes]
+        opt = optim.AdamW(params, lr=3e-3, weight_decay=0.1, shadow_dtype=shadow_dtype)
+        for step in range(3):
+            for i, p in enumerate(params):
+                p.grad = torch.randn(p.shape, generator=g).to(dev) if (step, i) != (1, 0) else None  # steps of their own from here
+            versions = [p._version for p in params]
+            opt.step()
+            assert all((p._version > v) == (p.grad is not None) for p, v in zip(params, versions))
+        return [t for p in params for t in (p.detach(), opt.state[p]["exp_avg"], opt.state[p]["exp_avg_sq"], opt.shadow(p))]
+
+    def through():
+        counted.append(_Counted(native))
+        return counted[-1]
+
+    for sizes in ([(7,), (64, 33), (1000,)], [(7,), (0,), (64, 33)]):
+        del counted[:]
+        for a, b in zip(steps(through, sizes), steps(HandsBack, sizes)):
+            assert a is b is None or torch.equal(a, b)
+        served = sum(c.answers.get("adamw", (0, 0))[0] for c in counted)
+        assert served == (3 + 1 if (0,) not in sizes else 1)
+
+
+def test_a_body_that_raises_leaves_autocast_as_it_was():
+    """The node's body runs with autocast off, and the flag is back on whichever way the body ends."""
+    from tritonformer_amd._amp import amp_fwd
+
+    seen = []
+
+    class Ctx:
+        pass
+
+    @amp_fwd
+    def body(ctx, fail):
+        seen.append(torch.is_autocast_enabled("cuda"))
+        if fail:
+            raise RuntimeError("body")
+        return 1
+
+    was = torch.is_autocast_enabled("cuda")
+    try:
+        torch.set_autocast_enabled("cuda", True)
+        assert body(Ctx(), False) == 1 and torch.is_autocast_enabled("cuda")
+        with pytest.raises(RuntimeError, match="body"):
+            body(Ctx(), True)
+        assert torch.is_autocast_enabled("cuda")
+        torch.set_autocast_enabled("cuda", False)
+        with pytest.raises(RuntimeError, match="body"):
+            body(Ctx(), True)
+        assert not torch.is_autocast_enabled("cuda")
+    finally:
+        torch.set_autocast_enabled("cuda", was)
+    assert seen == [False, False, False]
+
+
 def test_pick_takes_what_the_exhaustive_search_takes():
     """The packing of pending weight gradients against the search over ways to reach a sum, written out."""
     import random

@@ -347,13 +347,15 @@ def test_small_tiles_give_the_bits_of_the_large_ones(layouts, M, N, dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (33, 129, 70), (200, 328, 192), (512, 768, 4096), (4096, 2304, 1024)])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (33, 129, 70), (200, 328, 192), (512, 768, 4096), (4096, 2304, 1024),
+                                   (4096, 6144, 1536)])
 def test_master_bias_is_the_bias_converted_ahead(dtype, M, N, K, dev):
     """A bias read as fp32 and rounded in the product: register-staged and direct-to-LDS kernels, split contractions, a product
-    cut along N, with ReLU and with sign bits -- the bits of the product with a converted bias."""
+    cut along N (the last: 4096 columns, then 2048), with ReLU and with sign bits -- the bits of the product with a converted
+    bias."""
     from tritonformer_amd import _lib
 
-    lib = _lib.load()
+    lib, launches = _lib.load(), _lib.load_diag().tf_diag_gemm_launch_count
     g = torch.Generator().manual_seed(N)
     x, w = torch.randn(M, K, generator=g).to(dtype).to(dev), (torch.randn(K, N, generator=g) / K ** 0.5).to(dtype).to(dev)
     bias = torch.randn(N, generator=g).to(dev)
@@ -370,11 +372,13 @@ def test_master_bias_is_the_bias_converted_ahead(dtype, M, N, K, dev):
         assert torch.equal(a, b), f"relu {relu}"
     if N % 8 == 0:
         ba, bb = (torch.zeros(M, N // 8, dtype=torch.uint8, device=dev) for _ in range(2))
+        before = launches()
         rc = [lib.tf_gemm_relu_bits(st, code, code, 0, 1, M, N, K, x.data_ptr(), K, w.data_ptr(), N, a.data_ptr(), N,
                                     low.data_ptr(), ba.data_ptr(), None, N // 8),
               lib.tf_gemm_master_bias(st, code, 0, 1, M, N, K, x.data_ptr(), K, w.data_ptr(), N, b.data_ptr(), N,
                                       bias.data_ptr(), 1, bb.data_ptr(), N // 8, None, 0)]
         assert rc == [0, 0] and torch.equal(a, b) and torch.equal(ba, bb)
+        assert launches() - before == (4 if N == 6144 else 2)
 
 
 @pytest.mark.parametrize("dims,use_bias", [((2, 128, 256, 1024), False), ((3, 77, 136, 264), True),
@@ -651,3 +655,35 @@ def test_sign_bit_rows_of_any_pitch_and_alignment(pitch, shift, dev):
                                None, bits.data_ptr(), pitch)
     assert rc == 0
     assert torch.equal(dh, K.mm(dy.view(1, m, d), w2.T, mask_act=want_h.view(1, m, f)).view(m, f))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", [2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("pitch,shift", [(32, 0), (40, 0), (48, 8), (37, 0)])
+def test_sign_bit_rows_on_every_tile(cfg, pitch, shift, dev):
+    """The test above on each tile configuration: bit rows that go in 16-byte pieces (32, 0) and those that cannot, full tiles
+    (512 x 256) and tiles that end in the middle (500 x 248), bias and none."""
+    import numpy as np
+    from tritonformer_amd import _lib
+
+    call = _lib.load_diag().tf_diag_gemm_relu_bits
+    st = _lib.stream_ptr()
+    for m, d, f, biased in ((512, 256, 256, True), (500, 192, 248, False)):
+        g = torch.Generator().manual_seed(43)
+        x, dy = (torch.randn(m, d, generator=g).half().to(dev) for _ in range(2))
+        w1 = (torch.randn(d, f, generator=g) / d ** 0.5).half().to(dev)
+        w2 = (torch.randn(f, d, generator=g) / f ** 0.5).half().to(dev)
+        bias = torch.randn(f, generator=g).half().to(dev) if biased else None
+        raw = torch.zeros(m * pitch + 64, dtype=torch.uint8, device=dev)
+        bits = raw[shift:shift + m * pitch].view(m, pitch)
+        hidden, dh = (torch.full((m + 1, f), 7.0, dtype=torch.float16, device=dev) for _ in range(2))
+        assert call(st, cfg, 0, 0, 0, 1, m, f, d, x.data_ptr(), d, w1.data_ptr(), f, hidden.data_ptr(), f,
+                    bias.data_ptr() if biased else None, bits.data_ptr(), None, pitch) == 0
+        want = K_mod.gemm(x.view(1, m, d), w1, bias, True).view(m, f)
+        assert torch.equal(hidden[:m], want) and (hidden[m] == 7).all()
+        assert np.array_equal(bits[:, : f // 8].cpu().numpy(), np.packbits((want > 0).cpu().numpy(), axis=1, bitorder="little"))
+        assert not bits[:, f // 8:].any() and not raw[shift + m * pitch:].any() and not raw[:shift].any()
+        assert call(st, cfg, 0, 0, 0, 0, m, f, d, dy.data_ptr(), d, w2.data_ptr(), d, dh.data_ptr(), f, None, None,
+                    bits.data_ptr(), pitch) == 0
+        assert torch.equal(dh[:m], K_mod.mm(dy.view(1, m, d), w2.T, mask_act=want.view(1, m, f)).view(m, f))
+        assert (dh[m] == 7).all()
