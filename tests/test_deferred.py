@@ -49,7 +49,7 @@ def test_packing_fills_whole_rounds():
     assert _simulate(2048, 8192, 24) == [512, 256] * 24
     # 840M: 252 of 256 or 504 of 512 but for the very last product; nothing lost, nothing launched twice
     l840 = _simulate(1536, 6144, 24)
-    assert sum(l840) == 24 * 432 and all(D._fill(s, 256) > 0.98 for s in l840[:-1])
+    assert sum(l840) == 24 * 432 and all(s / (-(-s // 256) * 256) > 0.98 for s in l840[:-1])
     # 160M: no combination of eight products makes a whole round; what goes goes at 91 % and more, and the
     # leftovers of the pass in launches of at most half a round, which the grouped GEMM splits to fill the chip
     l160 = _simulate(768, 3072, 12)

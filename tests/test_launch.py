@@ -401,7 +401,7 @@ def test_pick_takes_what_the_exhaustive_search_takes():
         best, best_rank = None, None
         for s, sub in reach.items():
             if sub:
-                f = 0.9 * s * (cus // s) / cus if split and 2 * s <= cus else D._fill(s, cus)
+                f = 0.9 * s * (cus // s) / cus if split and 2 * s <= cus else s / (-(-s // cus) * cus)
                 rank = (min(f, D._FILL), 0 in sub, s)
                 if best_rank is None or rank > best_rank:
                     best, best_rank = sub, rank

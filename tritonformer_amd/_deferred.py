@@ -81,10 +81,6 @@ def _round(device):
     return n
 
 
-def _fill(tiles, cus):
-    return tiles / (-(-tiles // cus) * cus)
-
-
 def _pick(items, cus, split=False):
     """Indices of up to _MAX_GROUP products (of the first one's kind) whose tiles best fill whole rounds;
     among equals the oldest, then the most tiles.  Returns (indices, fill).  ``split``: as if the grouped GEMM may split
