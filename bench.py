@@ -664,7 +664,8 @@ def main():
             "gemm_ms_per_step": round(total_ms / reps, 3),
             "measured": f"HIP events on the launch stream around each tf_gemm / tf_gemm_scaled / tf_gemm_relu_bits / tf_gemm_group call, {reps} instrumented steps "
                         "run after the timed ones (queued behind three plain steps so that the GPU never waits for the host); the event time of a call covers its GEMM kernel(s) and, for a split contraction, "
-                        "the reduce kernel; launches = GEMM kernels counted by the library",
+                        "the reduce kernel; launches = GEMM kernels counted by the library; attention and MLP blocks, which the timed steps launch in one native call each, go "
+                        "launch by launch in the instrumented ones, with fp32 biases of an MLP converted ahead of its products",
         }
         out["roofline"]["other_kernels"] = family_rooflines(gt.by_family, reps)
         out["roofline"]["other_kernels_measured"] = (
