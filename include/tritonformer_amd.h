@@ -12,7 +12,9 @@
  *    never allocates, frees, retains or synchronises; it reads no environment
  *    variable.  What it keeps between calls: the device's CU / XCD counts (read
  *    from the runtime once per device), the address of the scratch array of
- *    tf_colsum_noalloc (taken once per device), and a counter of GEMM launches
+ *    tf_colsum_noalloc (taken once per device), the tile choice of the products
+ *    it was asked for last (per thread, 256 at most, by extents and kind of
+ *    call, a pure function of these), and a counter of GEMM launches
  *    (a relaxed atomic that only tf_diag_gemm_launch_count reads); no result
  *    depends on any of them beyond tile choice.  Work is enqueued on
  *    `stream` (a hipStream_t passed as void*, NULL = the null stream);

@@ -149,6 +149,8 @@ __global__ __launch_bounds__(kCeThreads, NCH == 8 ? 4 : 1) void ce_fwd_regs(int 
       // wave takes (the empty statement keeps the moves from being made for every chunk).  Eight tested element loads in
       // its place held up the loads in flight.  bf16 with gradient, us: 4095 x 50257 190 -> 173, 2047 x 33001 70.7 -> 58,
       // 8192 x 1001 24.0 -> 20.5; forward alone 8192 x 4097 19.1 -> 16.7, 8192 x 1001 13.3 -> 11.9, 4095 x 50257 82 as before.
+      // (Fewer rows than CUs and 33000 columns and more lose a little: with gradient 256 x 50257 fp16 18.4 -> 19.4, 100 x 50257
+      // 15.5 -> 16.3; 600 x 33001 27.8 -> 23.9.)
       if (ANY && (c + 1) * 8 > V) {
         asm volatile("");
         raw[u] = Row<T, ANY>::template settle<true>(raw[u], c, V, (T)-INFINITY);

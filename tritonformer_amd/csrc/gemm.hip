@@ -1169,6 +1169,12 @@ static GemmPlan plan_for(int64_t cus, int cfg, int64_t M, int64_t N, int64_t K, 
 // made for whole rounds -- is 1.3 to 2 times too high: a fixed part plus a time per 64-wide step that rises with the
 // workgroups per CU (`fill`), since operands come faster and the clock is higher while few CUs work.  Fits to 348 products
 // of 16 to 4096 rows, 128 to 6144 columns and contractions of 64 to 8192, operand B from HBM.
+// Checked over 1400 others that leave CUs idle with the large tile (16 to 6144 rows, 64 to 9000 columns, all layouts, slices
+// and sign bits as they are in use): 1.44 times the large tile's speed (geometric mean; the best of the three tiles each time
+// 1.45), seven of them slower than the large tile, by 4 to 9 per cent, all of 300 workgroups and more with long contractions
+// (629 x 5120 x 8128 90 -> 98 us), where two workgroups of a CU take longer than 1.3 to 1.8 of them would.  Counted as two they
+// would cost others more (2087 x 1552 x 1024 12.8 -> 17.3).  Sign bits, which 64-wide tiles store byte by byte, cost these 0.2 to
+// 1.1 us; an extra 0.5 us for them changes nothing for the better.
 static double part_round_us(int64_t cus, const GemmPlan& pl, int64_t M, int64_t N) {
   const double steps = (double)(pl.k_per_split / pl.bk);
   const double fill = (double)((int64_t)pl.tiles_m * pl.tiles_n * pl.splits) / (double)cus;

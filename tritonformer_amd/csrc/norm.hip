@@ -34,7 +34,8 @@ template <int WPR> __device__ __forceinline__ float row_sum(float v, float (*red
 // moved down (Row::settle), so that no wave stands waiting for eight element loads in the midst of its prefetch.  fp16, us:
 // backward 31713 x 1021 68.0 -> 46.0 (1024 columns: 42.2), 31713 x 777 60.7 -> 41.8, 20000 x 2051 121 -> 99, 8000 x 8191
 // 156 -> 140; forward 31713 x 1021 33.0 -> 30.0, 8000 x 8191 69.7 -> 62.6; softmax 31713 x 1021 forward 26.3 -> 23.7, backward
-// 36.5 -> 31.6, 16000 x 3001 41.2 -> 39.1 and 58.5 -> 53.0 (fp32 46.5 -> 44.9, 77 -> 74).
+// 36.5 -> 31.6, 16000 x 3001 41.2 -> 39.1 and 58.5 -> 53.0 (fp32 46.5 -> 44.9, 77 -> 74; forward rows of 257 to 259, where one lane has
+// an upper chunk and three elements at the most, lose: 63488 x 259 24.1 -> 25.4, 261 to 511 gain 1 to 6 per cent).
 template <typename T, int NV, bool ANY, int FROM = NV / 2> struct RowEnds {
   typedef Row<T, ANY> R;
   static __device__ __forceinline__ u32x4 fetch(const T* row, int c, int i, int n, T fill = (T)0.f) {
