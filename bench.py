@@ -132,7 +132,7 @@ def gemm_table(by_shape, reps, workload, dtype_name):
     rows.sort(key=lambda r: -r[0])
     head = [f"# GEMM calls of one step by shape ({workload}, {dtype_name})", "",
             "Command (on the MI355X box, from the repository root):", "",
-            f"    python3 bench.py --workload {workload} --dtype {dtype_name} --no-cpu-baseline --no-extras --gemm-table gpurun_out/gemm_table.md",
+            f"    python3 bench.py --workload {workload} --dtype {dtype_name} --no-cpu-baseline --no-extras --gemm-table gemm_table.md",
             "", "M x N x K of `C[M,N] = sum_k A(m,k) B(n,k)`; time = HIP events on the launch stream around the call "
             f"(its GEMM kernel or kernels and, for a split contraction, the reduce pass), mean over {reps} instrumented steps.", "",
             "| product (M x N x K) | operand layout | calls / step | us / call | TFLOP/s | ms / step |", "|---|---|---:|---:|---:|---:|"]
@@ -462,7 +462,7 @@ def vendor_compare(workload, dtype, device, path, iters=30):
     text = "\n".join([
         f"# Dense products of the step against the vendor BLAS library ({workload}, {str(dtype).replace('torch.', '')})", "",
         "Command (on the MI355X box, from the repository root):", "",
-        f"    python3 bench.py --workload {workload} --vendor-compare gpurun_out/vendor_compare.md", "",
+        f"    python3 bench.py --workload {workload} --vendor-compare vendor_compare.md", "",
         f"Each product alone, {iters} back-to-back calls on N(0,1) activations / gradients and N(0,0.02) weights, HIP events around the "
         "calls (a split contraction includes its reduce pass; 16-bit results on both sides).  `torch.matmul` runs the BLAS "
         "library torch is built with (hipBLASLt / rocBLAS).  Back-to-back repeats keep the operands in the caches: both "

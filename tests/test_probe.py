@@ -1,5 +1,5 @@
 """The MFMA-rate probe behind `bench.py --mfma-probe` runs and reports a rate per kind of operand data
-(a diagnostic: nothing is asserted about the rates themselves, which depend on the box)."""
+(a diagnostic: nothing is asserted about the rates themselves, which depend on the card)."""
 import pytest
 import torch
 
