@@ -687,3 +687,35 @@ def test_sign_bit_rows_on_every_tile(cfg, pitch, shift, dev):
                     bits.data_ptr(), pitch) == 0
         assert torch.equal(dh[:m], K_mod.mm(dy.view(1, m, d), w2.T, mask_act=want.view(1, m, f)).view(m, f))
         assert (dh[m] == 7).all()
+
+
+@pytest.mark.parametrize("pitch", [1 << 22, (1 << 22) + 8, (1 << 22) + 3])
+@pytest.mark.parametrize("layouts", ["fwd", "dx", "dw"])
+def test_rows_at_and_beyond_the_pitch_that_32_bit_offsets_reach(layouts, pitch, dev):
+    """The direct-to-LDS kernels and the register-staged 256x256 tiles address a lane's chunks by 32-bit offsets; wider rows
+    take the 128x128 register-staged tiles.  One operand a narrow strip of a very wide matrix, whose other columns are NaN
+    where they are next to the strip; the sums run over the same steps in the same order whatever the tile, so the bits are
+    those of the operand by itself."""
+    from tritonformer_amd import _lib
+
+    d = _lib.load_diag()
+    M, N, K = 264, 72, 128
+    la, lb = {"fwd": (0, 1), "dx": (0, 0), "dw": (1, 1)}[layouts]
+    g = torch.Generator().manual_seed(41)
+    a = torch.randn((M, K) if la == 0 else (K, M), generator=g).half().to(dev)
+    b = (torch.randn((N, K) if lb == 0 else (K, N), generator=g) / K ** 0.5).half().to(dev)
+    wide = torch.empty(a.shape[0] * pitch, dtype=torch.float16, device=dev).view(a.shape[0], pitch)
+    wide[:, :a.shape[1] + 64] = float("nan")
+    wide[:, :a.shape[1]] = a
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(x, cfg):
+        out = torch.empty((M, N), dtype=torch.float16, device=dev)
+        _lib.check(d.tf_diag_gemm(stream, cfg, 1, 0, 0, 0, la, lb, M, N, K, x.data_ptr(), x.stride(0), b.data_ptr(), b.stride(0),
+                                  out.data_ptr(), N, None, 0, None, 0))
+        return out
+
+    base = run(a, 2)
+    assert_close(base, (a.float() if la == 0 else a.float().T) @ (b.float().T if lb == 0 else b.float()), name=layouts)
+    for cfg in range(8):
+        assert torch.equal(run(wide, cfg), base), f"cfg {cfg}"

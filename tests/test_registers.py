@@ -50,3 +50,10 @@ def test_cross_entropy_forward_of_whole_rows_holds_a_row_and_little_else(tmp_pat
     kernels = {k: v for k, v in kernels_of("ce", tmp_path).items() if re.search(r"ce_fwd_regsIDF16b?_?Li\d+ELb0ELb0E", k)}
     assert len(kernels) == 6
     assert {k: v for k, v in kernels.items() if v[0] > 5 * int(re.search(r"Li(\d+)E", k)[1]) + 8 or v[1]} == {}
+
+
+def test_direct_to_lds_gemm_keeps_two_waves_per_simd_and_spills_nothing(tmp_path):
+    """Fragments are in flight in registers that the compiler takes as written: a spill or a copy of one would read it too early."""
+    kernels = {k: v for k, v in kernels_of("gemm", tmp_path).items() if "gemm_dma_" in k}
+    assert len(kernels) == 2 * (4 * 6 + 1)  # two types; four operand layouts of six tiles, the grouped launch
+    assert {k: v for k, v in kernels.items() if v[0] > 256 or v[1]} == {}

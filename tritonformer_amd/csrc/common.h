@@ -97,6 +97,16 @@ __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// ---- MFMA 16x16x32, D(16x16 fp32) += A(16x32) * B(32x16) ------------------
+// Lane l supplies A[l%16][(l/16)*8 .. +8] and B[(l/16)*8 .. +8][l%16];
+// result register r of lane l is D[(l/16)*4 + r][l%16].
+__device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
 // ---- LDS access ------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void;
 

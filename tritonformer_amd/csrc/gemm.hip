@@ -11,7 +11,12 @@
 //  * gemm_reg_kernel, for anything those cannot take (ragged extents, unaligned pointers,
 //    a contraction that is not a multiple of BK): the same loop and write-out with the
 //    operands staged through registers in 16-byte chunks at any element address.
-// Both use v_mfma_f32_32x32x16_{f16,bf16} with fp32 accumulators.
+// Both use v_mfma_f32_16x16x32_{f16,bf16} with fp32 accumulators.  Real data holds the clock of the matrix pipes down (power),
+// and the smaller instruction needs less of it: it moves a quarter of the accumulators per multiplication.  The MFMA stream
+// of a 256x256x64 step alone on normal fp16 data: 1.29 us with 32x32x16, 1.13 with 16x16x32 (bf16 1.20 and 1.06); equal on zeros.
+// The results are the same bits.  Products on operands from HBM, fp16, with 32x32x16 and now: 8192 x 1024 x 4096 71.2 -> 64.9 us,
+// 8192 x 4096 x 1024 73.5 -> 69.9, 4096 x 8192 x 2048 125.2 -> 115.9, 8192 x 50304 x 1024 819 -> 772; 4096 x 4096 x 8192 225 -> 204:
+// the clock rises from 1.50 to 1.71 GHz, the matrix pipes are busy for three quarters of the cycles either way.
 //
 // Either operand may be stored with the contraction dimension contiguous
 // ("K-major": read from LDS with ds_read_b128) or strided ("K-minor": read with
@@ -111,6 +116,15 @@ template <> struct FragRegs<false> {
 
 
 
+// A wave-uniform address plus a lane's 32-bit offset, as one instruction takes them.  The empty statement keeps the
+// extension of the offset to 64 bits next to its use: hoisted out of the loop it costs a second register per offset and a
+// 64-bit addition per access.
+__device__ __forceinline__ const char* at_offset(const char* origin, uint32_t off) {
+  asm volatile("" : "+v"(off));
+  return origin + off;
+}
+__device__ __forceinline__ const char* at_offset(const char* origin, uint64_t off) { return origin + off; }
+
 template <typename T, int R, int BK, bool KMAJOR, int NW>
 struct DmaPanel {
   static constexpr int CPR = KMAJOR ? BK / 8 : R / 8;
@@ -122,66 +136,89 @@ struct DmaPanel {
   static_assert(WLOADS % NW == 0 && PER_WAVE >= 1, "panel must divide evenly over the waves");
   static_assert(KMAJOR ? (CPR == 4 || CPR == 8) : (CPR >= 4), "unsupported panel shape");
 
-  // K-minor: a transposing read takes 32 bytes of each of four neighbouring rows per 16 lanes.  Rows of 256 bytes and
-  // more begin at the same bank, rows of 128 bytes at every other half of them; four rows of 64 bytes fill them.
+  // K-major: 16 rows of one chunk column fill the banks once.  K-minor: a transposing read takes 32 bytes of each of four
+  // neighbouring rows per 16 lanes, and of the four rows eight further on in the next 16.  Rows of 256 bytes and more begin
+  // at the same bank, rows of 128 bytes at every other half of them.
   static __device__ __forceinline__ int swz(int lrow, int c) {
     if constexpr (KMAJOR) return c ^ ((lrow / (16 / CPR)) % CPR);
-    else if constexpr (CPR >= 16) return c ^ ((lrow & 3) << 2);
-    else if constexpr (CPR == 8) return c ^ ((lrow & 3) << 1);
-    else return c;
+    else if constexpr (CPR >= 16) return c ^ ((lrow & 3) << 2) ^ ((lrow >> 2) & 2);
+    else return c ^ ((lrow & 3) << 1) ^ ((lrow >> 2) & 2);
   }
 
-  // Global address of each of this lane's chunks for the step starting at kbeg.
-  static __device__ __forceinline__ void init(const T* (&ptrs)[PER_WAVE], const T* base, int64_t ld, int row0,
-                                              int rmax, int kbeg, int wave, int lane) {
+  // Byte offset of each of this lane's chunks from the panel's first element of a step (row row0, contraction index kbeg):
+  // the address is wave-uniform but for these 32 bits, which no step changes.
+  static __device__ __forceinline__ const char* origin(const T* base, int64_t ld, int row0, int kbeg) {
+    return (const char*)(KMAJOR ? base + (int64_t)row0 * ld + kbeg : base + (int64_t)kbeg * ld + row0);
+  }
+  static __device__ __forceinline__ void init(uint32_t (&offs)[PER_WAVE], int64_t ld, int row0, int rmax, int wave, int lane) {
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) {
       const int slot = (wave * PER_WAVE + j) * 64 + lane;
       const int lrow = slot / CPR;
       const int c = swz(lrow, slot % CPR);
-      if (KMAJOR) {
-        const int gr = min(row0 + lrow, rmax - 1);
-        ptrs[j] = base + (int64_t)gr * ld + kbeg + c * 8;
-      } else {
-        int gr = row0 + c * 8;
-        if (gr >= rmax) gr = row0;
-        ptrs[j] = base + (int64_t)(kbeg + lrow) * ld + gr;
-      }
+      if (KMAJOR) offs[j] = ((uint32_t)(min(row0 + lrow, rmax - 1) - row0) * (uint32_t)ld + (uint32_t)c * 8u) * 2u;
+      else offs[j] = ((uint32_t)lrow * (uint32_t)ld + (row0 + c * 8 < rmax ? (uint32_t)c * 8u : 0u)) * 2u;
     }
   }
-  static __device__ __forceinline__ void issue(const T* (&ptrs)[PER_WAVE], char* lds, int wave) {
+  static __device__ __forceinline__ void issue_one(const char* org, const uint32_t (&offs)[PER_WAVE], char* lds, int wave, int j) {
+    __builtin_amdgcn_global_load_lds((gptr_void*)at_offset(org, offs[j]), (lds_void*)(lds + (wave * PER_WAVE + j) * 1024), 16, 0, 0);
+  }
+  static __device__ __forceinline__ void issue(const char* org, const uint32_t (&offs)[PER_WAVE], char* lds, int wave) {
 #pragma unroll
-    for (int j = 0; j < PER_WAVE; ++j)
-      __builtin_amdgcn_global_load_lds((gptr_void*)ptrs[j], (lds_void*)(lds + (wave * PER_WAVE + j) * 1024), 16, 0, 0);
+    for (int j = 0; j < PER_WAVE; ++j) issue_one(org, offs, lds, wave, j);
   }
-  static __device__ __forceinline__ void issue_one(const T* (&ptrs)[PER_WAVE], char* lds, int wave, int j) {
-    __builtin_amdgcn_global_load_lds((gptr_void*)ptrs[j], (lds_void*)(lds + (wave * PER_WAVE + j) * 1024), 16, 0, 0);
-  }
-  static __device__ __forceinline__ void advance(const T* (&ptrs)[PER_WAVE], int64_t ld) {
-#pragma unroll
-    for (int j = 0; j < PER_WAVE; ++j) ptrs[j] += KMAJOR ? (int64_t)BK : (int64_t)BK * ld;
-  }
+  // bytes from one step's panel to the next one's
+  static __device__ __forceinline__ int64_t stride(int64_t ld) { return (KMAJOR ? (int64_t)BK : (int64_t)BK * ld) * 2; }
+
   static constexpr int READS_PER_FRAG = KMAJOR ? 1 : 2;
-  // MFMA operand for the 32 rows starting at rb, contraction step ks (16 wide), read with volatile asm from the panel at
-  // LDS byte address `base`: lane l gets elements (row rb + l%32, k = ks*16 + (l/32)*8 + 0..7).
-  static __device__ __forceinline__ void frag_issue(FragRegs<KMAJOR>& f, uint32_t base, int rb, int ks, int lane) {
+  // MFMA operands: fragment F holds the 16 rows from rb0 + 16 F on (rb0: first row of the wave's tile) for the 32-wide
+  // contraction step KS, lane l elements (row l % 16, k = KS * 32 + (l / 16) * 8 + 0..7), read with volatile asm.
+  // frag_lane: the lane's part of the address; the swizzle and F share bits of it, the rest is the instruction's offset.
+  static __device__ __forceinline__ uint32_t frag_lane(int rb0, int lane) {
     if constexpr (KMAJOR) {
-      const int row = rb + (lane & 31);
-      const int c = ks * 2 + (lane >> 5);
-      const uint32_t a = base + (row * CPR + swz(row, c)) * 16;
-      asm volatile("ds_read_b128 %0, %1" : "=v"(f.q) : "v"(a));
+      const int row = rb0 + (lane & 15);
+      return (uint32_t)(row * CPR + swz(row, lane >> 4)) * 16u;
     } else {
-      const int i = lane & 15;
-      const int col = rb + 16 * ((lane >> 4) & 1) + (i & 3) * 4;
-      const int kk0 = ks * 16 + 8 * (lane >> 5) + (i >> 2);
-      const int kk1 = kk0 + 4;
-      const uint32_t a0 = base + (kk0 * CPR + swz(kk0, col >> 3)) * 16 + (col & 7) * 2;
-      const uint32_t a1 = base + (kk1 * CPR + swz(kk1, col >> 3)) * 16 + (col & 7) * 2;
-      asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(f.lo) : "v"(a0));
-      asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(f.hi) : "v"(a1));
+      const int i = lane & 15, lrow = 8 * (lane >> 4) + (i >> 2);
+      return (uint32_t)(lrow * CPR + swz(lrow, rb0 / 8 + ((i >> 1) & 1))) * 16u + (uint32_t)(i & 1) * 8u;
+    }
+  }
+  template <int F, int KS> static __device__ __forceinline__ void frag_issue(FragRegs<KMAJOR>& f, uint32_t base, uint32_t lane_part) {
+    static_assert(BK == 64, "offsets of a 64-wide step");
+    if constexpr (KMAJOR) {
+      lds_read128_at<F * 16 * CPR * 16>(f.q, base + (lane_part ^ (uint32_t)(KS * 64)));
+    } else {
+      const uint32_t a = base + (lane_part ^ (uint32_t)(F % 8 * 32));
+      lds_read64_tr_at<F / 8 * 256 + KS * 32 * CPR * 16>(f.lo, a);
+      lds_read64_tr_at<F / 8 * 256 + (KS * 32 + 4) * CPR * 16>(f.hi, a);
     }
   }
 };
+
+// Where the LDS reads of the next 32-wide step go among the TM x TN MFMAs of a step (row by row): B's fragments (items 0 to
+// TN - 1), which every row needs, into a second set of registers behind the first MFMAs; A's (the items after them) into the
+// registers that the row just multiplied has left.  `from`: first MFMA that may carry reads (behind a hand-over to the next
+// stage: then two at a time).
+template <int TM, int TN> struct ReadSlots {
+  int slot[TN + TM];  // ascending
+  constexpr ReadSlots(int from) : slot() {
+    int at = from, n = 0;
+    for (int q = 0; q < TN + TM; ++q) {
+      const int earliest = q < TN ? 0 : TN * (q - TN) + TN - 1, most = q < TN && from == 0 ? 1 : 2;
+      if (at < earliest) { at = earliest; n = 0; }
+      if (n == most && at < TM * TN - 1) { ++at; n = 0; }
+      ++n;
+      slot[q] = at;
+    }
+  }
+  constexpr int before(int m) const {  // items that go behind MFMAs ahead of m
+    int q = 0;
+    while (q < TN + TM && slot[q] < m) ++q;
+    return q;
+  }
+};
+// MFMA rows of a stage's last step that come ahead of the hand-over to the next stage
+constexpr int hand_rows(int tm) { return tm >= 8 ? 5 : tm >= 4 ? 2 : 1; }
 
 // bias[n .. n + 3] in T
 template <typename T> __device__ __forceinline__ typename Vec<T>::v4 bias4(const GemmParams& p, int n) {
@@ -206,7 +243,7 @@ template <typename T> __device__ __forceinline__ T bias1(const void* bias, int f
 // ANY: rows of C, the bias and the mask start at any element and N is any number (register-staged kernel):
 // the same 16-byte accesses at element alignment, the chunk that crosses the end of a row by elements.
 template <typename T, typename TO, int TM, int TN, int WTM, int WTN, bool PLAIN = false, bool FULL = false, bool ANY = false>
-__device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&acc)[TM][TN], char* smem, int m0,
+__device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x4 (&acc)[TM][TN], char* smem, int m0,
                                                   int n0, int wm, int wn, int wave, int lane,
                                                   const uint8_t (*sign_bytes)[4] = nullptr) {
   constexpr int ES = (int)sizeof(TO);
@@ -231,39 +268,37 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
   // ... and so is the row part of its first store; the others lie whole multiples of ldc further on
   TO* const row0 = C + (int64_t)(m0 + wm * WTM + lane / CH) * p.ldc + col_off;
   // this lane's bias values: the same for every 32-row block, requested once ahead of the loop
-  typename Vec<T>::v4 bvals[TN][4] = {};
+  typename Vec<T>::v4 bvals[TN] = {};
   if (bias) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int j = 0; j < TN; ++j) {
+      const int nl = j * 16 + (lane >> 4) * 4;
+      if constexpr (ANY) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int nl = j * 32 + g * 8 + (lane >> 5) * 4;
-        if constexpr (ANY) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (nbase + nl + e < p.N) bvals[j][g][e] = bias1<T>(bias, p.bias_f32, nbase + nl + e);
-        } else {
-          if (nbase + nl < p.N) bvals[j][g] = bias4<T>(p, nbase + nl);
-        }
+        for (int e = 0; e < 4; ++e)
+          if (nbase + nl + e < p.N) bvals[j][e] = bias1<T>(bias, p.bias_f32, nbase + nl + e);
+      } else {
+        if (nbase + nl < p.N) bvals[j] = bias4<T>(p, nbase + nl);
       }
+    }
   }
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
+  for (int i = 0; i < TM / 2; ++i) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int nl = j * 32 + g * 8 + (lane >> 5) * 4;
+      for (int j = 0; j < TN; ++j) {
+        const int r = h * 16 + (lane & 15), nl = j * 16 + (lane >> 4) * 4;
         float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][g * 4 + e];
+        for (int e = 0; e < 4; ++e) v[e] = acc[i * 2 + h][j][e];
         if (!PLAIN) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] *= alpha;
         }
         if (bias) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += (float)bvals[j][g][e];
+          for (int e = 0; e < 4; ++e) v[e] += (float)bvals[j][e];
         }
         if (relu) {
 #pragma unroll
@@ -271,12 +306,12 @@ __device__ __forceinline__ void gemm_epilogue_lds(const GemmParams& p, f32x16 (&
         }
         if (ES == 4) {
           f32x4 o = {v[0], v[1], v[2], v[3]};
-          *reinterpret_cast<f32x4*>(mine + (lane & 31) * ROWB + nl * 4) = o;
+          *reinterpret_cast<f32x4*>(mine + r * ROWB + nl * 4) = o;
         } else {
           typename Vec<T>::v4 o;
 #pragma unroll
           for (int e = 0; e < 4; ++e) o[e] = (T)v[e];
-          *reinterpret_cast<typename Vec<T>::v4*>(mine + (lane & 31) * ROWB + nl * 2) = o;
+          *reinterpret_cast<typename Vec<T>::v4*>(mine + r * ROWB + nl * 2) = o;
         }
       }
     }
@@ -390,7 +425,7 @@ __device__ __forceinline__ u32x4 keep_by_bits8(u32x4 v, unsigned bits) {
 //            eight to a row, a partial write of eight lines each.
 //  !BITS_OUT: C = bit ? acc : 0, the bytes requested before the main loop (sign_bytes).
 template <typename T, int BM, int BN, int TM, int TN, int WTM, int WTN, bool BITS_OUT>
-__device__ __forceinline__ void gemm_epilogue_bits(const GemmParams& p, f32x16 (&acc)[TM][TN], char* smem, int m0, int n0,
+__device__ __forceinline__ void gemm_epilogue_bits(const GemmParams& p, f32x4 (&acc)[TM][TN], char* smem, int m0, int n0,
                                                    int wm, int wn, int wave, int lane, const uint8_t (*sign_bytes)[4]) {
   constexpr int ROWB = WTN * 2 + 16, CH = WTN * 2 / 16, RPI = 64 / CH;
   constexpr int NW = (BM / WTM) * (BN / WTN);
@@ -401,27 +436,25 @@ __device__ __forceinline__ void gemm_epilogue_bits(const GemmParams& p, f32x16 (
   const int nbase = n0 + wn * WTN;
   const int n_lane = nbase + (lane % CH) * 8;
   T* const row0 = C + (int64_t)(m0 + wm * WTM + lane / CH) * p.ldc + n_lane + (int64_t)(n_lane / p.chunk_n) * p.chunk_skip;
-  typename Vec<T>::v4 bvals[TN][4] = {};
+  typename Vec<T>::v4 bvals[TN] = {};
   if (BITS_OUT && p.bias) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) bvals[j][g] = bias4<T>(p, nbase + j * 32 + g * 8 + (lane >> 5) * 4);
+    for (int j = 0; j < TN; ++j) bvals[j] = bias4<T>(p, nbase + j * 16 + (lane >> 4) * 4);
   }
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
+  for (int i = 0; i < TM / 2; ++i) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+      for (int j = 0; j < TN; ++j) {
         typename Vec<T>::v4 o;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          float v = acc[i][j][g * 4 + e];
-          if (BITS_OUT) v = fmaxf(v + (float)bvals[j][g][e], 0.f);
+          float v = acc[i * 2 + h][j][e];
+          if (BITS_OUT) v = fmaxf(v + (float)bvals[j][e], 0.f);
           o[e] = (T)v;
         }
-        *reinterpret_cast<typename Vec<T>::v4*>(mine + (lane & 31) * ROWB + (j * 32 + g * 8 + (lane >> 5) * 4) * 2) = o;
+        *reinterpret_cast<typename Vec<T>::v4*>(mine + (h * 16 + (lane & 15)) * ROWB + (j * 16 + (lane >> 4) * 4) * 2) = o;
       }
     u32x4 vals[32 / RPI];
 #pragma unroll
@@ -456,17 +489,16 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
   static_assert(NS == 2 || NS == 3, "two or three pipeline stages");
   constexpr int NW = WM * WN;
   constexpr int WTM = BM / WM, WTN = BN / WN;
-  constexpr int TM = WTM / 32, TN = WTN / 32;
+  constexpr int TM = WTM / 16, TN = WTN / 16;
   constexpr int GROUP_M = 8;
-  constexpr int KSTEPS = BK / 16;
+  constexpr int KSTEPS = BK / 32;
   typedef DmaPanel<T, BM, BK, A_KMAJOR, NW> PA;
   typedef DmaPanel<T, BN, BK, B_KMAJOR, NW> PB;
   typedef typename Vec<T>::v8 v8;
   constexpr int STAGE = PA::BYTES + PB::BYTES;      // two stages, ping-pong
   constexpr int LPS = PA::PER_WAVE + PB::PER_WAVE;  // loads per wave per stage
   constexpr int NEARLY = LPS / 2;  // loads of a stage issued right after the hand-over to the stage before it
-  static_assert(KSTEPS >= 3, "the loop deals its loads and pointer updates over the first two steps and the last one");
-  static_assert(KSTEPS % 2 == 0, "operand register ping-pong needs an even number of contraction steps");
+  static_assert(KSTEPS == 2, "B's fragments alternate between two sets of registers");
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   const int lane = threadIdx.x & 63;
@@ -487,28 +519,31 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
   const int kend = min(p.K, kbeg + p.k_per_split);
   const int nk = (kend - kbeg) / BK;
 
-  const T* pa[PA::PER_WAVE];
-  const T* pb[PB::PER_WAVE];
-  PA::init(pa, (const T*)p.A, p.lda, m0, p.M, kbeg, wave, lane);
-  PB::init(pb, (const T*)p.B, p.ldb, n0, p.N, kbeg, wave, lane);
+  uint32_t oa[PA::PER_WAVE], ob[PB::PER_WAVE];
+  PA::init(oa, p.lda, m0, p.M, wave, lane);
+  PB::init(ob, p.ldb, n0, p.N, wave, lane);
+  const char* pa = PA::origin((const T*)p.A, p.lda, m0, kbeg);
+  const char* pb = PB::origin((const T*)p.B, p.ldb, n0, kbeg);
+  const int64_t sa = PA::stride(p.lda), sb = PB::stride(p.ldb);
+  const uint32_t la = PA::frag_lane(wm * WTM, lane), lb = PA::BYTES + PB::frag_lane(wn * WTN, lane);
 
-  f32x16 acc[TM][TN];
+  f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
   // Mask bits of a 16-bit result: this lane's bytes (one per 8-element chunk it will store, in the
   // order of the write-out) are requested here, a whole main loop ahead of their use -- loaded in
   // the write-out they would sit between every LDS read and the store that needs both.
   static_assert(WTN == 64 || WTN == 32, "four or two wave-wide stores per 32-row block of a 16-bit result");
-  uint8_t sign_bytes[TM][4] = {};
+  uint8_t sign_bytes[TM / 2][4] = {};
   if (p.sign_in && !p.out_f32) {
     constexpr int CH16 = WTN * 2 / 16, RPI16 = 64 / CH16;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM / 2; ++i)
 #pragma unroll
       for (int rr = 0; rr < 32 / RPI16; ++rr) {
         const int m = m0 + wm * WTM + i * 32 + rr * RPI16 + lane / CH16, n = n0 + wn * WTN + (lane % CH16) * 8;
@@ -523,37 +558,38 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  FragRegs<A_KMAJOR> fa[2][TM];
+  FragRegs<A_KMAJOR> fa[TM];
   FragRegs<B_KMAJOR> fb[2][TN];
-  auto read_operands = [&](const char* stage, int ks, int buf) {
-    const uint32_t sa_addr = lds_address(stage), sb_addr = sa_addr + PA::BYTES;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) PA::frag_issue(fa[buf][i], sa_addr, wm * WTM + i * 32, ks, lane);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) PB::frag_issue(fb[buf][j], sb_addr, wn * WTN + j * 32, ks, lane);
+  const uint32_t lds0 = lds_address(smem);
+  // operand fragment for 32-wide step KS of the stage at LDS offset `at`: item q < TN is B's (into set KS), the others A's
+  auto read_item = [&](uint32_t at, auto ks_c, auto q_c) {
+    constexpr int ks = decltype(ks_c)::value, q = decltype(q_c)::value;
+    if constexpr (q < TN) PB::template frag_issue<q, ks>(fb[ks][q], lds0 + at, lb);
+    else PA::template frag_issue<q - TN, ks>(fa[q - TN], lds0 + at, la);
+  };
+  auto load_item = [&](uint32_t at, int q) {
+    if (q < PA::PER_WAVE) PA::issue_one(pa, oa, smem + at, wave, q);
+    else PB::issue_one(pb, ob, smem + at + PA::BYTES, wave, q - PA::PER_WAVE);
+  };
+  auto load_all = [&](uint32_t at) {
+    PA::issue(pa, oa, smem + at, wave);
+    PB::issue(pb, ob, smem + at + PA::BYTES, wave);
+    pa += sa;
+    pb += sb;
   };
 
   // ---- prologue: step 0 into stage 0, then its first operands and the head of step 1
   if (nk > 0) {
-    PA::issue(pa, smem, wave);
-    PB::issue(pb, smem + PA::BYTES, wave);
-    PA::advance(pa, p.lda);
-    PB::advance(pb, p.ldb);
+    load_all(0);
     // the head of step 1 goes out before step 0 is waited for: the two travel together through
     // the cold start instead of one after the other
     if constexpr (NS == 3) {
       // three buffers: all of step 1 and the head of step 2
       if (nk > 1) {
-        PA::issue(pa, smem + STAGE, wave);
-        PB::issue(pb, smem + STAGE + PA::BYTES, wave);
-        PA::advance(pa, p.lda);
-        PB::advance(pb, p.ldb);
+        load_all(STAGE);
         if (nk > 2) {
 #pragma unroll
-          for (int q = 0; q < NEARLY; ++q) {
-            if (q < PA::PER_WAVE) PA::issue_one(pa, smem + 2 * STAGE, wave, q);
-            else PB::issue_one(pb, smem + 2 * STAGE + PA::BYTES, wave, q - PA::PER_WAVE);
-          }
+          for (int q = 0; q < NEARLY; ++q) load_item(2 * STAGE, q);
           wait_vmcnt<LPS + NEARLY>();  // loads complete in order: all but the youngest LPS + NEARLY = step 0
         } else {
           wait_vmcnt<LPS>();
@@ -563,113 +599,94 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
       }
     } else if (nk > 1) {
 #pragma unroll
-      for (int q = 0; q < NEARLY; ++q) {
-        if (q < PA::PER_WAVE) PA::issue_one(pa, smem + STAGE, wave, q);
-        else PB::issue_one(pb, smem + STAGE + PA::BYTES, wave, q - PA::PER_WAVE);
-      }
+      for (int q = 0; q < NEARLY; ++q) load_item(STAGE, q);
       wait_vmcnt<NEARLY>();  // loads complete in order: all but the NEARLY youngest = step 0
     } else {
       wait_vmcnt<0>();
     }
     barrier();
-    read_operands(smem, 0, 0);
+    static_for<TN + TM>([&](auto q_c) { read_item(0, std::integral_constant<int, 0>(), q_c); });
   }
 
-  // ---- main loop.  Every LDS read, load and pointer update sits behind an MFMA, pinned there by
-  // scheduling barriers: the matrix pipe is busy for 32 cycles per MFMA and the wave is free to
-  // issue meanwhile.  Per 16-wide step there are NMFMA slots; the operand reads of the next step
-  // go behind the first ones (register ping-pong: the MFMAs of step ks read set ks % 2), the extras
-  // of the step behind the rest -- half of the next stage's loads at step 0, the pointer updates
-  // at step 1, and in the last step the hand-over (wait for this wave's loads, barrier) followed
-  // by the first operand reads of the next stage and the other half of the loads, which go into
-  // the buffer everyone has just left.
+  // ---- main loop.  Every LDS read and load sits behind an MFMA, pinned there by scheduling barriers: the matrix pipe is
+  // busy for 16 cycles per MFMA and the wave is free to issue meanwhile.  A stage is two steps of 32, a step TM x TN MFMAs,
+  // row by row and back and forth along the rows, so that every MFMA has one operand in common with the one before it (the
+  // MFMA stream alone draws less power that way: 1.13 -> 1.10 us per 256x256x64); ReadSlots says where the reads of the next step go.  An LDS read has most of a step to land: ahead of row i
+  // the wait leaves in flight what was requested after A's fragment i (B's are older).  Of the next stage's loads the first
+  // half goes out behind the hand-over (wait for this wave's loads and reads, barrier), into the buffer everyone has just
+  // left, the rest at the head of step 0.
   constexpr int NMFMA = TM * TN;
-  constexpr int NR = TM + TN;                                       // read items (one fragment each)
-  constexpr int RPS = (NR + NMFMA - 1) / NMFMA;                     // read items per slot
-  constexpr int RSLOTS = (NR + RPS - 1) / RPS;                      // slots that carry reads
-  constexpr int HAND = NMFMA - RSLOTS >= 4 ? 2 : 0;                 // MFMAs of the last step ahead of the barrier
-  static_assert(HAND + RSLOTS <= NMFMA, "the reads of a step must fit behind its MFMAs");
+  constexpr int HAND = hand_rows(TM) * TN;  // MFMAs of the last step ahead of the hand-over
+  constexpr int RA = PA::READS_PER_FRAG, RB = PB::READS_PER_FRAG;
   static_assert(LPS % 2 == 0, "loads go out in two halves");
-  auto read_item = [&](const char* stage, int ks, int buf, int item) {
-    const uint32_t sa_addr = lds_address(stage), sb_addr = sa_addr + PA::BYTES;
-    if (item < TM) PA::frag_issue(fa[buf][item], sa_addr, wm * WTM + item * 32, ks, lane);
-    else PB::frag_issue(fb[buf][item - TM], sb_addr, wn * WTN + (item - TM) * 32, ks, lane);
-  };
-  auto load_item = [&](char* dst, int q) {
-    if (q < PA::PER_WAVE) PA::issue_one(pa, dst, wave, q);
-    else PB::issue_one(pb, dst + PA::BYTES, wave, q - PA::PER_WAVE);
-  };
-  auto advance_item = [&](int q) {
-    if (q < PA::PER_WAVE) pa[q] += A_KMAJOR ? (int64_t)BK : (int64_t)BK * p.lda;
-    else pb[q - PA::PER_WAVE] += B_KMAJOR ? (int64_t)BK : (int64_t)BK * p.ldb;
-  };
   // One 64-wide stage.  MORE: another stage follows (hand over to it); MORE2: and one after that
   // (its first loads go out).  Compile-time, so the steady state of the loop has no branch.
   // With three buffers (NS == 3) everything that is loaded lies one stage further ahead: step 0 sends the
   // rest of the stage after the next one into the third buffer `far`, the last step the head of the stage
   // after that into `cur`; MORE3: that stage exists.  The hand-over then waits for all but the youngest
   // stage's loads.
-  auto stage = [&](char* cur, char* nxt, char* far, auto more_c, auto more2_c, auto more3_c) {
+  auto stage = [&](uint32_t cur, uint32_t nxt, uint32_t far, auto more_c, auto more2_c, auto more3_c) {
     constexpr bool MORE = decltype(more_c)::value, MORE2 = decltype(more2_c)::value, MORE3 = decltype(more3_c)::value;
-    constexpr bool LOAD0 = NS == 3 ? MORE2 : MORE;    // step 0 has loads to send (and step 1 pointers to move)
+    constexpr bool LOAD0 = NS == 3 ? MORE2 : MORE;    // step 0 has loads to send
     constexpr bool LOADL = NS == 3 ? MORE3 : MORE2;   // the last step has
-    char* const dst0 = NS == 3 ? far : nxt;
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      const bool last = ks + 1 == KSTEPS;
-      const int first = last ? HAND : 0;                 // first slot that carries work of this step
-      const int xfirst = first + RSLOTS < NMFMA ? first + RSLOTS : NMFMA - 1;  // extras: behind the reads
-      const int xslots = NMFMA - xfirst;
-      const int nx = last ? (LOADL ? NEARLY : 0) : !LOAD0 ? 0 : ks == 0 ? LPS - NEARLY : ks == 1 ? LPS : 0;
-      wait_lgkmcnt<0>();  // the operands of this step were requested a whole step ago
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int m = 0; m < NMFMA; ++m) {
-        const int i = m / TN, j = m % TN;
-        if (last && m == HAND && MORE) {
-          wait_vmcnt<(NS == 3 && MORE2) ? LPS : 0>();  // this wave's loads of the next stage have landed
-          barrier();        // ... and everyone's; everyone has read the last operands of `cur`
+    const uint32_t dst0 = NS == 3 ? far : nxt;
+    static_for<KSTEPS>([&](auto ks_c) {
+      constexpr int ks = decltype(ks_c)::value;
+      constexpr bool last = ks + 1 == KSTEPS, hands = last && MORE;
+      typedef std::integral_constant<int, last ? 0 : ks + 1> next_ks;
+      constexpr ReadSlots<TM, TN> slots(hands ? HAND : 0);
+      static_for<NMFMA>([&](auto m_c) {
+        constexpr int m = decltype(m_c)::value, i = m / TN, j = i % 2 ? TN - 1 - m % TN : m % TN;
+        if constexpr (hands && m == HAND) {
+          wait_lgkmcnt<0>();  // this wave has read the last operands of `cur`
+          wait_vmcnt<(NS == 3 && MORE2) ? LPS : 0>();  // its loads of the next stage have landed
+          barrier();                                   // ... and everyone's
+          __builtin_amdgcn_sched_barrier(0);
+        } else if constexpr (m % TN == 0 && (!hands || m < HAND)) {
+          constexpr int flying = (TM - 1 - i) * RA + (last || i == 0 ? 0 : TN * RB + i * RA);
+          wait_lgkmcnt<(flying < 15 ? flying : 15)>();
           __builtin_amdgcn_sched_barrier(0);
         }
-        acc[i][j] = mfma32(fb[ks & 1][j].template get<v8>(), fa[ks & 1][i].template get<v8>(), acc[i][j]);
+        acc[i][j] = mfma16(fb[ks][j].template get<v8>(), fa[i].template get<v8>(), acc[i][j]);
         __builtin_amdgcn_sched_barrier(0);
-        if (m >= first && (!last || MORE)) {
-#pragma unroll
-          for (int r = (m - first) * RPS; r < (m - first + 1) * RPS && r < NR; ++r) {
-            if (last) read_item(nxt, 0, 0, r);
-            else read_item(cur, ks + 1, (ks + 1) & 1, r);
-          }
+        if constexpr (!last || MORE) {
+          constexpr int q0 = slots.before(m), q1 = slots.before(m + 1);
+          static_for<q1 - q0>([&](auto q) {
+            read_item(last ? nxt : cur, next_ks(), std::integral_constant<int, q0 + decltype(q)::value>());
+          });
         }
-        if (m >= xfirst) {
+        if constexpr (ks == 0 && LOAD0) {  // the rest of the next stage (NS == 3: of the one after it)
 #pragma unroll
-          for (int q = (m - xfirst) * nx / xslots; q < (m - xfirst + 1) * nx / xslots; ++q) {
-            if (last) load_item(cur, q);                 // first half of the stage after the next one (NS == 3: one further)
-            else if (ks == 0) load_item(dst0, NEARLY + q);  // the rest of the next stage (NS == 3: of the one after it)
-            else advance_item(q);
-          }
+          for (int q = 0; q < LPS - NEARLY; ++q)
+            if (TN + 2 * q == m || (TN + 2 * q > m && m == NMFMA - 1)) load_item(dst0, NEARLY + q);
+        }
+        if constexpr (last && LOADL) {     // first half of the stage after the next one (NS == 3: one further)
+          if constexpr (m == HAND) { pa += sa; pb += sb; }
+#pragma unroll
+          for (int q = 0; q < NEARLY; ++q)
+            if (HAND + 4 + 2 * q == m || (HAND + 4 + 2 * q > m && m == NMFMA - 1)) load_item(cur, q);
         }
         __builtin_amdgcn_sched_barrier(0);
-      }
-    }
+      });
+    });
   };
   typedef std::integral_constant<bool, true> yes_t;
   typedef std::integral_constant<bool, false> no_t;
   int kt = 0;
   if constexpr (NS == 3) {
-    int o0 = 0, o1 = STAGE, o2 = 2 * STAGE;   // buffers of this stage, the next one and the one after it
-    auto rotate = [&]() { const int t = o0; o0 = o1; o1 = o2; o2 = t; ++kt; };
-    for (; kt + 3 < nk; rotate()) stage(smem + o0, smem + o1, smem + o2, yes_t(), yes_t(), yes_t());
-    if (kt + 2 < nk) { stage(smem + o0, smem + o1, smem + o2, yes_t(), yes_t(), no_t()); rotate(); }
-    if (kt + 1 < nk) { stage(smem + o0, smem + o1, smem + o2, yes_t(), no_t(), no_t()); rotate(); }
-    if (kt < nk) stage(smem + o0, smem + o1, smem + o2, no_t(), no_t(), no_t());
+    uint32_t o0 = 0, o1 = STAGE, o2 = 2 * STAGE;   // buffers of this stage, the next one and the one after it
+    auto rotate = [&]() { const uint32_t t = o0; o0 = o1; o1 = o2; o2 = t; ++kt; };
+    for (; kt + 3 < nk; rotate()) stage(o0, o1, o2, yes_t(), yes_t(), yes_t());
+    if (kt + 2 < nk) { stage(o0, o1, o2, yes_t(), yes_t(), no_t()); rotate(); }
+    if (kt + 1 < nk) { stage(o0, o1, o2, yes_t(), no_t(), no_t()); rotate(); }
+    if (kt < nk) stage(o0, o1, o2, no_t(), no_t(), no_t());
   } else {
-    for (; kt + 2 < nk; ++kt)
-      stage(smem + (kt & 1) * STAGE, smem + ((kt + 1) & 1) * STAGE, nullptr, yes_t(), yes_t(), no_t());
+    for (; kt + 2 < nk; ++kt) stage((kt & 1) * STAGE, (~kt & 1) * STAGE, 0, yes_t(), yes_t(), no_t());
     if (kt + 1 < nk) {
-      stage(smem + (kt & 1) * STAGE, smem + ((kt + 1) & 1) * STAGE, nullptr, yes_t(), no_t(), no_t());
+      stage((kt & 1) * STAGE, (~kt & 1) * STAGE, 0, yes_t(), no_t(), no_t());
       ++kt;
     }
-    if (kt < nk) stage(smem + (kt & 1) * STAGE, smem + ((kt + 1) & 1) * STAGE, nullptr, no_t(), no_t(), no_t());
+    if (kt < nk) stage((kt & 1) * STAGE, (~kt & 1) * STAGE, 0, no_t(), no_t(), no_t());
   }
 
   static_assert(NW * 32 * (WTN * 4 + 16) <= NS * STAGE, "epilogue staging must fit in the pipeline LDS");
@@ -737,26 +754,23 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_dma_kernel(GemmParams p
 // gradient 103 -> 56, weight gradient 121 -> 59; 8192 x 50257 x 1024 forward 4232 -> 1057 (of the element-wise one),
 // 798 TFLOP/s; 8192 x 1024 x 2056 (all aligned, K % 64 != 0) 58 -> 46.
 // ---------------------------------------------------------------------------
-template <typename T, int R, int BK, bool KMAJOR, int NW>
+template <typename T, int R, int BK, bool KMAJOR, int NW, typename Off>
 struct RegPanel {
   typedef DmaPanel<T, R, BK, KMAJOR, NW> D;
   static constexpr int PER = D::PER_WAVE;  // chunks per thread
   static constexpr int NT = NW * 64;
   static constexpr int ROWS = NT / D::CPR;  // LDS rows between a thread's chunks
   static_assert(NT % D::CPR == 0 && D::NCHUNK == PER * NT, "panel must divide evenly over the threads");
-  static_assert(KMAJOR ? (ROWS / (16 / D::CPR)) % D::CPR == 0 : ROWS % 4 == 0, "a thread's chunks share one swizzle");
+  static_assert(KMAJOR ? (ROWS / (16 / D::CPR)) % D::CPR == 0 : ROWS % 16 == 0, "a thread's chunks share one swizzle");
 
   // Thread t owns the LDS slots t, t + NT, ... and fetches the chunk that the swizzle puts there.
-  static __device__ __forceinline__ void init(const T* (&ptrs)[PER], const T* base, int64_t ld, int row0, int rmax, int kbeg) {
+  // Offsets in bytes from D::origin.
+  static __device__ __forceinline__ void init(Off (&offs)[PER], int64_t ld, int row0, int rmax) {
     const int t = threadIdx.x, lrow = t / D::CPR, c = D::swz(lrow, t % D::CPR);
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      if (KMAJOR) {
-        ptrs[j] = base + (int64_t)min(row0 + lrow + j * ROWS, rmax - 1) * ld + kbeg + c * 8;
-      } else {
-        const int gr = row0 + c * 8 < rmax ? row0 + c * 8 : row0;
-        ptrs[j] = base + (int64_t)(kbeg + lrow + j * ROWS) * ld + gr;
-      }
+      if (KMAJOR) offs[j] = ((Off)(min(row0 + lrow + j * ROWS, rmax - 1) - row0) * (Off)ld + (Off)(c * 8)) * 2;
+      else offs[j] = ((Off)(lrow + j * ROWS) * (Off)ld + (Off)(row0 + c * 8 < rmax ? c * 8 : 0)) * 2;
     }
   }
   static __device__ __forceinline__ u32x4 fetch(const T* ptr) {
@@ -781,15 +795,17 @@ template <typename T, int BM, int BN, int BK, int WM, int WN, int WPE, bool A_KM
 __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_reg_kernel(GemmParams p) {
   constexpr int NW = WM * WN, NT = NW * 64;
   constexpr int WTM = BM / WM, WTN = BN / WN;
-  constexpr int TM = WTM / 32, TN = WTN / 32;
+  constexpr int TM = WTM / 16, TN = WTN / 16;
   constexpr int GROUP_M = 8;
-  constexpr int KSTEPS = BK / 16;
-  typedef RegPanel<T, BM, BK, A_KMAJOR, NW> PA;
-  typedef RegPanel<T, BN, BK, B_KMAJOR, NW> PB;
+  constexpr int KSTEPS = BK / 32;
+  // the 256-row panels keep 32-bit offsets (kMaxPitch): with 64 bits the kernel spills
+  typedef std::conditional_t<(BM > 128), uint32_t, uint64_t> Off;
+  typedef RegPanel<T, BM, BK, A_KMAJOR, NW, Off> PA;
+  typedef RegPanel<T, BN, BK, B_KMAJOR, NW, Off> PB;
   typedef typename Vec<T>::v8 v8;
   constexpr int STAGE = PA::D::BYTES + PB::D::BYTES;
   constexpr int LPS = PA::PER + PB::PER;  // chunks per thread per stage
-  static_assert(KSTEPS == 4, "stores, loads and hand-over are dealt over four contraction steps");
+  static_assert(KSTEPS == 2, "stores, loads and hand-over are dealt over two contraction steps");
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   const int lane = threadIdx.x & 63;
@@ -813,29 +829,35 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_reg_kernel(GemmParams p
   // stages that need no test: all but the last one, none where a row may be shorter than a chunk
   const int nfree = (A_KMAJOR || p.lda >= 8) && (B_KMAJOR || p.ldb >= 8) ? nk - 1 : 0;
 
-  const T* pa[PA::PER];
-  const T* pb[PB::PER];
-  PA::init(pa, (const T*)p.A, p.lda, m0, p.M, kbeg);
-  PB::init(pb, (const T*)p.B, p.ldb, n0, p.N, kbeg);
+  Off oa[PA::PER], ob[PB::PER];
+  PA::init(oa, p.lda, m0, p.M);
+  PB::init(ob, p.ldb, n0, p.N);
+  const char* pa = PA::D::origin((const T*)p.A, p.lda, m0, kbeg);
+  const char* pb = PB::D::origin((const T*)p.B, p.ldb, n0, kbeg);
+  const int64_t sa = PA::D::stride(p.lda), sb = PB::D::stride(p.ldb);
 
-  f32x16 acc[TM][TN];
+  f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
   u32x4 regs[LPS];
   // chunk q of the next stage to be fetched (which starts at contraction index k0) into its register
   auto load_item = [&](int q, int k0, auto tested_c) {
     constexpr bool TESTED = decltype(tested_c)::value;
     if (q < PA::PER) {
-      regs[q] = TESTED ? PA::fetch_tested(pa[q], q, k0, kend, m0, p.M) : PA::fetch(pa[q]);
-      pa[q] += A_KMAJOR ? (int64_t)BK : (int64_t)BK * p.lda;
+      const T* ptr = (const T*)at_offset(pa, oa[q]);
+      regs[q] = TESTED ? PA::fetch_tested(ptr, q, k0, kend, m0, p.M) : PA::fetch(ptr);
     } else {
-      regs[q] = TESTED ? PB::fetch_tested(pb[q - PA::PER], q - PA::PER, k0, kend, n0, p.N) : PB::fetch(pb[q - PA::PER]);
-      pb[q - PA::PER] += B_KMAJOR ? (int64_t)BK : (int64_t)BK * p.ldb;
+      const T* ptr = (const T*)at_offset(pb, ob[q - PA::PER]);
+      regs[q] = TESTED ? PB::fetch_tested(ptr, q - PA::PER, k0, kend, n0, p.N) : PB::fetch(ptr);
+    }
+    if (q == LPS - 1) {
+      pa += sa;
+      pb += sb;
     }
   };
   auto store_item = [&](char* dst, int q) {
@@ -847,16 +869,14 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_reg_kernel(GemmParams p
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  FragRegs<A_KMAJOR> fa[2][TM];
+  FragRegs<A_KMAJOR> fa[TM];
   FragRegs<B_KMAJOR> fb[2][TN];
-  constexpr int NMFMA = TM * TN;
-  constexpr int NR = TM + TN;
-  constexpr int RPS = (NR + NMFMA - 1) / NMFMA;
-  constexpr int RSLOTS = (NR + RPS - 1) / RPS;
-  auto read_item = [&](const char* stage, int ks, int buf, int item) {
-    const uint32_t sa_addr = lds_address(stage), sb_addr = sa_addr + PA::D::BYTES;
-    if (item < TM) PA::D::frag_issue(fa[buf][item], sa_addr, wm * WTM + item * 32, ks, lane);
-    else PB::D::frag_issue(fb[buf][item - TM], sb_addr, wn * WTN + (item - TM) * 32, ks, lane);
+  const uint32_t lds0 = lds_address(smem);
+  const uint32_t la = PA::D::frag_lane(wm * WTM, lane), lb = PA::D::BYTES + PB::D::frag_lane(wn * WTN, lane);
+  auto read_item = [&](uint32_t at, auto ks_c, auto q_c) {
+    constexpr int ks = decltype(ks_c)::value, q = decltype(q_c)::value;
+    if constexpr (q < TN) PB::D::template frag_issue<q, ks>(fb[ks][q], lds0 + at, lb);
+    else PA::D::template frag_issue<q - TN, ks>(fa[q - TN], lds0 + at, la);
   };
   typedef std::integral_constant<bool, true> yes_t;
   typedef std::integral_constant<bool, false> no_t;
@@ -878,54 +898,63 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_reg_kernel(GemmParams p
   }
   wait_lgkmcnt<0>();
   barrier();
-#pragma unroll
-  for (int r = 0; r < NR; ++r) read_item(smem, 0, 0, r);
+  static_for<TN + TM>([&](auto q_c) { read_item(0, std::integral_constant<int, 0>(), q_c); });
 
-  // ---- one stage: everything that is not an MFMA sits behind one, pinned by scheduling barriers.
-  // MORE: another stage follows (its chunks are in the registers: stored behind steps 0 and 1);
-  // LOAD: and one after that, whose chunks are requested behind steps 1 and 2 (TESTED: by extents).
-  auto stage = [&](char* cur, char* nxt, int k2, auto more_c, auto load_c, auto tested_c) {
-    constexpr bool MORE = decltype(more_c)::value, LOAD = decltype(load_c)::value;
+  // ---- one stage, as in the direct-to-LDS kernel: everything that is not an MFMA sits behind one, pinned by scheduling
+  // barriers.  MORE: another stage follows (its chunks are in the registers: stored behind the MFMAs of step 0); LOAD: and one
+  // after that, whose chunks are requested into the registers a store has left (TESTED: by extents).  The waits for
+  // fragments count reads alone: with stores among them they leave less in flight than they might, never more.
+  constexpr int NMFMA = TM * TN;
+  constexpr int HAND = hand_rows(TM) * TN;
+  constexpr int RA = PA::D::READS_PER_FRAG, RB = PB::D::READS_PER_FRAG;
+  auto stage = [&](uint32_t cur, uint32_t nxt, int k2, auto more_c, auto load_c, auto tested_c) {
+    constexpr bool MORE = decltype(more_c)::value, LOAD = decltype(load_c)::value, TESTED = decltype(tested_c)::value;
+    static_for<KSTEPS>([&](auto ks_c) {
+      constexpr int ks = decltype(ks_c)::value;
+      constexpr bool last = ks + 1 == KSTEPS, hands = last && MORE;
+      typedef std::integral_constant<int, last ? 0 : ks + 1> next_ks;
+      constexpr ReadSlots<TM, TN> slots(hands ? HAND : 0);
+      static_for<NMFMA>([&](auto m_c) {
+        constexpr int m = decltype(m_c)::value, i = m / TN, j = i % 2 ? TN - 1 - m % TN : m % TN;
+        if constexpr (hands && m == HAND) {
+          wait_lgkmcnt<0>();  // this wave's stores of the next stage are in, it has read the last operands of `cur`
+          barrier();          // ... and everyone
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (LOAD && TESTED) {  // branches: here, where no read is in flight whose register a branch might move
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      const bool last = ks + 1 == KSTEPS;
-      wait_lgkmcnt<0>();  // this step's operands, requested a step ago; at the last step also the stores
-      __builtin_amdgcn_sched_barrier(0);
-      if (last && MORE) {
-        barrier();  // everyone's stores of the next stage are in, everyone has read the last operands of `cur`
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int m = 0; m < NMFMA; ++m) {
-        const int i = m / TN, j = m % TN;
-        acc[i][j] = mfma32(fb[ks & 1][j].template get<v8>(), fa[ks & 1][i].template get<v8>(), acc[i][j]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (!last || MORE) {
-#pragma unroll
-          for (int r = m * RPS; r < (m + 1) * RPS && r < NR; ++r) {
-            if (last) read_item(nxt, 0, 0, r);
-            else read_item(cur, ks + 1, (ks + 1) & 1, r);
+            for (int q = 0; q < LPS; ++q) load_item(q, k2, tested_c);
+            __builtin_amdgcn_sched_barrier(0);
           }
+        } else if constexpr (m % TN == 0 && (!hands || m < HAND)) {
+          constexpr int flying = (TM - 1 - i) * RA + (last || i == 0 ? 0 : TN * RB + i * RA);
+          wait_lgkmcnt<(flying < 15 ? flying : 15)>();
+          __builtin_amdgcn_sched_barrier(0);
         }
-        // the extras of steps 0 to 2, dealt over their MFMAs: half of the stores, the other half and half of the
-        // loads, the other half of the loads
-        constexpr int H = LPS / 2;
-        const int q0 = m * H / NMFMA, q1 = (m + 1) * H / NMFMA;
-#pragma unroll
-        for (int q = q0; q < q1; ++q) {
-          if (MORE && ks == 0) store_item(nxt, q);
-          if (MORE && ks == 1) store_item(nxt, H + q);
-          if (LOAD && ks == 1) load_item(q, k2, tested_c);
-          if (LOAD && ks == 2) load_item(H + q, k2, tested_c);
-        }
+        acc[i][j] = mfma16(fb[ks][j].template get<v8>(), fa[i].template get<v8>(), acc[i][j]);
         __builtin_amdgcn_sched_barrier(0);
-      }
-    }
+        if constexpr (!last || MORE) {
+          constexpr int q0 = slots.before(m), q1 = slots.before(m + 1);
+          static_for<q1 - q0>([&](auto q) {
+            read_item(last ? nxt : cur, next_ks(), std::integral_constant<int, q0 + decltype(q)::value>());
+          });
+        }
+        // step 0: store and load of chunk q, the load half a step behind its store where the step is long enough; the loads
+        // that are left in the last step
+        constexpr int T0 = m * LPS / NMFMA, T1 = (m + 1) * LPS / NMFMA;
+        static_for<T1 - T0>([&](auto q_c) {
+          constexpr int q = T0 + decltype(q_c)::value;
+          if constexpr (!last && MORE) store_item(smem + nxt, q);
+          if constexpr (!last && LOAD && !TESTED && q >= LPS / 2) load_item(q - LPS / 2, k2, tested_c);
+          if constexpr (last && LOAD && !TESTED && q < LPS / 2) load_item(q + LPS / 2, k2, tested_c);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
   };
-  static_assert(LPS % 2 == 0 && RSLOTS <= NMFMA, "halves of a stage's chunks; a step's reads fit behind its MFMAs");
+  static_assert(LPS % 2 == 0, "halves of a stage's chunks");
   int kt = 0;
-  auto cur = [&]() { return smem + (kt & 1) * STAGE; };
-  auto nxt = [&]() { return smem + ((kt + 1) & 1) * STAGE; };
+  auto cur = [&]() { return (uint32_t)((kt & 1) * STAGE); };
+  auto nxt = [&]() { return (uint32_t)((~kt & 1) * STAGE); };
   for (; kt + 2 < nfree; ++kt) stage(cur(), nxt(), 0, yes_t(), yes_t(), no_t());
   for (; kt + 2 < nk; ++kt) stage(cur(), nxt(), kbeg + (kt + 2) * BK, yes_t(), yes_t(), yes_t());
   if (kt + 1 < nk) {
@@ -1275,6 +1304,9 @@ static int launch_dma(hipStream_t st, const GemmParams& p) {
 // The register-staged kernel handles everything (ragged extents, unaligned
 // pointers); the direct-to-LDS kernel needs the vector conditions and a
 // contraction extent that is a multiple of its BK.
+// Leading dimensions up to which a lane's part of an operand address (255 rows and a chunk) fits 32 bits, by half.
+constexpr int64_t kMaxPitch = 1 << 22;
+
 constexpr int kStagesNarrow = 3;  // LDS stages of the configurations below 256x256 but 128x128
 
 template <typename T, bool AK, bool BKM>
@@ -1289,9 +1321,16 @@ static int launch_cfg(hipStream_t st, bool vec, const GemmPlan& pl, const GemmPa
       case 7: return launch_dma<T, 128, 64, 64, 4, 1, 2, AK, BKM, kStagesNarrow>(st, p);
     }
   }
-  if (pl.bm == 256 && pl.bn == 256) return launch_reg<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
-  if (pl.bm == 128 && pl.bn == 128) return launch_reg<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, p);
-  return TF_EINVAL;
+  if (pl.bm == 256 && pl.bn == 256 && p.lda <= kMaxPitch && p.ldb <= kMaxPitch)
+    return launch_reg<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
+  if (pl.bm == 256) {  // wider rows than the 256x256 kernel addresses: the same slices on the smaller tiles
+    GemmParams q = p;
+    q.tiles_m = (q.M + 127) / 128;
+    q.tiles_n = (q.N + 127) / 128;
+    if ((int64_t)q.tiles_m * q.tiles_n * q.splits > 0x7fffffff) return TF_EINVAL;
+    return launch_reg<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, q);
+  }
+  return launch_reg<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, p);
 }
 
 // Second pass of a split contraction (no-op when the contraction was not split).
@@ -1523,7 +1562,7 @@ static int gemm_entry(void* stream, int dtype, int out_dtype, int layout_a, int 
        reinterpret_cast<uintptr_t>(bias)) & 1)
     return TF_EALIGN;
 
-  const bool vec = aligned16(A) && aligned16(B) && aligned16(C) && (!bias || aligned16(bias)) && a_contig % 8 == 0 &&
+  const bool vec = lda <= kMaxPitch && ldb <= kMaxPitch && aligned16(A) && aligned16(B) && aligned16(C) && (!bias || aligned16(bias)) && a_contig % 8 == 0 &&
                    b_contig % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && N % 8 == 0 && ldc % 8 == 0 &&
                    (!mask_act || (aligned16(mask_act) && ld_mask % 8 == 0));
   const bool forced = force.cfg >= 0 || force.splits > 0 || (force.flags & 64);
@@ -1685,7 +1724,7 @@ bool group_problem_ok(const tf_gemm_problem& q) {
 // Fast-path preconditions of the direct-to-LDS kernel for a (K-minor, K-minor) problem.
 bool group_problem_fast(const tf_gemm_problem& q) {
   const int64_t cn = (q.chunk_n <= 0 || q.chunk_n >= q.N) ? q.N : q.chunk_n;
-  return aligned16(q.A) && aligned16(q.B) && aligned16(q.C) && q.M % 8 == 0 && q.N % 8 == 0 && q.lda % 8 == 0 &&
+  return q.lda <= kMaxPitch && q.ldb <= kMaxPitch && aligned16(q.A) && aligned16(q.B) && aligned16(q.C) && q.M % 8 == 0 && q.N % 8 == 0 && q.lda % 8 == 0 &&
          q.ldb % 8 == 0 && q.ldc % 8 == 0 && q.K % 64 == 0 && q.lda >= q.M && q.ldb >= q.N && q.ldc >= cn &&
          q.N % cn == 0 && cn % 8 == 0 && (cn == q.N || (q.chunk_stride % 8 == 0 && q.chunk_stride >= (q.M - 1) * q.ldc + cn));
 }
