@@ -135,3 +135,23 @@ def test_alibi_closed_form_against_oracle_and_argument_checks(dev):
         T.fast_causal_attention_with_bias.apply(q.to(dev), k.to(dev), v.to(dev), torch.ones(3, dtype=torch.float16, device=dev))
     with pytest.raises(ValueError):   # float16 slopes, the precision the reference's matrix is built from
         T.fast_causal_attention_with_bias.apply(q.to(dev), k.to(dev), v.to(dev), torch.ones(4, dtype=torch.float32, device=dev))
+
+
+@pytest.mark.parametrize("form", ["none", "dense", "slopes", "masked"])
+@pytest.mark.parametrize("dims", [(1, 2, 512, 64), (1, 1, 576, 32), (2, 1, 640, 64), (1, 3, 1088, 32), (1, 1, 1984, 64)])
+def test_two_groups_of_waves(dims, form, dev):
+    """Few heads and long chains of blocks, the forms whose workgroups have two groups of waves (from 512 keys on forward, 640
+    backward): even and odd numbers of blocks, and rows that see no key in one group's blocks or in all of the other's."""
+    from tritonformer_amd.transformer import get_slopes
+
+    b, nh, s, hd = dims
+    bias = None if form == "none" else R.alibi_mask(s, nh)
+    slopes = torch.tensor(get_slopes(nh), dtype=torch.float16) if form == "slopes" else None
+    if form == "masked":
+        keys, rows = torch.arange(s), torch.arange(s)
+        odd = (keys // 64) % 2 == 1
+        bias[:, rows >= 128] = bias[:, rows >= 128].masked_fill(odd, float("-inf"))     # the first group's keys alone
+        own = (keys[None] // 64) == (rows[:, None] // 64)
+        late = (rows // 64) % 4 == 3                                                  # these rows: the second group's alone
+        bias[:, late] = R.alibi_mask(s, nh)[:, late].masked_fill(~own[late], float("-inf"))
+    run_case(dims, torch.float16, dev, bias=bias, kernel_bias=slopes)

@@ -18,6 +18,7 @@
 //     ds_read_b64_tr_b16.
 // The 16 contraction slots of lane-half h in step t map to sequence offsets
 // 16t + 8(s/4) + 4h + s%4 (s = 0..7), on both operands alike.
+#include <algorithm>
 #include <type_traits>
 #include "rowops.h"
 
@@ -62,10 +63,10 @@ struct SeqTile {
   // Direct-to-LDS loads: thread t's j-th 16-byte load lands in LDS slot t + 256 j of the tile,
   // so the chunk swizzle is applied to the global address.  ptr[j] = address of that chunk in
   // the tile whose first row is row0 of a (seq, hd) matrix with row stride ss.
-  static __device__ __forceinline__ void stream_init(const T* (&ptr)[PER_THREAD], const T* base, int64_t ss, int row0) {
+  static __device__ __forceinline__ void stream_init(const T* (&ptr)[PER_THREAD], const T* base, int64_t ss, int row0, int tid) {
 #pragma unroll
     for (int j = 0; j < PER_THREAD; ++j) {
-      const int id = threadIdx.x + j * 256;
+      const int id = tid + j * 256;
       const int row = id / CPR, c = (id % CPR) ^ swz(row);
       ptr[j] = base + (int64_t)(row0 + row) * ss + c * 8;
     }
@@ -75,10 +76,10 @@ struct SeqTile {
   // allocation -- are moved 32 rows back: the tile then holds rows 0 .. 31 twice.  No valid query ever
   // sees the copies (keys beyond the sequence lie above every diagonal; queries beyond it are skipped),
   // they only have to be readable and finite.
-  static __device__ __forceinline__ void stream_tail(const T* (&ptr)[PER_THREAD], int64_t ss) {
+  static __device__ __forceinline__ void stream_tail(const T* (&ptr)[PER_THREAD], int64_t ss, int tid) {
 #pragma unroll
     for (int j = 0; j < PER_THREAD; ++j)
-      if ((int)threadIdx.x + j * 256 >= 32 * CPR) ptr[j] -= 32 * ss;
+      if (tid + j * 256 >= 32 * CPR) ptr[j] -= 32 * ss;
   }
   // LDS destination of a wave's j-th load into the tile at `tile`
   static __device__ __forceinline__ char* stream_slot(char* tile, int wave, int j) {
@@ -156,30 +157,30 @@ template <typename T> __device__ __forceinline__ void alibi4(float d0, float ste
 struct BiasTile {
   static constexpr int BYTES = 128 * 64 * 2;
   template <typename T>
-  static __device__ __forceinline__ void init(const T* (&bp)[4], const T* bias_head, int64_t row_stride, int q0, int S) {
+  static __device__ __forceinline__ void init(const T* (&bp)[4], const T* bias_head, int64_t row_stride, int q0, int S, int tid) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int id = threadIdx.x + j * 256;
+      const int id = tid + j * 256;
       const int row = id >> 3, c = (id & 7) ^ ((row >> 1) & 7);
       const int qrow = min(q0 + row, S - 1);  // rows past the sequence are never read back
       bp[j] = bias_head + (int64_t)qrow * row_stride + c * 8;
     }
   }
   // last block of a sequence that ends half way through it: chunks of key columns 32 .. 63 read 32 columns back
-  template <typename T> static __device__ __forceinline__ void tail(const T* (&bp)[4]) {
+  template <typename T> static __device__ __forceinline__ void tail(const T* (&bp)[4], int tid) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int id = threadIdx.x + j * 256;
+      const int id = tid + j * 256;
       const int row = id >> 3, c = (id & 7) ^ ((row >> 1) & 7);
       if (c >= 4) bp[j] -= 32;
     }
   }
-  // next 64 keys into the tile at `dst`; advances the pointers
-  template <typename T> static __device__ __forceinline__ void load(const T* (&bp)[4], char* dst, int wave) {
+  // 64 keys into the tile at `dst`; advances the pointers by `step` columns
+  template <typename T> static __device__ __forceinline__ void load(const T* (&bp)[4], char* dst, int wave, int step) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       __builtin_amdgcn_global_load_lds((gptr_void*)bp[j], (lds_void*)(dst + (j * 256 + wave * 64) * 16), 16, 0, 0);
-      bp[j] += 64;
+      bp[j] += step;
     }
   }
   // LDS address (relative to the tile) of keys chunk*8 + 4*half .. +3 of query row r
@@ -239,8 +240,18 @@ __device__ __forceinline__ void store_rows32(char* slab, T* dst, int64_t row_str
 // ===========================================================================
 constexpr float kRescaleThreshold = 8.0f;  // log2 domain
 
-template <typename T, int HD, int BMODE, bool TAIL>
-__global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE == kDenseBias ? 2 : 3)) void attn_fwd_kernel(AttnParams p) {
+// G groups of four waves: group g takes the blocks g, g + G, ... of its workgroup's loop, with LDS stages of its own, and the
+// groups' results are merged through LDS at the end, in the order of the groups.  A grid that does not fill the chip waits for
+// its longest chain of blocks with one wave per SIMD: two groups halve the chain and put a second wave beside the first.
+#define ATTN_GROUP_SETUP(STAGE_BYTES)                                                                                         \
+  const int grp = G > 1 ? (int)(threadIdx.x >> 8) : 0, tid = G > 1 ? (int)(threadIdx.x & 255) : (int)threadIdx.x;             \
+  const int lane = threadIdx.x & 63, wave = tid >> 6;                                                                         \
+  /* the same numbers as scalars: LDS slot addresses of the tile loads stay scalar arithmetic */                              \
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave), grp_u = G > 1 ? __builtin_amdgcn_readfirstlane(grp) : 0;           \
+  char* const gmem = smem + grp_u * (2 * (STAGE_BYTES))
+
+template <typename T, int HD, int BMODE, bool TAIL, int G = 1>
+__global__ __launch_bounds__(256 * G, HD > 64 ? 1 : (G > 1 || BMODE == kDenseBias ? 2 : 3)) void attn_fwd_kernel(AttnParams p) {
   constexpr bool HAS_BIAS = BMODE == kDenseBias, ALIBI = BMODE == kAlibi;
   typedef SeqTile<T, 64, HD> KT;
   typedef typename Vec<T>::v8 v8;
@@ -251,8 +262,7 @@ __global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE == kDenseBias ? 2 : 3)) v
   constexpr int PT = KT::PER_THREAD;  // 16-byte chunks per thread per 64-row tile
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);  // the same number as a scalar: LDS slot addresses of the tile loads stay scalar arithmetic
+  ATTN_GROUP_SETUP(STAGE);
   const int nbh = p.B * p.nh;
   const int nqb = (p.S + 127) / 128;
   const int qblk = nqb - 1 - (int)(blockIdx.x / nbh);  // heaviest query blocks first
@@ -294,41 +304,41 @@ __global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE == kDenseBias ? 2 : 3)) v
 
   // K and V (and bias) tiles go from global memory straight into LDS, no register staging
   const T* kp[PT];
-  KT::stream_init(kp, K, p.ss, 0);
+  KT::stream_init(kp, K, p.ss, grp * 64, tid);
   const int64_t v_minus_k = V - K;
   const T* bp[4];
-  if (HAS_BIAS) BiasTile::init(bp, (const T*)p.bias + (int64_t)h * p.bias_sh, p.bias_sr, q0, p.S);
+  if (HAS_BIAS) BiasTile::init(bp, (const T*)p.bias + (int64_t)h * p.bias_sh + grp * 64, p.bias_sr, q0, p.S, tid);
   auto load_tile = [&](int stage_off) {  // next 64 keys / values (/ bias columns) into the stage at byte offset stage_off
 #pragma unroll
     for (int j = 0; j < PT; ++j) {
-      __builtin_amdgcn_global_load_lds((gptr_void*)kp[j], (lds_void*)KT::stream_slot(smem + stage_off, wave_u, j), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((gptr_void*)kp[j], (lds_void*)KT::stream_slot(gmem + stage_off, wave_u, j), 16, 0, 0);
       __builtin_amdgcn_global_load_lds((gptr_void*)(kp[j] + v_minus_k),
-                                       (lds_void*)KT::stream_slot(smem + stage_off + KT::BYTES, wave_u, j), 16, 0, 0);
-      kp[j] += (int64_t)64 * p.ss;
+                                       (lds_void*)KT::stream_slot(gmem + stage_off + KT::BYTES, wave_u, j), 16, 0, 0);
+      kp[j] += (int64_t)(64 * G) * p.ss;
     }
-    if (HAS_BIAS) BiasTile::load(bp, smem + stage_off + 2 * KT::BYTES, wave_u);
+    if (HAS_BIAS) BiasTile::load(bp, gmem + stage_off + 2 * KT::BYTES, wave_u, 64 * G);
   };
   // the loads of key block jb: if the sequence ends inside it (TAIL: S = 32 mod 64, an instantiation of its
   // own, so that whole-block sequences pay nothing), rows / bias columns 32 .. 63 are taken 32 earlier
   auto load_block_of = [&](int jb, int stage_off) {
     if (TAIL && (jb + 1) * 64 > p.S) {
-      KT::stream_tail(kp, p.ss);
-      if (HAS_BIAS) BiasTile::tail(bp);
+      KT::stream_tail(kp, p.ss, tid);
+      if (HAS_BIAS) BiasTile::tail(bp, tid);
     }
     load_tile(stage_off);
   };
   uint32_t ka[KS], va[DT][2];
-  const uint32_t lds0 = lds_address(smem);
+  const uint32_t lds0 = lds_address(gmem);
   KT::operand_addrs(ka, va, lds0, lane);
 
-  load_block_of(0, 0);
+  if (grp < nkv) load_block_of(grp, 0);
   __syncthreads();
 
   // One 64-key block out of the stage at byte offset SOFF.
   auto step = [&](auto stage_tag, int j) {
     constexpr int SOFF = decltype(stage_tag)::value * STAGE;
     constexpr int VOFF = SOFF + KT::BYTES;
-    if (j + 1 < nkv) load_block_of(j + 1, STAGE - SOFF);
+    if (j + G < nkv) load_block_of(j + G, STAGE - SOFF);
     const int kb = j * 64;
     if (active && kb <= q0w + 31) {
       auto block = [&](auto diag_tag) {
@@ -438,12 +448,43 @@ __global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE == kDenseBias ? 2 : 3)) v
     __syncthreads();  // waits for this thread's tile loads, then for everyone's; all reads of this stage are done
   };
 
-  for (int j = 0; j < nkv; j += 2) {
-    step(std::integral_constant<int, 0>{}, j);
-    if (j + 1 < nkv) step(std::integral_constant<int, 1>{}, j + 1);
+  for (int j = 0; j < nkv; j += 2 * G) {  // the same number of steps in every group; one that has no block left only meets the barriers
+    step(std::integral_constant<int, 0>{}, j + grp);
+    if (j + G < nkv) step(std::integral_constant<int, 1>{}, j + G + grp);
   }
 
-  if (active) {
+  if constexpr (G > 1) {
+    // running maxima, sums and results of groups 1 .. G - 1 to group 0, register by register of every lane
+    constexpr int REGS = DT * 16 + 2;
+    float* const mine = (float*)smem + (size_t)wave * (REGS * 64) + lane;
+    if (grp > 0) {
+      float* x = mine + (size_t)(grp - 1) * (4 * REGS * 64);
+      x[0] = m_ref;
+      x[64] = lacc[0];
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[(2 + d * 16 + r) * 64] = oacc[d][r];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int g = 1; g < G; ++g) {
+        const float* x = mine + (size_t)(g - 1) * (4 * REGS * 64);
+        const float m_new = fmaxf(m_ref, x[0]), m_use = m_new == -INFINITY ? 0.f : m_new;
+        const float a0 = fast_exp2(m_ref - m_use), a1 = fast_exp2(x[0] - m_use);  // exp2(-inf) = 0: a group without a live key
+        lacc[0] = lacc[0] * a0 + x[64] * a1;
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) oacc[d][r] = oacc[d][r] * a0 + x[(2 + d * 16 + r) * 64] * a1;
+        m_ref = m_new;
+      }
+    }
+    __syncthreads();  // the slabs below lie where the groups' results were
+  }
+
+  if (active && grp == 0) {
     const float l_tot = lacc[0];
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
     if (lane < 32) p.lse[(int64_t)bh * p.S + myq] = m_ref + log2f(l_tot);
@@ -456,8 +497,8 @@ __global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE == kDenseBias ? 2 : 3)) v
 // dK/dV pass.  Workgroup: 4 waves x 32 keys; query blocks of 64 from the
 // diagonal downwards.  Q and dO tiles (+ their lse / delta) go through LDS.
 // ===========================================================================
-template <typename T, int HD, int BMODE, bool TAIL>
-__global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_dkdv_kernel(AttnParams p) {
+template <typename T, int HD, int BMODE, bool TAIL, int G = 1>
+__global__ __launch_bounds__(256 * G, HD <= 64 ? 2 : 1) void attn_dkdv_kernel(AttnParams p) {
   constexpr bool HAS_BIAS = BMODE == kDenseBias, ALIBI = BMODE == kAlibi;
   typedef SeqTile<T, 64, HD> QT;
   typedef typename Vec<T>::v8 v8;
@@ -471,8 +512,7 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_dkdv_kernel(AttnPa
   static_assert(4 * 32 * (HD * 2 + 16) <= 2 * STAGE, "the result slabs of the four waves reuse the pipeline stages");
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);  // the same number as a scalar: LDS slot addresses of the tile loads stay scalar arithmetic
+  ATTN_GROUP_SETUP(STAGE);
   const int nbh = p.B * p.nh;
   const int kblk = (int)(blockIdx.x / nbh);  // lowest key blocks (longest loops) first
   const int bh = blockIdx.x % nbh;
@@ -513,44 +553,44 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_dkdv_kernel(AttnPa
   // waves 0 and 1) and, with a bias, its [64][128] tile in plain row-major order.
   const T* qp[PT];
   const T* dop[PT];
-  QT::stream_init(qp, Q, p.ss, k0);
-  QT::stream_init(dop, dO, p.oss, k0);
-  const float* statp = (wave == 0 ? p.lse : p.delta) + (int64_t)bh * p.S + k0 + lane;  // waves 0, 1 only
+  QT::stream_init(qp, Q, p.ss, k0 + grp * 64, tid);
+  QT::stream_init(dop, dO, p.oss, k0 + grp * 64, tid);
+  const float* statp = (wave == 0 ? p.lse : p.delta) + (int64_t)bh * p.S + k0 + grp * 64 + lane;  // waves 0, 1 only
   const T* bp[4];
   if (HAS_BIAS) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int id = threadIdx.x + j * 256;
+      const int id = tid + j * 256;
       const int row = id >> 4;
       int col = k0 + (id & 15) * 8;
       if (col >= p.S) col = k0;  // keys past the sequence belong to inactive waves: any in-bounds column will do
-      bp[j] = (const T*)p.bias + (int64_t)h * p.bias_sh + (int64_t)(k0 + row) * p.bias_sr + col;
+      bp[j] = (const T*)p.bias + (int64_t)h * p.bias_sh + (int64_t)(k0 + grp * 64 + row) * p.bias_sr + col;
     }
   }
   auto load_block = [&](int stage_off) {  // next 64 queries into the stage at byte offset stage_off
 #pragma unroll
     for (int j = 0; j < PT; ++j) {
-      __builtin_amdgcn_global_load_lds((gptr_void*)qp[j], (lds_void*)QT::stream_slot(smem + stage_off, wave_u, j), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((gptr_void*)dop[j], (lds_void*)QT::stream_slot(smem + stage_off + QT::BYTES, wave_u, j),
+      __builtin_amdgcn_global_load_lds((gptr_void*)qp[j], (lds_void*)QT::stream_slot(gmem + stage_off, wave_u, j), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((gptr_void*)dop[j], (lds_void*)QT::stream_slot(gmem + stage_off + QT::BYTES, wave_u, j),
                                        16, 0, 0);
-      qp[j] += (int64_t)64 * p.ss;
-      dop[j] += (int64_t)64 * p.oss;
+      qp[j] += (int64_t)(64 * G) * p.ss;
+      dop[j] += (int64_t)(64 * G) * p.oss;
     }
     if (wave < 2) {
-      __builtin_amdgcn_global_load_lds((gptr_void*)statp, (lds_void*)(smem + stage_off + STAT + wave_u * 256), 4, 0, 0);
-      statp += 64;
+      __builtin_amdgcn_global_load_lds((gptr_void*)statp, (lds_void*)(gmem + stage_off + STAT + wave_u * 256), 4, 0, 0);
+      statp += 64 * G;
     }
     if (HAS_BIAS) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        __builtin_amdgcn_global_load_lds((gptr_void*)bp[j], (lds_void*)(smem + stage_off + BIAS + (j * 256 + wave_u * 64) * 16),
+        __builtin_amdgcn_global_load_lds((gptr_void*)bp[j], (lds_void*)(gmem + stage_off + BIAS + (j * 256 + wave_u * 64) * 16),
                                          16, 0, 0);
-        bp[j] += (int64_t)64 * p.bias_sr;
+        bp[j] += (int64_t)(64 * G) * p.bias_sr;
       }
     }
   };
   // lane-dependent parts of the LDS addresses
-  const uint32_t lds0 = lds_address(smem);
+  const uint32_t lds0 = lds_address(gmem);
   uint32_t ra[KS], ha[DT][2];
   QT::operand_addrs(ra, ha, lds0, lane);
   const uint32_t sa = lds0 + STAT + 16 * (lane >> 5);  // statistics of queries g*8 + 4*(lane/32) .. +3
@@ -560,25 +600,25 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_dkdv_kernel(AttnPa
   // are taken 32 earlier; the sub-tile they fill is never used
   auto load_block_of = [&](int ib, int stage_off) {
     if (TAIL && k0 + (ib + 1) * 64 > p.S) {
-      QT::stream_tail(qp, p.ss);
-      QT::stream_tail(dop, p.oss);
+      QT::stream_tail(qp, p.ss, tid);
+      QT::stream_tail(dop, p.oss, tid);
       if (lane >= 32) statp -= 32;
       if (HAS_BIAS) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (((threadIdx.x + j * 256) >> 4) >= 32) bp[j] -= (int64_t)32 * p.bias_sr;
+          if (((tid + j * 256) >> 4) >= 32) bp[j] -= (int64_t)32 * p.bias_sr;
       }
     }
     load_block(stage_off);
   };
-  if (nq > 0) load_block_of(0, 0);
+  if (grp < nq) load_block_of(grp, 0);
   __syncthreads();
 
   auto step = [&](auto stage_tag, int it) {
     constexpr int SOFF = decltype(stage_tag)::value * STAGE;
-    if (it + 1 < nq) load_block_of(it + 1, STAGE - SOFF);
+    if (it + G < nq) load_block_of(it + G, STAGE - SOFF);
     const int qb = k0 + it * 64;
-    if (active) {
+    if (active && (G == 1 || it < nq)) {
       static_for<2>([&](auto qt_tag) {
         constexpr int qt = decltype(qt_tag)::value;
         const int qs = qb + qt * 32;      // first query of this 32-row sub-tile
@@ -680,19 +720,43 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_dkdv_kernel(AttnPa
     }
     __syncthreads();  // this thread's block loads have landed, then everyone's; all reads of this stage are done
   };
-  for (int it = 0; it < nq; it += 2) {
-    step(std::integral_constant<int, 0>{}, it);
-    if (it + 1 < nq) step(std::integral_constant<int, 1>{}, it + 1);
+  for (int it = 0; it < nq; it += 2 * G) {
+    step(std::integral_constant<int, 0>{}, it + grp);
+    if (it + G < nq) step(std::integral_constant<int, 1>{}, it + G + grp);
   }
 
+  if constexpr (G > 1) {
+    // group 0 sums and stores dK, group 1 dV: each hands its part of the other's over
+    static_assert(G == 2, "one result for each group");
+    float* const mine = (float*)smem + (size_t)wave * (DT * 16 * 64) + lane;
+    float* const out = mine + (grp ? 0 : 4 * DT * 16 * 64);
+    const float* const in = mine + (grp ? 4 * DT * 16 * 64 : 0);
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) out[(d * 16 + r) * 64] = grp ? dk[d][r] : dv[d][r];
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float x = in[(d * 16 + r) * 64];
+        dk[d][r] = grp ? x + dv[d][r] : dk[d][r] + x;  // the sum this group stores, group 0's part first
+      }
+    __syncthreads();  // the slabs lie where the results were
+  }
   if (active) {
     T* dK = (T*)p.dk + base;
     T* dV = (T*)p.dv + base;
     // the pipeline stages are free: every wave is past the last barrier of the loop
-    char* slab = smem + wave * (32 * (HD * 2 + 16));
+    char* slab = smem + (grp * 4 + wave) * (32 * (HD * 2 + 16));
     const int64_t row0 = (int64_t)(mykey - (lane & 31)) * p.ss;
-    store_rows32<T, HD>(slab, dK + row0, p.ss, dk, p.scale, lane);
-    store_rows32<T, HD>(slab, dV + row0, p.ss, dv, 1.0f, lane);
+    if (G > 1) {
+      store_rows32<T, HD>(slab, (grp ? dV : dK) + row0, p.ss, dk, grp ? 1.0f : p.scale, lane);
+    } else {
+      store_rows32<T, HD>(slab, dK + row0, p.ss, dk, p.scale, lane);
+      store_rows32<T, HD>(slab, dV + row0, p.ss, dv, 1.0f, lane);
+    }
   }
 }
 
@@ -700,8 +764,8 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_dkdv_kernel(AttnPa
 // dQ pass.  Workgroup: 4 waves x 32 queries; key/value blocks of 64 up to the
 // diagonal, K and V tiles through LDS.
 // ===========================================================================
-template <typename T, int HD, int BMODE, bool TAIL>
-__global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE != kNoBias ? 2 : 3)) void attn_dq_kernel(AttnParams p) {
+template <typename T, int HD, int BMODE, bool TAIL, int G = 1>
+__global__ __launch_bounds__(256 * G, HD > 64 ? 1 : (G > 1 || BMODE != kNoBias ? 2 : 3)) void attn_dq_kernel(AttnParams p) {
   constexpr bool HAS_BIAS = BMODE == kDenseBias, ALIBI = BMODE == kAlibi;
   typedef SeqTile<T, 64, HD> KT;
   typedef typename Vec<T>::v8 v8;
@@ -711,8 +775,7 @@ __global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE != kNoBias ? 2 : 3)) void
   static_assert(4 * 32 * (HD * 2 + 16) <= 2 * STAGE, "the result slabs of the four waves reuse the pipeline stages");
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);  // the same number as a scalar: LDS slot addresses of the tile loads stay scalar arithmetic
+  ATTN_GROUP_SETUP(STAGE);
   const int nbh = p.B * p.nh;
   const int nqb = (p.S + 127) / 128;
   const int qblk = nqb - 1 - (int)(blockIdx.x / nbh);
@@ -760,7 +823,7 @@ __global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE != kNoBias ? 2 : 3)) void
     const auto both = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // own half and the partner's
     const unsigned u0 = both[0], u1 = both[1];
     neg_delta = -(__builtin_bit_cast(float, u0) + __builtin_bit_cast(float, u1));
-    if (lane < 32) p.delta[(int64_t)bh * p.S + myq] = neg_delta;
+    if (lane < 32 && grp == 0) p.delta[(int64_t)bh * p.S + myq] = neg_delta;
   }
   f32x16 dq[DT];
 #pragma unroll
@@ -771,40 +834,40 @@ __global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE != kNoBias ? 2 : 3)) void
   // K and V (and bias) tiles go from global memory straight into LDS
   constexpr int PT = KT::PER_THREAD;
   const T* kp[PT];
-  KT::stream_init(kp, K, p.ss, 0);
+  KT::stream_init(kp, K, p.ss, grp * 64, tid);
   const int64_t v_minus_k = V - K;
   const T* bp[4];
-  if (HAS_BIAS) BiasTile::init(bp, (const T*)p.bias + (int64_t)h * p.bias_sh, p.bias_sr, q0, p.S);
+  if (HAS_BIAS) BiasTile::init(bp, (const T*)p.bias + (int64_t)h * p.bias_sh + grp * 64, p.bias_sr, q0, p.S, tid);
   auto load_tile = [&](int stage_off) {
 #pragma unroll
     for (int j = 0; j < PT; ++j) {
-      __builtin_amdgcn_global_load_lds((gptr_void*)kp[j], (lds_void*)KT::stream_slot(smem + stage_off, wave_u, j), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((gptr_void*)kp[j], (lds_void*)KT::stream_slot(gmem + stage_off, wave_u, j), 16, 0, 0);
       __builtin_amdgcn_global_load_lds((gptr_void*)(kp[j] + v_minus_k),
-                                       (lds_void*)KT::stream_slot(smem + stage_off + KT::BYTES, wave_u, j), 16, 0, 0);
-      kp[j] += (int64_t)64 * p.ss;
+                                       (lds_void*)KT::stream_slot(gmem + stage_off + KT::BYTES, wave_u, j), 16, 0, 0);
+      kp[j] += (int64_t)(64 * G) * p.ss;
     }
-    if (HAS_BIAS) BiasTile::load(bp, smem + stage_off + 2 * KT::BYTES, wave_u);
+    if (HAS_BIAS) BiasTile::load(bp, gmem + stage_off + 2 * KT::BYTES, wave_u, 64 * G);
   };
   // the loads of key block jb: if the sequence ends inside it (TAIL: S = 32 mod 64, an instantiation of its
   // own, so that whole-block sequences pay nothing), rows / bias columns 32 .. 63 are taken 32 earlier
   auto load_block_of = [&](int jb, int stage_off) {
     if (TAIL && (jb + 1) * 64 > p.S) {
-      KT::stream_tail(kp, p.ss);
-      if (HAS_BIAS) BiasTile::tail(bp);
+      KT::stream_tail(kp, p.ss, tid);
+      if (HAS_BIAS) BiasTile::tail(bp, tid);
     }
     load_tile(stage_off);
   };
   // row operands of K and V, hd operands of K
   uint32_t ra[KS], ha[DT][2];
-  const uint32_t lds0 = lds_address(smem);
+  const uint32_t lds0 = lds_address(gmem);
   KT::operand_addrs(ra, ha, lds0, lane);
 
-  load_block_of(0, 0);
+  if (grp < nkv) load_block_of(grp, 0);
   __syncthreads();
 
   auto step = [&](auto stage_tag, int j) {
     constexpr int SOFF = decltype(stage_tag)::value * STAGE;
-    if (j + 1 < nkv) load_block_of(j + 1, STAGE - SOFF);
+    if (j + G < nkv) load_block_of(j + G, STAGE - SOFF);
     const int kb = j * 64;
     if (active) {
       static_for<2>([&](auto jt_tag) {
@@ -889,12 +952,33 @@ __global__ __launch_bounds__(256, HD > 64 ? 1 : (BMODE != kNoBias ? 2 : 3)) void
     }
     __syncthreads();  // this thread's tile loads have landed, then everyone's; all reads of this stage are done
   };
-  for (int j = 0; j < nkv; j += 2) {
-    step(std::integral_constant<int, 0>{}, j);
-    if (j + 1 < nkv) step(std::integral_constant<int, 1>{}, j + 1);
+  for (int j = 0; j < nkv; j += 2 * G) {  // the same number of steps in every group; one that has no block left only meets the barriers
+    step(std::integral_constant<int, 0>{}, j + grp);
+    if (j + G < nkv) step(std::integral_constant<int, 1>{}, j + G + grp);
   }
 
-  if (active) {
+  if constexpr (G > 1) {
+    float* const mine = (float*)smem + (size_t)wave * (DT * 16 * 64) + lane;
+    if (grp > 0) {
+      float* x = mine + (size_t)(grp - 1) * (4 * DT * 16 * 64);
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[(d * 16 + r) * 64] = dq[d][r];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int g = 1; g < G; ++g)
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) dq[d][r] += mine[(size_t)(g - 1) * (4 * DT * 16 * 64) + (d * 16 + r) * 64];
+    }
+    __syncthreads();
+  }
+
+  if (active && grp == 0) {
     T* dQ = (T*)p.dq + base;
     // the pipeline stages are free: every wave is past the last barrier of the loop
     store_rows32<T, HD>(smem + wave * (32 * (HD * 2 + 16)), dQ + (int64_t)(myq - (lane & 31)) * p.ss, p.ss, dq, p.scale,
@@ -911,47 +995,78 @@ static void allow_lds(K kernel, int bytes) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
-template <typename T, int HD, int MODE, bool TAIL>
+// LDS of a workgroup: its groups' stages, or what they hand over at the end (`regs` floats per lane and wave of those that do)
+constexpr int attn_lds(int stage, int groups, int handing, int regs) {
+  return std::max(groups * 2 * stage, groups > 1 ? handing * 4 * regs * 64 * 4 : 0);
+}
+
+template <typename T, int HD, int MODE, bool TAIL, int G>
 static int fwd_launch(hipStream_t st, const AttnParams& p) {
-  constexpr int lds = 2 * (2 * SeqTile<T, 64, HD>::BYTES + (MODE == kDenseBias ? BiasTile::BYTES : 0));
-  auto kernel = attn_fwd_kernel<T, HD, MODE, TAIL>;
+  constexpr int stage = 2 * SeqTile<T, 64, HD>::BYTES + (MODE == kDenseBias ? BiasTile::BYTES : 0);
+  constexpr int lds = attn_lds(stage, G, G - 1, HD / 2 + 2);
+  static_assert(lds <= 160 * 1024, "LDS budget");
+  auto kernel = attn_fwd_kernel<T, HD, MODE, TAIL, G>;
   static bool once = (allow_lds(kernel, lds), true);
   (void)once;
   const unsigned grid = (unsigned)(((p.S + 127) / 128) * p.B * p.nh);
-  kernel<<<dim3(grid), dim3(256), lds, st>>>(p);
+  kernel<<<dim3(grid), dim3(256 * G), lds, st>>>(p);
   TF_CHECK_LAUNCH();
   return TF_OK;
 }
 
 // dQ pass first: it also produces the -delta rows that the dK/dV pass reads.
-template <typename T, int HD, int MODE, bool TAIL>
+template <typename T, int HD, int MODE, bool TAIL, int G>
 static int bwd_launch(hipStream_t st, const AttnParams& p) {
   const unsigned grid = (unsigned)(((p.S + 127) / 128) * p.B * p.nh);
   {
-    constexpr int lds = 2 * (2 * SeqTile<T, 64, HD>::BYTES + (MODE == kDenseBias ? BiasTile::BYTES : 0));
-    auto kernel = attn_dq_kernel<T, HD, MODE, TAIL>;
+    constexpr int stage = 2 * SeqTile<T, 64, HD>::BYTES + (MODE == kDenseBias ? BiasTile::BYTES : 0);
+    constexpr int lds = attn_lds(stage, G, G - 1, HD / 2);
+    static_assert(lds <= 160 * 1024, "LDS budget");
+    auto kernel = attn_dq_kernel<T, HD, MODE, TAIL, G>;
     static bool once = (allow_lds(kernel, lds), true);
     (void)once;
-    kernel<<<dim3(grid), dim3(256), lds, st>>>(p);
+    kernel<<<dim3(grid), dim3(256 * G), lds, st>>>(p);
     TF_CHECK_LAUNCH();
   }
   {
-    constexpr int lds = 2 * (2 * SeqTile<T, 64, HD>::BYTES + 2 * 64 * 4 + (MODE == kDenseBias ? 64 * 128 * 2 : 0));
-    auto kernel = attn_dkdv_kernel<T, HD, MODE, TAIL>;
+    constexpr int stage = 2 * SeqTile<T, 64, HD>::BYTES + 2 * 64 * 4 + (MODE == kDenseBias ? 64 * 128 * 2 : 0);
+    constexpr int lds = attn_lds(stage, G, G, HD / 2);
+    static_assert(lds <= 160 * 1024 && G * 4 * 32 * (HD * 2 + 16) <= lds, "LDS budget, slabs of the write-out");
+    auto kernel = attn_dkdv_kernel<T, HD, MODE, TAIL, G>;
     static bool once = (allow_lds(kernel, lds), true);
     (void)once;
-    kernel<<<dim3(grid), dim3(256), lds, st>>>(p);
+    kernel<<<dim3(grid), dim3(256 * G), lds, st>>>(p);
     TF_CHECK_LAUNCH();
   }
   return TF_OK;
 }
 
+// Two groups of waves per workgroup where the longest chain of blocks is what a launch waits for.  fp16, head_dim 64, us forward /
+// both backward passes.  One workgroup per CU or less: 24 heads of 1024 16.2 -> 13.3 / 38.1 -> 34.7 (dense bias 20.2 -> 18.4 / 45.9 ->
+// 41.9), 16 of 2048 29.1 -> 23.0 / 69.0 -> 59.8, one of 2560 32.8 -> 24.8 / 82 -> 68, 12 of 1024 and head_dim 32 21.1 -> 17.3 / 54.3 ->
+// 41.8; a short chain loses to handing over at the end what it gains: 64 of 512 10.2 -> 9.2 / 23.3 -> 23.3, 36 of 320 7.3 -> 7.3 / 16.8 ->
+// 18.3, 192 of 128 5.9 -> 6.1 / 12.4 -> 14.8.  Up to two per CU the longer sequences: 12 of 4096 54 -> 42 / 144 -> 117, 24 of 2048 29.3
+// -> 23.5 / 77 -> 64, 32 of 2048 31.6 -> 28.4 / 86 -> 79, but 48 of 1024 17.0 -> 16.5 / 43.7 -> 43.6, 64 of 1024 17.8 -> 18.8 / 48 -> 52.
+// Only for whole blocks and head_dim <= 64: at 128 the passes hold more registers than two waves per SIMD have, and the
+// stages of two groups do not fit the LDS beside a bias.
+static bool attn_two_groups(const AttnParams& p, bool fwd) {
+  const int64_t wgs = (int64_t)((p.S + 127) / 128) * p.B * p.nh;
+  return p.S >= (fwd ? 512 : 640) && wgs * 1024 <= (int64_t)device_shape().cus * std::min(std::max(p.S, 1024), 2048);
+}
+template <typename T, int HD, bool FWD, int MODE, bool TAIL>
+static int attn_launch(hipStream_t st, const AttnParams& p) {
+  if constexpr (HD <= 64 && !TAIL) {
+    if (attn_two_groups(p, FWD)) return FWD ? fwd_launch<T, HD, MODE, TAIL, 2>(st, p) : bwd_launch<T, HD, MODE, TAIL, 2>(st, p);
+  }
+  return FWD ? fwd_launch<T, HD, MODE, TAIL, 1>(st, p) : bwd_launch<T, HD, MODE, TAIL, 1>(st, p);
+}
+
 template <typename T, bool FWD, int MODE, bool TAIL>
 static int attn_dispatch_tail(hipStream_t st, int hd, const AttnParams& p) {
   switch (hd) {
-    case 32: return FWD ? fwd_launch<T, 32, MODE, TAIL>(st, p) : bwd_launch<T, 32, MODE, TAIL>(st, p);
-    case 64: return FWD ? fwd_launch<T, 64, MODE, TAIL>(st, p) : bwd_launch<T, 64, MODE, TAIL>(st, p);
-    case 128: return FWD ? fwd_launch<T, 128, MODE, TAIL>(st, p) : bwd_launch<T, 128, MODE, TAIL>(st, p);
+    case 32: return attn_launch<T, 32, FWD, MODE, TAIL>(st, p);
+    case 64: return attn_launch<T, 64, FWD, MODE, TAIL>(st, p);
+    case 128: return attn_launch<T, 128, FWD, MODE, TAIL>(st, p);
   }
   return TF_ESHAPE;
 }
