@@ -21,7 +21,7 @@ extern "C" {
 
 /* tf_gemm_out (include/tritonformer_amd.h) with the tile choice imposed on THIS call:
  *   cfg    -1 = cost model; 0 / 1 = register-staged 256x256 / 128x128;
- *          2..7 = direct-to-LDS 256x256, 128x128, 256x128, 128x256, 64x64, 128x64
+ *          2..7 = direct-to-LDS 256x256, 128x128, 256x128, 128x256, 64x64, 128x64; 8 = register-staged 256x128
  *          (a direct-to-LDS cfg falls back to its register-staged twin when the operands
  *          do not meet its preconditions);
  *   splits 0 = chosen by the library, n > 0 = contraction cut into n slices;

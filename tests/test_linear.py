@@ -719,3 +719,30 @@ def test_rows_at_and_beyond_the_pitch_that_32_bit_offsets_reach(layouts, pitch, 
     assert_close(base, (a.float() if la == 0 else a.float().T) @ (b.float().T if lb == 0 else b.float()), name=layouts)
     for cfg in range(8):
         assert torch.equal(run(wide, cfg), base), f"cfg {cfg}"
+
+
+@pytest.mark.parametrize("layouts", ["fwd", "dx", "dw"])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (255, 127, 65), (257, 129, 63), (300, 200, 193), (513, 385, 320), (256, 128, 2051)])
+def test_register_staged_256x128_gives_the_bits_of_128x128(layouts, M, N, K, dev):
+    """Edges of the tile, contractions that end within a step, odd pitches, with bias and ReLU: unsplit, both sum the same steps in
+    the same order."""
+    from tritonformer_amd import _lib
+
+    d = _lib.load_diag()
+    g = torch.Generator().manual_seed(43)
+    la, lb = {"fwd": (0, 1), "dx": (0, 0), "dw": (1, 1)}[layouts]
+    a = torch.randn((M, K + 3) if la == 0 else (K, M + 3), generator=g).half().to(dev)
+    b = (torch.randn((N, K + 1) if lb == 0 else (K, N + 1), generator=g) / K ** 0.5).half().to(dev)
+    bias = torch.randn(N, generator=g).half().to(dev)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(cfg, epilogue):
+        out = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+        _lib.check(d.tf_diag_gemm(stream, cfg, 1, 0, 0, 0, la, lb, M, N, K, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+                                  out.data_ptr(), N, bias.data_ptr() if epilogue else None, int(epilogue), None, 0))
+        return out
+
+    want = (a[:, :K].float() if la == 0 else a[:, :M].float().T) @ (b[:, :K].float().T if lb == 0 else b[:, :N].float())
+    assert_close(run(8, False), want, name=layouts)
+    for epilogue in (False, True):
+        assert torch.equal(run(8, epilogue), run(1, epilogue))

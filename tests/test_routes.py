@@ -76,3 +76,18 @@ def test_route_rejects_bad_arguments():
     assert f(0, 64, 64, 64, 1, 0, rows, 1) == -1 and f(256, 0, 64, 64, 1, 0, rows, 1) == -1
     assert f(256, 64, 64, 64, 1, 4, rows, 1) == -1 and f(256, 64, 64, 64, 1, 0, None, 1) == -1
     assert f(256, 8192, 3072, 1024, 1, 0, rows, 1) == -1  # two launches, room for one
+
+
+@pytest.mark.parametrize("m,n,k,vec,want", [
+    # operands of any alignment: 256x128 tiles where these fill one round, 256x256 tiles for whole rounds, 128x128 for few
+    (4113, 1733, 2051, False, [(1733, 8, 1)]),
+    (2051, 1733, 4113, False, [(1733, 8, 2)]),
+    (8192, 50257, 1024, False, [(50257, 0, 1)]),
+    (100, 5001, 129, False, [(5001, 1, 1)]),
+    # a short contraction is mostly start and write-out, which 128x128 tiles overlap; a long one holds 256x128 tiles up
+    (7488, 2624, 64, True, [(2624, 3, 1)]),
+    (4096, 2048, 8192, True, [(2048, 4, 1)]),
+    (8192, 1024, 50304, True, [(1024, 2, 2)]),
+])
+def test_rates_of_the_tiles(m, n, k, vec, want):
+    assert route(m, n, k, vec=vec) == want

@@ -1121,6 +1121,7 @@ static const TileCfg kCfgs[] = {
     {128, 256, 64, 8, 1},  // 5: direct-to-LDS, three stages = 144 KB LDS, waves 2x4, wave tile 64x64
     {64, 64, 64, 4, 1},    // 6: direct-to-LDS, three stages = 48 KB LDS, waves 2x2, wave tile 32x32: few tiles
     {128, 64, 64, 4, 1},   // 7: direct-to-LDS, three stages = 72 KB LDS, waves 4x1, wave tile 32x64: few tiles
+    {256, 128, 64, 8, 0},  // 8: register-staged, waves 4x2, wave tile 64x64, any shape / alignment
 };
 constexpr int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
 
@@ -1153,13 +1154,19 @@ static GemmPlan plan_for(int64_t cus, int cfg, int64_t M, int64_t N, int64_t K, 
   // gradients: few output tiles, long contraction); never beyond one full round of
   // workgroups, and every slice keeps at least 16 steps so that the fp32 partial
   // traffic stays small.
-  const double fixed = pl.bm * pl.bn >= 256 * 256 ? 10.0 : 7.0;
-  // register-staged: 8192 x 1024 x 50257 takes 393 steps of 256x256 tiles in 911 us, 786 of 128x128 in 1340
-  // (with the figures of the direct-to-LDS tiles 960 x 768 x 50257 ran on 128x128 tiles: 160 us instead of 129)
-  // Over 46 products of odd extents (64 to 16384, 64 to 8192, 64 to 4096, all layouts) the choice was within a tenth of the
-  // better tile every time.
-  const double per_step = !kCfgs[cfg].dma ? (pl.bm * pl.bn >= 256 * 256 ? 2.25 : 1.6)
-                          : pl.bm * pl.bn >= 256 * 256 ? 1.65 : (pl.bm * pl.bn >= 256 * 128 ? 1.0 : 1.1);
+  // Microseconds of a round of workgroups beside its steps and per 64-wide step, by configuration.  Found over 550 products of
+  // odd extents (16 to 16384 rows, 64 to 8192 columns, contractions of 64 to 4096, all layouts) and 730 of whole multiples of 64, every
+  // tile timed: the tiles chosen take 0.7 and 1.3 per cent longer (geometric mean) than the best of those at hand; with the
+  // figures of the 32x32x16 kernels (10 and 2.25, 7 and 1.6 register-staged; 10 and 1.65, 7 and 1.1, 7 and 1.0) it was 1.5 and
+  // 3.0, up to 25 where a contraction is short (7488 x 2624 x 64 13.9 -> 11.3 us) or 256x128 tiles fill one round (768 x 7040 x 3648
+  // 52.5 -> 42.0).
+  static const struct { double fixed, per_step; } rates[] = {{8.9, 1.63}, {3.1, 1.14}, {10.1, 1.62}, {5.0, 1.13}, {9.7, 0.78},
+                                                             {9.7, 0.78}, {5.0, 1.13}, {5.0, 1.13}, {10.1, 0.92}};
+  static_assert(sizeof(rates) / sizeof(rates[0]) == sizeof(kCfgs) / sizeof(kCfgs[0]), "a rate for each configuration");
+  // 256x128 tiles pay for a long contraction, which holds the clock down, with their share of loads: 0.79 us per step of 128
+  // (4096 x 2048 x 8192 125 us on 256x256 tiles in two slices, 111 on these), 0.91 of 786 (8192 x 1024 x 50304 687 and 725)
+  const bool held = (cfg == 4 || cfg == 5) && ksteps >= 256;
+  const double fixed = rates[cfg].fixed, per_step = held ? 0.91 : rates[cfg].per_step;
   auto cost_of = [&](int64_t nsplit, int64_t steps) {
     const int64_t rounds = (tiles * nsplit + slots - 1) / slots;
     double c = (double)rounds * (fixed + per_step * (double)steps);
@@ -1196,9 +1203,11 @@ static GemmPlan plan_for(int64_t cus, int cfg, int64_t M, int64_t N, int64_t K, 
 
 // Time (microseconds) of a direct-to-LDS launch that leaves CUs or their second workgroup idle, where the cost above --
 // made for whole rounds -- is 1.3 to 2 times too high: a fixed part plus a time per 64-wide step that rises with the
-// workgroups per CU (`fill`), since operands come faster and the clock is higher while few CUs work.  Fits to 348 products
-// of 16 to 4096 rows, 128 to 6144 columns and contractions of 64 to 8192, operand B from HBM.
-// Checked over 1400 others that leave CUs idle with the large tile (16 to 6144 rows, 64 to 9000 columns, all layouts, slices
+// workgroups per CU (`fill`), since operands come faster and the clock is higher while few CUs work.  Fits to 650 products that
+// leave CUs idle (16 to 16384 rows, 64 to 8192 columns, contractions of 64 to 4096 and more, all layouts): the tile taken is 1.4 per
+// cent slower than the best of the five at hand (geometric mean), 2.5 with the figures of the 32x32x16 kernels; 2752 x 512 x 1792
+// 14.8 -> 12.2 us, 384 x 3392 x 2048 18.7 -> 15.5.
+// With those kernels it was checked over 1400 others that leave CUs idle with the large tile (16 to 6144 rows, 64 to 9000 columns, all layouts, slices
 // and sign bits as they are in use): 1.44 times the large tile's speed (geometric mean; the best of the three tiles each time
 // 1.45), seven of them slower than the large tile, by 4 to 9 per cent, all of 300 workgroups and more with long contractions
 // (629 x 5120 x 8128 90 -> 98 us), where two workgroups of a CU take longer than 1.3 to 1.8 of them would.  Counted as two they
@@ -1211,11 +1220,11 @@ static double part_round_us(int64_t cus, const GemmPlan& pl, int64_t M, int64_t 
   const double more = 0.7 * std::max(0.0, fill - 1);  // start and write-out of every further workgroup of a CU
   double c = 0;
   switch (pl.cfg) {
-    case 2: c = 5.4 + steps * (0.95 + 0.70 * rise(fill, 0.35, 1)); break;
-    case 3: c = 2.5 + steps * (0.67 + 0.43 * rise(fill, 0.6, 2)); break;
-    case 4: c = 3.8 + steps * (0.64 + 0.36 * rise(fill, 0.25, 1)); break;
-    case 6: c = 2.7 + more + steps * std::max(0.27 + 0.05 * rise(fill, 0.5, 1), 0.27 * fill); break;
-    case 7: c = 2.9 + more + steps * std::max(0.36 + 0.14 * rise(fill, 0.5, 1), 0.40 * fill); break;
+    case 2: c = 4.4 + steps * (0.85 + 1.05 * rise(fill, 0.31, 1.14)); break;
+    case 3: c = 2.1 + steps * (0.81 + 0.59 * rise(fill, 0.73, 2.2)); break;
+    case 4: c = 3.6 + steps * (0.63 + 0.47 * rise(fill, 0.285, 1.15)); break;
+    case 6: c = 2.8 + more + steps * std::max(0.26 + 0.04 * rise(fill, 0.5, 1), 0.35 * fill); break;
+    case 7: c = 2.6 + more + steps * std::max(0.36 + 0.12 * rise(fill, 0.5, 1), 0.43 * fill); break;
   }
   if (pl.splits > 1) c += 3.0 + (pl.splits + 0.5) * (double)M * (double)N * 4.0 / 5.0e6;
   return c;
@@ -1230,15 +1239,14 @@ static GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec
     if (kCfgs[cfg].dma && !dma) cfg = kCfgs[cfg].bm * kCfgs[cfg].bn >= 256 * 256 ? 0 : 1;  // register-staged twin
     return plan_for(cus, cfg, M, N, K, nullptr, allow_split, force.splits);
   }
-  // candidates: 256x256 and 256x128 / 128x128 tiles, direct-to-LDS kernels when their
+  // candidates: 256x256, 256x128 and 128x128 tiles, direct-to-LDS kernels when their
   // preconditions hold, the register-staged twins otherwise
   const int cand_dma[3] = {2, 4, 3};
-  const int cand_reg[2] = {0, 1};
+  const int cand_reg[3] = {0, 8, 1};
   const int* cand = dma ? cand_dma : cand_reg;
-  const int ncand = dma ? 3 : 2;
   GemmPlan best = plan_for(cus, cand[0], M, N, K, nullptr, allow_split, force.splits);
   double best_cost = 1e30;
-  for (int i = 0; i < ncand; ++i) {
+  for (int i = 0; i < 3; ++i) {
     double c;
     const GemmPlan pl = plan_for(cus, cand[i], M, N, K, &c, allow_split, force.splits);
     if (c < best_cost) { best_cost = c; best = pl; }
@@ -1254,7 +1262,7 @@ static GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec
   const int64_t wgs = (int64_t)best.tiles_m * best.tiles_n * best.splits;
   if (dma && wgs <= cus * (best.cfg == 3 ? 2 : 1)) {
     const GemmPlan best_large = best;
-    double best_us = 0.95 * part_round_us(cus, best, M, N);
+    double best_us = 1.05 * part_round_us(cus, best, M, N);
     for (int cfg : {6, 7}) {
       const GemmPlan pl = plan_for(cus, cfg, M, N, K, nullptr, allow_split, best_large.splits);
       const double us = part_round_us(cus, pl, M, N);
@@ -1323,7 +1331,9 @@ static int launch_cfg(hipStream_t st, bool vec, const GemmPlan& pl, const GemmPa
   }
   if (pl.bm == 256 && pl.bn == 256 && p.lda <= kMaxPitch && p.ldb <= kMaxPitch)
     return launch_reg<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
-  if (pl.bm == 256) {  // wider rows than the 256x256 kernel addresses: the same slices on the smaller tiles
+  if (pl.bm == 256 && pl.bn == 128 && p.lda <= kMaxPitch && p.ldb <= kMaxPitch)
+    return launch_reg<T, 256, 128, 64, 4, 2, 2, AK, BKM>(st, p);
+  if (pl.bm == 256) {  // wider rows than the 256-row tiles address: the same slices on the smaller tiles
     GemmParams q = p;
     q.tiles_m = (q.M + 127) / 128;
     q.tiles_n = (q.N + 127) / 128;
