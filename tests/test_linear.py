@@ -746,3 +746,28 @@ def test_register_staged_256x128_gives_the_bits_of_128x128(layouts, M, N, K, dev
     assert_close(run(8, False), want, name=layouts)
     for epilogue in (False, True):
         assert torch.equal(run(8, epilogue), run(1, epilogue))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [1, 127, 128, 513, 1024, 1025])
+@pytest.mark.parametrize("cols,pitch", [(1, 1), (8, 8), (63, 64), (64, 72), (72, 72), (777, 777), (3072, 3072)])
+def test_column_sums_of_few_rows(rows, cols, pitch, dtype, dev):
+    """One launch up to 1024 rows (512 of odd pitch), two beyond: every remainder of its 128 rows and 64 columns, rows whose end is no whole chunk,
+    with and without a mask, against 64 bits.  At most 32 additions deep: 2^-19 of the sum of magnitudes."""
+    from tritonformer_amd import _lib
+
+    lib, st, code = _lib.load(), _lib.stream_ptr(), _lib.dtype_code(dtype)
+    g = torch.Generator().manual_seed(47)
+    x, act = (torch.randn(rows, pitch, generator=g).to(dtype).to(dev) for _ in range(2))
+    nb = lib.tf_colsum_partial_bytes(rows, cols)
+    part = torch.empty(max(nb, 16), dtype=torch.uint8, device=dev)
+    masked = torch.full((rows, pitch), 7.0, dtype=dtype, device=dev)
+    sums, msums, again = (torch.full((cols,), float("nan"), device=dev) for _ in range(3))
+    _lib.check(lib.tf_colsum(st, code, 2, rows, cols, x.data_ptr(), pitch, sums.data_ptr(), part.data_ptr(), nb))
+    _lib.check(lib.tf_relu_mask_colsum(st, code, 2, rows, cols, x.data_ptr(), pitch, act.data_ptr(), pitch, masked.data_ptr(), pitch,
+                                       msums.data_ptr(), part.data_ptr(), nb))
+    _lib.check(lib.tf_colsum(st, code, 2, rows, cols, masked.data_ptr(), pitch, again.data_ptr(), part.data_ptr(), nb))
+    xs, kept = x[:, :cols].double(), torch.where(act > 0, x, torch.zeros_like(x))[:, :cols]
+    assert ((sums.double() - xs.sum(0)).abs() <= 2.0 ** -19 * xs.abs().sum(0)).all()
+    assert torch.equal(masked[:, :cols], kept) and (masked[:, cols:] == 7).all() and torch.equal(msums, again)
+    assert ((msums.double() - kept.double().sum(0)).abs() <= 2.0 ** -19 * kept.double().abs().sum(0)).all()

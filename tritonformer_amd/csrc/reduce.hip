@@ -111,6 +111,76 @@ __global__ __launch_bounds__(256) void colsum_final(int groups, int cols, const 
   }
 }
 
+// Few rows: both stages in one launch, a workgroup of 1024 threads per 64 columns (one line of a row), 128 rows at a time and four
+// of a thread's requested together.  Bound by the latency of its loads; the second launch cost more than the idle CUs do: both
+// stages and this one, us in a graph, fp16: 512 x 1024 4.35 -> 2.47, 960 x 768 4.57 -> 3.17, 960 x 3072 5.98 -> 4.92, 1024 x 8192
+// 7.98 -> 5.39.  Rows at odd addresses, whose pieces of 128 bytes lie in two lines, up to half as many: 1000 x 777 5.28 -> 5.65.
+constexpr int64_t kCsFewRows = 1024;
+constexpr int kCsFewCols = 64, kCsFewSlices = 128;
+template <typename T, typename TO, bool ANY, bool MASK>
+__global__ __launch_bounds__(1024) void colsum_few(int rows, int cols, const T* __restrict__ x, int64_t ldx, TO* __restrict__ sums,
+                                                   const T* __restrict__ act, int64_t lda, T* __restrict__ out, int64_t ldo) {
+  typedef Row<T, ANY> R;
+  __shared__ __align__(16) float red[kCsFewSlices][kCsFewCols + 4];
+  __shared__ float part[16][kCsFewCols];
+  const int lane8 = threadIdx.x & 7, slice = threadIdx.x >> 3;
+  const int chunk = blockIdx.x * (kCsFewCols / 8) + lane8;
+  float acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  if (chunk * 8 < cols) {
+    auto add = [&](int r, u32x4 rx, u32x4 ra) {
+      float v[8];
+      unpack8<T>(R::template settle<true>(rx, chunk, cols), v);
+      if constexpr (MASK) {
+        float a[8];
+        unpack8<T>(R::template settle<true>(ra, chunk, cols), a);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = a[e] > 0.f ? v[e] : 0.f;
+        R::template store<true>(out + (int64_t)r * ldo, chunk, cols, pack8<T>(v));
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += v[e];
+    };
+    auto fetch_x = [&](int r) { return R::template fetch<true>(x + (int64_t)r * ldx, chunk, cols); };
+    auto fetch_a = [&](int r, u32x4 rx) { return MASK ? R::template fetch<true>(act + (int64_t)r * lda, chunk, cols) : rx; };
+    int r = slice;
+    for (; r + 3 * kCsFewSlices < rows; r += 4 * kCsFewSlices) {
+      u32x4 rx[4], ra[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        rx[k] = fetch_x(r + k * kCsFewSlices);
+        ra[k] = fetch_a(r + k * kCsFewSlices, rx[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) add(r + k * kCsFewSlices, rx[k], ra[k]);
+    }
+    for (; r < rows; r += kCsFewSlices) {
+      const u32x4 rx = fetch_x(r);
+      add(r, rx, fetch_a(r, rx));
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; e += 4) {
+    const f32x4 v = {acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
+    *reinterpret_cast<f32x4*>(&red[slice][lane8 * 8 + e]) = v;
+  }
+  __syncthreads();
+  const int col = threadIdx.x & 63, p = threadIdx.x >> 6;
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < kCsFewSlices / 16; ++k) s += red[p * (kCsFewSlices / 16) + k][col];
+  part[p][col] = s;
+  __syncthreads();
+  const int c = blockIdx.x * kCsFewCols + col;
+  if (p == 0 && c < cols) {
+    s = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) s += part[k][col];
+    sums[c] = (TO)s;
+  }
+}
+
 template <typename T, bool ANY>
 __global__ __launch_bounds__(256) void relu_mask_kernel(int64_t rows, int cols, const T* __restrict__ grad,
                                                          int64_t ldg, const T* __restrict__ act, int64_t lda,
@@ -136,17 +206,30 @@ template <typename T>
 static int colsum_launch(hipStream_t st, int64_t rows, int64_t cols, const void* x, int64_t ldx, void* out,
                          bool out_f32, float* partial, const void* act = nullptr, int64_t lda = 0,
                          void* masked = nullptr, int64_t ldm = 0) {
+  const bool vec = row_vectorizable<T>(x, cols, ldx) && (!masked || (row_vectorizable<T>(act, cols, lda) && row_vectorizable<T>(masked, cols, ldm)));
+  if (rows <= (vec ? kCsFewRows : kCsFewRows / 2)) {
+    const dim3 few((unsigned)ceil_div(cols, kCsFewCols));
+#define COLSUM_FEW(TO, ANY, MASK)                                                                                    \
+  colsum_few<T, TO, ANY, MASK><<<few, dim3(1024), 0, st>>>((int)rows, (int)cols, (const T*)x, ldx, (TO*)out, (const T*)act, lda, \
+                                                           (T*)masked, ldm)
+#define COLSUM_FEW_MASK(TO, ANY) do { if (masked) COLSUM_FEW(TO, ANY, true); else COLSUM_FEW(TO, ANY, false); } while (0)
+    if (out_f32) { if (vec) COLSUM_FEW_MASK(float, false); else COLSUM_FEW_MASK(float, true); }
+    else { if (vec) COLSUM_FEW_MASK(T, false); else COLSUM_FEW_MASK(T, true); }
+#undef COLSUM_FEW_MASK
+#undef COLSUM_FEW
+    TF_CHECK_LAUNCH();
+    return TF_OK;
+  }
   const int groups = colsum_groups(rows, cols);
   const int rpg = (int)((rows + groups - 1) / groups);
   const dim3 grid((unsigned)ceil_div(cols, kCsColsPerBlock), (unsigned)groups), block(256);
 #define COLSUM(ANY, MASK)                                                                                       \
   colsum_partial<T, ANY, MASK><<<grid, block, 0, st>>>(rows, (int)cols, (const T*)x, ldx, partial, rpg, (const T*)act, \
                                                        lda, (T*)masked, ldm)
-  const bool vec = row_vectorizable<T>(x, cols, ldx);
   if (!masked) {
     if (vec) COLSUM(false, false);
     else COLSUM(true, false);
-  } else if (vec && row_vectorizable<T>(act, cols, lda) && row_vectorizable<T>(masked, cols, ldm)) {
+  } else if (vec) {
     COLSUM(false, true);
   } else {
     COLSUM(true, true);
