@@ -131,6 +131,13 @@ int tf_gemm_relu_bits(void* stream, int dtype, int out_dtype, int layout_a, int 
                       const void* A, int64_t lda, const void* B, int64_t ldb,
                       void* C, int64_t ldc, const void* bias,
                       void* bits_out, const void* bits_in, int64_t ld_bits);
+/* C (M, count * each) = A (M, K; K contiguous) . [B[0] | ... | B[count - 1]], up to three matrices (K, each) of leading dimension
+ * ldb (`B`: HOST array of device pointers) as one product: the three projections of tritonformer/transformer.py:158-160 over
+ * weights that lie apart, without a copy that lays them side by side.  The product that tf_gemm would make of such a copy, the
+ * same bits.  TF_ESHAPE (nothing launched) when it would not run on tiles that each lie in one of the matrices
+ * of the direct-to-LDS kernels; workspace: tf_gemm_workspace_bytes() of the whole product. */
+int tf_gemm_side_by_side(void* stream, int dtype, int64_t M, int64_t each, int count, int64_t K, const void* A, int64_t lda,
+                         const void* const* B, int64_t ldb, void* C, int64_t ldc, void* workspace, int64_t workspace_bytes);
 /* tf_gemm (bits_out null) or tf_gemm_relu_bits with bits_out, with the bias as its fp32 master: each value is
  * rounded to the operand dtype where it is read, so the results are those of the call with a bias converted
  * before it.  With bits_out no workspace is needed. */

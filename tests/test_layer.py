@@ -1,0 +1,131 @@
+"""A decoder layer as one autograd node against the four nodes it stands for: the same kernels in the same order, so the same
+bits -- but for the gradient of the embeddings, where the first layer's two summands are rounded once instead of twice."""
+import pytest
+import torch
+
+import tritonformer_amd.transformer as TM
+from tests.util import rel_l2
+from tritonformer_amd.transformer import Transformer, TransformerConfig
+
+pytestmark = pytest.mark.gpu
+
+
+def build(dev, bias=False, alibi=False, param_dtype=torch.float32, layers=3, d=128, heads=2):
+    torch.manual_seed(5)
+    m = Transformer(TransformerConfig(512, d, 64, heads, d // heads, 3 * d, layers, bias, alibi), device=dev, param_dtype=param_dtype)
+    with torch.no_grad():
+        m.logits_out.weight.normal_(0, 0.02)
+        for p in m.parameters():
+            if p.ndim == 1:
+                p.add_(torch.randn_like(p) * 0.05)
+    return m
+
+
+def step(m, fused, amp=None, passes=1, retain=False):
+    ids = torch.randint(0, 512, (2, 64), generator=torch.Generator().manual_seed(7)).to(m.embed_tokens.weight.device)
+    m.zero_grad(set_to_none=True)
+    TM.FUSE_LAYER = fused
+    try:
+        for _ in range(passes):
+            with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+                logits, loss = m(ids, ids)
+            if retain:
+                (loss * 256).backward(retain_graph=True)
+            (loss * 256).backward()
+    finally:
+        TM.FUSE_LAYER = True
+    return logits, loss, {n: None if p.grad is None else p.grad.clone() for n, p in m.named_parameters()}
+
+
+def assert_same(one, four, dtype):
+    assert torch.equal(one[0], four[0]) and torch.equal(one[1], four[1])
+    assert one[2].keys() == four[2].keys()
+    for name, g in four[2].items():
+        if g is None:
+            assert one[2][name] is None, name
+        elif name.startswith("embed"):  # a rounding to 16 bits more or less: half a unit of the last place per element
+            assert rel_l2(one[2][name], g) < (2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7), name
+        else:
+            assert torch.equal(one[2][name], g), name
+
+
+@pytest.mark.parametrize("bias,alibi", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("param_dtype,amp", [(torch.float32, torch.float16), (torch.float32, torch.bfloat16), (torch.float16, None)])
+def test_one_node_gives_the_bits_of_four(bias, alibi, param_dtype, amp, dev):
+    m = build(dev, bias, alibi, param_dtype)
+    assert_same(step(m, True, amp), step(m, False, amp), amp or param_dtype)
+    with torch.no_grad():
+        ids = torch.arange(64, device=dev)[None]
+        one = m(ids, None) if amp is None else None
+        TM.FUSE_LAYER = False
+        try:
+            assert one is None or torch.equal(one, m(ids, None))
+        finally:
+            TM.FUSE_LAYER = True
+
+
+def test_accumulated_and_repeated_passes(dev):
+    m = build(dev, bias=True)
+    assert_same(step(m, True, torch.float16, passes=2), step(m, False, torch.float16, passes=2), torch.float16)
+    assert_same(step(m, True, torch.float16, retain=True), step(m, False, torch.float16, retain=True), torch.float16)
+
+
+@pytest.mark.parametrize("train", ["mlp.", "attention.v_proj", "layernorm", "layer_list.2", "layer_list.0.input_layernorm",
+                                   "layer_list.1.mlp.dense_4h_to_h.bias", "embed"])
+def test_frozen_parameters(train, dev):
+    m = build(dev, bias=True)
+    for name, p in m.named_parameters():
+        p.requires_grad_(train in name)
+    assert_same(step(m, True, torch.float16), step(m, False, torch.float16), torch.float16)
+
+
+def test_gradients_without_the_queue(dev):
+    m = build(dev)
+    TM.DEFER_DW = False
+    try:
+        assert_same(step(m, True, torch.float16), step(m, False, torch.float16), torch.float16)
+    finally:
+        TM.DEFER_DW = True
+
+
+def test_saved_tensor_hooks_see_what_the_layer_keeps(dev):
+    m = build(dev)
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(t.shape), t.clone())[1], lambda t: t):
+        hooked = step(m, True, torch.float16)
+    assert len(seen) > 3 * 12
+    assert_same(hooked, step(m, True, torch.float16), torch.float16)
+
+
+def test_watched_or_replaced_modules_are_called(dev):
+    m = build(dev)
+    plain = step(m, False, torch.float16)
+    calls = []
+    hooks = [m.layer_list[0].input_layernorm.register_forward_hook(lambda *_: calls.append("ln")),
+             m.layer_list[1].attention.register_forward_pre_hook(lambda *_: calls.append("attention")),
+             m.layer_list[2].mlp.register_full_backward_hook(lambda *_: calls.append("mlp"))]
+    assert_same(step(m, True, torch.float16), plain, torch.float16)
+    assert sorted(calls) == ["attention", "ln", "mlp"]
+    for h in hooks:
+        h.remove()
+
+    class Doubled(TM.MLPBlock):
+        def forward(self, x):
+            return 2 * super().forward(x)
+
+    m.layer_list[1].mlp.__class__ = Doubled
+    assert not torch.equal(step(m, True, torch.float16)[0], plain[0])
+
+
+def test_graph_of_a_step_goes_with_its_outputs(dev):
+    """An output that the node held beside its saved tensors would keep the whole pass alive."""
+    m = build(dev)
+    step(m, True, torch.float16)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    for _ in range(3):
+        ids = torch.zeros((2, 64), dtype=torch.long, device=dev)
+        with torch.autocast("cuda", dtype=torch.float16):
+            out = m(ids, ids)
+        del out, ids
+    assert torch.cuda.memory_allocated() == before

@@ -1,0 +1,106 @@
+"""A product over matrices that lie apart against the product over their copy side by side, and a layer of which nothing is kept
+against the graph nodes it stands for: the same bits."""
+import pytest
+import torch
+
+import tritonformer_amd.transformer as TM
+from tests.test_layer import build
+from tritonformer_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,each,K,count", [(1, 64, 64, 3), (65, 128, 192, 3), (128, 1024, 1024, 3), (300, 256, 2048, 2), (960, 768, 768, 3),
+                                            (8192, 256, 64, 3), (64, 192, 4096, 1), (700, 64, 128, 3)])
+def test_side_by_side_gives_the_bits_of_the_copy(M, each, K, count, dtype, dev):
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(11)
+    a = torch.randn(M, K, generator=g).to(dtype).to(dev)
+    parts = [(torch.randn(K, each, generator=g) / K ** 0.5).to(dtype).to(dev) for _ in range(count)]
+    n, code, st = each * count, _lib.dtype_code(dtype), _lib.stream_ptr()
+    nb = lib.tf_gemm_workspace_bytes(0, 1, M, n, K)
+    ws = torch.empty(max(nb, 16), dtype=torch.uint8, device=dev)
+    whole, apart = torch.empty(M, n, dtype=dtype, device=dev), torch.full((M, n), float("nan"), dtype=dtype, device=dev)
+    copy = torch.cat(parts, 1)
+    _lib.check(lib.tf_gemm(st, code, 0, 1, M, n, K, a.data_ptr(), K, copy.data_ptr(), n, whole.data_ptr(), n, None, 0, ws.data_ptr(), nb))
+    ptrs = (_lib._vp * count)(*[p.data_ptr() for p in parts])
+    rc = lib.tf_gemm_side_by_side(st, code, M, each, count, K, a.data_ptr(), K, ptrs, each, apart.data_ptr(), n, ws.data_ptr(), nb)
+    if rc == -4:  # tiles wider than a part
+        assert each % 64 or M > 256
+        return
+    _lib.check(rc)
+    assert torch.equal(apart, whole)
+
+
+def test_side_by_side_refuses_what_it_does_not_serve(dev):
+    lib = _lib.load()
+    a = torch.randn(128, 128, device=dev).half()
+    w = torch.randn(128, 128, device=dev).half()
+    c = torch.empty(128, 384, device=dev).half()
+    st = _lib.stream_ptr()
+
+    def run(each=128, K=128, off=0, count=3, ldb=128):
+        ptrs = (_lib._vp * 3)(w.data_ptr() + off, w.data_ptr(), w.data_ptr())
+        return lib.tf_gemm_side_by_side(st, 0, 128, each, count, K, a.data_ptr(), 128, ptrs, ldb, c.data_ptr(), 384, None, 0)
+
+    assert run() == 0
+    assert run(each=96) == run(each=60) == run(K=96) == run(off=2) == run(ldb=64) == -4
+    assert run(count=4) == run(count=0) == -1
+
+
+@pytest.mark.parametrize("bias,alibi", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,heads", [(128, 2), (96, 3), (256, 4)])
+def test_a_layer_in_one_call_gives_the_bits_of_its_nodes(bias, alibi, dtype, d, heads, dev, monkeypatch):
+    m = build(dev, bias, alibi, dtype, d=d, heads=heads)
+    ids = torch.arange(128, device=dev).view(2, 64) * 3
+    calls = []
+    native = _lib.launch().layer
+
+    class Counting:
+        def __getattr__(self, name):
+            if name == "layer":
+                return lambda *a: (calls.append(1), native(*a))[1]
+            return getattr(_lib.launch(), name)
+
+    monkeypatch.setattr(TM, "launch", lambda: Counting())
+    with torch.no_grad():
+        one = m(ids, None)
+        assert len(calls) == 3
+        TM.FUSE_LAYER = False
+        try:
+            nodes = m(ids, None)
+        finally:
+            TM.FUSE_LAYER = True
+    assert torch.equal(one, nodes) and len(calls) == 3
+    assert torch.equal(m(ids, None).detach(), nodes) and len(calls) == 3     # a graph is built: its nodes run
+    with torch.inference_mode():
+        assert torch.equal(m(ids, None), nodes)
+
+
+def test_a_layer_in_one_call_leaves_other_forms_to_the_nodes(dev):
+    """Tangents, traces, autocast and weights of another type: the graph nodes decide."""
+    m = build(dev, param_dtype=torch.float16)
+    ids = torch.arange(64, device=dev)[None]
+    with torch.no_grad():
+        plain = m(ids, None)
+        layer = m.layer_list[0]
+        x = torch.randn(1, 64, 128, device=dev).half()
+        args = (x, None, layer.input_layernorm.weight, layer.input_layernorm.bias, 1e-5,
+                [getattr(layer.attention, n).weight for n in ("q_proj", "k_proj", "v_proj", "out_proj")], 2, None,
+                layer.post_attention_layernorm.weight, layer.post_attention_layernorm.bias, 1e-5,
+                layer.mlp.dense_h_to_4h.weight, None, layer.mlp.dense_4h_to_h.weight, None)
+        call = _lib.launch().layer
+        assert call(*args) is not None
+        for i, other in ((0, x.float()), (0, x.transpose(1, 2)), (0, x[0]), (1, x[:, :32]), (2, args[2][:64]), (6, 3), (11, args[13]),
+                         (12, torch.zeros(128, device=dev)), (7, torch.zeros(2, 8, 8, device=dev).half())):
+            assert call(*args[:i], other, *args[i + 1:]) is None, i
+        import torch.autograd.forward_ad as fwAD
+
+        with fwAD.dual_level():
+            assert call(fwAD.make_dual(x, torch.ones_like(x)), *args[1:]) is None
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert torch.equal(m(ids, None), plain)
+        traced = torch.jit.trace(lambda t: t * (1.0 if call(t, *args[1:]) is None else 0.0), (x,), check_trace=False)
+        assert torch.equal(traced(x), x)

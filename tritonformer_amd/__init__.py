@@ -11,6 +11,7 @@ from .crossentropy import CrossEntropyLoss as cross_entropy_loss
 from .crossentropy import LMHeadLoss as lm_head_loss
 from .crossentropy import ShiftedCrossEntropyLoss as shifted_cross_entropy_loss
 from .embedding import EmbeddingSum as embedding_sum
+from .layer import DecoderLayer as decoder_layer
 from .layernorm import AddLayerNorm as add_layer_norm
 from .layernorm import LayerNorm as layer_norm
 from .linear import LinearBias as linear_bias

@@ -73,6 +73,11 @@ struct GemmParams {
   // to the fp32 sums before bias / rounding.  A pointer, so that a value computed on the GPU (the
   // upstream gradient of a mean loss) needs no host round trip.
   const float* alpha;
+  // B as up to three matrices side by side (K-minor, leading dimension ldb): columns [i * b_each, (i + 1) * b_each) are
+  // those of B, B1, B2; b_each is a multiple of the tile's width, so a tile reads one of them.  0: B alone.
+  const void* B1 = nullptr;
+  const void* B2 = nullptr;
+  int b_each = 0;
 };
 
 // Round-robin XCD dispatch -> compact per-XCD ranges, then grouped raster.
@@ -521,9 +526,17 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
 
   uint32_t oa[PA::PER_WAVE], ob[PB::PER_WAVE];
   PA::init(oa, p.lda, m0, p.M, wave, lane);
-  PB::init(ob, p.ldb, n0, p.N, wave, lane);
+  const T* B = (const T*)p.B;
+  int nb = n0, nend = p.N;  // the tile's columns in B
+  if (!B_KMAJOR && p.b_each) {
+    const int i = n0 / p.b_each;
+    B = (const T*)(i == 0 ? p.B : i == 1 ? p.B1 : p.B2);
+    nb = n0 - i * p.b_each;
+    nend = p.b_each;
+  }
+  PB::init(ob, p.ldb, nb, nend, wave, lane);
   const char* pa = PA::origin((const T*)p.A, p.lda, m0, kbeg);
-  const char* pb = PB::origin((const T*)p.B, p.ldb, n0, kbeg);
+  const char* pb = PB::origin(B, p.ldb, nb, kbeg);
   const int64_t sa = PA::stride(p.lda), sb = PB::stride(p.ldb);
   const uint32_t la = PA::frag_lane(wm * WTM, lane), lb = PA::BYTES + PB::frag_lane(wn * WTN, lane);
 
@@ -1660,6 +1673,41 @@ extern "C" int tf_gemm_scaled(void* stream, int dtype, int out_dtype, int layout
   if (!alpha) return TF_EINVAL;
   return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, N, K, A, lda, B, ldb, C, ldc, 0, 0, nullptr, 0,
                     nullptr, 0, workspace, workspace_bytes, nullptr, nullptr, 0, kNoForce, alpha);
+}
+
+extern "C" int tf_gemm_side_by_side(void* stream, int dtype, int64_t M, int64_t each, int count, int64_t K, const void* A,
+                                    int64_t lda, const void* const* B, int64_t ldb, void* C, int64_t ldc, void* workspace,
+                                    int64_t workspace_bytes) {
+  if (!A || !B || !C || M <= 0 || each <= 0 || K <= 0 || count < 1 || count > 3) return TF_EINVAL;
+  if (M > 0x7fffff00 || each > 0x7fffff00 / 3 || K > 0x7fffff00) return TF_EINVAL;
+  if (dtype != TF_F16 && dtype != TF_BF16) return TF_EDTYPE;
+  const int64_t N = each * count;
+  bool vec = lda <= kMaxPitch && ldb <= kMaxPitch && aligned16(A) && aligned16(C) && K % 8 == 0 && each % 8 == 0 && lda % 8 == 0 &&
+             ldb % 8 == 0 && ldc % 8 == 0;
+  for (int i = 0; i < count; ++i) {
+    if (!B[i]) return TF_EINVAL;
+    vec = vec && aligned16(B[i]);
+  }
+  if (lda < K || ldb < each || ldc < N || !vec) return TF_ESHAPE;
+  const Route rt = route(M, N, K, true, kRoutePlain);
+  const GemmPlan& pl = rt.plan;
+  if (rt.tail > 0 || !kCfgs[pl.cfg].dma || K % pl.bk != 0 || each % pl.bn != 0) return TF_ESHAPE;
+  const int64_t need = plan_need(pl, M, N);
+  if (need > 0 && (!workspace || workspace_bytes < need)) return TF_EWORKSPACE;
+  if (need > 0 && !aligned16(workspace)) return TF_EALIGN;
+  if ((int64_t)pl.tiles_m * pl.tiles_n * pl.splits > 0x7fffffff) return TF_EINVAL;
+  GemmParams p = {};
+  p.A = A; p.B = B[0]; p.C = C; p.partial = (float*)workspace;
+  p.B1 = B[count > 1 ? 1 : 0]; p.B2 = B[count > 2 ? 2 : 0]; p.b_each = (int)each;
+  p.M = (int)M; p.N = (int)N; p.K = (int)K;
+  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+  p.splits = pl.splits; p.k_per_split = pl.k_per_split;
+  p.tiles_m = pl.tiles_m; p.tiles_n = pl.tiles_n;
+  p.xcds = device_shape().xcds;
+  p.chunk_n = (int)N;
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == TF_F16) return gemm_dispatch<f16>(st, TF_OP_KMAJOR, TF_OP_KMINOR, true, pl, p);
+  return gemm_dispatch<bf16>(st, TF_OP_KMAJOR, TF_OP_KMINOR, true, pl, p);
 }
 
 // Diagnostic twin of tf_gemm_out_chunked: the same call with a tile configuration, a contraction

@@ -702,6 +702,98 @@ TF_FN(mlp, 7) {
   return t;
 }
 
+// No operand carries a tangent of forward-mode differentiation and no trace records the calls: for functions that stand in
+// for graph nodes.
+bool untraced(std::initializer_list<const Tensor*> ts) {
+  if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer)) return false;
+  for (const Tensor* t : ts)
+    if (t && t->_fw_grad(0).defined()) return false;
+  return true;
+}
+
+// layer(x (B, S, d), pending | None, g1, b1, eps1, [wq, wk, wv, wo], heads, bias | None, g2, b2, eps2, w1, c1 | None, w2,
+// c2 | None) -> (x + pending + attention branch, MLP branch): a decoder layer of which nothing is kept for a backward pass,
+// weights and biases in x's dtype.  The launches of the Functions in their order, but for the copy that lays the projections'
+// weights side by side where the product reads them where they are.
+TF_FN(layer, 15) {
+  const Tensor *x = dense(args.a[0]), *pending = nullptr, *bias, *ln[4] = {dense(args.a[2]), dense(args.a[3]), dense(args.a[8]), dense(args.a[9])};
+  if (!x || x->dim() != 3 || !is16(*x) || !aligned(*x) || !PyList_Check(args.a[5]) || PyList_GET_SIZE(args.a[5]) != 4) Py_RETURN_NONE;
+  const at::ScalarType type = x->scalar_type();
+  const int64_t b = x->size(0), s = x->size(1), d = x->size(2), m = b * s, nh = PyLong_AsLongLong(args.a[6]);
+  if (nh == -1 && PyErr_Occurred()) return nullptr;
+  if (nh <= 0 || d % nh || !attn_sizes(s, d / nh) || !attn_bias(args.a[7], *x, nh, s, &bias)) Py_RETURN_NONE;
+  if (args.a[1] != Py_None) {
+    pending = dense(args.a[1]);
+    if (!pending || pending->sizes() != x->sizes() || pending->scalar_type() != type) Py_RETURN_NONE;
+  }
+  for (int i = 0; i < 4; ++i)
+    if (!ln_param(ln[i], *x) || ln[i]->scalar_type() != ln[i ^ 1]->scalar_type()) Py_RETURN_NONE;
+  auto weight = [&](PyObject* o, int64_t rows, int64_t cols) {
+    const Tensor* t = dense(o);
+    return t && t->dim() == 2 && (rows < 0 || t->size(0) == rows) && (cols < 0 || t->size(1) == cols) && t->scalar_type() == type ? t : nullptr;
+  };
+  const Tensor* w[4];
+  for (int i = 0; i < 4; ++i)
+    if (!(w[i] = weight(PyList_GET_ITEM(args.a[5], i), d, d))) Py_RETURN_NONE;
+  const Tensor *w1 = weight(args.a[11], d, -1), *w2 = weight(args.a[13], -1, d), *c[2] = {nullptr, nullptr};
+  if (!w1 || !w2 || w2->size(0) != w1->size(1)) Py_RETURN_NONE;
+  const int64_t f = w1->size(1), hd = d / nh;
+  for (int i = 0; i < 2; ++i) {
+    if (args.a[12 + 2 * i] == Py_None) continue;
+    c[i] = dense(args.a[12 + 2 * i]);
+    if (!c[i] || c[i]->dim() != 1 || c[i]->size(0) != (i ? d : f) || c[i]->scalar_type() != type) Py_RETURN_NONE;
+  }
+  if (!untraced({x, pending, ln[0], ln[1], ln[2], ln[3], w[0], w[1], w[2], w[3], w1, c[0], w2, c[1], bias})) Py_RETURN_NONE;
+  const double eps1 = PyFloat_AsDouble(args.a[4]), eps2 = PyFloat_AsDouble(args.a[10]);
+  if (PyErr_Occurred()) return nullptr;
+
+  const int dt = code(type);
+  Tensor stats = make({2, m}, *x, at::kFloat), normed = make(x->sizes(), *x), qkv = make({b, s, 3, nh, hd}, *x),
+         attn = make({b, s, d}, *x), lse = make({b, nh, s}, *x, at::kFloat), branch = make({b, s, d}, *x),
+         stream_out = make(x->sizes(), *x), hidden = make({b, s, f}, *x), out = make({b, s, d}, *x);
+  Tensor total = pending ? make(x->sizes(), *x) : *x;
+  float *mean = stats.data_ptr<float>(), *rstd = mean + m;
+  auto add_norm = [&](const Tensor& a, const Tensor& r, Tensor& sum, const Tensor* const* p, double eps) {
+    return call([&] {
+      return tf_add_layernorm_fwd(stream(), dt, code(p[0]->scalar_type()), m, d, a.data_ptr(), d, r.data_ptr(), d, sum.data_ptr(), d,
+                                  p[0]->data_ptr(), p[1]->data_ptr(), (float)eps, normed.data_ptr(), d, mean, rstd);
+    });
+  };
+  if (pending) {
+    if (!add_norm(*x, *pending, total, ln, eps1)) return nullptr;
+  } else if (!call([&] {
+               return tf_layernorm_fwd(stream(), dt, code(ln[0]->scalar_type()), m, d, x->data_ptr(), d, ln[0]->data_ptr(),
+                                       ln[1]->data_ptr(), (float)eps1, normed.data_ptr(), d, mean, rstd);
+             })) {
+    return nullptr;
+  }
+  const int64_t bytes = tf_gemm_workspace_bytes(TF_OP_KMAJOR, TF_OP_KMINOR, m, 3 * d, d);
+  Tensor ws = scratch(bytes, *x);
+  const void* parts[3] = {w[0]->data_ptr(), w[1]->data_ptr(), w[2]->data_ptr()};
+  int rc = TF_OK;
+  if (!call([&] {
+        return tf_gemm_side_by_side(stream(), dt, m, d, 3, d, normed.data_ptr(), d, parts, d, qkv.data_ptr(), 3 * d, ptr(ws), bytes);
+      }, TF_ESHAPE, &rc))
+    return nullptr;
+  if (rc == TF_ESHAPE) {
+    Tensor packed;
+    if (!pack(w, 3, d, d, type, &packed)) {
+      if (PyErr_Occurred()) return nullptr;
+      Py_RETURN_NONE;
+    }
+    if (!product(*x, TF_OP_KMINOR, m, 3 * d, d, normed.data_ptr(), packed.data_ptr(), 3 * d, qkv.data_ptr())) return nullptr;
+  }
+  const char* q = static_cast<const char*>(qkv.data_ptr());
+  if (!attn_forward(dt, b, nh, s, hd, q, q + 2 * d, q + 4 * d, attn.data_ptr(), {s * 3 * d, hd, 3 * d}, {s * d, hd, d},
+                    lse.data_ptr<float>(), bias) ||
+      !product(*x, TF_OP_KMINOR, m, d, d, attn.data_ptr(), w[3]->data_ptr(), d, branch.data_ptr()) ||
+      !add_norm(total, branch, stream_out, ln + 2, eps2) ||
+      !product(*x, TF_OP_KMINOR, m, f, d, normed.data_ptr(), w1->data_ptr(), f, hidden.data_ptr(), c[0], 1) ||
+      !product(*x, TF_OP_KMINOR, m, d, f, hidden.data_ptr(), w2->data_ptr(), d, out.data_ptr(), c[1]))
+    return nullptr;
+  return tuple_of({&stream_out, &out});
+}
+
 // ------------------------------------------------------------------------------------------ optimizer
 // adamw([params], [grads], [first moments], [second moments], [16-bit copies] | None, dtype of the copies, lr, beta1, beta2,
 // eps, weight decay, step): dense float32 tensors of one size each (the copies 16-bit); nothing is returned but True
@@ -800,7 +892,7 @@ PyMethodDef methods[] = {
     TF_ENTRY(linear), TF_ENTRY(linear_bits), TF_ENTRY(linear_masked), TF_ENTRY(weight_grad), TF_ENTRY(cast_pack),
     TF_ENTRY(attn_fwd), TF_ENTRY(attn_bwd), TF_ENTRY(attn_packed_fwd), TF_ENTRY(attn_packed_bwd), TF_ENTRY(layernorm),
     TF_ENTRY(layernorm_bwd), TF_ENTRY(softmax_fwd), TF_ENTRY(softmax_bwd), TF_ENTRY(relu_mask), TF_ENTRY(relu_mask_colsum),
-    TF_ENTRY(colsum), TF_ENTRY(attn_block), TF_ENTRY(attn_block_dqkv), TF_ENTRY(mlp), TF_ENTRY(pick), TF_ENTRY(adamw),
+    TF_ENTRY(colsum), TF_ENTRY(attn_block), TF_ENTRY(attn_block_dqkv), TF_ENTRY(mlp), TF_ENTRY(layer), TF_ENTRY(pick), TF_ENTRY(adamw),
     {"set_check", set_check, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

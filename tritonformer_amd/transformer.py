@@ -21,6 +21,7 @@ import torch.nn as nn
 from . import (
     add_layer_norm,
     attention_block,
+    decoder_layer,
     embedding_sum,
     fast_causal_attention,
     fast_causal_attention_qkvpacked,
@@ -32,6 +33,7 @@ from . import (
 )
 from . import _deferred
 from . import nn as tnn
+from ._lib import launch
 
 
 @dataclass(frozen=True)
@@ -88,6 +90,9 @@ FUSE_ATTN_BLOCK = True
 # kernel: no separate elementwise addition kernels.  False: `residual + hidden_states`
 # as the reference writes it (transformer.py:245-250).
 FUSE_ADD_LN = True
+# True (with the four above): a layer is one autograd node, where its attention and MLP modules are those of this file and nobody
+# watches them (hooks); False: four nodes.
+FUSE_LAYER = True
 # True: token gather, position gather, their addition and the rounding to the compute type are
 # one kernel, and the table gradients a chain-ordered scatter-add; False: two nn.Embedding
 # calls and an addition as in the reference (transformer.py:311-323).
@@ -206,12 +211,36 @@ class TransformerLayer(nn.Module):
         hidden_states = hidden_states + self.attention(self.input_layernorm(hidden_states), attn_bias)
         return hidden_states + self.mlp(self.post_attention_layernorm(hidden_states))
 
+    def _plain(self, first: bool) -> bool:
+        """True when calling the layer's modules would do nothing but run their own forward."""
+        if torch.nn.modules.module._has_any_global_hook():
+            return False
+        called = [(self.attention, CausalAttention), (self.mlp, MLPBlock)]
+        if first:
+            called.append((self.input_layernorm, tnn.LayerNorm))
+        return all(type(m) is kind and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+                   and m._compiled_call_impl is None and "forward" not in m.__dict__ for m, kind in called)
+
     def forward_deferred(self, hidden_states: torch.Tensor, pending: Optional[torch.Tensor],
                          attn_bias: Optional[torch.Tensor] = None):
         """Same block with the additions folded into the LayerNorms: takes the residual stream
         and a branch output not yet added to it (None for the first block), returns the stream
         after the attention residual and this block's MLP output, still to be added."""
         ln1, ln2 = self.input_layernorm, self.post_attention_layernorm
+        if FUSE_LAYER and FUSE_QKV and FUSE_ATTN_BLOCK and FUSE_MLP and self._plain(pending is None):
+            att, mlp = self.attention, self.mlp
+            up, down = mlp.dense_h_to_4h, mlp.dense_4h_to_h
+            if not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda"):
+                # nothing is kept for a backward pass: the layer's launches in one native call
+                result = launch().layer(hidden_states, pending, ln1.weight, ln1.bias, ln1.eps,
+                                        [att.q_proj.weight, att.k_proj.weight, att.v_proj.weight, att.out_proj.weight],
+                                        att.num_attention_heads, attn_bias, ln2.weight, ln2.bias, ln2.eps, up.weight, up.bias,
+                                        down.weight, down.bias)
+                if result is not None:
+                    return result
+            return decoder_layer.apply(hidden_states, pending, ln1.weight, ln1.bias, ln1.eps, att.q_proj.weight, att.k_proj.weight,
+                                       att.v_proj.weight, att.out_proj.weight, att.num_attention_heads, attn_bias, ln2.weight,
+                                       ln2.bias, ln2.eps, up.weight, up.bias, down.weight, down.bias)
         if pending is None:
             normed = ln1(hidden_states)
         else:
