@@ -403,7 +403,7 @@ def mfma_probe(dtype, device, iters=20000):
         "normal, std 0.02 (weights)": torch.randn(24576, generator=gen) * 0.02,
         "normal, std 1": torch.randn(24576, generator=gen),
     }
-    out = {"probe": f"v_mfma_f32_32x32x16 stream of one 256x256x64 GEMM step per trip, {wgs} workgroups x 8 waves, "
+    out = {"probe": f"v_mfma_f32_16x16x32 stream of one 256x256x64 GEMM step per trip, {wgs} workgroups x 8 waves, "
                     "no memory traffic", "dtype": str(dtype).replace("torch.", ""), "iters": iters, "tflops": {}}
     flops = lib.tf_diag_mfma_rate_flops(iters, wgs)
     for name, vals in kinds.items():
