@@ -197,3 +197,24 @@ def test_param_grads_of_many_layernorms_in_one_launch(pdtype, dev):
     assert out.shape == (70, 2, d) and out.dtype == pdtype
     for i, (da, db) in enumerate(want):
         assert torch.equal(out[i, 0], da) and torch.equal(out[i, 1], db), i
+
+
+@pytest.mark.parametrize("pdtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("d", [8, 512, 520, 1024, 1032, 2048, 2056, 4096, 4104, 8192])
+def test_few_rows_are_the_rows_of_many(d, pdtype, dev):
+    """One row per wave (of a workgroup above 2048 columns) in at most two workgroups per CU is a kernel of its own, with gamma and
+    beta requested beside x: the same operations, so the same bits as the same rows among many, at the ends of each number of chunks
+    per lane and on both sides of the bound."""
+    many = 4096 + 5 if d <= 2048 else 1024 + 5
+    bound = 2 * torch.cuda.get_device_properties(dev).multi_processor_count * (4 if d <= 2048 else 1)
+    g = torch.Generator().manual_seed(d)
+    x, r = ((1.0 + torch.randn(1, many, d, generator=g)).half().to(dev) for _ in range(2))
+    gamma, beta = (torch.randn(d, generator=g).to(pdtype).to(dev) for _ in range(2))
+    y = T.layer_norm.apply(x, gamma, beta, 1e-5)
+    total, z = T.add_layer_norm.apply(x, r, gamma, beta, 1e-5)
+    assert_close(y[:, :8], R.layer_norm(x[:, :8].cpu(), gamma.cpu(), beta.cpu(), 1e-5), name=f"y {d}")
+    for rows in (1, 5, bound, bound + 1):
+        few, few_r = x[:, :rows].contiguous(), r[:, :rows].contiguous()
+        assert torch.equal(T.layer_norm.apply(few, gamma, beta, 1e-5), y[:, :rows])
+        few_total, few_z = T.add_layer_norm.apply(few, few_r, gamma, beta, 1e-5)
+        assert torch.equal(few_total, total[:, :rows]) and torch.equal(few_z, z[:, :rows])

@@ -61,7 +61,7 @@ template <typename T, int NV, bool ANY, int FROM = NV / 2> struct RowEnds {
 // With ADD the normalised row is s = x + res, rounded to T and also written to `sum`
 // (the residual stream after the addition); the statistics are those of the rounded s,
 // so the result equals an addition kernel followed by the plain forward.
-template <typename T, typename TP, int NV, int WPR, bool ADD, bool ANY>
+template <typename T, typename TP, int NV, int WPR, bool ADD, bool ANY, bool ONCE>
 __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* __restrict__ x, int64_t ldx,
                                                    const T* __restrict__ res, int64_t ldres,
                                                    T* __restrict__ sum, int64_t ldsum,
@@ -98,6 +98,19 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
   };
   int64_t row = (int64_t)blockIdx.x * RPB + (WPR == 1 ? threadIdx.x >> 6 : 0);
   if (row < rows) fetch(row);
+  // ONCE: no wave has a second row.  gamma and beta are then requested here, behind x, and arrive beside it
+  float g[NV][8], b[NV][8];
+  auto params = [&](int i, int c) {
+    E::template load8<TP>(gamma, c, i, d, g[i]);
+    E::template load8<TP>(beta, c, i, d, b[i]);
+  };
+  if (ONCE) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = lane + i * LANES;
+      if (c < nchunk) params(i, c);
+    }
+  }
   for (; row < rows; row += stride) {
     float v[NV][8];
     float s = 0.f;
@@ -122,7 +135,7 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
         for (int e = 0; e < 8; ++e) v[i][e] = 0.f;
       }
     }
-    if (row + stride < rows) fetch(row + stride);
+    if (!ONCE && row + stride < rows) fetch(row + stride);
     const float mean = row_sum<WPR>(s, red, 0) / (float)d;
     float q = 0.f;
 #pragma unroll
@@ -149,14 +162,13 @@ __global__ __launch_bounds__(256) void ln_fwd_vec(int64_t rows, int d, const T* 
     for (int i = 0; i < NV; ++i) {
       const int c = lane + i * LANES;
       if (c < nchunk) {
-        // (gamma and beta are fetched per row: held in registers across the rows a wave walks they
+        // (gamma and beta are fetched per row where there are several: held in registers across the rows a wave walks they
         // cost a wave of occupancy, 98 against 86 VGPRs, and the kernel 0.5 us at d = 1024)
-        float g[8], b[8], o[8];
-        E::template load8<TP>(gamma, c, i, d, g);
-        E::template load8<TP>(beta, c, i, d, b);
+        if (!ONCE) params(i, c);
+        float o[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          o[e] = __builtin_fmaf((v[i][e] - mean) * rstd, g[e], b[e]);
+          o[e] = __builtin_fmaf((v[i][e] - mean) * rstd, g[i][e], b[i][e]);
           // the fp32 value is pinned before the rounding to 16 bits: left alone, the compiler turns
           // some of these into v_fma_mix*_f16 (one rounding straight to 16 bits) and others not,
           // differently per instantiation, and the two forms differ in one element in 50 000
@@ -798,12 +810,20 @@ static int ln_fwd_launch(hipStream_t st, int64_t rows, int64_t d, const void* x,
   const int64_t fill = (int64_t)device_shape().cus * 4;
   if (walkers < fill) walkers = ceil_div(rows, rpb) < fill ? ceil_div(rows, rpb) : fill;
   const dim3 wgrid((unsigned)walkers);
+  // One row per wave and at most two workgroups per CU: gamma and beta beside x, not after the statistics, in registers that
+  // nobody else needs.  A launch of few rows is a chain of latencies, and this was a whole one.  fp16 with a residual, fp32
+  // parameters, us: 128 x 768 3.75 -> 3.09, 128 x 1024 3.69 -> 3.10 (fp16 parameters 3.64 -> 3.21), 960 x 768 4.43 -> 3.83,
+  // 512 x 1536 5.21 -> 4.14, 128 x 2048 5.37 -> 3.95, 2048 x 2048 10.5 -> 8.9, 512 x 8192 10.7 -> 9.3.  With four workgroups
+  // per CU the registers cost waves: 4096 x 1024 9.05 -> 9.54, 4096 x 2048 16.1 -> 17.5, without a residual 9.3 -> 10.6.
+  // (One chunk per lane of 16-bit parameters, 960 x 256, 3.22 -> 3.29: as before.)
+  const bool once = vec && rows <= walkers * rpb && walkers <= fill / 2;
 #define LN_ARGS                                                                                                    \
   (rows, (int)d, (const T*)x, ldx, (const T*)res, ldres, (T*)sum, ldsum, (const TP*)gamma, (const TP*)beta, eps, (T*)y, \
    ldy, mean, rstd)
 #define LN_FWD(NV, WPR)                                                        \
-  if (vec) ln_fwd_vec<T, TP, NV, WPR, ADD, false><<<wgrid, block, 0, st>>>LN_ARGS; \
-  else ln_fwd_vec<T, TP, NV, WPR, ADD, true><<<wgrid, block, 0, st>>>LN_ARGS
+  if (once) ln_fwd_vec<T, TP, NV, WPR, ADD, false, (NV > 1 || sizeof(TP) == 4)><<<wgrid, block, 0, st>>>LN_ARGS; \
+  else if (vec) ln_fwd_vec<T, TP, NV, WPR, ADD, false, false><<<wgrid, block, 0, st>>>LN_ARGS; \
+  else ln_fwd_vec<T, TP, NV, WPR, ADD, true, false><<<wgrid, block, 0, st>>>LN_ARGS
   switch (nv * 10 + wpr) {
     case 11: LN_FWD(1, 1); break;
     case 21: LN_FWD(2, 1); break;
