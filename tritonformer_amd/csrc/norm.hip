@@ -814,7 +814,8 @@ static int ln_fwd_launch(hipStream_t st, int64_t rows, int64_t d, const void* x,
   // nobody else needs.  A launch of few rows is a chain of latencies, and this was a whole one.  fp16 with a residual, fp32
   // parameters, us: 128 x 768 3.75 -> 3.09, 128 x 1024 3.69 -> 3.10 (fp16 parameters 3.64 -> 3.21), 960 x 768 4.43 -> 3.83,
   // 512 x 1536 5.21 -> 4.14, 128 x 2048 5.37 -> 3.95, 2048 x 2048 10.5 -> 8.9, 512 x 8192 10.7 -> 9.3.  With four workgroups
-  // per CU the registers cost waves: 4096 x 1024 9.05 -> 9.54, 4096 x 2048 16.1 -> 17.5, without a residual 9.3 -> 10.6.
+  // per CU the registers cost waves: 4096 x 1024 9.05 -> 9.54, 4096 x 2048 16.1 -> 17.5, without a residual 9.3 -> 10.6.  (Both sides
+  // with the sums through the LDS crossbar; either is 0.3 shorter with wave_sum as it is.)
   // (One chunk per lane of 16-bit parameters, 960 x 256, 3.22 -> 3.29: as before.)
   const bool once = vec && rows <= walkers * rpb && walkers <= fill / 2;
 #define LN_ARGS                                                                                                    \
