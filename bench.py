@@ -208,7 +208,7 @@ NATIVE_CALLS = {
     "layernorm": lambda x, res, *rest: ("layernorm", (4.0 if res is None else 8.0) * x.numel()),
     "layernorm_bwd": lambda g, s, x, *rest: ("layernorm", (6.0 if s is None else 8.0) * x.numel()),
     # several launches in one call: the instrumented steps decline it, so that the block goes launch by launch
-    "attn_block": DECLINED, "attn_block_dqkv": DECLINED, "mlp": DECLINED,
+    "attn_block": DECLINED, "attn_block_dqkv": DECLINED, "mlp": DECLINED, "layer": DECLINED,
     "pick": None, "adamw": None, "cast_pack": None, "softmax_fwd": None, "softmax_bwd": None, "relu_mask": None, "relu_mask_colsum": None, "colsum": None,
 }
 
