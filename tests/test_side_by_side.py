@@ -5,7 +5,7 @@ import torch
 
 import tritonformer_amd.transformer as TM
 from tests.test_layer import build
-from tritonformer_amd import _lib
+from tritonformer_amd import _lib, linear
 
 pytestmark = pytest.mark.gpu
 
@@ -104,3 +104,32 @@ def test_a_layer_in_one_call_leaves_other_forms_to_the_nodes(dev):
             assert torch.equal(m(ids, None), plain)
         traced = torch.jit.trace(lambda t: t * (1.0 if call(t, *args[1:]) is None else 0.0), (x,), check_trace=False)
         assert torch.equal(traced(x), x)
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,heads,batch", [(2048, 16, 1), (2048, 16, 4), (1024, 16, 2)])
+def test_few_tokens_of_a_wide_layer_give_the_bits_of_the_nodes(d, heads, batch, bias, dtype, dev):
+    """The first MLP product of these (2048 wide): two slices of the contraction without sign bits, one with them."""
+    m = build(dev, bias, False, dtype, layers=2, d=d, heads=heads)
+    ids = (torch.arange(64 * batch, device=dev) * 7 % 512).view(batch, 64)
+    with torch.no_grad():
+        one = m(ids, None)
+        TM.FUSE_LAYER = False
+        try:
+            nodes = m(ids, None)
+        finally:
+            TM.FUSE_LAYER = True
+    assert torch.equal(one, nodes)
+    assert torch.equal(m(ids, None).detach(), nodes)
+
+
+def test_products_without_sign_bits_are_left_to_the_nodes(dev, monkeypatch):
+    """With RELU_BITS off the nodes take the product that may split its contraction."""
+    m = build(dev, False, False, torch.float16, layers=2, d=2048, heads=16)
+    ids = torch.arange(64, device=dev)[None]
+    monkeypatch.setattr(linear, "RELU_BITS", False)
+    with torch.no_grad():
+        one = m(ids, None)
+        monkeypatch.setattr(TM, "FUSE_LAYER", False)
+        assert torch.equal(one, m(ids, None))

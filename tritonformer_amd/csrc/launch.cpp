@@ -644,6 +644,28 @@ TF_FN(attn_block_dqkv, 6) {
   return THPVariable_Wrap(dqkv);
 }
 
+// hidden (m, f) = relu(x w + bias); with `with_bits` as the product that writes its sign bits, which go to `bits`, where one serves
+// the shape.  That product splits no contraction: whoever is to give the bits of the other's results takes it too.
+bool up_projection(const Tensor& like, int64_t m, int64_t f, int64_t k, const void* x, const void* w, const Tensor* bias, void* hidden,
+                   bool with_bits, Tensor* bits) {
+  int rc = TF_ESHAPE;
+  if (with_bits && f % 8 == 0) {
+    *bits = make({m, f / 8}, like, at::kByte);
+    const int dt = code(like.scalar_type());
+    if (!call([&] {
+          if (bias && bias->scalar_type() == at::kFloat)
+            return tf_gemm_master_bias(stream(), dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x, k, w, f, hidden, f,
+                                       bias->data_ptr<float>(), 1, bits->data_ptr(), f / 8, nullptr, 0);
+          return tf_gemm_relu_bits(stream(), dt, dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x, k, w, f, hidden, f,
+                                   bias ? bias->data_ptr() : nullptr, bits->data_ptr(), nullptr, f / 8);
+        }, TF_ESHAPE, &rc))
+      return false;
+  }
+  if (rc == TF_OK) return true;
+  *bits = Tensor();
+  return product(like, TF_OP_KMINOR, m, f, k, x, w, f, hidden, bias, 1);
+}
+
 // mlp(x (B, S, k), w1 (k, f), b1 | None, w2 (f, n), b2 | None, with_bits, master_biases: fp32 ones are taken as well)
 //   -> (relu(x w1 + b1) w2 + b2, hidden, sign bits | None, w1 and w2 in x's dtype)
 TF_FN(mlp, 7) {
@@ -676,22 +698,9 @@ TF_FN(mlp, 7) {
     c1 = both.narrow(1, 0, each).view({k, f}), c2 = both.narrow(1, each, each).view({f, n});
   }
   Tensor hidden = make({x->size(0), x->size(1), f}, *x), out = make({x->size(0), x->size(1), n}, *x), bits;
-  int rc = TF_ESHAPE;
-  if (args.a[5] == Py_True && f % 8 == 0) {
-    bits = make({m, f / 8}, *x, at::kByte);
-    const int dt = code(x->scalar_type());
-    if (!call([&] {
-          if (b1 && b1->scalar_type() == at::kFloat)
-            return tf_gemm_master_bias(stream(), dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x->data_ptr(), k, c1.data_ptr(), f,
-                                       hidden.data_ptr(), f, b1->data_ptr<float>(), 1, bits.data_ptr(), f / 8, nullptr, 0);
-          return tf_gemm_relu_bits(stream(), dt, dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x->data_ptr(), k, c1.data_ptr(), f,
-                                   hidden.data_ptr(), f, b1 ? b1->data_ptr() : nullptr, bits.data_ptr(), nullptr, f / 8);
-        }, TF_ESHAPE, &rc))
-      return nullptr;
-  }
-  if (rc != TF_OK && !product(*x, TF_OP_KMINOR, m, f, k, x->data_ptr(), c1.data_ptr(), f, hidden.data_ptr(), b1, 1)) return nullptr;
+  if (!up_projection(*x, m, f, k, x->data_ptr(), c1.data_ptr(), b1, hidden.data_ptr(), args.a[5] == Py_True, &bits)) return nullptr;
   if (!product(*x, TF_OP_KMINOR, m, n, f, hidden.data_ptr(), c2.data_ptr(), n, out.data_ptr(), b2)) return nullptr;
-  if (rc == TF_OK) return tuple_of({&out, &hidden, &bits, &c1, &c2});
+  if (bits.defined()) return tuple_of({&out, &hidden, &bits, &c1, &c2});
   PyObject* t = tuple_of({&out, &hidden, &hidden, &c1, &c2});
   if (t) {
     Py_INCREF(Py_None);
@@ -713,8 +722,9 @@ bool untraced(std::initializer_list<const Tensor*> ts) {
 
 // layer(x (B, S, d), pending | None, g1, b1, eps1, [wq, wk, wv, wo], heads, bias | None, g2, b2, eps2, w1, c1 | None, w2,
 // c2 | None) -> (x + pending + attention branch, MLP branch): a decoder layer of which nothing is kept for a backward pass,
-// weights and biases in x's dtype.  The launches of the Functions in their order, but for the copy that lays the projections'
-// weights side by side where the product reads them where they are.
+// weights and biases in x's dtype.  The launches of the Functions in their order, the sign bits of the first MLP product
+// included (a product without them may split its contraction: other bits), but for the copy that lays the projections' weights
+// side by side where the product reads them where they are.
 TF_FN(layer, 15) {
   const Tensor *x = dense(args.a[0]), *pending = nullptr, *bias, *ln[4] = {dense(args.a[2]), dense(args.a[3]), dense(args.a[8]), dense(args.a[9])};
   if (!x || x->dim() != 3 || !is16(*x) || !aligned(*x) || !PyList_Check(args.a[5]) || PyList_GET_SIZE(args.a[5]) != 4) Py_RETURN_NONE;
@@ -750,7 +760,7 @@ TF_FN(layer, 15) {
   const int dt = code(type);
   Tensor stats = make({2, m}, *x, at::kFloat), normed = make(x->sizes(), *x), qkv = make({b, s, 3, nh, hd}, *x),
          attn = make({b, s, d}, *x), lse = make({b, nh, s}, *x, at::kFloat), branch = make({b, s, d}, *x),
-         stream_out = make(x->sizes(), *x), hidden = make({b, s, f}, *x), out = make({b, s, d}, *x);
+         stream_out = make(x->sizes(), *x), hidden = make({b, s, f}, *x), out = make({b, s, d}, *x), bits;
   Tensor total = pending ? make(x->sizes(), *x) : *x;
   float *mean = stats.data_ptr<float>(), *rstd = mean + m;
   auto add_norm = [&](const Tensor& a, const Tensor& r, Tensor& sum, const Tensor* const* p, double eps) {
@@ -788,7 +798,7 @@ TF_FN(layer, 15) {
                     lse.data_ptr<float>(), bias) ||
       !product(*x, TF_OP_KMINOR, m, d, d, attn.data_ptr(), w[3]->data_ptr(), d, branch.data_ptr()) ||
       !add_norm(total, branch, stream_out, ln + 2, eps2) ||
-      !product(*x, TF_OP_KMINOR, m, f, d, normed.data_ptr(), w1->data_ptr(), f, hidden.data_ptr(), c[0], 1) ||
+      !up_projection(*x, m, f, d, normed.data_ptr(), w1->data_ptr(), c[0], hidden.data_ptr(), true, &bits) ||
       !product(*x, TF_OP_KMINOR, m, d, f, hidden.data_ptr(), w2->data_ptr(), d, out.data_ptr(), c[1]))
     return nullptr;
   return tuple_of({&stream_out, &out});

@@ -31,7 +31,7 @@ from . import (
     mlp_fused_relu,
     shifted_cross_entropy_loss,
 )
-from . import _deferred
+from . import _deferred, linear
 from . import nn as tnn
 from ._lib import launch
 
@@ -230,7 +230,7 @@ class TransformerLayer(nn.Module):
         if FUSE_LAYER and FUSE_QKV and FUSE_ATTN_BLOCK and FUSE_MLP and self._plain(pending is None):
             att, mlp = self.attention, self.mlp
             up, down = mlp.dense_h_to_4h, mlp.dense_4h_to_h
-            if not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda"):
+            if not torch.is_grad_enabled() and not torch.is_autocast_enabled("cuda") and linear.RELU_BITS:
                 # nothing is kept for a backward pass: the layer's launches in one native call
                 result = launch().layer(hidden_states, pending, ln1.weight, ln1.bias, ln1.eps,
                                         [att.q_proj.weight, att.k_proj.weight, att.v_proj.weight, att.out_proj.weight],
