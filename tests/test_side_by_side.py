@@ -133,3 +133,20 @@ def test_products_without_sign_bits_are_left_to_the_nodes(dev, monkeypatch):
         one = m(ids, None)
         monkeypatch.setattr(TM, "FUSE_LAYER", False)
         assert torch.equal(one, m(ids, None))
+
+
+@pytest.mark.parametrize("first", [False, True])
+def test_a_layer_in_one_call_holds_no_more_than_its_nodes(first, dev, monkeypatch):
+    m = build(dev, False, False, torch.float16, layers=1, d=256, heads=4)
+    x, pending = torch.randn(2, 128, 64, 256, device=dev).half().unbind(0)
+    peaks = []
+    for fused in (True, False):
+        monkeypatch.setattr(TM, "FUSE_LAYER", fused)
+        for _ in range(2):
+            with torch.no_grad():
+                torch.cuda.reset_peak_memory_stats()
+                before = torch.cuda.memory_allocated()
+                out = m.layer_list[0].forward_deferred(x, None if first else pending)
+            peaks.append(torch.cuda.max_memory_allocated() - before)
+            del out
+    assert peaks[1] <= peaks[3], peaks

@@ -758,10 +758,9 @@ TF_FN(layer, 15) {
   if (PyErr_Occurred()) return nullptr;
 
   const int dt = code(type);
-  Tensor stats = make({2, m}, *x, at::kFloat), normed = make(x->sizes(), *x), qkv = make({b, s, 3, nh, hd}, *x),
-         attn = make({b, s, d}, *x), lse = make({b, nh, s}, *x, at::kFloat), branch = make({b, s, d}, *x),
-         stream_out = make(x->sizes(), *x), hidden = make({b, s, f}, *x), out = make({b, s, d}, *x), bits;
-  Tensor total = pending ? make(x->sizes(), *x) : *x;
+  // each made where it is first written and let go behind its last reader, as between the nodes: a long batch is bound by the
+  // memory that lives at once
+  Tensor stats = make({2, m}, *x, at::kFloat), normed = make(x->sizes(), *x), total = pending ? make(x->sizes(), *x) : *x;
   float *mean = stats.data_ptr<float>(), *rstd = mean + m;
   auto add_norm = [&](const Tensor& a, const Tensor& r, Tensor& sum, const Tensor* const* p, double eps) {
     return call([&] {
@@ -777,30 +776,44 @@ TF_FN(layer, 15) {
              })) {
     return nullptr;
   }
-  const int64_t bytes = tf_gemm_workspace_bytes(TF_OP_KMAJOR, TF_OP_KMINOR, m, 3 * d, d);
-  Tensor ws = scratch(bytes, *x);
-  const void* parts[3] = {w[0]->data_ptr(), w[1]->data_ptr(), w[2]->data_ptr()};
-  int rc = TF_OK;
-  if (!call([&] {
-        return tf_gemm_side_by_side(stream(), dt, m, d, 3, d, normed.data_ptr(), d, parts, d, qkv.data_ptr(), 3 * d, ptr(ws), bytes);
-      }, TF_ESHAPE, &rc))
-    return nullptr;
-  if (rc == TF_ESHAPE) {
-    Tensor packed;
-    if (!pack(w, 3, d, d, type, &packed)) {
-      if (PyErr_Occurred()) return nullptr;
-      Py_RETURN_NONE;
+  Tensor branch;
+  {
+    Tensor qkv = make({b, s, 3, nh, hd}, *x);
+    {
+      const int64_t bytes = tf_gemm_workspace_bytes(TF_OP_KMAJOR, TF_OP_KMINOR, m, 3 * d, d);
+      Tensor ws = scratch(bytes, *x), packed;
+      const void* parts[3] = {w[0]->data_ptr(), w[1]->data_ptr(), w[2]->data_ptr()};
+      int rc = TF_OK;
+      if (!call([&] {
+            return tf_gemm_side_by_side(stream(), dt, m, d, 3, d, normed.data_ptr(), d, parts, d, qkv.data_ptr(), 3 * d, ptr(ws), bytes);
+          }, TF_ESHAPE, &rc))
+        return nullptr;
+      if (rc == TF_ESHAPE) {
+        ws = Tensor();
+        if (!pack(w, 3, d, d, type, &packed)) {
+          if (PyErr_Occurred()) return nullptr;
+          Py_RETURN_NONE;
+        }
+        if (!product(*x, TF_OP_KMINOR, m, 3 * d, d, normed.data_ptr(), packed.data_ptr(), 3 * d, qkv.data_ptr())) return nullptr;
+      }
     }
-    if (!product(*x, TF_OP_KMINOR, m, 3 * d, d, normed.data_ptr(), packed.data_ptr(), 3 * d, qkv.data_ptr())) return nullptr;
+    Tensor attn = make({b, s, d}, *x), lse = make({b, nh, s}, *x, at::kFloat);
+    const char* q = static_cast<const char*>(qkv.data_ptr());
+    if (!attn_forward(dt, b, nh, s, hd, q, q + 2 * d, q + 4 * d, attn.data_ptr(), {s * 3 * d, hd, 3 * d}, {s * d, hd, d},
+                      lse.data_ptr<float>(), bias))
+      return nullptr;
+    qkv = lse = Tensor();
+    branch = make({b, s, d}, *x);
+    if (!product(*x, TF_OP_KMINOR, m, d, d, attn.data_ptr(), w[3]->data_ptr(), d, branch.data_ptr())) return nullptr;
   }
-  const char* q = static_cast<const char*>(qkv.data_ptr());
-  if (!attn_forward(dt, b, nh, s, hd, q, q + 2 * d, q + 4 * d, attn.data_ptr(), {s * 3 * d, hd, 3 * d}, {s * d, hd, d},
-                    lse.data_ptr<float>(), bias) ||
-      !product(*x, TF_OP_KMINOR, m, d, d, attn.data_ptr(), w[3]->data_ptr(), d, branch.data_ptr()) ||
-      !add_norm(total, branch, stream_out, ln + 2, eps2) ||
-      !up_projection(*x, m, f, d, normed.data_ptr(), w1->data_ptr(), c[0], hidden.data_ptr(), true, &bits) ||
-      !product(*x, TF_OP_KMINOR, m, d, f, hidden.data_ptr(), w2->data_ptr(), d, out.data_ptr(), c[1]))
-    return nullptr;
+  Tensor stream_out = make(x->sizes(), *x);
+  if (!add_norm(total, branch, stream_out, ln + 2, eps2)) return nullptr;
+  total = branch = Tensor();
+  Tensor hidden = make({b, s, f}, *x), out, bits;
+  if (!up_projection(*x, m, f, d, normed.data_ptr(), w1->data_ptr(), c[0], hidden.data_ptr(), true, &bits)) return nullptr;
+  normed = bits = Tensor();
+  out = make({b, s, d}, *x);
+  if (!product(*x, TF_OP_KMINOR, m, d, f, hidden.data_ptr(), w2->data_ptr(), d, out.data_ptr(), c[1])) return nullptr;
   return tuple_of({&stream_out, &out});
 }
 
