@@ -117,6 +117,23 @@ def test_watched_or_replaced_modules_are_called(dev):
     assert not torch.equal(step(m, True, torch.float16)[0], plain[0])
 
 
+@pytest.mark.parametrize("kind,name,calls_per_pass", [(TM.CausalAttention, "forward", 3), (TM.MLPBlock, "forward", 3), (TM.tnn.LayerNorm, "forward", 1),
+                                                      (torch.nn.Module, "__call__", 8)])
+def test_classes_patched_by_the_caller_are_called(kind, name, calls_per_pass, dev, monkeypatch):
+    m = build(dev)
+    ids = torch.zeros((2, 64), dtype=torch.long, device=dev)
+    plain = step(m, False, torch.float16)
+    own, calls = getattr(kind, name), []
+    monkeypatch.setattr(kind, name, lambda self, *a, **k: (calls.append(type(self)), own(self, *a, **k))[1])
+    assert_same(step(m, True, torch.float16), plain, torch.float16)
+    assert len(calls) == calls_per_pass
+    calls.clear()
+    m.half()
+    with torch.no_grad():
+        m(ids, ids)
+    assert len(calls) == calls_per_pass
+
+
 def test_graph_of_a_step_goes_with_its_outputs(dev):
     """An output that the node held beside its saved tensors would keep the whole pass alive."""
     m = build(dev)

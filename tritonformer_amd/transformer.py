@@ -197,6 +197,11 @@ class MLPBlock(nn.Module):
         return self.dense_4h_to_h(self.dense_h_to_4h(hidden_states))
 
 
+# what calling these modules runs unless somebody patches the classes
+_OWN_FORWARD = {kind: kind.forward for kind in (CausalAttention, MLPBlock, tnn.LayerNorm)}
+_MODULE_CALL = nn.Module.__call__
+
+
 class TransformerLayer(nn.Module):
     """Pre-LN block (reference transformer.py:220-251)."""
 
@@ -219,7 +224,8 @@ class TransformerLayer(nn.Module):
         if first:
             called.append((self.input_layernorm, tnn.LayerNorm))
         return all(type(m) is kind and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
-                   and m._compiled_call_impl is None and "forward" not in m.__dict__ for m, kind in called)
+                   and m._compiled_call_impl is None and "forward" not in m.__dict__
+                   and kind.forward is _OWN_FORWARD[kind] and kind.__call__ is _MODULE_CALL for m, kind in called)
 
     def forward_deferred(self, hidden_states: torch.Tensor, pending: Optional[torch.Tensor],
                          attn_bias: Optional[torch.Tensor] = None):
