@@ -117,6 +117,47 @@ def test_watched_or_replaced_modules_are_called(dev):
     assert not torch.equal(step(m, True, torch.float16)[0], plain[0])
 
 
+def test_a_backward_pass_holds_no_more_than_that_of_four_nodes(dev, monkeypatch):
+    """What a part of the layer kept goes when its gradients are there."""
+    m = build(dev, param_dtype=torch.float16, layers=1, d=256, heads=4)
+    monkeypatch.setattr(TM, "DEFER_DW", False)
+    peaks = []
+    for fused in (True, False):
+        monkeypatch.setattr(TM, "FUSE_LAYER", fused)
+        for _ in range(2):
+            m.zero_grad(set_to_none=True)
+            x, pending = (torch.randn(128, 64, 256, device=dev).half().requires_grad_() for _ in range(2))
+            out = m.layer_list[0].forward_deferred(x, pending)
+            grads = [torch.ones_like(t) for t in out]
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            torch.autograd.backward(out, grads)
+            peaks.append(torch.cuda.max_memory_allocated() - before)
+            del x, pending, out, grads
+    assert peaks[1] <= peaks[3], peaks
+
+
+def test_saved_tensors_that_were_packed_away_come_back_a_part_at_a_time(dev):
+    """Bytes that live at once between their unpacking and the release by the engine."""
+    m = build(dev, layers=1, d=256, heads=4)
+    x = torch.randn(128, 64, 256, device=dev).half().requires_grad_()
+    peaks = []
+    for fused in (True, False):
+        TM.FUSE_LAYER = fused
+        try:
+            m.zero_grad(set_to_none=True)
+            with torch.autograd.graph.save_on_cpu(), torch.autocast("cuda", dtype=torch.float16):
+                out = m.layer_list[0].forward_deferred(x, x)
+        finally:
+            TM.FUSE_LAYER = True
+        grads = [torch.ones_like(t) for t in out]
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        torch.autograd.backward(out, grads)
+        peaks.append(torch.cuda.max_memory_allocated() - before)
+    assert peaks[0] <= peaks[1], peaks
+
+
 @pytest.mark.parametrize("kind,name,calls_per_pass", [(TM.CausalAttention, "forward", 3), (TM.MLPBlock, "forward", 3), (TM.tnn.LayerNorm, "forward", 1),
                                                       (torch.nn.Module, "__call__", 8)])
 def test_classes_patched_by_the_caller_are_called(kind, name, calls_per_pass, dev, monkeypatch):

@@ -77,18 +77,19 @@ class DecoderLayer(Function):
         for part, count, needed in zip(ctx.parts, ctx.counts, (True, need1, True, need2)):
             parts.append(part.restored(tensors[at:at + count], needed))
             at += count
-        del tensors
-        ln1, attn, ln2, mlp = parts
-        parts = None
-        d_normed, d_w1, d_c1, d_w2, d_c2 = _MLP[1](mlp, grad_out)
+        # what the parts kept goes with each of them, as it does from node to node: the gradients of a part take its place
+        ctx.maybe_clear_saved_tensors()
+        del tensors, part
+        d_normed, d_w1, d_c1, d_w2, d_c2 = _MLP[1](parts.pop(), grad_out)
         mlp_grads = (d_w1, d_c1, d_w2, d_c2)
         if not need2:
             return (None,) * 14 + mlp_grads
-        dx, _, d_g2, d_b2, _ = _ADD_LN[1](ln2, grad_stream, d_normed)
-        d_normed, d_wq, d_wk, d_wv, d_wo, _, _ = _ATTENTION[1](attn, dx)
+        dx, _, d_g2, d_b2, _ = _ADD_LN[1](parts.pop(), grad_stream, d_normed)
+        d_normed = None
+        d_normed, d_wq, d_wk, d_wv, d_wo, _, _ = _ATTENTION[1](parts.pop(), dx)
         grads = (d_wq, d_wk, d_wv, d_wo, None, None, d_g2, d_b2, None) + mlp_grads
         if not need1:
             return (None,) * 5 + grads
         # LayerNorm keeps what AddLayerNorm keeps: in the first layer this adds the gradient that x has beside its LayerNorm
-        dx, _, d_g1, d_b1, _ = _ADD_LN[1](ln1, dx, d_normed)
+        dx, _, d_g1, d_b1, _ = _ADD_LN[1](parts.pop(), dx, d_normed)
         return (dx, None if ctx.first else dx, d_g1, d_b1, None) + grads

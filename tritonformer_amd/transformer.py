@@ -244,9 +244,12 @@ class TransformerLayer(nn.Module):
                                         down.weight, down.bias)
                 if result is not None:
                     return result
-            return decoder_layer.apply(hidden_states, pending, ln1.weight, ln1.bias, ln1.eps, att.q_proj.weight, att.k_proj.weight,
-                                       att.v_proj.weight, att.out_proj.weight, att.num_attention_heads, attn_bias, ln2.weight,
-                                       ln2.bias, ln2.eps, up.weight, up.bias, down.weight, down.bias)
+            # hooks that pack saved tensors away (offloading, checkpointing) get them back node by node: four times a part of
+            # the layer's, not all of them together
+            if torch._C._autograd._top_saved_tensors_default_hooks(False) is None:
+                return decoder_layer.apply(hidden_states, pending, ln1.weight, ln1.bias, ln1.eps, att.q_proj.weight,
+                                           att.k_proj.weight, att.v_proj.weight, att.out_proj.weight, att.num_attention_heads,
+                                           attn_bias, ln2.weight, ln2.bias, ln2.eps, up.weight, up.bias, down.weight, down.bias)
         if pending is None:
             normed = ln1(hidden_states)
         else:
