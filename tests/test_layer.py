@@ -5,6 +5,7 @@ import torch
 
 import tritonformer_amd.transformer as TM
 from tests.util import rel_l2
+from tritonformer_amd import layer
 from tritonformer_amd.transformer import Transformer, TransformerConfig
 
 pytestmark = pytest.mark.gpu
@@ -156,6 +157,57 @@ def test_saved_tensors_that_were_packed_away_come_back_a_part_at_a_time(dev):
         torch.autograd.backward(out, grads)
         peaks.append(torch.cuda.max_memory_allocated() - before)
     assert peaks[0] <= peaks[1], peaks
+
+
+@pytest.mark.parametrize("train", ["", "mlp", "post_attention_layernorm", "attention", "input_layernorm"])
+@pytest.mark.parametrize("used", [0, 1])
+def test_one_output_used(train, used, dev):
+    """Of an output that nobody reads no gradient comes: parameters behind it alone have none, where zeros would be one."""
+    m = build(dev, bias=True, layers=1)
+    for name, p in m.named_parameters():
+        p.requires_grad_(train in name)
+    results = []
+    for fused in (True, False):
+        TM.FUSE_LAYER = fused
+        m.zero_grad(set_to_none=True)
+        torch.manual_seed(3)
+        x, pending = (torch.randn(2, 64, 128, device=dev).half().requires_grad_(not train) for _ in range(2))
+        try:
+            with torch.autocast("cuda", dtype=torch.float16):
+                out = m.layer_list[0].forward_deferred(x, pending)[used]
+        finally:
+            TM.FUSE_LAYER = True
+        if not out.requires_grad or (used == 0 and train in ("mlp", "post_attention_layernorm")):
+            continue  # nothing to train stands before this output (of one node all outputs require a gradient)
+        out.backward(torch.randn_like(out))
+        results.append([out] + [t.grad for t in (x, pending)] + [p.grad for p in m.layer_list[0].parameters()])
+    for one, four in zip(*results) if results else ():
+        assert (one is None) == (four is None)
+        assert one is None or torch.equal(one, four)
+
+
+def test_a_pass_without_a_graph_holds_no_more_than_four_nodes(dev, monkeypatch):
+    m = build(dev, layers=1, d=256, heads=4)
+    x, pending = torch.randn(2, 128, 64, 256, device=dev).half().unbind(0)
+    peaks = []
+    for fused in (True, False):
+        monkeypatch.setattr(TM, "FUSE_LAYER", fused)
+        for _ in range(2):
+            with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+                torch.cuda.reset_peak_memory_stats()
+                before = torch.cuda.memory_allocated()
+                out = m.layer_list[0].forward_deferred(x, pending)
+            peaks.append(torch.cuda.max_memory_allocated() - before)
+            del out
+    assert peaks[1] <= peaks[3], peaks
+
+
+def test_attention_with_nothing_to_train_before_it_is_not_differentiated(dev, monkeypatch):
+    m = build(dev, bias=True, layers=1)
+    for name, p in m.named_parameters():
+        p.requires_grad_("mlp" in name or "post_attention_layernorm" in name)
+    monkeypatch.setattr(layer, "_ATTENTION", (layer._ATTENTION[0], None))
+    assert step(m, True, torch.float16)[2]["layer_list.0.post_attention_layernorm.weight"] is not None
 
 
 @pytest.mark.parametrize("kind,name,calls_per_pass", [(TM.CausalAttention, "forward", 3), (TM.MLPBlock, "forward", 3), (TM.tnn.LayerNorm, "forward", 1),

@@ -12,11 +12,11 @@ class _Part:
     beyond it (an output held by the node that made it would keep itself alive): these go through the layer's own
     ``save_for_backward``, in the order of the parts."""
 
-    def __init__(self, arg_dtypes, amp_active):
-        self.arg_dtypes, self.amp_active = arg_dtypes, amp_active
+    def __init__(self, arg_dtypes, amp_active, keep):
+        self.arg_dtypes, self.amp_active, self.keep = arg_dtypes, amp_active, keep
 
     def save_for_backward(self, *tensors):
-        self.saved_tensors = tensors
+        self.saved_tensors = tensors if self.keep else ()
 
     def set_materialize_grads(self, value):
         pass
@@ -52,8 +52,10 @@ class DecoderLayer(Function):
     @amp_fwd(keep=tuple(range(2, 18)))
     def forward(ctx, x, pending, g1, b1, eps1, wq, wk, wv, wo, heads, attn_bias, g2, b2, eps2, w1, c1, w2, c2):
         dt, amp = ctx.arg_dtypes, ctx.amp_active
-        ln1, attn, ln2, mlp = parts = [_Part(dt[:1] + dt[2:5], amp), _Part(dt[:1] + dt[5:11], amp), _Part(dt[:2] + dt[11:14], amp),
-                                       _Part(dt[:1] + dt[14:], amp)]
+        # the node has its edges by now: none where no graph is built, and nothing is then kept beyond its last reader
+        ln1, attn, ln2, mlp = parts = [_Part(types, amp, bool(ctx.next_functions))
+                                       for types in (dt[:1] + dt[2:5], dt[:1] + dt[5:11], dt[:2] + dt[11:14], dt[:1] + dt[14:])]
+        ctx.set_materialize_grads(False)  # an unused output arrives as None, not as zeros
         ctx.first = pending is None
         if pending is None:
             normed = _LN[0](ln1, x, g1, b1, eps1)
@@ -61,6 +63,7 @@ class DecoderLayer(Function):
             x, normed = _ADD_LN[0](ln1, x, pending, g1, b1, eps1)
         branch = _ATTENTION[0](attn, normed, wq, wk, wv, wo, heads, attn_bias)
         stream, normed = _ADD_LN[0](ln2, x, branch, g2, b2, eps2)
+        del x, branch
         out = _MLP[0](mlp, normed, w1, c1, w2, c2)
         saved = [part.release() for part in parts]
         ctx.parts, ctx.counts = parts, [len(t) for t in saved]
@@ -71,8 +74,9 @@ class DecoderLayer(Function):
     @amp_bwd
     def backward(ctx, grad_stream, grad_out):
         need = ctx.needs_input_grad
-        need1 = need[0] or need[1] or need[2] or need[3]              # the LayerNorm ahead of the attention
-        need2 = need1 or any(need[5:9]) or need[11] or need[12]       # the one ahead of the MLP
+        need1 = any(need[:4])                         # the LayerNorm ahead of the attention
+        attended = need1 or any(need[5:9])            # the attention
+        need2 = attended or need[11] or need[12]      # the LayerNorm ahead of the MLP
         tensors, parts, at = ctx.saved_tensors, [], 0
         for part, count, needed in zip(ctx.parts, ctx.counts, (True, need1, True, need2)):
             parts.append(part.restored(tensors[at:at + count], needed))
@@ -80,16 +84,17 @@ class DecoderLayer(Function):
         # what the parts kept goes with each of them, as it does from node to node: the gradients of a part take its place
         ctx.maybe_clear_saved_tensors()
         del tensors, part
-        d_normed, d_w1, d_c1, d_w2, d_c2 = _MLP[1](parts.pop(), grad_out)
-        mlp_grads = (d_w1, d_c1, d_w2, d_c2)
-        if not need2:
-            return (None,) * 14 + mlp_grads
-        dx, _, d_g2, d_b2, _ = _ADD_LN[1](parts.pop(), grad_stream, d_normed)
-        d_normed = None
-        d_normed, d_wq, d_wk, d_wv, d_wo, _, _ = _ATTENTION[1](parts.pop(), dx)
-        grads = (d_wq, d_wk, d_wv, d_wo, None, None, d_g2, d_b2, None) + mlp_grads
-        if not need1:
-            return (None,) * 5 + grads
-        # LayerNorm keeps what AddLayerNorm keeps: in the first layer this adds the gradient that x has beside its LayerNorm
-        dx, _, d_g1, d_b1, _ = _ADD_LN[1](parts.pop(), dx, d_normed)
-        return (dx, None if ctx.first else dx, d_g1, d_b1, None) + grads
+        grads, d_normed, mlp = [None] * 18, None, parts.pop()
+        if grad_out is not None:
+            d_normed, *grads[14:] = _MLP[1](mlp, grad_out)
+        del mlp, grad_out
+        if need2:
+            dx, _, *grads[11:14] = _ADD_LN[1](parts.pop(), grad_stream, d_normed)
+            d_normed = None
+        if attended:
+            d_normed, *grads[5:11] = _ATTENTION[1](parts.pop(), dx)
+        if need1:
+            # LayerNorm keeps what AddLayerNorm keeps: in the first layer this adds the gradient that x has beside its LayerNorm
+            dx, _, *grads[2:5] = _ADD_LN[1](parts.pop(), dx, d_normed)
+            grads[:2] = dx, None if ctx.first else dx
+        return tuple(grads)
