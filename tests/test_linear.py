@@ -691,11 +691,12 @@ def test_sign_bit_rows_on_every_tile(cfg, pitch, shift, dev):
 
 @pytest.mark.parametrize("pitch", [1 << 22, (1 << 22) + 8, (1 << 22) + 3])
 @pytest.mark.parametrize("layouts", ["fwd", "dx", "dw"])
-def test_rows_at_and_beyond_the_pitch_that_32_bit_offsets_reach(layouts, pitch, dev):
-    """The direct-to-LDS kernels and the register-staged 256x256 tiles address a lane's chunks by 32-bit offsets; wider rows
-    take the 128x128 register-staged tiles.  One operand a narrow strip of a very wide matrix, whose other columns are NaN
-    where they are next to the strip; the sums run over the same steps in the same order whatever the tile, so the bits are
-    those of the operand by itself."""
+@pytest.mark.parametrize("which", ["A", "B"])
+def test_rows_at_and_beyond_the_pitch_that_32_bit_offsets_reach(which, layouts, pitch, dev):
+    """The direct-to-LDS kernels and the register-staged tiles of 256 rows address a lane's chunks by 32-bit offsets; wider rows
+    take 128x128 tiles with 64-bit ones, direct to LDS or register-staged.  One operand a narrow strip of a very wide matrix, whose
+    other columns are NaN where they are next to the strip; the sums run over the same steps in the same order whatever the tile, so the
+    bits are those of the operand by itself."""
     from tritonformer_amd import _lib
 
     d = _lib.load_diag()
@@ -704,21 +705,52 @@ def test_rows_at_and_beyond_the_pitch_that_32_bit_offsets_reach(layouts, pitch, 
     g = torch.Generator().manual_seed(41)
     a = torch.randn((M, K) if la == 0 else (K, M), generator=g).half().to(dev)
     b = (torch.randn((N, K) if lb == 0 else (K, N), generator=g) / K ** 0.5).half().to(dev)
-    wide = torch.empty(a.shape[0] * pitch, dtype=torch.float16, device=dev).view(a.shape[0], pitch)
-    wide[:, :a.shape[1] + 64] = float("nan")
-    wide[:, :a.shape[1]] = a
+    strip = a if which == "A" else b
+    wide = torch.empty(strip.shape[0] * pitch, dtype=torch.float16, device=dev).view(strip.shape[0], pitch)
+    wide[:, :strip.shape[1] + 64] = float("nan")
+    wide[:, :strip.shape[1]] = strip
     stream = torch.cuda.current_stream().cuda_stream
 
-    def run(x, cfg):
+    def run(a, b, cfg, splits=1):
         out = torch.empty((M, N), dtype=torch.float16, device=dev)
-        _lib.check(d.tf_diag_gemm(stream, cfg, 1, 0, 0, 0, la, lb, M, N, K, x.data_ptr(), x.stride(0), b.data_ptr(), b.stride(0),
-                                  out.data_ptr(), N, None, 0, None, 0))
+        ws = torch.empty(M * N * 4 * splits, dtype=torch.uint8, device=dev)
+        _lib.check(d.tf_diag_gemm(stream, cfg, splits, 0, 0, 0, la, lb, M, N, K, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+                                  out.data_ptr(), N, None, 0, ws.data_ptr(), ws.numel()))
         return out
 
-    base = run(a, 2)
+    pair = (wide, b) if which == "A" else (a, wide)
+    base = run(a, b, 2)
     assert_close(base, (a.float() if la == 0 else a.float().T) @ (b.float().T if lb == 0 else b.float()), name=layouts)
-    for cfg in range(8):
-        assert torch.equal(run(wide, cfg), base), f"cfg {cfg}"
+    for cfg in range(9):
+        assert torch.equal(run(*pair, cfg), base), f"cfg {cfg}"
+    assert torch.equal(run(*pair, 2, 2), run(a, b, 2, 2))
+
+
+@pytest.mark.parametrize("which", ["A", "B"])
+@pytest.mark.parametrize("pitch", [1 << 22, (1 << 22) + 8])
+def test_sign_bits_of_products_with_very_wide_rows(which, pitch, dev):
+    """The sign bits exist in the direct-to-LDS kernels alone, whose 64-bit offsets these rows need."""
+    from tritonformer_amd import _lib
+
+    call, st = _lib.load().tf_gemm_relu_bits, _lib.stream_ptr()
+    M, N, K = 300, 136, 128
+    g = torch.Generator().manual_seed(53)
+    x, w = torch.randn(M, K, generator=g).half().to(dev), (torch.randn(K, N, generator=g) / K ** 0.5).half().to(dev)
+    dy = torch.randn(M, K, generator=g).half().to(dev)
+    strip = x if which == "A" else w
+    wide = torch.empty(strip.shape[0] * pitch, dtype=torch.float16, device=dev).view(strip.shape[0], pitch)
+    wide[:, :strip.shape[1]] = strip
+    bits = []
+    for a, b in ((x, w), (wide, w) if which == "A" else (x, wide)):
+        h, dh = (torch.full((M, N), float("nan"), dtype=torch.float16, device=dev) for _ in range(2))
+        signs = torch.zeros(M, N // 8, dtype=torch.uint8, device=dev)
+        _lib.check(call(st, 0, 0, 0, 1, M, N, K, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), h.data_ptr(), N, None,
+                        signs.data_ptr(), None, N // 8))
+        _lib.check(call(st, 0, 0, 0, 1, M, N, K, dy.data_ptr(), K, b.data_ptr(), b.stride(0), dh.data_ptr(), N, None, None,
+                        signs.data_ptr(), N // 8))
+        bits.append((h, signs, dh))
+    for got, want in zip(bits[1], bits[0]):
+        assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("layouts", ["fwd", "dx", "dw"])

@@ -151,24 +151,27 @@ struct DmaPanel {
   }
 
   // Byte offset of each of this lane's chunks from the panel's first element of a step (row row0, contraction index kbeg):
-  // the address is wave-uniform but for these 32 bits, which no step changes.
+  // the address is wave-uniform but for these 32 bits (64 for rows beyond kMaxPitch), which no step changes.
   static __device__ __forceinline__ const char* origin(const T* base, int64_t ld, int row0, int kbeg) {
     return (const char*)(KMAJOR ? base + (int64_t)row0 * ld + kbeg : base + (int64_t)kbeg * ld + row0);
   }
-  static __device__ __forceinline__ void init(uint32_t (&offs)[PER_WAVE], int64_t ld, int row0, int rmax, int wave, int lane) {
+  template <typename Off>
+  static __device__ __forceinline__ void init(Off (&offs)[PER_WAVE], int64_t ld, int row0, int rmax, int wave, int lane) {
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) {
       const int slot = (wave * PER_WAVE + j) * 64 + lane;
       const int lrow = slot / CPR;
       const int c = swz(lrow, slot % CPR);
-      if (KMAJOR) offs[j] = ((uint32_t)(min(row0 + lrow, rmax - 1) - row0) * (uint32_t)ld + (uint32_t)c * 8u) * 2u;
-      else offs[j] = ((uint32_t)lrow * (uint32_t)ld + (row0 + c * 8 < rmax ? (uint32_t)c * 8u : 0u)) * 2u;
+      if (KMAJOR) offs[j] = ((Off)(min(row0 + lrow, rmax - 1) - row0) * (Off)ld + (Off)(c * 8)) * 2;
+      else offs[j] = ((Off)lrow * (Off)ld + (Off)(row0 + c * 8 < rmax ? c * 8 : 0)) * 2;
     }
   }
-  static __device__ __forceinline__ void issue_one(const char* org, const uint32_t (&offs)[PER_WAVE], char* lds, int wave, int j) {
+  template <typename Off>
+  static __device__ __forceinline__ void issue_one(const char* org, const Off (&offs)[PER_WAVE], char* lds, int wave, int j) {
     __builtin_amdgcn_global_load_lds((gptr_void*)at_offset(org, offs[j]), (lds_void*)(lds + (wave * PER_WAVE + j) * 1024), 16, 0, 0);
   }
-  static __device__ __forceinline__ void issue(const char* org, const uint32_t (&offs)[PER_WAVE], char* lds, int wave) {
+  template <typename Off>
+  static __device__ __forceinline__ void issue(const char* org, const Off (&offs)[PER_WAVE], char* lds, int wave) {
 #pragma unroll
     for (int j = 0; j < PER_WAVE; ++j) issue_one(org, offs, lds, wave, j);
   }
@@ -489,7 +492,7 @@ __device__ __forceinline__ void gemm_epilogue_bits(const GemmParams& p, f32x4 (&
 // being multiplied, and have one stage's time to arrive.  3: a stage's loads are requested two stages ahead
 // and have two stages' time: for tiles whose stage is short (256x128: half the MFMAs of 256x256 per stage)
 // one stage's time does not cover the latency of operands that come from HBM rather than from the L2.
-template <typename T, int BM, int BN, int BK, int WM, int WN, bool A_KMAJOR, bool B_KMAJOR, int NS = 2>
+template <typename T, int BM, int BN, int BK, int WM, int WN, bool A_KMAJOR, bool B_KMAJOR, int NS = 2, typename Off = uint32_t>
 __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid) {
   static_assert(NS == 2 || NS == 3, "two or three pipeline stages");
   constexpr int NW = WM * WN;
@@ -524,7 +527,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams& p, const int pid
   const int kend = min(p.K, kbeg + p.k_per_split);
   const int nk = (kend - kbeg) / BK;
 
-  uint32_t oa[PA::PER_WAVE], ob[PB::PER_WAVE];
+  Off oa[PA::PER_WAVE], ob[PB::PER_WAVE];
   PA::init(oa, p.lda, m0, p.M, wave, lane);
   const T* B = (const T*)p.B;
   int nb = n0, nend = p.N;  // the tile's columns in B
@@ -748,6 +751,14 @@ template <typename T, int BM, int BN, int BK, int WM, int WN, int WPE, bool A_KM
 __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_dma_kernel(GemmParams p) {
   const int pid = (p.flags & 1) ? (int)blockIdx.x : remap_xcd(blockIdx.x, p.tiles_m * p.tiles_n * p.splits, p.xcds);
   gemm_dma_body<T, BM, BN, BK, WM, WN, A_KMAJOR, B_KMAJOR, NS>(p, pid);
+}
+
+// Operands with rows beyond kMaxPitch: 64-bit offsets, which the 128x128 tile has the registers for.  Same steps, same order of
+// sums as any other tile of these kernels.
+template <typename T, bool A_KMAJOR, bool B_KMAJOR>
+__global__ __launch_bounds__(256, 2) void gemm_wide_kernel(GemmParams p) {
+  const int pid = (p.flags & 1) ? (int)blockIdx.x : remap_xcd(blockIdx.x, p.tiles_m * p.tiles_n * p.splits, p.xcds);
+  gemm_dma_body<T, 128, 128, 64, 2, 2, A_KMAJOR, B_KMAJOR, 2, uint64_t>(p, pid);
 }
 
 // ---------------------------------------------------------------------------
@@ -1295,17 +1306,22 @@ static void allow_big_lds(K kernel, int bytes) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
+template <typename K>
+static int launch_tiles(hipStream_t st, K kernel, int threads, int lds, const GemmParams& p) {
+  const unsigned grid = (unsigned)(p.tiles_m * p.tiles_n * p.splits);
+  kernel<<<dim3(grid), dim3(threads), lds, st>>>(p);
+  TF_CHECK_LAUNCH();
+  g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
+  return TF_OK;
+}
+
 template <typename T, int BM, int BN, int BK, int WM, int WN, int WPE, bool AK, bool BKM>
 static int launch_reg(hipStream_t st, const GemmParams& p) {
   constexpr int lds = 2 * (BM + BN) * BK * 2;
   auto kernel = gemm_reg_kernel<T, BM, BN, BK, WM, WN, WPE, AK, BKM>;
   static bool once = (allow_big_lds(kernel, lds), true);
   (void)once;
-  const unsigned grid = (unsigned)(p.tiles_m * p.tiles_n * p.splits);
-  kernel<<<dim3(grid), dim3(WM * WN * 64), lds, st>>>(p);
-  TF_CHECK_LAUNCH();
-  g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
-  return TF_OK;
+  return launch_tiles(st, kernel, WM * WN * 64, lds, p);
 }
 
 template <typename T, int BM, int BN, int BK, int WM, int WN, int WPE, bool AK, bool BKM, int NS = 2>
@@ -1315,11 +1331,18 @@ static int launch_dma(hipStream_t st, const GemmParams& p) {
   auto kernel = gemm_dma_kernel<T, BM, BN, BK, WM, WN, WPE, AK, BKM, NS>;
   static bool once = (allow_big_lds(kernel, lds), true);
   (void)once;
-  const unsigned grid = (unsigned)(p.tiles_m * p.tiles_n * p.splits);
-  kernel<<<dim3(grid), dim3(WM * WN * 64), lds, st>>>(p);
-  TF_CHECK_LAUNCH();
-  g_gemm_launches.fetch_add(1, std::memory_order_relaxed);
-  return TF_OK;
+  return launch_tiles(st, kernel, WM * WN * 64, lds, p);
+}
+
+// Whatever the plan's tiles: the same slices on 128x128 tiles, whose kernels take rows of any pitch.
+template <typename T, bool AK, bool BKM>
+static int launch_any_pitch(hipStream_t st, bool dma, const GemmParams& p) {
+  GemmParams q = p;
+  q.tiles_m = (q.M + 127) / 128;
+  q.tiles_n = (q.N + 127) / 128;
+  if ((int64_t)q.tiles_m * q.tiles_n * q.splits > 0x7fffffff) return TF_EINVAL;
+  if (dma) return launch_tiles(st, gemm_wide_kernel<T, AK, BKM>, 256, 2 * (128 + 128) * 64 * 2, q);
+  return launch_reg<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, q);
 }
 
 // The register-staged kernel handles everything (ragged extents, unaligned
@@ -1332,7 +1355,9 @@ constexpr int kStagesNarrow = 3;  // LDS stages of the configurations below 256x
 
 template <typename T, bool AK, bool BKM>
 static int launch_cfg(hipStream_t st, bool vec, const GemmPlan& pl, const GemmParams& p) {
-  if (kCfgs[pl.cfg].dma && vec && p.K % pl.bk == 0) {
+  const bool dma = kCfgs[pl.cfg].dma && vec && p.K % pl.bk == 0;
+  if (p.lda > kMaxPitch || p.ldb > kMaxPitch) return launch_any_pitch<T, AK, BKM>(st, dma, p);
+  if (dma) {
     switch (pl.cfg) {
       case 2: return launch_dma<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
       case 3: return launch_dma<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, p);
@@ -1342,18 +1367,10 @@ static int launch_cfg(hipStream_t st, bool vec, const GemmPlan& pl, const GemmPa
       case 7: return launch_dma<T, 128, 64, 64, 4, 1, 2, AK, BKM, kStagesNarrow>(st, p);
     }
   }
-  if (pl.bm == 256 && pl.bn == 256 && p.lda <= kMaxPitch && p.ldb <= kMaxPitch)
-    return launch_reg<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
-  if (pl.bm == 256 && pl.bn == 128 && p.lda <= kMaxPitch && p.ldb <= kMaxPitch)
-    return launch_reg<T, 256, 128, 64, 4, 2, 2, AK, BKM>(st, p);
-  if (pl.bm == 256) {  // wider rows than the 256-row tiles address: the same slices on the smaller tiles
-    GemmParams q = p;
-    q.tiles_m = (q.M + 127) / 128;
-    q.tiles_n = (q.N + 127) / 128;
-    if ((int64_t)q.tiles_m * q.tiles_n * q.splits > 0x7fffffff) return TF_EINVAL;
-    return launch_reg<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, q);
-  }
-  return launch_reg<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, p);
+  if (pl.bm == 256 && pl.bn == 256) return launch_reg<T, 256, 256, 64, 2, 4, 2, AK, BKM>(st, p);
+  if (pl.bm == 256 && pl.bn == 128) return launch_reg<T, 256, 128, 64, 4, 2, 2, AK, BKM>(st, p);
+  if (pl.bm == 128 && pl.bn == 128) return launch_reg<T, 128, 128, 64, 2, 2, 2, AK, BKM>(st, p);
+  return TF_EINVAL;
 }
 
 // Second pass of a split contraction (no-op when the contraction was not split).
@@ -1585,7 +1602,7 @@ static int gemm_entry(void* stream, int dtype, int out_dtype, int layout_a, int 
        reinterpret_cast<uintptr_t>(bias)) & 1)
     return TF_EALIGN;
 
-  const bool vec = lda <= kMaxPitch && ldb <= kMaxPitch && aligned16(A) && aligned16(B) && aligned16(C) && (!bias || aligned16(bias)) && a_contig % 8 == 0 &&
+  const bool vec = aligned16(A) && aligned16(B) && aligned16(C) && (!bias || aligned16(bias)) && a_contig % 8 == 0 &&
                    b_contig % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && N % 8 == 0 && ldc % 8 == 0 &&
                    (!mask_act || (aligned16(mask_act) && ld_mask % 8 == 0));
   const bool forced = force.cfg >= 0 || force.splits > 0 || (force.flags & 64);
