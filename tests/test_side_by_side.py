@@ -150,3 +150,30 @@ def test_a_layer_in_one_call_holds_no_more_than_its_nodes(first, dev, monkeypatc
             peaks.append(torch.cuda.max_memory_allocated() - before)
             del out
     assert peaks[1] <= peaks[3], peaks
+
+
+@pytest.mark.parametrize("odd", range(4))
+def test_projections_at_odd_addresses_are_left_to_the_nodes(odd, dev, monkeypatch):
+    """Views of one flat buffer, as optimizers and checkpoints make them: the nodes copy such weights to an aligned matrix."""
+    m = build(dev, False, False, torch.float16, layers=1, d=2048, heads=16)
+    att = m.layer_list[0].attention
+    weight = getattr(att, ("q_proj", "k_proj", "v_proj", "out_proj")[odd]).weight
+    flat = torch.empty(weight.numel() + 1, dtype=torch.float16, device=dev)
+    flat[1:] = weight.detach().flatten()
+    weight.data = flat[1:].view_as(weight)
+    ids = torch.arange(128, device=dev).view(2, 64)
+    answers = []
+    native = _lib.launch().layer
+
+    class Watching:
+        def __getattr__(self, name):
+            if name == "layer":
+                return lambda *a: (answers.append(native(*a)), answers[-1])[1]
+            return getattr(_lib.launch(), name)
+
+    monkeypatch.setattr(TM, "launch", lambda: Watching())
+    with torch.no_grad():
+        one = m(ids, None)
+        assert answers == [None]
+        monkeypatch.setattr(TM, "FUSE_LAYER", False)
+        assert torch.equal(one, m(ids, None))

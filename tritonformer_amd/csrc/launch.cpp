@@ -744,7 +744,8 @@ TF_FN(layer, 15) {
   };
   const Tensor* w[4];
   for (int i = 0; i < 4; ++i)
-    if (!(w[i] = weight(PyList_GET_ITEM(args.a[5], i), d, d))) Py_RETURN_NONE;
+    // at an odd address the products would go through registers, where the nodes read the aligned copy that they make
+    if (!(w[i] = weight(PyList_GET_ITEM(args.a[5], i), d, d)) || !aligned(*w[i])) Py_RETURN_NONE;
   const Tensor *w1 = weight(args.a[11], d, -1), *w2 = weight(args.a[13], -1, d), *c[2] = {nullptr, nullptr};
   if (!w1 || !w2 || w2->size(0) != w1->size(1)) Py_RETURN_NONE;
   const int64_t f = w1->size(1), hd = d / nh;
