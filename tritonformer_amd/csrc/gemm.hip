@@ -139,7 +139,7 @@ struct DmaPanel {
   static constexpr int WLOADS = NCHUNK / 64;   // wave-level loads per panel
   static constexpr int PER_WAVE = WLOADS / NW;
   static_assert(WLOADS % NW == 0 && PER_WAVE >= 1, "panel must divide evenly over the waves");
-  static_assert(KMAJOR ? (CPR == 4 || CPR == 8) : (CPR >= 4), "unsupported panel shape");
+  static_assert(KMAJOR ? (CPR == 4 || CPR == 8) : (CPR >= 8), "the swizzle stays within the row");
 
   // K-major: 16 rows of one chunk column fill the banks once.  K-minor: a transposing read takes 32 bytes of each of four
   // neighbouring rows per 16 lanes, and of the four rows eight further on in the next 16.  Rows of 256 bytes and more begin
