@@ -12,7 +12,7 @@
 //    a contraction that is not a multiple of BK): the same loop and write-out with the
 //    operands staged through registers in 16-byte chunks at any element address.
 // Both use v_mfma_f32_16x16x32_{f16,bf16} with fp32 accumulators.  Real data holds the clock of the matrix pipes down (power),
-// and the smaller instruction needs less of it: it moves a quarter of the accumulators per multiplication.  The MFMA stream
+// and the smaller instruction needs less of it: it moves half the accumulators per multiplication.  The MFMA stream
 // of a 256x256x64 step alone on normal fp16 data: 1.29 us with 32x32x16, 1.13 with 16x16x32 (bf16 1.20 and 1.06); equal on zeros.
 // The results are the same bits.  Products on operands from HBM, fp16, with 32x32x16 and now: 8192 x 1024 x 4096 71.2 -> 64.9 us,
 // 8192 x 4096 x 1024 73.5 -> 69.9, 4096 x 8192 x 2048 125.2 -> 115.9, 8192 x 50304 x 1024 819 -> 772; 4096 x 4096 x 8192 225 -> 204:
@@ -822,7 +822,9 @@ __global__ __launch_bounds__(WM* WN * 64, WPE) void gemm_reg_kernel(GemmParams p
   constexpr int TM = WTM / 16, TN = WTN / 16;
   constexpr int GROUP_M = 8;
   constexpr int KSTEPS = BK / 32;
-  // the 256-row panels keep 32-bit offsets (kMaxPitch): with 64 bits the kernel spills
+  // the tiles of 256 rows keep 32-bit offsets (kMaxPitch): 64 bits are eight registers more, and 256x256 has none left.  It holds all
+  // 256, and where just one operand is contraction-strided it parks seven in scratch around the stages that test extents, not in
+  // the loop over whole stages
   typedef std::conditional_t<(BM > 128), uint32_t, uint64_t> Off;
   typedef RegPanel<T, BM, BK, A_KMAJOR, NW, Off> PA;
   typedef RegPanel<T, BN, BK, B_KMAJOR, NW, Off> PB;
