@@ -91,3 +91,25 @@ def test_route_rejects_bad_arguments():
 ])
 def test_rates_of_the_tiles(m, n, k, vec, want):
     assert route(m, n, k, vec=vec) == want
+
+
+@pytest.mark.parametrize("m,n,k,kind,vec,want", [
+    # two rounds of 256x128 tiles take longer than one of 256x256, and long contractions longer than short ones by the step
+    (8192, 2048, 12288, PLAIN, True, (2, 1)),
+    (14976, 1984, 12800, PLAIN, True, (2, 1)),
+    (11136, 960, 12224, PLAIN, True, (2, 1)),
+    # one or two steps are start and write-out, which more and smaller tiles have less of; 128x64 tiles on just over one workgroup per CU
+    (40, 1536, 64, PLAIN, True, (6, 1)),
+    (7296, 560, 832, PLAIN, True, (4, 1)),
+    (7432, 144, 3968, PLAIN, True, (4, 3)),
+    # operands of any alignment, unsplit: 128x128 tiles up to one per CU, 256x128 where they would be more
+    (1509, 105, 7035, MASK, False, (1, 1)),
+    (2334, 1614, 9044, MASK, False, (1, 1)),
+    (1563, 2665, 5116, MASK, False, (8, 1)),
+    # split: 256x256 in slices
+    (10712, 616, 6012, PLAIN, False, (0, 2)),
+    (966, 7598, 9983, PLAIN, False, (0, 2)),
+])
+def test_tiles_that_were_the_slower_ones(m, n, k, kind, vec, want):
+    """Each of these ran 1.05 to 1.5 times as long on the tiles that a fit to warm operands had taken."""
+    assert route(m, n, k, kind, vec) == [(n, *want)]

@@ -1180,22 +1180,24 @@ static GemmPlan plan_for(int64_t cus, int cfg, int64_t M, int64_t N, int64_t K, 
   // gradients: few output tiles, long contraction); never beyond one full round of
   // workgroups, and every slice keeps at least 16 steps so that the fp32 partial
   // traffic stays small.
-  // Microseconds of a round of workgroups beside its steps and per 64-wide step, by configuration.  Found over 550 products of
-  // odd extents (16 to 16384 rows, 64 to 8192 columns, contractions of 64 to 4096, all layouts) and 730 of whole multiples of 64, every
-  // tile timed: the tiles chosen take 0.7 and 1.3 per cent longer (geometric mean) than the best of those at hand; with the
-  // figures of the 32x32x16 kernels (10 and 2.25, 7 and 1.6 register-staged; 10 and 1.65, 7 and 1.1, 7 and 1.0) it was 1.5 and
-  // 3.0, up to 25 where a contraction is short (7488 x 2624 x 64 13.9 -> 11.3 us) or 256x128 tiles fill one round (768 x 7040 x 3648
-  // 52.5 -> 42.0).
-  static const struct { double fixed, per_step; } rates[] = {{8.9, 1.63}, {3.1, 1.14}, {10.1, 1.62}, {5.0, 1.13}, {9.7, 0.78},
-                                                             {9.7, 0.78}, {5.0, 1.13}, {5.0, 1.13}, {10.1, 0.92}};
-  static_assert(sizeof(rates) / sizeof(rates[0]) == sizeof(kCfgs) / sizeof(kCfgs[0]), "a rate for each configuration");
-  // 256x128 tiles pay for a long contraction, which holds the clock down, with their share of loads: 0.79 us per step of 128
-  // (4096 x 2048 x 8192 125 us on 256x256 tiles in two slices, 111 on these), 0.91 of 786 (8192 x 1024 x 50304 687 and 725)
-  const bool held = (cfg == 4 || cfg == 5) && ksteps >= 256;
-  const double fixed = rates[cfg].fixed, per_step = held ? 0.91 : rates[cfg].per_step;
+  // Microseconds of a round of workgroups beside its steps and per 64-wide step (`alone`: of a round with one workgroup per CU at
+  // the most, where two of 128x128 share one otherwise), by configuration.  Found over 2300 products of 2 to 16384 rows, 64 to 8192
+  // columns and contractions of 64 to 16384, all layouts, odd extents and whole multiples of 8 and 64, shapes of decoders among them,
+  // operands from HBM, every tile timed with and without slices; over 1400 others the tile taken is 1.0 per cent slower than the best of
+  // those at hand (geometric mean; 0.5 where the contraction is not split), 0.2 to 0.4 with operands of any alignment.
+  // With the figures of the 32x32x16 kernels (2: 10 and 1.65, 4: 7 and 1.0, 3: 7 and 1.1, 0: 10 and 2.25, 1: 7 and 1.6, no 8) it
+  // is 1.3, 0.9 and 0.6 to 0.7.  A step of 256x128 tiles at 0.78 us, what it is where a contraction is short, took long ones to them:
+  // 14976 x 1984 x 12800 643 us on 256x256 tiles and 768 on 256x128, 8192 x 2048 x 12288 319 and 348.
+  // Register-staged 256x128 tiles pay where 128x128 tiles are more than one and less than two per CU: 1563 x 2665 x 5116 106 us on
+  // these and 82, but with fewer than one per CU 1509 x 105 x 7035 119 and 179.
+  static const struct { double fixed, per_step, alone; } rates[] = {
+      {13.9, 1.93, 1.93}, {5.1, 1.47, 1.25}, {10.8, 1.55, 1.55}, {5.8, 1.09, 1.09}, {7.3, 0.88, 0.88},
+      {7.3, 0.88, 0.88},  {5.8, 1.09, 1.09}, {5.8, 1.09, 1.09},  {8.7, 1.31, 1.31}};
+  static_assert(sizeof(rates) / sizeof(rates[0]) == sizeof(kCfgs) / sizeof(kCfgs[0]), "rates for each configuration");
   auto cost_of = [&](int64_t nsplit, int64_t steps) {
-    const int64_t rounds = (tiles * nsplit + slots - 1) / slots;
-    double c = (double)rounds * (fixed + per_step * (double)steps);
+    const int64_t wgs = tiles * nsplit, rounds = (wgs + slots - 1) / slots;
+    double c = (double)rounds * (rates[cfg].fixed + rates[cfg].per_step * (double)steps);
+    if (wgs - (rounds - 1) * slots <= cus) c -= (rates[cfg].per_step - rates[cfg].alone) * (double)steps;
     if (nsplit > 1) c += 3.0 + (nsplit + 0.5) * (double)M * (double)N * 4.0 / 5.0e6;
     return c;
   };
@@ -1229,28 +1231,25 @@ static GemmPlan plan_for(int64_t cus, int cfg, int64_t M, int64_t N, int64_t K, 
 
 // Time (microseconds) of a direct-to-LDS launch that leaves CUs or their second workgroup idle, where the cost above --
 // made for whole rounds -- is 1.3 to 2 times too high: a fixed part plus a time per 64-wide step that rises with the
-// workgroups per CU (`fill`), since operands come faster and the clock is higher while few CUs work.  Fits to 650 products that
-// leave CUs idle (16 to 16384 rows, 64 to 8192 columns, contractions of 64 to 4096 and more, all layouts): the tile taken is 1.4 per
-// cent slower than the best of the five at hand (geometric mean), 2.5 with the figures of the 32x32x16 kernels; 2752 x 512 x 1792
-// 14.8 -> 12.2 us, 384 x 3392 x 2048 18.7 -> 15.5.
-// With those kernels it was checked over 1400 others that leave CUs idle with the large tile (16 to 6144 rows, 64 to 9000 columns, all layouts, slices
-// and sign bits as they are in use): 1.44 times the large tile's speed (geometric mean; the best of the three tiles each time
-// 1.45), seven of them slower than the large tile, by 4 to 9 per cent, all of 300 workgroups and more with long contractions
-// (629 x 5120 x 8128 90 -> 98 us), where two workgroups of a CU take longer than 1.3 to 1.8 of them would.  Counted as two they
-// would cost others more (2087 x 1552 x 1024 12.8 -> 17.3).  Sign bits, which 64-wide tiles store byte by byte, cost these 0.2 to
-// 1.1 us; an extra 0.5 us for them changes nothing for the better.
+// workgroups per CU (`fill`), since operands come faster and the clock is higher while few CUs work.  Fits to the products above
+// that leave CUs idle.  Over 300 others (16 to 8192 rows and columns, contractions of 64 to 8192, all layouts) the tile taken has 1.47 times
+// the speed of the large one (geometric mean) and is 0.6 per cent slower than the best of the five (1.5 with the fit named below).  The
+// few that are slower, by up to a fifth, are long contractions on just over one workgroup per CU (192 x 1536 x 6144 in six slices 18.4 us
+// on 64x64 and 21.9 on 128x64 tiles), where two of a CU take longer than `fill` of them would; counted as two they would cost others more.
+// A first fit to these kernels (2.8 and 0.26 for 64x64 tiles, 2.6 and 0.36 for 128x64), to operands that lay in the caches, took products of
+// a step or two and products of 256x128 tiles to 128x64: 40 x 1536 x 64 2.8 us on 64x64 and 3.6, 7296 x 560 x 832 13.7 on 256x128 and 17.1.
 static double part_round_us(int64_t cus, const GemmPlan& pl, int64_t M, int64_t N) {
   const double steps = (double)(pl.k_per_split / pl.bk);
   const double fill = (double)((int64_t)pl.tiles_m * pl.tiles_n * pl.splits) / (double)cus;
   auto rise = [](double x, double from, double to) { return x <= from ? 0.0 : x >= to ? 1.0 : (x - from) / (to - from); };
-  const double more = 0.7 * std::max(0.0, fill - 1);  // start and write-out of every further workgroup of a CU
+  const double more = std::max(0.0, fill - 1);  // further workgroups of a CU: their start and write-out
   double c = 0;
   switch (pl.cfg) {
-    case 2: c = 4.4 + steps * (0.85 + 1.05 * rise(fill, 0.31, 1.14)); break;
-    case 3: c = 2.1 + steps * (0.81 + 0.59 * rise(fill, 0.73, 2.2)); break;
-    case 4: c = 3.6 + steps * (0.63 + 0.47 * rise(fill, 0.285, 1.15)); break;
-    case 6: c = 2.8 + more + steps * std::max(0.26 + 0.04 * rise(fill, 0.5, 1), 0.35 * fill); break;
-    case 7: c = 2.6 + more + steps * std::max(0.36 + 0.12 * rise(fill, 0.5, 1), 0.43 * fill); break;
+    case 2: c = 5.14 + steps * (0.82 + 0.71 * rise(fill, 0.35, 0.84)); break;
+    case 3: c = 3.38 + steps * (0.717 + 0.407 * rise(fill, 0.654, 2.19)); break;
+    case 4: c = 4.04 + steps * (0.588 + 0.36 * rise(fill, 0.16, 1.05)); break;
+    case 6: c = 2.59 + more * 0.6 + steps * std::max(0.277 + 0.05 * rise(fill, 0.5, 1), 0.306 * fill); break;
+    case 7: c = 2.84 + more * 0.7 + steps * std::max(0.322 + 0.138 * rise(fill, 0.5, 1), 0.378 * fill); break;
   }
   if (pl.splits > 1) c += 3.0 + (pl.splits + 0.5) * (double)M * (double)N * 4.0 / 5.0e6;
   return c;
@@ -1288,7 +1287,7 @@ static GemmPlan make_plan(int64_t cus, int64_t M, int64_t N, int64_t K, bool vec
   const int64_t wgs = (int64_t)best.tiles_m * best.tiles_n * best.splits;
   if (dma && wgs <= cus * (best.cfg == 3 ? 2 : 1)) {
     const GemmPlan best_large = best;
-    double best_us = 1.05 * part_round_us(cus, best, M, N);
+    double best_us = 0.95 * part_round_us(cus, best, M, N);
     for (int cfg : {6, 7}) {
       const GemmPlan pl = plan_for(cus, cfg, M, N, K, nullptr, allow_split, best_large.splits);
       const double us = part_round_us(cus, pl, M, N);
