@@ -803,3 +803,27 @@ def test_column_sums_of_few_rows(rows, cols, pitch, dtype, dev):
     assert ((sums.double() - xs.sum(0)).abs() <= 2.0 ** -19 * xs.abs().sum(0)).all()
     assert torch.equal(masked[:, :cols], kept) and (masked[:, cols:] == 7).all() and torch.equal(msums, again)
     assert ((msums.double() - kept.double().sum(0)).abs() <= 2.0 ** -19 * kept.double().abs().sum(0)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [256, 257, 353, 512, 513, 641, 1024, 1025])
+@pytest.mark.parametrize("cols,shifts", [(64, (0, 1, 0)), (72, (1, 0, 0)), (72, (0, 0, 1)), (777, (0, 0, 0)), (1000, (0, 8, 0)), (8200, (0, 0, 0)),
+                                         (16400, (8, 8, 8)), (32776, (0, 0, 0))])
+def test_masked_sums_are_those_of_the_masked_matrix(cols, shifts, rows, dtype, dev):
+    """The bits of a mask pass followed by a sum pass, whatever the alignment of the three matrices: the sum pass sees the masked one
+    alone.  Sums of one CU per 64 columns, in sixteen parts and in two stages."""
+    from tritonformer_amd import _lib
+
+    lib, st, code = _lib.load(), _lib.stream_ptr(), _lib.dtype_code(dtype)
+    raw = [torch.randn(rows * cols + 16, device=dev).to(dtype) for _ in range(3)]
+    x, act, masked = (t[s:s + rows * cols].view(rows, cols) for t, s in zip(raw, shifts))
+    nb = lib.tf_colsum_partial_bytes(rows, cols)
+    part = torch.full((nb // 4 + 16,), 7.0, device=dev)
+    sums, again = (torch.full((cols,), float("nan"), device=dev) for _ in range(2))
+    _lib.check(lib.tf_relu_mask_colsum(st, code, 2, rows, cols, x.data_ptr(), cols, act.data_ptr(), cols, masked.data_ptr(), cols,
+                                       sums.data_ptr(), part.data_ptr(), nb))
+    _lib.check(lib.tf_colsum(st, code, 2, rows, cols, masked.data_ptr(), cols, again.data_ptr(), part.data_ptr(), nb))
+    assert torch.equal(masked, torch.where(act > 0, x, torch.zeros_like(x)))
+    assert torch.equal(sums, again) and (part[nb // 4:] == 7).all()
+    # 8 rows to a slice, 8 slices, 16 parts; or 8 slices of a row group, 8 of the groups: 64 additions deep at the most
+    assert ((sums.double() - masked.double().sum(0)).abs() <= 2.0 ** -18 * masked.double().abs().sum(0)).all()

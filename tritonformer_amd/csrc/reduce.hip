@@ -24,6 +24,15 @@ static int colsum_groups(int64_t rows, int64_t cols) {
   return (int)want;
 }
 
+// Rows whose sums may be made in parts (below) have scratch for sixteen of them, up to where the columns alone fill the chip.
+constexpr int64_t kCsFewRows = 1024;
+constexpr int kCsFewSlices = 128, kCsParts = 16;
+static int colsum_scratch_groups(int64_t rows, int64_t cols) {
+  const int groups = colsum_groups(rows, cols);
+  return rows > kCsFewRows / 4 && rows <= kCsFewRows && cols <= 32768 && groups < kCsParts ? kCsParts : groups;
+}
+static bool on_lines(const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) % 128 == 0 && ld % 64 == 0; }  // 16-bit rows
+
 // grid (col_blocks, groups).  Thread (slice, lane32) sums 8 adjacent columns
 // over rows  group_begin + slice, + 8, ...; slices are combined through LDS.
 // MASK: x is masked by act > 0 first and written to `out` on the way -- the sums take the same values in the same
@@ -111,20 +120,24 @@ __global__ __launch_bounds__(256) void colsum_final(int groups, int cols, const 
   }
 }
 
-// Few rows: both stages in one launch, a workgroup of 1024 threads per 64 columns (one line of a row), 128 rows at a time and four
-// of a thread's requested together.  Bound by the latency of its loads; the second launch cost more than the idle CUs do: both
-// stages and this one, us in a graph, fp16: 512 x 1024 4.35 -> 2.47, 960 x 768 4.57 -> 3.17, 960 x 3072 5.98 -> 4.92, 1024 x 8192
-// 7.98 -> 5.39.  Rows at odd addresses, whose pieces of 128 bytes lie in two lines, up to half as many: 1000 x 777 5.28 -> 5.65.
-constexpr int64_t kCsFewRows = 1024;
-constexpr int kCsFewCols = 64, kCsFewSlices = 128;
-template <typename T, typename TO, bool ANY, bool MASK>
-__global__ __launch_bounds__(1024) void colsum_few(int rows, int cols, const T* __restrict__ x, int64_t ldx, TO* __restrict__ sums,
-                                                   const T* __restrict__ act, int64_t lda, T* __restrict__ out, int64_t ldo) {
+// Up to 1024 rows (512 of ragged columns): 128 slices of every 128th row, eight slices to a part, sixteen parts; slices and parts are
+// added in their order by either form, so that a sum has the same bits with and without a mask.  Four rows of a thread are requested
+// together.
+// WHOLE: a workgroup of 1024 threads takes 64 columns (one line of a row), all slices, and writes the sums.  Bound by the latency of its
+// loads; the second launch cost more than the idle CUs do: both stages as they are beyond 1024 rows and this one, us in a graph, fp16: 512 x
+// 1024 4.35 -> 2.47, 960 x 768 4.57 -> 3.17, 960 x 3072 5.98 -> 4.92, 1024 x 8192 7.98 -> 5.39.
+// !WHOLE: a workgroup of 256 threads takes 256 columns and the slices of one part (blockIdx.y), which it leaves to colsum_parts: where one
+// CU has too many bytes to move, and where rows do not start on a line, which makes pieces of 128 bytes two lines each.
+template <typename T, typename TO, bool ANY, bool MASK, bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? 1024 : 256) void colsum_few(int rows, int cols, const T* __restrict__ x, int64_t ldx,
+                                                                 TO* __restrict__ sums, const T* __restrict__ act, int64_t lda,
+                                                                 T* __restrict__ out, int64_t ldo) {
   typedef Row<T, ANY> R;
-  __shared__ __align__(16) float red[kCsFewSlices][kCsFewCols + 4];
-  __shared__ float part[16][kCsFewCols];
-  const int lane8 = threadIdx.x & 7, slice = threadIdx.x >> 3;
-  const int chunk = blockIdx.x * (kCsFewCols / 8) + lane8;
+  constexpr int COLS = WHOLE ? 64 : 256, LANES = COLS / 8, PARTS = WHOLE ? kCsParts : 1, PER = kCsFewSlices / kCsParts, SLICES = PARTS * PER;
+  __shared__ __align__(16) float red[SLICES][COLS + 4];
+  __shared__ float part[PARTS][COLS];
+  const int lane8 = threadIdx.x % LANES, local = threadIdx.x / LANES, slice = (WHOLE ? 0 : blockIdx.y * PER) + local;
+  const int chunk = blockIdx.x * LANES + lane8;
   float acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
@@ -163,22 +176,38 @@ __global__ __launch_bounds__(1024) void colsum_few(int rows, int cols, const T* 
 #pragma unroll
   for (int e = 0; e < 8; e += 4) {
     const f32x4 v = {acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
-    *reinterpret_cast<f32x4*>(&red[slice][lane8 * 8 + e]) = v;
+    *reinterpret_cast<f32x4*>(&red[local][lane8 * 8 + e]) = v;
   }
   __syncthreads();
-  const int col = threadIdx.x & 63, p = threadIdx.x >> 6;
+  const int col = threadIdx.x % COLS, p = threadIdx.x / COLS, c = blockIdx.x * COLS + col;
   float s = 0.f;
 #pragma unroll
-  for (int k = 0; k < kCsFewSlices / 16; ++k) s += red[p * (kCsFewSlices / 16) + k][col];
-  part[p][col] = s;
-  __syncthreads();
-  const int c = blockIdx.x * kCsFewCols + col;
-  if (p == 0 && c < cols) {
-    s = 0.f;
+  for (int k = 0; k < PER; ++k) s += red[p * PER + k][col];
+  if constexpr (WHOLE) {
+    part[p][col] = s;
+    __syncthreads();
+    if (p == 0 && c < cols) {
+      s = 0.f;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) s += part[k][col];
-    sums[c] = (TO)s;
+      for (int k = 0; k < kCsParts; ++k) s += part[k][col];
+      sums[c] = (TO)s;
+    }
+  } else if (c < cols) {
+    sums[(int64_t)blockIdx.y * cols + c] = (TO)s;
   }
+}
+
+// The sixteen parts of colsum_few, in their order.
+template <typename TO>
+__global__ __launch_bounds__(64) void colsum_parts(int cols, const float* __restrict__ parts, TO* __restrict__ sums) {
+  const int c = blockIdx.x * 64 + threadIdx.x;
+  if (c >= cols) return;
+  float v[kCsParts], s = 0.f;
+#pragma unroll
+  for (int k = 0; k < kCsParts; ++k) v[k] = parts[(int64_t)k * cols + c];
+#pragma unroll
+  for (int k = 0; k < kCsParts; ++k) s += v[k];
+  sums[c] = (TO)s;
 }
 
 template <typename T, bool ANY>
@@ -207,20 +236,38 @@ static int colsum_launch(hipStream_t st, int64_t rows, int64_t cols, const void*
                          bool out_f32, float* partial, const void* act = nullptr, int64_t lda = 0,
                          void* masked = nullptr, int64_t ldm = 0) {
   const bool vec = row_vectorizable<T>(x, cols, ldx) && (!masked || (row_vectorizable<T>(act, cols, lda) && row_vectorizable<T>(masked, cols, ldm)));
-  if (rows <= (vec ? kCsFewRows : kCsFewRows / 2)) {
-    const dim3 few((unsigned)ceil_div(cols, kCsFewCols));
-#define COLSUM_FEW(TO, ANY, MASK)                                                                                    \
-  colsum_few<T, TO, ANY, MASK><<<few, dim3(1024), 0, st>>>((int)rows, (int)cols, (const T*)x, ldx, (TO*)out, (const T*)act, lda, \
-                                                           (T*)masked, ldm)
-#define COLSUM_FEW_MASK(TO, ANY) do { if (masked) COLSUM_FEW(TO, ANY, true); else COLSUM_FEW(TO, ANY, false); } while (0)
-    if (out_f32) { if (vec) COLSUM_FEW_MASK(float, false); else COLSUM_FEW_MASK(float, true); }
-    else { if (vec) COLSUM_FEW_MASK(T, false); else COLSUM_FEW_MASK(T, true); }
-#undef COLSUM_FEW_MASK
+  const int groups = colsum_groups(rows, cols);
+  // The order of the sums follows from the matrix that is summed alone (its alignment, for the two stages are the faster ones for long
+  // ragged columns): the masked one where there is a mask, which a call without one reads.
+  const bool few = rows <= (row_vectorizable<T>(masked ? masked : x, cols, masked ? ldm : ldx) ? kCsFewRows : kCsFewRows / 2);
+  if (few) {
+    // With a mask a row is three pieces.  us on one CU per 64 columns, apart, and in the two stages: 1024 x 3072 7.9, 5.2, 5.8; 1024 x 16384
+    // 17.3, 17.8, 20.0; 640 x 1024 5.0, 5.0, 5.4.  Rows that do not start on a line: 1024 x 7208 13.0, 9.7, 10.6; 450 x 3071 7.9, 5.5,
+    // 6.2; 400 x 777 4.9, 5.7, 6.6; 300 x 12345 6.8, 7.0, 7.3.  Without a mask: 1024 x 7208 4.7, 4.8, 5.9; 700 x 7208 3.4, 4.5, 4.9.
+    const bool lines = vec && on_lines(x, ldx) && on_lines(act, lda) && on_lines(masked, ldm);
+    const bool apart = masked && colsum_scratch_groups(rows, cols) >= kCsParts &&
+                       (lines ? rows > 640 && cols <= 8192 : rows > 256 && (rows > 352 || cols > 16384));
+    const dim3 grid((unsigned)ceil_div(cols, apart ? 256 : 64), apart ? kCsParts : 1), block(apart ? 256 : 1024);
+#define COLSUM_FEW(TO, ANY, MASK, WHOLE, RES)                                                                          \
+  colsum_few<T, TO, ANY, MASK, WHOLE><<<grid, block, 0, st>>>((int)rows, (int)cols, (const T*)x, ldx, (TO*)(RES), (const T*)act, lda, \
+                                                              (T*)masked, ldm)
+#define COLSUM_FEW_FORM(TO, WHOLE, RES)                                                                                \
+  do {                                                                                                                 \
+    if (!masked) { if (vec) COLSUM_FEW(TO, false, false, true, RES); else COLSUM_FEW(TO, true, false, true, RES); }    \
+    else { if (vec) COLSUM_FEW(TO, false, true, WHOLE, RES); else COLSUM_FEW(TO, true, true, WHOLE, RES); }            \
+  } while (0)
+    if (apart) COLSUM_FEW_FORM(float, false, partial);
+    else if (out_f32) COLSUM_FEW_FORM(float, true, out);
+    else COLSUM_FEW_FORM(T, true, out);
+#undef COLSUM_FEW_FORM
 #undef COLSUM_FEW
+    TF_CHECK_LAUNCH();
+    if (!apart) return TF_OK;
+    if (out_f32) colsum_parts<float><<<dim3(ceil_div(cols, 64)), dim3(64), 0, st>>>((int)cols, partial, (float*)out);
+    else colsum_parts<T><<<dim3(ceil_div(cols, 64)), dim3(64), 0, st>>>((int)cols, partial, (T*)out);
     TF_CHECK_LAUNCH();
     return TF_OK;
   }
-  const int groups = colsum_groups(rows, cols);
   const int rpg = (int)((rows + groups - 1) / groups);
   const dim3 grid((unsigned)ceil_div(cols, kCsColsPerBlock), (unsigned)groups), block(256);
 #define COLSUM(ANY, MASK)                                                                                       \
@@ -309,7 +356,7 @@ using namespace tfa;
 
 extern "C" int64_t tf_colsum_partial_bytes(int64_t rows, int64_t cols) {
   if (rows <= 0 || cols <= 0) return 0;
-  return (int64_t)colsum_groups(rows, cols) * cols * (int64_t)sizeof(float);
+  return (int64_t)colsum_scratch_groups(rows, cols) * cols * (int64_t)sizeof(float);
 }
 
 extern "C" int tf_colsum(void* stream, int dtype, int out_dtype, int64_t rows, int64_t cols, const void* x,
