@@ -155,3 +155,16 @@ def test_two_groups_of_waves(dims, form, dev):
         late = (rows // 64) % 4 == 3                                                  # these rows: the second group's alone
         bias[:, late] = R.alibi_mask(s, nh)[:, late].masked_fill(~own[late], float("-inf"))
     run_case(dims, torch.float16, dev, bias=bias, kernel_bias=slopes)
+
+
+@pytest.mark.parametrize("dtype,dims,form", [
+    (torch.bfloat16, (1, 2, 640, 64), "none"), (torch.bfloat16, (1, 3, 640, 32), "slopes"), (torch.bfloat16, (2, 2, 1088, 64), "dense"),
+    (torch.bfloat16, (1, 2, 1088, 32), "none"), (torch.bfloat16, (1, 2, 2048, 64), "slopes"), (torch.bfloat16, (1, 1, 2560, 64), "dense"),
+    # one to two workgroups per CU, which sequences from 2048 keys on take
+    (torch.float16, (1, 17, 2048, 64), "none"), (torch.bfloat16, (1, 18, 2048, 32), "slopes")])
+def test_two_groups_of_waves_in_either_type_and_beyond_one_workgroup_per_cu(dtype, dims, form, dev):
+    from tritonformer_amd.transformer import get_slopes
+
+    bias = None if form == "none" else R.alibi_mask(dims[2], dims[1]).to(dtype)
+    slopes = torch.tensor(get_slopes(dims[1]), dtype=torch.float16) if form == "slopes" else None
+    run_case(dims, dtype, dev, bias=bias, kernel_bias=slopes)

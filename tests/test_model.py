@@ -354,3 +354,33 @@ def test_weight_cast_cache_gives_the_same_step_and_follows_updates(dev):
         assert same(step(), plain)
     finally:
         T.set_weight_cast_cache(False)
+
+
+@pytest.mark.parametrize("vocab,d,ctx,heads,ffn,layers,bias,alibi,batch,dtype", [
+    (1000, 128, 640, 2, 512, 3, False, False, 2, torch.bfloat16),    # attention in two groups of waves, both directions
+    (50257, 192, 896, 3, 576, 2, True, True, 1, torch.float16),      # ... with slopes; a vocabulary no tile divides
+    (777, 256, 128, 4, 1024, 3, True, False, 3, torch.bfloat16),     # few tokens: small tiles, column sums in one launch
+    (512, 2048, 64, 16, 4096, 1, False, False, 2, torch.float16),    # contractions in slices
+    (1111, 64, 1024, 2, 264, 2, False, False, 4, torch.bfloat16),
+])
+def test_a_step_repeats_its_bits(vocab, d, ctx, heads, ffn, layers, bias, alibi, batch, dtype, dev):
+    """Every sum runs in a fixed order: the same step gives the same logits, loss and gradients each time, in memory that other steps
+    have left.  A difference between two runs is an error of synchronisation or lifetime, not of rounding."""
+    torch.manual_seed(9)
+    m = Transformer(TransformerConfig(vocab, d, ctx, heads, d // heads, ffn, layers, bias, alibi), device=dev, param_dtype=torch.float32)
+    with torch.no_grad():
+        m.logits_out.weight.normal_(0, 0.02)
+    ids = torch.randint(0, vocab, (batch, ctx), device=dev)
+    first = None
+    for run in range(4):
+        m.zero_grad(set_to_none=True)
+        junk = [torch.full((1 << 22,), float("nan"), device=dev) for _ in range(run)]
+        del junk
+        with torch.autocast("cuda", dtype=dtype):
+            logits, loss = m(ids, ids)
+        (loss * LOSS_SCALE).backward()
+        now = [logits.detach(), loss.detach()] + [p.grad for p in m.parameters()]
+        if first is None:
+            first = now
+        for i, (a, b) in enumerate(zip(first, now)):
+            assert torch.equal(a, b), (run, i)
