@@ -131,6 +131,10 @@ int tf_gemm_relu_bits(void* stream, int dtype, int out_dtype, int layout_a, int 
                       const void* A, int64_t lda, const void* B, int64_t ldb,
                       void* C, int64_t ldc, const void* bias,
                       void* bits_out, const void* bits_in, int64_t ld_bits);
+/* tf_gemm_relu_bits with bits_out, but no bits are written: the same launches and the same bits of C, for passes of which nothing is
+ * kept; the status of that call. */
+int tf_gemm_relu(void* stream, int dtype, int layout_a, int layout_b, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
+                 const void* B, int64_t ldb, void* C, int64_t ldc, const void* bias);
 /* C (M, count * each) = A (M, K; K contiguous) . [B[0] | ... | B[count - 1]], up to three matrices (K, each) of leading dimension
  * ldb (`B`: HOST array of device pointers) as one product: the three projections of tritonformer/transformer.py:158-160 over
  * weights that lie apart, without a copy that lays them side by side.  The product that tf_gemm would make of such a copy, the

@@ -174,3 +174,27 @@ def test_projections_at_odd_addresses_are_left_to_the_nodes(odd, dev, monkeypatc
         assert answers == [None]
         monkeypatch.setattr(TM, "FUSE_LAYER", False)
         assert torch.equal(one, m(ids, None))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,biased", [(1, 64, 64, True), (128, 6144, 2048, False), (300, 1000, 512, True), (2048, 8192, 2048, True),
+                                          (1024, 37376, 128, False)])
+def test_relu_without_its_bits_gives_the_bits_of_the_one_with(M, N, K, biased, dtype, dev):
+    """The last two: whole rounds of large tiles, and columns that are cut off."""
+    lib, st, code = _lib.load(), _lib.stream_ptr(), _lib.dtype_code(dtype)
+    a, b = torch.randn(M, K, device=dev).to(dtype), (torch.randn(K, N, device=dev) / K ** 0.5).to(dtype)
+    bias = torch.randn(N, device=dev).to(dtype) if biased else None
+    ptr = bias.data_ptr() if biased else None
+    c = [torch.full((M, N), float("nan"), dtype=dtype, device=dev) for _ in range(2)]
+    bits = torch.empty(M, N // 8, dtype=torch.uint8, device=dev)
+    _lib.check(lib.tf_gemm_relu_bits(st, code, code, 0, 1, M, N, K, a.data_ptr(), K, b.data_ptr(), N, c[0].data_ptr(), N, ptr, bits.data_ptr(),
+                                     None, N // 8))
+    _lib.check(lib.tf_gemm_relu(st, code, 0, 1, M, N, K, a.data_ptr(), K, b.data_ptr(), N, c[1].data_ptr(), N, ptr))
+    assert torch.equal(*c)
+    # where the one with bits is refused, so is this one
+    for n, k in ((N, K - 8), (N - 4, K)):
+        got = [f(n, k) for f in (
+            lambda n, k: lib.tf_gemm_relu_bits(st, code, code, 0, 1, M, n, k, a.data_ptr(), K, b.data_ptr(), N, c[0].data_ptr(), N, ptr,
+                                               bits.data_ptr(), None, N // 8),
+            lambda n, k: lib.tf_gemm_relu(st, code, 0, 1, M, n, k, a.data_ptr(), K, b.data_ptr(), N, c[1].data_ptr(), N, ptr))]
+        assert got[0] == got[1] != 0

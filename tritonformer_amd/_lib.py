@@ -31,6 +31,7 @@ SIGNATURES = {
     "tf_gemm_master_bias": (_i, [_vp, _i, _i, _i, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i, _vp, _i64,
                                  _vp, _i64]),
     "tf_gemm_side_by_side": (_i, [_vp, _i, _i64, _i64, _i, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64]),
+    "tf_gemm_relu": (_i, [_vp, _i, _i, _i, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp]),
     "tf_gemm_relu_bits": (_i, [_vp, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp,
                                _i64]),
     "tf_gemm_scaled": (_i, [_vp, _i, _i, _i, _i, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64]),

@@ -1576,11 +1576,11 @@ static int gemm_entry(void* stream, int dtype, int out_dtype, int layout_a, int 
                       int64_t chunk_n, int64_t chunk_stride, const void* bias, int relu, const void* mask_act,
                       int64_t ld_mask, void* workspace, int64_t workspace_bytes, void* sign_out, const void* sign_in,
                       int64_t ld_sign, const GemmForce& force = kNoForce, const float* alpha = nullptr,
-                      bool bias_f32 = false) {
+                      bool bias_f32 = false, bool like_signs = false) {
   if (!A || !B || !C) return TF_EINVAL;
   if (bias_f32 && (reinterpret_cast<uintptr_t>(bias) & 3)) return TF_EALIGN;
   if (alpha && (reinterpret_cast<uintptr_t>(alpha) & 3)) return TF_EALIGN;
-  const bool signs = sign_out || sign_in;
+  const bool signs = sign_out || sign_in || like_signs;  // like_signs: the launches of a product with sign bits, none written
   if (signs) {
     if ((sign_out && sign_in) || mask_act || N % 8 != 0 || ld_sign < N / 8 || (chunk_n != 0 && chunk_n < N)) return TF_EINVAL;
     if (sign_out && (!relu || out_dtype != dtype)) return TF_EINVAL;
@@ -1618,11 +1618,12 @@ static int gemm_entry(void* stream, int dtype, int out_dtype, int layout_a, int 
     void* so2 = sign_out ? (char*)sign_out + n1 / 8 : nullptr;
     const void* si2 = sign_in ? (const char*)sign_in + n1 / 8 : nullptr;
     const int rc = gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, n1, K, A, lda, B, ldb, C, ldc, 0, 0, bias,
-                              relu, nullptr, 0, workspace, workspace_bytes, sign_out, sign_in, ld_sign, force, alpha, bias_f32);
+                              relu, nullptr, 0, workspace, workspace_bytes, sign_out, sign_in, ld_sign, force, alpha, bias_f32,
+                              like_signs);
     if (rc != TF_OK) return rc;
     return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, tail, K, A, lda, b2, ldb, (char*)C + n1 * osz,
                       ldc, 0, 0, bias2, relu, nullptr, 0, workspace, workspace_bytes, so2, si2, ld_sign, force, alpha,
-                      bias_f32);
+                      bias_f32, like_signs);
   }
   const GemmPlan pl = rt.plan;
   // the sign bits exist in the write-out of the direct-to-LDS kernels only
@@ -1674,6 +1675,12 @@ extern "C" int tf_gemm_relu_bits(void* stream, int dtype, int out_dtype, int lay
   if (!bits_out && !bits_in) return TF_EINVAL;
   return gemm_entry(stream, dtype, out_dtype, layout_a, layout_b, M, N, K, A, lda, B, ldb, C, ldc, 0, 0, bias,
                     bits_out ? 1 : 0, nullptr, 0, nullptr, 0, bits_out, bits_in, ld_bits);
+}
+
+extern "C" int tf_gemm_relu(void* stream, int dtype, int layout_a, int layout_b, int64_t M, int64_t N, int64_t K, const void* A,
+                            int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, const void* bias) {
+  return gemm_entry(stream, dtype, dtype, layout_a, layout_b, M, N, K, A, lda, B, ldb, C, ldc, 0, 0, bias, 1, nullptr, 0, nullptr, 0,
+                    nullptr, nullptr, N / 8, kNoForce, nullptr, false, true);
 }
 
 extern "C" int tf_gemm_master_bias(void* stream, int dtype, int layout_a, int layout_b, int64_t M, int64_t N, int64_t K,

@@ -644,25 +644,27 @@ TF_FN(attn_block_dqkv, 6) {
   return THPVariable_Wrap(dqkv);
 }
 
-// hidden (m, f) = relu(x w + bias); with `with_bits` as the product that writes its sign bits, which go to `bits`, where one serves
-// the shape.  That product splits no contraction: whoever is to give the bits of the other's results takes it too.
+// hidden (m, f) = relu(x w + bias).  `like_bits`: by the product that writes its sign bits, where one serves the shape; it splits no
+// contraction, so whoever is to give the bits of its results takes it too.  The sign bits go to `bits` unless that is null.
 bool up_projection(const Tensor& like, int64_t m, int64_t f, int64_t k, const void* x, const void* w, const Tensor* bias, void* hidden,
-                   bool with_bits, Tensor* bits) {
+                   bool like_bits, Tensor* bits) {
   int rc = TF_ESHAPE;
-  if (with_bits && f % 8 == 0) {
-    *bits = make({m, f / 8}, like, at::kByte);
+  if (like_bits && f % 8 == 0) {
+    if (bits) *bits = make({m, f / 8}, like, at::kByte);
     const int dt = code(like.scalar_type());
+    const void* b = bias ? bias->data_ptr() : nullptr;
     if (!call([&] {
-          if (bias && bias->scalar_type() == at::kFloat)
+          if (bits && bias && bias->scalar_type() == at::kFloat)
             return tf_gemm_master_bias(stream(), dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x, k, w, f, hidden, f,
                                        bias->data_ptr<float>(), 1, bits->data_ptr(), f / 8, nullptr, 0);
-          return tf_gemm_relu_bits(stream(), dt, dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x, k, w, f, hidden, f,
-                                   bias ? bias->data_ptr() : nullptr, bits->data_ptr(), nullptr, f / 8);
+          if (!bits) return tf_gemm_relu(stream(), dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x, k, w, f, hidden, f, b);
+          return tf_gemm_relu_bits(stream(), dt, dt, TF_OP_KMAJOR, TF_OP_KMINOR, m, f, k, x, k, w, f, hidden, f, b, bits->data_ptr(),
+                                   nullptr, f / 8);
         }, TF_ESHAPE, &rc))
       return false;
   }
   if (rc == TF_OK) return true;
-  *bits = Tensor();
+  if (bits) *bits = Tensor();
   return product(like, TF_OP_KMINOR, m, f, k, x, w, f, hidden, bias, 1);
 }
 
@@ -722,9 +724,9 @@ bool untraced(std::initializer_list<const Tensor*> ts) {
 
 // layer(x (B, S, d), pending | None, g1, b1, eps1, [wq, wk, wv, wo], heads, bias | None, g2, b2, eps2, w1, c1 | None, w2,
 // c2 | None) -> (x + pending + attention branch, MLP branch): a decoder layer of which nothing is kept for a backward pass,
-// weights and biases in x's dtype.  The launches of the Functions in their order, the sign bits of the first MLP product
-// included (a product without them may split its contraction: other bits), but for the copy that lays the projections' weights
-// side by side where the product reads them where they are.
+// weights and biases in x's dtype.  The launches of the Functions in their order, the first MLP product as the one that
+// writes sign bits but without them (the plain product may split its contraction: other bits), but for the copy that lays the
+// projections' weights side by side where the product reads them where they are.
 TF_FN(layer, 15) {
   const Tensor *x = dense(args.a[0]), *pending = nullptr, *bias, *ln[4] = {dense(args.a[2]), dense(args.a[3]), dense(args.a[8]), dense(args.a[9])};
   if (!x || x->dim() != 3 || !is16(*x) || !aligned(*x) || !PyList_Check(args.a[5]) || PyList_GET_SIZE(args.a[5]) != 4) Py_RETURN_NONE;
@@ -810,10 +812,10 @@ TF_FN(layer, 15) {
   Tensor stream_out = make(x->sizes(), *x);
   if (!add_norm(total, branch, stream_out, ln + 2, eps2)) return nullptr;
   total = branch = Tensor();
-  Tensor hidden = make({b, s, f}, *x), out, bits;
-  if (!up_projection(*x, m, f, d, normed.data_ptr(), w1->data_ptr(), c[0], hidden.data_ptr(), true, &bits)) return nullptr;
-  normed = bits = Tensor();
-  out = make({b, s, d}, *x);
+  Tensor hidden = make({b, s, f}, *x);
+  if (!up_projection(*x, m, f, d, normed.data_ptr(), w1->data_ptr(), c[0], hidden.data_ptr(), true, nullptr)) return nullptr;
+  normed = Tensor();
+  Tensor out = make({b, s, d}, *x);
   if (!product(*x, TF_OP_KMINOR, m, d, f, hidden.data_ptr(), w2->data_ptr(), d, out.data_ptr(), c[1])) return nullptr;
   return tuple_of({&stream_out, &out});
 }
