@@ -825,5 +825,11 @@ def test_masked_sums_are_those_of_the_masked_matrix(cols, shifts, rows, dtype, d
     _lib.check(lib.tf_colsum(st, code, 2, rows, cols, masked.data_ptr(), cols, again.data_ptr(), part.data_ptr(), nb))
     assert torch.equal(masked, torch.where(act > 0, x, torch.zeros_like(x)))
     assert torch.equal(sums, again) and (part[nb // 4:] == 7).all()
+    # less scratch, as much as the sums of row groups take: the same bits
+    least = 4 * cols * max(1, min(-(-2048 // -(-cols // 256)), -(-rows // 32)))
+    part.fill_(7.0)
+    _lib.check(lib.tf_relu_mask_colsum(st, code, 2, rows, cols, x.data_ptr(), cols, act.data_ptr(), cols, masked.data_ptr(), cols,
+                                       again.data_ptr(), part.data_ptr(), least))
+    assert torch.equal(sums, again) and (part[least // 4:] == 7).all()
     # 8 rows to a slice, 8 slices, 16 parts; or 8 slices of a row group, 8 of the groups: 64 additions deep at the most
     assert ((sums.double() - masked.double().sum(0)).abs() <= 2.0 ** -18 * masked.double().abs().sum(0)).all()

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void relu_mask_kernel(int64_t rows, int cols, 
 // `masked` non-null: the sums are those of where(act > 0, x, 0), which is written there
 template <typename T>
 static int colsum_launch(hipStream_t st, int64_t rows, int64_t cols, const void* x, int64_t ldx, void* out,
-                         bool out_f32, float* partial, const void* act = nullptr, int64_t lda = 0,
+                         bool out_f32, float* partial, int64_t partial_bytes, const void* act = nullptr, int64_t lda = 0,
                          void* masked = nullptr, int64_t ldm = 0) {
   const bool vec = row_vectorizable<T>(x, cols, ldx) && (!masked || (row_vectorizable<T>(act, cols, lda) && row_vectorizable<T>(masked, cols, ldm)));
   const int groups = colsum_groups(rows, cols);
@@ -245,7 +245,7 @@ static int colsum_launch(hipStream_t st, int64_t rows, int64_t cols, const void*
     // 17.3, 17.8, 20.0; 640 x 1024 5.0, 5.0, 5.4.  Rows that do not start on a line: 1024 x 7208 13.0, 9.7, 10.6; 450 x 3071 7.9, 5.5,
     // 6.2; 400 x 777 4.9, 5.7, 6.6; 300 x 12345 6.8, 7.0, 7.3.  Without a mask: 1024 x 7208 4.7, 4.8, 5.9; 700 x 7208 3.4, 4.5, 4.9.
     const bool lines = vec && on_lines(x, ldx) && on_lines(act, lda) && on_lines(masked, ldm);
-    const bool apart = masked && colsum_scratch_groups(rows, cols) >= kCsParts &&
+    const bool apart = masked && colsum_scratch_groups(rows, cols) >= kCsParts && partial_bytes >= kCsParts * cols * (int64_t)sizeof(float) &&
                        (lines ? rows > 640 && cols <= 8192 : rows > 256 && (rows > 352 || cols > 16384));
     const dim3 grid((unsigned)ceil_div(cols, apart ? 256 : 64), apart ? kCsParts : 1), block(apart ? 256 : 1024);
 #define COLSUM_FEW(TO, ANY, MASK, WHOLE, RES)                                                                          \
@@ -354,6 +354,9 @@ static int cast_pack_launch(hipStream_t st, int count, int64_t rows, int64_t col
 
 using namespace tfa;
 
+// what a call cannot do without; with what tf_colsum_partial_bytes answers it may take the faster form
+static int64_t colsum_least_bytes(int64_t rows, int64_t cols) { return (int64_t)colsum_groups(rows, cols) * cols * (int64_t)sizeof(float); }
+
 extern "C" int64_t tf_colsum_partial_bytes(int64_t rows, int64_t cols) {
   if (rows <= 0 || cols <= 0) return 0;
   return (int64_t)colsum_scratch_groups(rows, cols) * cols * (int64_t)sizeof(float);
@@ -365,10 +368,10 @@ extern "C" int tf_colsum(void* stream, int dtype, int out_dtype, int64_t rows, i
   if (rows <= 0 || cols <= 0 || cols > (1 << 30) || ldx < cols) return TF_EINVAL;
   if (dtype != TF_F16 && dtype != TF_BF16) return TF_EDTYPE;
   if (out_dtype != dtype && out_dtype != TF_F32) return TF_EDTYPE;
-  if (!partial || partial_bytes < tf_colsum_partial_bytes(rows, cols)) return TF_EWORKSPACE;
+  if (!partial || partial_bytes < colsum_least_bytes(rows, cols)) return TF_EWORKSPACE;
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == TF_F16) return colsum_launch<f16>(st, rows, cols, x, ldx, out, out_dtype == TF_F32, partial);
-  return colsum_launch<bf16>(st, rows, cols, x, ldx, out, out_dtype == TF_F32, partial);
+  if (dtype == TF_F16) return colsum_launch<f16>(st, rows, cols, x, ldx, out, out_dtype == TF_F32, partial, partial_bytes);
+  return colsum_launch<bf16>(st, rows, cols, x, ldx, out, out_dtype == TF_F32, partial, partial_bytes);
 }
 
 // Device address of `scratch` on the current device, looked up once per device (with that device
@@ -399,14 +402,14 @@ extern "C" int tf_colsum_noalloc(void* stream, int dtype, int out_dtype, int64_t
   if (rows <= 0 || cols <= 0 || cols > (1 << 30) || ldx < cols) return TF_EINVAL;
   if (dtype != TF_F16 && dtype != TF_BF16) return TF_EDTYPE;
   if (out_dtype != dtype && out_dtype != TF_F32) return TF_EDTYPE;
-  if (tf_colsum_partial_bytes(rows, cols) > kNoAllocScratchBytes) return TF_EWORKSPACE;  // beyond the fixed scratch
+  if (colsum_least_bytes(rows, cols) > kNoAllocScratchBytes) return TF_EWORKSPACE;  // beyond the fixed scratch
   float* partial = noalloc_scratch();
   if (!partial) return TF_ELAUNCH;
   hipStream_t st = (hipStream_t)stream;
   // every partial sum the second stage reads is written by the first stage of the same call:
   // nothing has to start at zero, whatever an earlier (larger) call left behind
-  if (dtype == TF_F16) return colsum_launch<f16>(st, rows, cols, x, ldx, out, out_dtype == TF_F32, partial);
-  return colsum_launch<bf16>(st, rows, cols, x, ldx, out, out_dtype == TF_F32, partial);
+  if (dtype == TF_F16) return colsum_launch<f16>(st, rows, cols, x, ldx, out, out_dtype == TF_F32, partial, kNoAllocScratchBytes);
+  return colsum_launch<bf16>(st, rows, cols, x, ldx, out, out_dtype == TF_F32, partial, kNoAllocScratchBytes);
 }
 
 extern "C" int tf_relu_mask(void* stream, int dtype, int64_t rows, int64_t cols, const void* grad, int64_t ldg,
@@ -427,11 +430,11 @@ extern "C" int tf_relu_mask_colsum(void* stream, int dtype, int out_dtype, int64
   if (rows <= 0 || cols <= 0 || cols > (1 << 30) || ldg < cols || lda < cols || ldm < cols) return TF_EINVAL;
   if (dtype != TF_F16 && dtype != TF_BF16) return TF_EDTYPE;
   if (out_dtype != dtype && out_dtype != TF_F32) return TF_EDTYPE;
-  if (!partial || partial_bytes < tf_colsum_partial_bytes(rows, cols)) return TF_EWORKSPACE;
+  if (!partial || partial_bytes < colsum_least_bytes(rows, cols)) return TF_EWORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == TF_F16)
-    return colsum_launch<f16>(st, rows, cols, grad, ldg, sums, out_dtype == TF_F32, partial, act, lda, masked, ldm);
-  return colsum_launch<bf16>(st, rows, cols, grad, ldg, sums, out_dtype == TF_F32, partial, act, lda, masked, ldm);
+    return colsum_launch<f16>(st, rows, cols, grad, ldg, sums, out_dtype == TF_F32, partial, partial_bytes, act, lda, masked, ldm);
+  return colsum_launch<bf16>(st, rows, cols, grad, ldg, sums, out_dtype == TF_F32, partial, partial_bytes, act, lda, masked, ldm);
 }
 
 extern "C" int tf_cast_pack(void* stream, int src_dtype, int dst_dtype, int count, int64_t rows, int64_t cols,
