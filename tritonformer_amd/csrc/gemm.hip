@@ -16,7 +16,7 @@
 // of a 256x256x64 step alone on normal fp16 data: 1.29 us with 32x32x16, 1.13 with 16x16x32 (bf16 1.20 and 1.06); equal on zeros.
 // The results are the same bits.  Products on operands from HBM, fp16, with 32x32x16 and now: 8192 x 1024 x 4096 71.2 -> 64.9 us,
 // 8192 x 4096 x 1024 73.5 -> 69.9, 4096 x 8192 x 2048 125.2 -> 115.9, 8192 x 50304 x 1024 819 -> 772; 4096 x 4096 x 8192 225 -> 204:
-// the clock rises from 1.50 to 1.71 GHz, the matrix pipes are busy for three quarters of the cycles either way.
+// the clock rises from 1.51 to 1.64 GHz and more, the matrix pipes are busy for three quarters of the cycles either way.
 //
 // Either operand may be stored with the contraction dimension contiguous
 // ("K-major": read from LDS with ds_read_b128) or strided ("K-minor": read with
